@@ -19,7 +19,9 @@
 // below); partial sums go to the caller's workspace (helix_workspace_bytes) and are added in partition order by
 // the last workgroup of a tile to finish (all partitions of a tile run on one XCD, common/helix_splitk.h) or,
 // where that is not available (K-group configurations among them), by a second kernel; same bits either way.
-// Without the workspace the problem runs unpartitioned.  The reference's FP32 template has no K partition.
+// Where that is shorter still, only the tiles beyond the whole rounds of 256 are partitioned (tail_splits below,
+// common/helix_tail.h).  Without the workspace the problem runs unpartitioned.  The reference's FP32 template has no
+// K partition.
 //
 // LDS layout: A stage is [BK][BM + 32] floats, B stage [BK][BN + 32]; a fragment read takes lanes 0-31
 // from row k and lanes 32-63 from row k+1, and the 32-float row padding puts the two half-waves on
@@ -34,6 +36,7 @@
 #include "helix_im2col.h"
 #include "helix_fastdiv.h"
 #include "helix_splitk.h"
+#include "helix_tail.h"
 
 #ifndef BM
 #define BM 128
@@ -125,6 +128,7 @@ struct Params {
     int splits;      // K partitions of this launch
     int k_per;       // K extent of one partition, a multiple of BK
     helix_splitk::Plan plan;   // how the partitions of a tile are added
+    helix_tail::Plan tail;     // the last round's partition, where that is what is partitioned
     ConvGeom g;
 };
 
@@ -153,19 +157,29 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
 
     // workgroup id -> tile number (the round-robin deal over the 8 XCDs undone: each XCD is given a compact run of
     // tile numbers) and K partition, then walk groups of tile rows
-    const helix_splitk::Unit unit = helix_splitk::unit_of_workgroup(p.plan, p.tiles_m * p.tiles_n, p.splits);
-    if (unit.idle) return;
-    const int pid = unit.tile;
-    const int group_tiles = GROUP_ROWS * p.tiles_n;
-    const int first_m = (pid / group_tiles) * GROUP_ROWS;
-    const int gsize = (p.tiles_m - first_m) < GROUP_ROWS ? (p.tiles_m - first_m) : GROUP_ROWS;
-    const int tile_m = first_m + (pid % group_tiles) % gsize;
-    const int tile_n = (pid % group_tiles) / gsize;
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    int pid, split, k_per = p.k_per, tail_tile = -1;   // tail_tile: number of this workgroup's partitioned tile, if it has one
+    if (KG == 1 && p.tail.tiles) {
+        const helix_tail::Unit unit = helix_tail::unit_of_workgroup(p.tail, p.tiles_m * p.tiles_n);
+        if (unit.idle) return;
+        pid = unit.tile;
+        split = 0;
+        if (unit.split >= 0) {
+            split = unit.split;
+            k_per = p.tail.k_per;
+            tail_tile = unit.tail_tile;
+        }
+    } else {
+        const helix_splitk::Unit unit = helix_splitk::unit_of_workgroup(p.plan, p.tiles_m * p.tiles_n, p.splits);
+        if (unit.idle) return;
+        pid = unit.tile;
+        split = unit.split;
+    }
+    const int2 tile_at = helix_tail::tile_position<GROUP_ROWS>(pid, p.tiles_m, p.tiles_n);
+    const int m0 = tile_at.x * BM, n0 = tile_at.y * BN;
 
     // K range of this workgroup
-    const int k_lo = unit.split * p.k_per;
-    const int k_hi = (k_lo + p.k_per) < p.K ? (k_lo + p.k_per) : p.K;
+    const int k_lo = split * k_per;
+    const int k_hi = (k_lo + k_per) < p.K ? (k_lo + k_per) : p.K;
 
     constexpr int NA = CONV ? AC_ITERS : A_ITERS;
     constexpr int NB = CONV ? BC_ITERS : B_ITERS;
@@ -395,6 +409,18 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
 
     // lane l holds column (l % 32); rows 8*(v/4) + 4*(l/32) + (v%4)
     const int col_l = lane & 31, row_l = (lane >> 5) * 4;
+    if (KG == 1 && tail_tile >= 0) {   // a piece of a partitioned tile: the whole partial tile, edges included
+        float* part = p.ws + ((size_t)tail_tile * p.tail.splits + split) * (BM * BN);
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    part[(wave_m * WAVE_M + i * 32 + (v / 4) * 8 + row_l + (v % 4)) * BN + wave_n * WAVE_N + j * 32 + col_l] =
+                        acc[i][j][v];
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < TM; i++) {
 #pragma unroll
@@ -404,7 +430,7 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
             for (int v = 0; v < 16; v++) {
                 const int row = m0 + wave_m * WAVE_M + i * 32 + (v / 4) * 8 + row_l + (v % 4);
                 if (row < p.M && col < p.N) {
-                    if (p.splits > 1) p.ws[((size_t)unit.split * p.M + row) * p.N + col] = acc[i][j][v];
+                    if (p.splits > 1) p.ws[((size_t)split * p.M + row) * p.N + col] = acc[i][j][v];
                     else __builtin_nontemporal_store(acc[i][j][v], &p.C[(size_t)row * p.ldc + col]);   // not read again by this launch
                 }
             }
@@ -475,7 +501,11 @@ constexpr double SPLITK_MFMA_FRACTION = 0.8, SPLITK_FP32_MFMA_FLOPS = 157.3e12, 
                  SPLITK_REDUCE_LAUNCH_S = 4e-6, SPLITK_MIN_GAIN = 0.98;
 constexpr int SPLITK_MIN_K_BALANCE = 128, SPLITK_COMPUTE_UNITS = 256;
 
-inline int split_factor(long long M, long long N, long long K) {
+constexpr double SPLITK_PER_K = 2.0 * BM * BN * SPLITK_COMPUTE_UNITS / (SPLITK_MFMA_FRACTION * SPLITK_FP32_MFMA_FLOPS),
+                 SPLITK_FIXED_S = 1e-6 + 1.5e-6 * (BM * BN) / (128.0 * 128.0);
+
+// seconds: the predicted time behind the choice (more than SPLITK_FEW_TILES tiles only)
+inline int split_factor(long long M, long long N, long long K, double* seconds = nullptr) {
     const long long tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     if (tiles <= 0) return 1;
     if (tiles <= SPLITK_FEW_TILES) {
@@ -485,8 +515,7 @@ inline int split_factor(long long M, long long N, long long K) {
         if (s > K / min_k) s = K / min_k;
         return s < 1 ? 1 : (int)s;
     }
-    const double per_k = 2.0 * BM * BN * SPLITK_COMPUTE_UNITS / (SPLITK_MFMA_FRACTION * SPLITK_FP32_MFMA_FLOPS);
-    const double fixed = 1e-6 + 1.5e-6 * (BM * BN) / (128.0 * 128.0);
+    const double per_k = SPLITK_PER_K, fixed = SPLITK_FIXED_S;
     const long long ktiles = (K + BK - 1) / BK;
     int best = 1;
     double best_t = 0.0;
@@ -500,13 +529,44 @@ inline int split_factor(long long M, long long N, long long K) {
             best = s;
         }
     }
+    if (seconds) *seconds = best_t;
     return best;
 }
 
-// Partial sums of the K partitions; a caller that passes less runs the problem unpartitioned.
-inline size_t workspace_bytes(int M, int N, int K) {
+// Pieces per tile of the last round when only that is partitioned (common/helix_tail.h), 0 where the rule above is the
+// better one or nothing is to be gained: the same expression for the rounds, with the whole rounds unpartitioned and the
+// second kernel's traffic that of the partitioned tiles alone.  Measured on the launches it takes, us unpartitioned / with the
+// last round partitioned: 25088 x 128 x 1152 in 64 x 64 tiles (784 tiles) 77 / 66, 1500 x 768 x 2304 (288) 81 / 58;
+// 4000 x 2300 x 770 in 128 x 128 (576) 147 / 121; 661 x 11008 x 1024 in 128 x 64 (1032) 163 / 140.
+// Workgroups of one or two waves are left out: two of them run side by side on a compute unit's four SIMDs, so a round is
+// not 256 of them (64 x 32 tiles: 0.99 - 1.03 of the unpartitioned time).  The predicted gain has to reach a tenth: where a
+// compute unit holds several workgroups, the last round of a plain launch is shorter than the model's (1134 tiles of 64 x
+// 128, predicted 0.93, measured 0.96; 392 tiles of 64 x 64 or 128 x 64, 0.86 - 0.9, 0.93 - 0.97).
+constexpr double TAIL_GAIN = 0.9;
+constexpr int TAIL_MIN_WAVES = 4;
+inline int tail_splits(long long M, long long N, long long K) {
+    if (KG != 1 || NWAVES < TAIL_MIN_WAVES) return 0;   // (the K-group configurations already divide K among their waves)
+    const long long tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    if (tiles <= SPLITK_COMPUTE_UNITS) return 0;
+    double unpartitioned = 0.0;
+    split_factor(M, N, K, &unpartitioned);
+    const helix_tail::Model m{SPLITK_PER_K, SPLITK_FIXED_S, SPLITK_REDUCE_LAUNCH_S, SPLITK_REDUCE_BYTES_PER_S, SPLITK_MIN_K_BALANCE};
+    return helix_tail::choose(m, tiles, BM * BN, (int)K, BK, unpartitioned, TAIL_GAIN, nullptr);
+}
+
+// Partial sums of the partitions of whole problems ...
+inline size_t partition_bytes(int M, int N, int K) {
     const int s = split_factor(M, N, K);
     return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+inline size_t tail_bytes(int M, int N, int K) {
+    return helix_tail::workspace_bytes((long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN), BM * BN, tail_splits(M, N, K));
+}
+// ... or of the last round, whichever is more (the first runs where the second's bytes are not passed); a caller that
+// passes less than either runs the problem unpartitioned.
+inline size_t workspace_bytes(int M, int N, int K) {
+    const size_t all = partition_bytes(M, N, K), tail = tail_bytes(M, N, K);
+    return all > tail ? all : tail;
 }
 
 inline void bench_layout(int M, int N, int K, size_t* ae, size_t* be, size_t* ce, int* lda, int* ldb, int* ldc) {
@@ -522,13 +582,24 @@ inline int launch(Params& p, void* ws, size_t ws_bytes, hipStream_t s) {
     if (rc) return rc;
     const long long ntiles = (long long)p.tiles_m * p.tiles_n;
     if (ntiles > 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;
+    p.ws = (float*)ws;
+    p.plan = helix_splitk::Plan{0, 0u, nullptr};
+    p.tail = helix_tail::Plan{0, 0, 0, 0};
+    const int tail = ws && ((uintptr_t)ws & 15) == 0 ? tail_splits(p.M, p.N, p.K) : 0;
+    if (tail && ws_bytes >= helix_tail::workspace_bytes(ntiles, BM * BN, tail)) {
+        p.splits = 1;
+        p.k_per = (p.K + BK - 1) / BK * BK;
+        p.tail = helix_tail::make_plan(ntiles, p.K, BK, tail);
+        hipLaunchKernelGGL(helix_sgemm_f32_kernel<CONV>, dim3(helix_tail::grid(p.tail, ntiles)), dim3(NTHREADS), LDS_BYTES, s, p);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+        return helix_tail::reduce<float, BM, BN, GROUP_ROWS>(p.tail, p.ws, p.C, p.M, p.N, p.ldc, p.tiles_m, p.tiles_n, s);
+    }
     p.splits = split_factor(p.M, p.N, p.K);
-    if (p.splits > 1 && (!ws || ((uintptr_t)ws & 3) || ws_bytes < workspace_bytes(p.M, p.N, p.K))) p.splits = 1;
+    if (p.splits > 1 && (!ws || ((uintptr_t)ws & 3) || ws_bytes < partition_bytes(p.M, p.N, p.K))) p.splits = 1;
     const int ktiles = (p.K + BK - 1) / BK;
     p.k_per = ((ktiles + p.splits - 1) / p.splits) * BK;
-    p.ws = (float*)ws;
     // partitions added inside the launch where that is available (one-dimensional grid), else by the second kernel
-    p.plan = helix_splitk::Plan{0, 0u, nullptr};
     const unsigned fused = KG == 1 ? helix_splitk::plan_launch(p.plan, ntiles, p.splits, p.M, p.N) : 0u;
     const dim3 grid = fused ? dim3(fused, 1, 1) : dim3((unsigned)ntiles, (unsigned)p.splits, 1);
     hipLaunchKernelGGL(helix_sgemm_f32_kernel<CONV>, grid, dim3(NTHREADS), LDS_BYTES, s, p);
@@ -565,19 +636,25 @@ inline int gemm(const void* A, const void* B, void* C, int M, int N, int K, int 
 // Convolutions whose channel count is not a multiple of 4 run on channel-padded copies of activations and
 // weights in the workspace, or (IC = 1, where padding would quadruple the work) through a column buffer (K x M,
 // the A layout of this template) and transposed weights (K x N) there, then through the GEMM above.
-inline size_t conv_workspace_bytes(int batch, int H, int W, int IC, int OC, int kH, int kW, int stride, int pad) {
+// `sums`: the bytes of a GEMM's partial sums, all it can use (workspace_bytes) or what it must be given
+// (partition_bytes).
+inline size_t conv_bytes(int batch, int H, int W, int IC, int OC, int kH, int kW, int stride, int pad,
+                         size_t (*sums)(int, int, int)) {
     const int OH = (H + 2 * pad - kH) / stride + 1, OW = (W + 2 * pad - kW) / stride + 1;
     const long long M = (long long)batch * OH * OW, K = (long long)kH * kW * IC;
     if (M > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
-    if (IC % 4 == 0) return workspace_bytes((int)M, OC, (int)K);
+    if (IC % 4 == 0) return sums((int)M, OC, (int)K);
     if (helix_im2col::pads_channels(batch, H, W, IC, 4, 4)) {
         const int ICp = helix_im2col::padded_channels(IC, 4);
         return helix_im2col::align256((size_t)batch * H * W * ICp * 4) +
-               helix_im2col::align256((size_t)OC * kH * kW * ICp * 4) + workspace_bytes((int)M, OC, ICp * kH * kW);
+               helix_im2col::align256((size_t)OC * kH * kW * ICp * 4) + sums((int)M, OC, ICp * kH * kW);
     }
     const long long Mp = (M + 3) / 4 * 4, Np = (OC + 3) / 4 * 4;
     return helix_im2col::align256((size_t)K * Mp * 4) + helix_im2col::align256((size_t)K * Np * 4) +
-           workspace_bytes((int)M, OC, (int)K);
+           sums((int)M, OC, (int)K);
+}
+inline size_t conv_workspace_bytes(int batch, int H, int W, int IC, int OC, int kH, int kW, int stride, int pad) {
+    return conv_bytes(batch, H, W, IC, OC, kH, kW, stride, pad, workspace_bytes);
 }
 
 inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W, int IC, int OC, int kH, int kW,
@@ -590,7 +667,7 @@ inline int conv2d_padded_channels(const void* x, const void* w, void* y, int bat
     if (taps * (ICp / 4) > 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;
     const size_t xp_bytes = helix_im2col::align256((size_t)pixels * ICp * 4);
     const size_t wp_bytes = helix_im2col::align256((size_t)taps * ICp * 4);
-    if (!ws || ws_bytes < conv_workspace_bytes(batch, H, W, IC, OC, kH, kW, stride, pad)) return HELIX_ERR_WORKSPACE;
+    if (!ws || ws_bytes < conv_bytes(batch, H, W, IC, OC, kH, kW, stride, pad, partition_bytes)) return HELIX_ERR_WORKSPACE;
     if ((uintptr_t)ws & 15) return HELIX_ERR_INVALID_VALUE;
     float* xp = (float*)ws;
     float* wp = (float*)((unsigned char*)ws + xp_bytes);
@@ -614,7 +691,7 @@ inline int conv2d_explicit(const void* x, const void* w, void* y, int batch, int
     if (M > 0x7fffffffLL - 4 || K > 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;
     const int Mp = (int)((M + 3) / 4 * 4), Np = (OC + 3) / 4 * 4;
     const size_t col_bytes = helix_im2col::align256((size_t)K * Mp * 4);
-    if (!ws || ws_bytes < conv_workspace_bytes(batch, H, W, IC, OC, kH, kW, stride, pad)) return HELIX_ERR_WORKSPACE;
+    if (!ws || ws_bytes < conv_bytes(batch, H, W, IC, OC, kH, kW, stride, pad, partition_bytes)) return HELIX_ERR_WORKSPACE;
     float* col = (float*)ws;
     float* wt = (float*)((unsigned char*)ws + col_bytes);
     const helix_im2col::Geom g = helix_im2col::make_geom(H, W, IC, OH, OW, kW, stride, pad, (int)M, (int)K);
@@ -654,4 +731,5 @@ inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W
 
 }  // namespace tpl
 
+#define HELIX_TPL_REQUIRED_BYTES tpl::partition_bytes   // the partial sums of a last round are used where they fit
 #include "helix_host.h"

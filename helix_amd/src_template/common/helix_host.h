@@ -169,6 +169,11 @@ int helix_conv2d(const void* x, const void* w, void* y, int batch, int H, int W,
 #ifndef HELIX_TPL_SCRATCH_BYTES
 #define HELIX_TPL_SCRATCH_BYTES HELIX_STATIC_SCRATCH_BYTES
 #endif
+// HELIX_TPL_REQUIRED_BYTES (likewise) names the function that says what a launch of this library must be given:
+// tpl::workspace_bytes unless part of that is optional.
+#ifndef HELIX_TPL_REQUIRED_BYTES
+#define HELIX_TPL_REQUIRED_BYTES tpl::workspace_bytes
+#endif
 static_assert(HELIX_TPL_SCRATCH_BYTES <= HELIX_STATIC_SCRATCH_BYTES, "the documented maximum bounds every library");
 static __device__ __align__(256) unsigned char scratch[HELIX_TPL_SCRATCH_BYTES];
 
@@ -201,7 +206,7 @@ extern "C" {
 int helix_gemm_static_scratch(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
                               void* stream) {
     if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0) return HELIX_ERR_INVALID_VALUE;
-    const size_t need = tpl::workspace_bytes(M, N, K);
+    const size_t need = HELIX_TPL_REQUIRED_BYTES(M, N, K);
     if (need > (size_t)HELIX_TPL_SCRATCH_BYTES) return HELIX_ERR_WORKSPACE;
     void* ws = nullptr;
     int rc = helix_host::static_scratch(&ws);

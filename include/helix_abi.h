@@ -62,7 +62,9 @@ extern "C" {
  * (scripts/Ampere_FP16/build_Ampere_FP16.py:13-27, scripts/Ampere_FP32/build_Ampere_FP32.py:18). */
 HELIX_API int helix_info(char* json, int cap);
 
-/* Bytes of device scratch `helix_gemm` needs for this shape (0 unless the template splits K).
+/* Bytes of device scratch `helix_gemm` needs for this shape (0 unless the template splits K).  The FP32 tile
+ * libraries run without it too, unpartitioned: for them it is what the launch can use, for the partial sums of
+ * K partitions or of the tiles beyond the last whole round of 256 (src_template/common/helix_tail.h).
  * Replaces: nothing -- the reference's split-K accumulates with FP16 atomics into C
  * (src_template/Ampere_FP16/gemm_splitK.cu:495-506); here partial sums go through an FP32 workspace and are
  * added in partition order, inside the launch by the last workgroup of a tile to finish or (environment
@@ -81,7 +83,9 @@ HELIX_API int helix_gemm(const void* A, const void* B, void* C, int M, int N, in
  * capture, tight serving loops, harnesses that forbid hipMalloc): the K-partition partial sums go to a
  * fixed array of HELIX_STATIC_SCRATCH_BYTES inside the library's device image, so the call allocates
  * nothing and needs no workspace argument.  Same kernels, same results as `helix_gemm` with the workspace
- * `helix_workspace_bytes` asks for.  A shape that needs more than HELIX_STATIC_SCRATCH_BYTES returns
+ * `helix_workspace_bytes` asks for (FP32 tile libraries whose last round of tiles is partitioned, see there: where
+ * its partial sums exceed the array, the sums are taken in the order of the launch without them).  A shape that
+ * needs more than HELIX_STATIC_SCRATCH_BYTES returns
  * HELIX_ERR_WORKSPACE and launches nothing; the vendor comparator libraries return HELIX_ERR_UNSUPPORTED.
  * All calls on one GPU share that GPU's array: calls that overlap on one GPU (different streams or host
  * threads) race on it; calls on one stream are ordered and safe.  The array keeps the last call's
