@@ -9,7 +9,7 @@
 // register-tiled SGEMM with macros BM, BN, BK, TM, TN, :60-93).  Here the contraction runs on
 // v_mfma_f32_32x32x2_f32: one wave64 owns a WAVE_M x WAVE_N tile made of 32x32 MFMA tiles, each MFMA
 // consuming two k values; products are accumulated in ascending k within a K partition, the order the CPU
-// path uses.
+// path uses (convolutions: in ascending groups of eight k, the pairs k, k + 4 within a group).
 //
 // Compile-time parameters: BM x BN workgroup tile, BK (K extent of one LDS stage), WAVE_M x WAVE_N, K_GROUPS
 // (waves per wave tile, each taking BK / K_GROUPS of every K tile; 1 unless the configuration is a K-group one).
@@ -23,10 +23,17 @@
 // common/helix_tail.h).  Without the workspace the problem runs unpartitioned.  The reference's FP32 template has no
 // K partition.
 //
-// LDS layout: A stage is [BK][BM + 32] floats, B stage [BK][BN + 32]; a fragment read takes lanes 0-31
+// LDS layout, GEMM: A stage is [BK][BM + 32] floats, B stage [BK][BN + 32]; a fragment read takes lanes 0-31
 // from row k and lanes 32-63 from row k+1, and the 32-float row padding puts the two half-waves on
-// different halves of the 64 banks.  In CONV mode operands arrive K-contiguous and are written
-// transposed into the same layout.
+// different halves of the 64 banks.
+// LDS layout, CONV: operands arrive K-contiguous and stay so, [BM][BK] and [BN][BK], 16-byte chunk c of row r at chunk
+// position c ^ key(r), key(r) = (r / rows_per_256B) mod chunks_per_row, which puts the 16 rows of one chunk column into 16
+// different 16-byte bank groups.  A lane reads 16 bytes, four k of its row, which are the operands of four MFMAs: it does
+// not matter which two k an MFMA contracts as long as both operands agree, and lanes 0-31 and 32-63 take chunk 2s and
+// 2s + 1.  One write and one read instruction where the transposed layout of the GEMM mode took four of each, and no
+// padding, which leaves room for more workgroups per compute unit.  Measured, us per launch of the fastest configuration,
+// transposed / K-contiguous: 3x3 at batch 32, 28x28x128 85 / 81, 56x56x64 76 / 71, 7x7x512 78 / 74; 5x5 stride 2 40x40x48
+// -> 96 at batch 16 75 / 65; 0.80 - 0.92 in the mean over 65 configurations of each layer.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -79,31 +86,28 @@ constexpr int WAVES_M = BM / WAVE_M, WAVES_N = BN / WAVE_N, WAVES_MN = WAVES_M *
               NTHREADS = 64 * NWAVES;
 constexpr int TM = WAVE_M / 32, TN = WAVE_N / 32;
 constexpr int KSTEPS = BK / 2 / KG;   // MFMA k steps (2 of K each) of one wave per K tile
-// LDS row strides in floats.  GEMM mode: +32, which puts the two half-waves of a fragment read on different bank
-// halves and keeps rows 16-byte aligned for the 128-bit tile writes.  CONV mode writes scalars, BK/4 lanes per
-// tile row along k: the extra 16 / (BK/4) floats make the rows those lanes write fall on different banks
-// (4 * stride = 64 / (BK/4) mod 64) instead of all on one; from BK = 64 on one extra float (an odd stride: 16
-// distinct banks for the 16 or 32 lanes of a row, where an even one put them all on the same bank).
-constexpr int CONV_PAD = 32 + (BK >= 64 ? 1 : BK >= 8 ? 64 / BK : 0);
-template <bool CONV> struct Lds {
-    static constexpr int LDA = BM + (CONV ? CONV_PAD : 32), LDB = BN + (CONV ? CONV_PAD : 32);
-    static constexpr int A_STAGE = BK * LDA, B_STAGE = BK * LDB;    // floats
-    static constexpr int STAGE = A_STAGE + B_STAGE;
-    static constexpr int BYTES = 2 * STAGE * 4;
-};
 constexpr int REDUCE_BYTES = (KG - 1) * BM * BN * 4;   // partial tiles of the wave groups beyond the first
-constexpr int STAGES_BYTES = Lds<true>::BYTES > Lds<false>::BYTES ? Lds<true>::BYTES : Lds<false>::BYTES;
-constexpr int LDS_BYTES = STAGES_BYTES > REDUCE_BYTES ? STAGES_BYTES : REDUCE_BYTES;
+// GEMM mode, row strides in floats: +32 puts the two half-waves of a fragment read on different bank halves and keeps
+// rows 16-byte aligned for the 128-bit tile writes
+template <bool CONV> struct Lds {
+    static constexpr int LDA = BM + 32, LDB = BN + 32;
+    static constexpr int A_STAGE = CONV ? BM * BK : BK * LDA, B_STAGE = CONV ? BN * BK : BK * LDB;    // floats
+    static constexpr int STAGE = A_STAGE + B_STAGE;
+    static constexpr int BYTES = 2 * STAGE * 4 > REDUCE_BYTES ? 2 * STAGE * 4 : REDUCE_BYTES;
+};
+constexpr int LDS_BYTES = Lds<false>::BYTES;           // the larger of the two
 // GEMM mode: tile rows are k, 16-byte chunks run along m / n
 constexpr int A_CPR = BM / 4, B_CPR = BN / 4;                // chunks per tile row
 constexpr int A_ITERS = BK * A_CPR / NTHREADS, B_ITERS = BK * B_CPR / NTHREADS;
 // CONV mode: tile rows are m / n, 16-byte chunks run along k
 constexpr int K_CPR = BK / 4;
+constexpr int CONV_RP = BK >= 64 ? 1 : 64 / BK;              // tile rows per 256 bytes of LDS
 constexpr int AC_ITERS = BM * K_CPR / NTHREADS, BC_ITERS = BN * K_CPR / NTHREADS;
 
 static_assert(BM % WAVE_M == 0 && BN % WAVE_N == 0, "block tile must be a multiple of the wave tile");
 static_assert(WAVE_M % 32 == 0 && WAVE_N % 32 == 0, "wave tile is built from 32x32 MFMA tiles");
-static_assert(BK % 4 == 0 && BK >= 4, "BK must be a multiple of 4");
+static_assert(BK % 8 == 0 && (BK & (BK - 1)) == 0, "BK must be a power of two, at least 8");
+static_assert((BK / KG) % 8 == 0, "a wave group's share of a K tile is whole pairs of 16-byte chunks");
 static_assert(KG >= 1 && (BK / 2) % KG == 0, "the k steps of a K tile must divide among the wave groups");
 static_assert(NTHREADS <= 1024, "too many waves");
 static_assert((BK * A_CPR) % NTHREADS == 0 && (BK * B_CPR) % NTHREADS == 0, "tile copy must divide evenly");
@@ -139,6 +143,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, un
 __device__ __forceinline__ floatx4 buf_load16(__amdgpu_buffer_rsrc_t r, int voff) {
     return __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
 }
+
+__device__ __forceinline__ int conv_key(int row) { return (row / CONV_RP) & (K_CPR - 1); }
 
 constexpr int OOB = 0x7fffffff;  // byte offset beyond any buffer: the load returns zeros
 
@@ -281,18 +287,16 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
                 *(floatx4*)(sb + (c / B_CPR) * LDB_S + (c % B_CPR) * 4) = stage_b[SET][i];
             }
         } else {
-            const int kc = (tid % K_CPR) * 4;
+            const int kc = tid % K_CPR;
 #pragma unroll
             for (int i = 0; i < NA; i++) {
                 const int m = (tid + i * NTHREADS) / K_CPR;
-#pragma unroll
-                for (int e = 0; e < 4; e++) sa[(kc + e) * LDA_S + m] = stage_a[SET][i][e];
+                *(floatx4*)(sa + m * BK + (kc ^ conv_key(m)) * 4) = stage_a[SET][i];
             }
 #pragma unroll
             for (int i = 0; i < NB; i++) {
                 const int n = (tid + i * NTHREADS) / K_CPR;
-#pragma unroll
-                for (int e = 0; e < 4; e++) sb[(kc + e) * LDB_S + n] = stage_b[SET][i][e];
+                *(floatx4*)(sb + n * BK + (kc ^ conv_key(n)) * 4) = stage_b[SET][i];
             }
         }
     };
@@ -309,6 +313,10 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
     const int frow = lane & 31, fk = lane >> 5;
     const int a_rd = (wave_kg * (BK / KG) + fk) * LDA_S + wave_m * WAVE_M + frow;
     const int b_rd = A_STAGE + (wave_kg * (BK / KG) + fk) * LDB_S + wave_n * WAVE_N + frow;
+
+    // CONV: row of the lane's fragments and, wave groups included, its first chunk; rows 32 apart have the same key
+    const int conv_a = (wave_m * WAVE_M + frow) * BK, conv_b = A_STAGE + (wave_n * WAVE_N + frow) * BK;
+    const int conv_chunk = wave_kg * (K_CPR / KG) + fk, conv_swz = conv_key(frow);
 
     const int ktiles = (k_hi - k_lo + BK - 1) / BK;
     constexpr std::integral_constant<int, 0> set0{};
@@ -342,6 +350,24 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
         }
 
         const float* sb = smem + SET * STAGE;
+        if constexpr (CONV) {
+#pragma unroll
+            for (int s = 0; s < KSTEPS / 4; s++) {
+                const int at = ((conv_chunk + 2 * s) ^ conv_swz) * 4;
+                floatx4 af[TM], bf[TN];
+#pragma unroll
+                for (int i = 0; i < TM; i++) af[i] = *(const floatx4*)(sb + conv_a + i * 32 * BK + at);
+#pragma unroll
+                for (int j = 0; j < TN; j++) bf[j] = *(const floatx4*)(sb + conv_b + j * 32 * BK + at);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+#pragma unroll
+                        for (int j = 0; j < TN; j++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][e], bf[j][e], acc[i][j], 0, 0, 0);
+            }
+        } else
 #pragma unroll
         for (int s = 0; s < KSTEPS; s++) {
             float af[TM], bf[TN];
@@ -439,7 +465,7 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
     if (KG == 1 && p.splits > 1 && p.plan.fused) {           // else helix_sgemm_splitk_reduce_kernel adds the partials
         // loads in flight while adding: what the main loop's registers already allow (32 where LDS keeps the kernel to
         // two waves per SIMD, 16 from 64 accumulator registers per lane on, else 8)
-        constexpr bool ROOMY = ((160 * 1024) / LDS_BYTES) * NWAVES <= 8;
+        constexpr bool ROOMY = ((160 * 1024) / Lds<CONV>::BYTES) * NWAVES <= 8;
         constexpr int LOADS = ROOMY ? 32 : (TM * TN * 16 >= 64 ? 16 : 8);
         helix_splitk::sum_partitions_if_last<float, BM, BN, NTHREADS, 8, LOADS>(
             p.plan, p.ws, p.C, p.M, p.N, p.ldc, p.splits, pid, m0, n0, tid, (unsigned char*)smem);
@@ -578,7 +604,7 @@ inline void bench_layout(int M, int N, int K, size_t* ae, size_t* be, size_t* ce
 template <bool CONV>
 inline int launch(Params& p, void* ws, size_t ws_bytes, hipStream_t s) {
     static int rc = (int)hipFuncSetAttribute((const void*)helix_sgemm_f32_kernel<CONV>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, Lds<CONV>::BYTES);
     if (rc) return rc;
     const long long ntiles = (long long)p.tiles_m * p.tiles_n;
     if (ntiles > 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;
@@ -590,7 +616,7 @@ inline int launch(Params& p, void* ws, size_t ws_bytes, hipStream_t s) {
         p.splits = 1;
         p.k_per = (p.K + BK - 1) / BK * BK;
         p.tail = helix_tail::make_plan(ntiles, p.K, BK, tail);
-        hipLaunchKernelGGL(helix_sgemm_f32_kernel<CONV>, dim3(helix_tail::grid(p.tail, ntiles)), dim3(NTHREADS), LDS_BYTES, s, p);
+        hipLaunchKernelGGL(helix_sgemm_f32_kernel<CONV>, dim3(helix_tail::grid(p.tail, ntiles)), dim3(NTHREADS), Lds<CONV>::BYTES, s, p);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
         return helix_tail::reduce<float, BM, BN, GROUP_ROWS>(p.tail, p.ws, p.C, p.M, p.N, p.ldc, p.tiles_m, p.tiles_n, s);
@@ -602,7 +628,7 @@ inline int launch(Params& p, void* ws, size_t ws_bytes, hipStream_t s) {
     // partitions added inside the launch where that is available (one-dimensional grid), else by the second kernel
     const unsigned fused = KG == 1 ? helix_splitk::plan_launch(p.plan, ntiles, p.splits, p.M, p.N) : 0u;
     const dim3 grid = fused ? dim3(fused, 1, 1) : dim3((unsigned)ntiles, (unsigned)p.splits, 1);
-    hipLaunchKernelGGL(helix_sgemm_f32_kernel<CONV>, grid, dim3(NTHREADS), LDS_BYTES, s, p);
+    hipLaunchKernelGGL(helix_sgemm_f32_kernel<CONV>, grid, dim3(NTHREADS), Lds<CONV>::BYTES, s, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     if (p.splits > 1 && !fused) {
