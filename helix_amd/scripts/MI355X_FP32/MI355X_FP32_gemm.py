@@ -39,7 +39,7 @@ SPLITK_MFMA_FRACTION, SPLITK_REDUCE_BYTES_PER_S, SPLITK_MIN_GAIN, SPLITK_MIN_K_B
 SPLITK_REDUCE_LAUNCH_S = 4e-6   # the reduction kernel of a K-partitioned launch
 
 
-TAIL_GAIN, TAIL_MAX_SPLITS, TAIL_MIN_WAVES = 0.9, 8, 4
+TAIL_GAIN, TAIL_MAX_SPLITS, TAIL_MIN_WAVES, TAIL_MAX_TILE = 0.9, 8, 4, 128 * 128
 
 
 def _split_factor(k, M, N, K):
@@ -75,7 +75,7 @@ def _round_model(BM, BN):
 def tail_splits(k, M, N, K):
     """Pieces per tile when the SGEMM libraries partition only the tiles beyond the whole rounds of 256 (same rule, same
     arithmetic as their host side, src_template/common/helix_tail.h); 0 when they do not."""
-    if k[2] == 0 or k[6] != 1 or (k[0] // k[3]) * (k[1] // k[4]) < TAIL_MIN_WAVES:
+    if k[2] == 0 or k[6] != 1 or (k[0] // k[3]) * (k[1] // k[4]) < TAIL_MIN_WAVES or k[0] * k[1] > TAIL_MAX_TILE:
         return 0
     BM, BN, BK = k[0], k[1], k[2]
     tiles = math.ceil(M / BM) * math.ceil(N / BN)

@@ -104,6 +104,11 @@ constexpr int K_CPR = BK / 4;
 constexpr int CONV_RP = BK >= 64 ? 1 : 64 / BK;              // tile rows per 256 bytes of LDS
 constexpr int AC_ITERS = BM * K_CPR / NTHREADS, BC_ITERS = BN * K_CPR / NTHREADS;
 
+// the last round may be partitioned (tail_splits below): not in K-group configurations, which divide K among their waves
+// already, nor with one or two waves, nor in tiles whose main loop leaves the second way out of the kernel no registers
+// (256 x 256: it spilled, 2048^3 15 % slower)
+constexpr bool TAIL = KG == 1 && NWAVES >= 4 && BM * BN <= 128 * 128;
+
 static_assert(BM % WAVE_M == 0 && BN % WAVE_N == 0, "block tile must be a multiple of the wave tile");
 static_assert(WAVE_M % 32 == 0 && WAVE_N % 32 == 0, "wave tile is built from 32x32 MFMA tiles");
 static_assert(BK % 8 == 0 && (BK & (BK - 1)) == 0, "BK must be a power of two, at least 8");
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
     // workgroup id -> tile number (the round-robin deal over the 8 XCDs undone: each XCD is given a compact run of
     // tile numbers) and K partition, then walk groups of tile rows
     int pid, split, k_per = p.k_per, tail_tile = -1;   // tail_tile: number of this workgroup's partitioned tile, if it has one
-    if (KG == 1 && p.tail.tiles) {
+    if (TAIL && p.tail.tiles) {
         const helix_tail::Unit unit = helix_tail::unit_of_workgroup(p.tail, p.tiles_m * p.tiles_n);
         if (unit.idle) return;
         pid = unit.tile;
@@ -442,7 +447,7 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
 
     // lane l holds column (l % 32); rows 8*(v/4) + 4*(l/32) + (v%4)
     const int col_l = lane & 31, row_l = (lane >> 5) * 4;
-    if (KG == 1 && tail_tile >= 0) {   // a piece of a partitioned tile: the whole partial tile, edges included
+    if (TAIL && tail_tile >= 0) {   // a piece of a partitioned tile: the whole partial tile, edges included
         float* part = p.ws + ((size_t)tail_tile * p.tail.splits + split) * (BM * BN);
 #pragma unroll
         for (int i = 0; i < TM; i++)
@@ -576,9 +581,8 @@ inline int split_factor(long long M, long long N, long long K, double* seconds =
 // compute unit holds several workgroups, the last round of a plain launch is shorter than the model's (1134 tiles of 64 x
 // 128, predicted 0.93, measured 0.96; 392 tiles of 64 x 64 or 128 x 64, 0.86 - 0.9, 0.93 - 0.97).
 constexpr double TAIL_GAIN = 0.9;
-constexpr int TAIL_MIN_WAVES = 4;
 inline int tail_splits(long long M, long long N, long long K) {
-    if (KG != 1 || NWAVES < TAIL_MIN_WAVES) return 0;   // (the K-group configurations already divide K among their waves)
+    if (!TAIL) return 0;
     const long long tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     if (tiles <= SPLITK_COMPUTE_UNITS) return 0;
     double unpartitioned = 0.0;
