@@ -103,6 +103,9 @@ constexpr int A_ITERS = BK * A_CPR / NTHREADS, B_ITERS = BK * B_CPR / NTHREADS;
 constexpr int K_CPR = BK / 4;
 constexpr int CONV_RP = BK >= 64 ? 1 : 64 / BK;              // tile rows per 256 bytes of LDS
 constexpr int AC_ITERS = BM * K_CPR / NTHREADS, BC_ITERS = BN * K_CPR / NTHREADS;
+constexpr int SLOT_ROWS = NTHREADS / K_CPR;                  // tile rows between two copy slots of a lane
+constexpr int KEY_PERIOD = CONV_RP * K_CPR;                  // tile rows after which the swizzle key (conv_key) repeats
+constexpr int KEY_SLOTS = KEY_PERIOD > SLOT_ROWS ? KEY_PERIOD / SLOT_ROWS : 1;   // ... in copy slots
 
 // the last round may be partitioned (tail_splits below): not in K-group configurations, which divide K among their waves
 // already, nor with one or two waves, nor in tiles whose main loop leaves the second way out of the kernel no registers
@@ -114,6 +117,8 @@ static_assert(WAVE_M % 32 == 0 && WAVE_N % 32 == 0, "wave tile is built from 32x
 static_assert(BK % 8 == 0 && (BK & (BK - 1)) == 0, "BK must be a power of two, at least 8");
 static_assert((BK / KG) % 8 == 0, "a wave group's share of a K tile is whole pairs of 16-byte chunks");
 static_assert(KG >= 1 && (BK / 2) % KG == 0, "the k steps of a K tile must divide among the wave groups");
+static_assert(NTHREADS % K_CPR == 0 && (KEY_SLOTS * SLOT_ROWS) % KEY_PERIOD == 0, "copy slots must step through the key evenly");
+static_assert(32 % KEY_PERIOD == 0, "rows 32 apart, the fragments of a wave tile, must share their key");
 static_assert(NTHREADS <= 1024, "too many waves");
 static_assert((BK * A_CPR) % NTHREADS == 0 && (BK * B_CPR) % NTHREADS == 0, "tile copy must divide evenly");
 static_assert((BM * K_CPR) % NTHREADS == 0 && (BN * K_CPR) % NTHREADS == 0, "conv tile copy must divide evenly");
@@ -228,7 +233,10 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
         for (int i = 0; i < NB; i++) row_b[i] = (((tid + i * NTHREADS) / K_CPR) * p.K + (tid % K_CPR) * 4) * 4;
     }
     // (no multiplication per copy slot: a row's and a weight row's part is kept in a register, the tap's part is one sum
-    // per tile -- 28x28x128 3x3 at batch 32 71.2 -> 68.5 us, seven layers 1 - 5 % with their fastest configurations)
+    // per tile -- 28x28x128 3x3 at batch 32 71.2 -> 68.5 us, seven layers 1 - 5 % with their fastest configurations.  Weight
+    // rows as a scalar beside one register: level, 1 - 3 % slower with K groups; only in the 128 x 128 wave tiles whose
+    // accumulators and staging leave fewer than 128 of 512 registers, which spill 200 - 260 bytes per lane less with it)
+    constexpr bool ONE_ROW_B = CONV && TM * TN * 16 + 2 * 4 * (AC_ITERS + BC_ITERS) > 384;
     auto conv_offsets = [&](int k0) {
         const int k = k0 + (tid % K_CPR) * 4;
         const bool dead = k >= k_hi;
@@ -248,7 +256,7 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
         }
 #pragma unroll
         for (int i = 0; i < NB; i++) {
-            const int off = row_b[i] + k0 * 4;
+            const int off = ONE_ROW_B ? row_b[0] + (k0 + i * SLOT_ROWS * p.K) * 4 : row_b[i] + k0 * 4;
             off_b[i] = dead ? OOB : off;
         }
     };
@@ -283,6 +291,21 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
         }
     };
 
+    // What LDS addresses are derived from, in tiles that have no registers to keep the addresses over the loop (accumulators
+    // and staging take 192 of the 256 that two waves per SIMD leave each): opaque to the compiler, so that it derives them
+    // again where they are used.  256 x 256 x 32 with eight waves spilled 9 - 42 registers otherwise: 3x3 56x56x256 at batch 8
+    // 411 -> 358 us, 7x7x512 at batch 32 189 -> 180; the same in the tiles that do not spill costs 3 - 8 %
+    constexpr bool SHORT_OF_REGISTERS = CONV && NWAVES > 4 && TM * TN * 16 + 2 * 4 * (AC_ITERS + BC_ITERS) >= 192;
+    auto in_loop = [&](int v) {
+        if (SHORT_OF_REGISTERS) asm volatile("" : "+v"(v));
+        return v;
+    };
+    // LDS place of a lane's copy slot: slots whose rows are a period of the key apart differ by a constant, so that one
+    // register holds the address of all of them (or two or four, where a workgroup copies less than a period at a time)
+    auto conv_slot = [&](int i) {
+        const int t = in_loop(tid), row = t / K_CPR + i % KEY_SLOTS * SLOT_ROWS;
+        return row * BK + ((t % K_CPR) ^ conv_key(row)) * 4 + i / KEY_SLOTS * KEY_SLOTS * SLOT_ROWS * BK;
+    };
     auto store_lds = [&](int stage, auto set_c) {
         constexpr int SET = decltype(set_c)::value;
         float* sa = smem + stage * STAGE;
@@ -299,17 +322,10 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
                 *(floatx4*)(sb + (c / B_CPR) * LDB_S + (c % B_CPR) * 4) = stage_b[SET][i];
             }
         } else {
-            const int kc = tid % K_CPR;
 #pragma unroll
-            for (int i = 0; i < NA; i++) {
-                const int m = (tid + i * NTHREADS) / K_CPR;
-                *(floatx4*)(sa + m * BK + (kc ^ conv_key(m)) * 4) = stage_a[SET][i];
-            }
+            for (int i = 0; i < NA; i++) *(floatx4*)(sa + conv_slot(i)) = stage_a[SET][i];
 #pragma unroll
-            for (int i = 0; i < NB; i++) {
-                const int n = (tid + i * NTHREADS) / K_CPR;
-                *(floatx4*)(sb + n * BK + (kc ^ conv_key(n)) * 4) = stage_b[SET][i];
-            }
+            for (int i = 0; i < NB; i++) *(floatx4*)(sb + conv_slot(i)) = stage_b[SET][i];
         }
     };
 
@@ -328,7 +344,7 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
 
     // CONV: row of the lane's fragments and, wave groups included, its first chunk; rows 32 apart have the same key
     const int conv_a = (wave_m * WAVE_M + frow) * BK, conv_b = A_STAGE + (wave_n * WAVE_N + frow) * BK;
-    const int conv_chunk = wave_kg * (K_CPR / KG) + fk, conv_swz = conv_key(frow);
+    const int conv_chunk = (wave_kg * (K_CPR / KG) + fk) ^ conv_key(frow);
 
     const int ktiles = (k_hi - k_lo + BK - 1) / BK;
     constexpr std::integral_constant<int, 0> set0{};
@@ -365,7 +381,7 @@ __global__ __launch_bounds__(NTHREADS) void helix_sgemm_f32_kernel(const Params 
         if constexpr (CONV) {
 #pragma unroll
             for (int s = 0; s < KSTEPS / 4; s++) {
-                const int at = ((conv_chunk + 2 * s) ^ conv_swz) * 4;
+                const int at = (in_loop(conv_chunk) ^ (2 * s)) * 4;   // the lane's first chunk has none of the bits of 2s
                 floatx4 af[TM], bf[TN];
 #pragma unroll
                 for (int i = 0; i < TM; i++) af[i] = *(const floatx4*)(sb + conv_a + i * 32 * BK + at);
