@@ -5,6 +5,7 @@ scripts/Ampere_FP16/build_Ampere_FP16.py:7-28) and once per measurement (`os.pop
 scripts/Ampere_FP16/profile_Ampere_FP16.py:36-38).  Here a configuration is a shared library that is
 compiled once, loaded once per process and called through ctypes.
 """
+import hashlib
 import json
 import os
 import re
@@ -258,9 +259,9 @@ def write_prof_dict(backend, prof_dict):
 # The cost model ranks configurations from two profile points each; the first few of its ranking lie within a few
 # per cent of each other in prediction and 5 - 25 % apart on the device.  The runners therefore time the first few
 # candidates the first time they meet a problem (a few dozen launches) and keep the winner in a dict file beside the
-# profile, {problem tuple: configuration key} plus one entry that names the profile by its contents; later calls under
-# the same profile, in this process or another, go straight to it; under any other profile the record starts afresh.  A
-# new profile file (write_prof_dict) discards the file.  HELIX_SELECTION=model switches this off: the cost model alone
+# profile, {problem tuple: configuration key} plus one entry that names the profile by its contents and the kernels and
+# selection rules by their sources; later calls under the same of all three, in this process or another, go straight to it;
+# under any other the record starts afresh.  A new profile file (write_prof_dict) discards the file.  HELIX_SELECTION=model switches this off: the cost model alone
 # picks, as in the reference (scripts/Ampere_FP16/Ampere_FP16_gemm.py:433-446).
 def winners_path(backend):
     return f"{root_path}/build/prof_dict/{backend}_winners.dict"
@@ -274,14 +275,33 @@ def selection_mode():
 
 
 _winners = {}
-PROFILE_TAG = ("profile",)     # the entry of a winners file that names the profile its winners were ranked and timed under
+PROFILE_TAG = ("profile",)     # the entry of a winners file that names what its winners were ranked and timed under
+_code_fingerprint = {}
+
+
+def code_fingerprint():
+    """Names the kernels and the rules that pick among them by the text of the kernel templates and of the backends' host
+    modules, read once per process: the fastest configuration of a problem may be another one after a change of either."""
+    if SRC_ROOT not in _code_fingerprint:
+        digest = hashlib.md5()
+        for top in (SRC_ROOT, _find_include_dir(), _SCRIPTS_DIR):
+            for directory, subdirectories, files in os.walk(top):
+                subdirectories.sort()
+                for name in sorted(files):
+                    if name.endswith((".hip", ".h", ".py")):
+                        path = os.path.join(directory, name)
+                        digest.update(os.path.relpath(path, top).encode() + b"\0")
+                        with open(path, "rb") as f:
+                            digest.update(hashlib.md5(f.read()).digest())
+        _code_fingerprint[SRC_ROOT] = digest.hexdigest()
+    return _code_fingerprint[SRC_ROOT]
 
 
 def profile_fingerprint(prof_dict):
-    """Names a profile by its contents: winners recorded under one profile are not handed out under another (a profile
-    of other libraries or another machine state, a hand-made dict in a test)."""
-    import hashlib
-    return hashlib.md5(repr(sorted(prof_dict.items())).encode()).hexdigest()
+    """Names a profile by its contents, together with the code it is used by: winners recorded under one profile are not
+    handed out under another (a profile of other libraries or another machine state, a hand-made dict in a test), nor
+    those of one state of the kernels and selection rules under another."""
+    return hashlib.md5((code_fingerprint() + repr(sorted(prof_dict.items()))).encode()).hexdigest()
 
 
 def read_winners(backend, prof_dict):
