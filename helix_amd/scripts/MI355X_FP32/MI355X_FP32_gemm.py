@@ -5,6 +5,7 @@ import math
 import os
 
 from utils.helix_runtime import load, tuned_config, fastest_of
+from utils.hip_ctypes import STATIC_SCRATCH_BYTES
 from utils.roofline import NUM_CU, HBM_BYTES_PER_S, gemm_bytes
 from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library
 from MI355X_FP32.profile_MI355X_FP32 import PROFILE_K, PROFILE_K_SHORT, GEMV_PROFILE_K
@@ -87,7 +88,7 @@ def tail_splits(k, M, N, K):
     whole = rounds * (ktiles * BK * per_k + fixed)
     best, best_t = 0, _split_factor(k, M, N, K)[1] * TAIL_GAIN
     s = 2
-    while s <= TAIL_MAX_SPLITS and K // s >= SPLITK_MIN_K_BALANCE:
+    while s <= TAIL_MAX_SPLITS and K // s >= SPLITK_MIN_K_BALANCE and rest * s * BM * BN * 4 <= STATIC_SCRATCH_BYTES:
         per = (ktiles + s - 1) // s
         if (ktiles + per - 1) // per == s:
             piece_rounds = (rest * s + NUM_CU - 1) // NUM_CU

@@ -595,7 +595,9 @@ inline int split_factor(long long M, long long N, long long K, double* seconds =
 // Workgroups of one or two waves are left out: two of them run side by side on a compute unit's four SIMDs, so a round is
 // not 256 of them (64 x 32 tiles: 0.99 - 1.03 of the unpartitioned time).  The predicted gain has to reach a tenth: where a
 // compute unit holds several workgroups, the last round of a plain launch is shorter than the model's (1134 tiles of 64 x
-// 128, predicted 0.93, measured 0.96; 392 tiles of 64 x 64 or 128 x 64, 0.86 - 0.9, 0.93 - 0.97).
+// 128, predicted 0.93, measured 0.96; 392 tiles of 64 x 64 or 128 x 64, 0.86 - 0.9, 0.93 - 0.97).  The partial tiles fit the
+// static scratch array, so that helix_gemm_static_scratch sums in the same order as a launch with the workspace: 256 pieces
+// of the largest tile, a whole round of them, just do; one choice in sixty over random shapes is another for it.
 constexpr double TAIL_GAIN = 0.9;
 inline int tail_splits(long long M, long long N, long long K) {
     if (!TAIL) return 0;
@@ -603,7 +605,8 @@ inline int tail_splits(long long M, long long N, long long K) {
     if (tiles <= SPLITK_COMPUTE_UNITS) return 0;
     double unpartitioned = 0.0;
     split_factor(M, N, K, &unpartitioned);
-    const helix_tail::Model m{SPLITK_PER_K, SPLITK_FIXED_S, SPLITK_REDUCE_LAUNCH_S, SPLITK_REDUCE_BYTES_PER_S, SPLITK_MIN_K_BALANCE};
+    const helix_tail::Model m{SPLITK_PER_K, SPLITK_FIXED_S, SPLITK_REDUCE_LAUNCH_S, SPLITK_REDUCE_BYTES_PER_S,
+                              SPLITK_MIN_K_BALANCE, HELIX_STATIC_SCRATCH_BYTES};
     return helix_tail::choose(m, tiles, BM * BN, (int)K, BK, unpartitioned, TAIL_GAIN, nullptr);
 }
 

@@ -93,10 +93,11 @@ __global__ __launch_bounds__(256) void helix_tail_reduce_kernel(const float* ws,
 
 // ---- host side --------------------------------------------------------------------------------------------------
 // What a template knows about its launches: seconds a round of 256 workgroups takes per column of K and besides that, the
-// shortest K range worth a workgroup, and the second kernel's cost.
+// shortest K range worth a workgroup, the second kernel's cost, and the bytes the partial tiles may take at most.
 struct Model {
     double per_k, fixed, reduce_launch, reduce_bytes_per_s;
     int min_k;
+    long long max_bytes;
 };
 
 // The pieces per tile that make a launch of `tiles` tiles of `elements` results shortest, and that launch's time in
@@ -113,6 +114,7 @@ inline int choose(const Model& m, long long tiles, int elements, int K, int bloc
     for (int s = 2; s <= MAX_SPLITS && K / s >= m.min_k; s++) {
         const int per = (ktiles + s - 1) / s;
         if ((ktiles + per - 1) / per != s) continue;          // the same pieces as a smaller s
+        if (rest * s * elements * 4 > m.max_bytes) break;
         const double piece_rounds = (double)((rest * s + COMPUTE_UNITS - 1) / COMPUTE_UNITS);
         const double t = whole + piece_rounds * ((double)(per * block_k) * m.per_k + m.fixed) + m.reduce_launch +
                          (s + 1.0) * (double)rest * elements * 4.0 / m.reduce_bytes_per_s;

@@ -83,9 +83,7 @@ HELIX_API int helix_gemm(const void* A, const void* B, void* C, int M, int N, in
  * capture, tight serving loops, harnesses that forbid hipMalloc): the K-partition partial sums go to a
  * fixed array of HELIX_STATIC_SCRATCH_BYTES inside the library's device image, so the call allocates
  * nothing and needs no workspace argument.  Same kernels, same results as `helix_gemm` with the workspace
- * `helix_workspace_bytes` asks for (FP32 tile libraries whose last round of tiles is partitioned, see there: where
- * its partial sums exceed the array, the sums are taken in the order of the launch without them).  A shape that
- * needs more than HELIX_STATIC_SCRATCH_BYTES returns
+ * `helix_workspace_bytes` asks for.  A shape that needs more than HELIX_STATIC_SCRATCH_BYTES returns
  * HELIX_ERR_WORKSPACE and launches nothing; the vendor comparator libraries return HELIX_ERR_UNSUPPORTED.
  * All calls on one GPU share that GPU's array: calls that overlap on one GPU (different streams or host
  * threads) race on it; calls on one stream are ordered and safe.  The array keeps the last call's
