@@ -50,11 +50,14 @@ constexpr int ROW_BYTES = BK * 2;
 constexpr int RP = ROW_BYTES >= 256 ? 1 : 256 / ROW_BYTES;  // rows per 256 bytes of LDS
 constexpr int A_ITERS = BM * KCH / NTHREADS, B_ITERS = BN * KCH / NTHREADS;
 constexpr int ROWS_PER_ITER = NTHREADS / KCH;
+constexpr int SWZ_PERIOD = RP * KCH;           // rows after which the swizzle key (swz_key) repeats
+constexpr int KEY_SLOTS = SWZ_PERIOD > ROWS_PER_ITER ? SWZ_PERIOD / ROWS_PER_ITER : 1;   // ... in copy slots
 constexpr int RING_BYTES = 2 * STAGE_BYTES;
 constexpr int LDS_BYTES = RING_BYTES > NWAVES * STRIP_BYTES ? RING_BYTES : NWAVES * STRIP_BYTES;
 
 static_assert(BK == 64 || BK == 128, "BLOCK_K holds an even number of 32-wide MFMA k-steps: 64 or 128");
 static_assert(NTHREADS % KCH == 0, "bad thread count");
+static_assert((KEY_SLOTS * ROWS_PER_ITER) % SWZ_PERIOD == 0, "copy slots must step through the swizzle key evenly");
 static_assert((BM * KCH) % NTHREADS == 0 && (BN * KCH) % NTHREADS == 0, "tile copy must divide evenly");
 static_assert(STAGES >= 2 && STAGES <= 4, "K_STAGES: one to three K tiles staged in registers behind the one in LDS");
 constexpr int RT = STAGES - 1;                 // K tiles in flight in staging registers
@@ -275,17 +278,31 @@ __global__ __launch_bounds__(NTHREADS) void helix_gemm_f16_kernel(const Params p
             const int kh = p.g.by_kW.div(t);
             const int kw = t - kh * p.g.kW;
             const int ih = cv_ih[i] + kh, iw = cv_iw[i] + kw;
-            // the chunk, and with it the tap, is the same for all copy slots of a lane (rows 16 apart share their swizzle
-            // key): per slot an addition and the bounds, no multiplication and no branches.  Against two multiplications
-            // and short-circuit bounds, us per launch of the fastest configuration: 28x28x96 3x3 -> 128 at batch 32 14.7 ->
-            // 12.5, 14x14x144 -> 288 at batch 8 10.3 -> 9.2, 40x40x48 5x5 stride 2 at batch 16 13.2 -> 12.2; 0.85 - 0.95
-            // in the mean over 23 configurations of nine such layers
+            // rows SWZ_PERIOD apart share their swizzle key, so a lane's copy slots have KEY_SLOTS different chunks, and with
+            // them taps, between them: one where a workgroup copies 16 rows at a time, two or four with one or two waves.  The
+            // tap is worked out once for each, per slot there is an addition and the bounds, no multiplication and no branches.
+            // Against two multiplications and short-circuit bounds, us per launch of the fastest configuration: 28x28x96 3x3 ->
+            // 128 at batch 32 14.7 -> 12.5, 14x14x144 -> 288 at batch 8 10.3 -> 9.2, 40x40x48 5x5 stride 2 at batch 16 13.2 ->
+            // 12.2; 0.85 - 0.95 in the mean over 23 configurations of nine such layers with one chunk, and over five layers
+            // 0.65 - 0.99 on the 50 configurations with two or four that do not spill
             const bool ok = !(narrow & (gch_a[i] * 8 >= width)) & ((unsigned)ih < (unsigned)p.g.H) & ((unsigned)iw < (unsigned)p.g.W);
             const int off = cv_base[i] + ((kh * p.g.W + kw) * p.g.IC + c) * 2;
             return ok ? off : OOB_OFFSET;
         }
     };
+    // MODE 1, one-wave tiles with four different chunks whose accumulators and staging take more than half of the 512
+    // registers: weight rows SWZ_PERIOD apart, which have the same chunk, are addressed from one register and a scalar, added
+    // where the load is (opaque to the compiler: it would work all of them out in front of the loop and spill them; 64 x 128 x
+    // 128 208 bytes per lane, none so; the one tile beyond 320, 128 x 96 x 128, spills a thousand either way)
+    constexpr int HELD = TM * TN * 4 + (A_ITERS + B_ITERS) * 4 * RT;
+    constexpr bool FEW_ROWS_B = MODE == 1 && KEY_SLOTS == 4 && HELD > 256 && HELD <= 320;
     auto b_offset = [&](int i, bool narrow, int width) -> int {
+        if (FEW_ROWS_B && i >= KEY_SLOTS) {
+            int first = voff_b[i % KEY_SLOTS];
+            asm volatile("" : "+v"(first));
+            const int off = first + i / KEY_SLOTS * KEY_SLOTS * ROWS_PER_ITER * p.ldb * 2;
+            return (narrow && gch_b[i % KEY_SLOTS] * 8 >= width) ? OOB_OFFSET : off;
+        }
         return (narrow && gch_b[i] * 8 >= width) ? OOB_OFFSET : voff_b[i];
     };
 
