@@ -37,7 +37,7 @@ def is_valid_config(BMt, BNt, BM, BN, BK=16, WAVE_M=64, WAVE_N=64, KG=1):
         return False
     # gfx950 resources
     threads = 64 * BMt * BNt * KG
-    if (BK // 2) % KG:                                             # whole MFMA k steps per wave group
+    if BK < 8 or BK & (BK - 1) or (BK // KG) % 8:                  # whole pairs of 16-byte chunks per wave group
         return False
     if (KG - 1) * BM * BN * 4 > LDS_LIMIT:                         # partial tiles of the groups, added through LDS
         return False
@@ -45,8 +45,11 @@ def is_valid_config(BMt, BNt, BM, BN, BK=16, WAVE_M=64, WAVE_N=64, KG=1):
         return False
     if (BM * BK // 4) % threads or (BN * BK // 4) % threads:       # conv tile copy, 16-byte chunks along K
         return False
-    conv_pad = 32 + max(64 // BK, 1)  # LDS row padding of the convolution mode, the wider of the two
-    if 2 * BK * (BM + conv_pad + BN + conv_pad) * 4 > LDS_LIMIT:
+    key_period, slot_rows = max(16, BK // 4), threads // (BK // 4)  # conv tile copy: its slots step through the swizzle key
+    if threads % (BK // 4) or max(key_period, slot_rows) % min(key_period, slot_rows) or 32 % key_period:
+        return False
+    # GEMM mode's padded rows; convolutions need less (two K-group points would fill the LDS to the last byte: never built)
+    if 2 * BK * (BM + 32 + BN + 32) * 4 >= LDS_LIMIT:
         return False
     if WAVE_M * WAVE_N // 64 > 256:
         return False
