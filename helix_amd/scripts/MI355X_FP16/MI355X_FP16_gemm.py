@@ -169,20 +169,39 @@ def run_config(k, M, N, K, warmup=10, iters=10, outer=1, copies=1):
     return avg
 
 
-# A model's layers take their weights in turn: from this many bytes on they are not in the 256 MB memory-side cache when
-# their layer is met again, and the leaders of a selection are timed that way too.  Repeating one launch makes 64-row tiles,
-# which read the weights once per 64 rows, look level with 256-row ones (661 x 11008 x 4096: 73 against 71 us, and 80
-# against 66 with three weight matrices in turn).
-COLD_WEIGHT_BYTES, COLD_COPIES = 64 << 20, 4
+# A model's layers take their weights in turn: large ones are not in the 256 MB memory-side cache when their layer is met
+# again, where a selection that repeats one launch finds them.  From COLD_WEIGHT_BYTES on the candidates are therefore timed
+# on as many copies of the weights as fill the cache (none beyond it: weights of its size are out of cache by themselves).
+# What the pick loses against the best of its twelve candidates, out of cache when timed in cache / in cache when timed out
+# of it, mean and worst: weights of 75 - 142 MB (16 problems, 8 - 8192 rows) 6.1 and 35 % (400 x 6144 x 6144) / 1.8 and
+# 6.6 % (661 x 8192 x 8192); 34 - 52 MB (7 problems) 2.7 and 7 % / 2.0 and 4 %, about even, hence the line.  FP32 problems
+# of 67 - 180 MB, bound by the matrix pipes, 2.8 and 6 % / 2.6 and 12 %: they stay timed in cache.
+COLD_WEIGHT_BYTES, CACHE_BYTES = 64 << 20, 256 << 20
+
+
+def weight_copies(N, K):
+    """Copies of the second operand a selection is timed on."""
+    weights = N * padded_k(K) * 2
+    return math.ceil(CACHE_BYTES / weights) if weights >= COLD_WEIGHT_BYTES else 1
 
 
 def verified_config(prof_dict, M, N, K, top=VERIFY_TOP):
     """The fastest of the cost model's first `top` configurations on this problem (utils.helix_runtime.fastest_of:
-    2 + 5 launches each, the leaders timed again)."""
-    copies = COLD_COPIES if N * K * 2 >= COLD_WEIGHT_BYTES else 1
-    return fastest_of(ranked_configs(prof_dict, M, N, K, top),
-                      lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters, copies=copies),
-                      f"{M}x{N}x{K}")
+    2 + 5 launches each, the leaders timed again).  Where the copies of the weights do not fit the device beside the
+    problem, one does."""
+    keys = ranked_configs(prof_dict, M, N, K, top)
+
+    def fastest(copies):
+        return fastest_of(keys, lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters, copies=copies),
+                          f"{M}x{N}x{K}")
+
+    copies = weight_copies(N, K)
+    if copies > 1:
+        try:
+            return fastest(copies)
+        except RuntimeError:
+            pass
+    return fastest(1)
 
 
 def select_config(prof_dict, M, N, K):

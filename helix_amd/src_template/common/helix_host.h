@@ -82,7 +82,10 @@ struct DeviceBuffers {
         *out = nullptr;
         if (bytes == 0) bytes = 256;
         hipError_t e = hipMalloc(out, bytes);
-        if (e != hipSuccess) return (int)e;
+        if (e != hipSuccess) {
+            (void)hipGetLastError();   // reported here: not by the next launch as well
+            return (int)e;
+        }
         ptrs.push_back(*out);
         return 0;
     }
