@@ -3,7 +3,7 @@
 //   GEMM : C[M x N] = A^T * B with A stored K x M and B stored K x N (row-major FP32), the operand
 //          convention of the reference FP32 kernel (src_template/Ampere_FP32/sgemm.cu:138,378-382).
 //   CONV : y[B,OH,OW,OC] = conv2d(x[B,H,W,IC], w[OC,kH,kW,IC]), FP32, == GEMM with M = B*OH*OW, N = OC,
-//          K = kH*kW*IC; both operands are then K-contiguous and are transposed on their way into LDS.
+//          K = kH*kW*IC; both operands are then K-contiguous and stay so in LDS.
 //
 // Role in the reference: src_template/Ampere_FP32/sgemm.cu:97-350 (`mySgemmCPAsyncTemplate`, a CUDA-core
 // register-tiled SGEMM with macros BM, BN, BK, TM, TN, :60-93).  Here the contraction runs on
@@ -20,8 +20,8 @@
 // the last workgroup of a tile to finish (all partitions of a tile run on one XCD, common/helix_splitk.h) or,
 // where that is not available (K-group configurations among them), by a second kernel; same bits either way.
 // Where that is shorter still, only the tiles beyond the whole rounds of 256 are partitioned (tail_splits below,
-// common/helix_tail.h).  Without the workspace the problem runs unpartitioned.  The reference's FP32 template has no
-// K partition.
+// common/helix_tail.h).  Without the workspace the problem runs unpartitioned (see workspace_bytes below).  The
+// reference's FP32 template has no K partition.
 //
 // LDS layout, GEMM: A stage is [BK][BM + 32] floats, B stage [BK][BN + 32]; a fragment read takes lanes 0-31
 // from row k and lanes 32-63 from row k+1, and the 32-float row padding puts the two half-waves on
@@ -607,7 +607,7 @@ inline int tail_splits(long long M, long long N, long long K) {
     split_factor(M, N, K, &unpartitioned);
     const helix_tail::Model m{SPLITK_PER_K, SPLITK_FIXED_S, SPLITK_REDUCE_LAUNCH_S, SPLITK_REDUCE_BYTES_PER_S,
                               SPLITK_MIN_K_BALANCE, HELIX_STATIC_SCRATCH_BYTES};
-    return helix_tail::choose(m, tiles, BM * BN, (int)K, BK, unpartitioned, TAIL_GAIN, nullptr);
+    return helix_tail::choose(m, tiles, BM * BN, (int)K, BK, unpartitioned, TAIL_GAIN);
 }
 
 // Partial sums of the partitions of whole problems ...
@@ -618,8 +618,8 @@ inline size_t partition_bytes(int M, int N, int K) {
 inline size_t tail_bytes(int M, int N, int K) {
     return helix_tail::workspace_bytes((long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN), BM * BN, tail_splits(M, N, K));
 }
-// ... or of the last round, whichever is more (the first runs where the second's bytes are not passed); a caller that
-// passes less than either runs the problem unpartitioned.
+// ... or of the last round, whichever is more.  A caller that passes too little for the partition of the last round gets the
+// one of the whole problem where there is one and it is passed enough for that; unpartitioned otherwise.
 inline size_t workspace_bytes(int M, int N, int K) {
     const size_t all = partition_bytes(M, N, K), tail = tail_bytes(M, N, K);
     return all > tail ? all : tail;
@@ -649,7 +649,7 @@ inline int launch(Params& p, void* ws, size_t ws_bytes, hipStream_t s) {
         hipLaunchKernelGGL(helix_sgemm_f32_kernel<CONV>, dim3(helix_tail::grid(p.tail, ntiles)), dim3(NTHREADS), Lds<CONV>::BYTES, s, p);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
-        return helix_tail::reduce<float, BM, BN, GROUP_ROWS>(p.tail, p.ws, p.C, p.M, p.N, p.ldc, p.tiles_m, p.tiles_n, s);
+        return helix_tail::reduce<BM, BN, GROUP_ROWS>(p.tail, p.ws, p.C, p.M, p.N, p.ldc, p.tiles_m, p.tiles_n, s);
     }
     p.splits = split_factor(p.M, p.N, p.K);
     if (p.splits > 1 && (!ws || ((uintptr_t)ws & 3) || ws_bytes < partition_bytes(p.M, p.N, p.K))) p.splits = 1;

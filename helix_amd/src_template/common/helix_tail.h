@@ -63,8 +63,8 @@ __device__ __forceinline__ int2 tile_position(int pid, int tiles_m, int tiles_n)
 namespace {   // internal linkage: every library carries its own copy
 
 // Adds the pieces of the partitioned tiles: thread = four consecutive columns of one tile row.
-template <typename OutT, int TILE_ROWS, int TILE_COLS, int GROUP>
-__global__ __launch_bounds__(256) void helix_tail_reduce_kernel(const float* ws, OutT* C, int M, int N, int ldc, int tiles_m,
+template <int TILE_ROWS, int TILE_COLS, int GROUP>
+__global__ __launch_bounds__(256) void helix_tail_reduce_kernel(const float* ws, float* C, int M, int N, int ldc, int tiles_m,
                                                                 int tiles_n, int first_tile, int splits) {
     constexpr int CHUNKS = TILE_ROWS * TILE_COLS / 4, PER_ROW = TILE_COLS / 4;
     const int c = (int)blockIdx.x * 256 + (int)threadIdx.x;
@@ -83,10 +83,10 @@ __global__ __launch_bounds__(256) void helix_tail_reduce_kernel(const float* ws,
         if (k < splits) {
             sum[0] += v[k][0]; sum[1] += v[k][1]; sum[2] += v[k][2]; sum[3] += v[k][3];
         }
-    OutT* dst = C + (size_t)row * ldc + col;
+    float* dst = C + (size_t)row * ldc + col;
 #pragma unroll
     for (int e = 0; e < 4; e++)
-        if (col + e < N) dst[e] = (OutT)sum[e];
+        if (col + e < N) dst[e] = sum[e];
 }
 
 }  // namespace
@@ -100,11 +100,10 @@ struct Model {
     long long max_bytes;
 };
 
-// The pieces per tile that make a launch of `tiles` tiles of `elements` results shortest, and that launch's time in
-// *seconds; 0 if the last round is not worth partitioning or would not be shorter than `unpartitioned` seconds by
-// 1 - `gain` of them.  (The host scripts' cost models evaluate the same expression.)
-inline int choose(const Model& m, long long tiles, int elements, int K, int block_k, double unpartitioned, double gain,
-                  double* seconds) {
+// The pieces per tile that make a launch of `tiles` tiles of `elements` results shortest; 0 if the last round is not worth
+// partitioning or would not be shorter than `unpartitioned` seconds by 1 - `gain` of them.  (The host scripts' cost models
+// evaluate the same expression.)
+inline int choose(const Model& m, long long tiles, int elements, int K, int block_k, double unpartitioned, double gain) {
     const long long rounds = tiles / COMPUTE_UNITS, rest = tiles % COMPUTE_UNITS;
     if (rounds < 1 || rest == 0) return 0;
     const int ktiles = (K + block_k - 1) / block_k;
@@ -123,7 +122,6 @@ inline int choose(const Model& m, long long tiles, int elements, int K, int bloc
             best = s;
         }
     }
-    if (best && seconds) *seconds = best_t;
     return best;
 }
 
@@ -143,10 +141,10 @@ inline size_t workspace_bytes(long long tiles, int elements, int splits) {
 
 inline unsigned grid(const Plan& p, long long tiles) { return (unsigned)(tiles - p.tiles + p.ids); }
 
-template <typename OutT, int TILE_ROWS, int TILE_COLS, int GROUP>
-inline int reduce(const Plan& p, const float* ws, OutT* C, int M, int N, int ldc, int tiles_m, int tiles_n, hipStream_t s) {
+template <int TILE_ROWS, int TILE_COLS, int GROUP>
+inline int reduce(const Plan& p, const float* ws, float* C, int M, int N, int ldc, int tiles_m, int tiles_n, hipStream_t s) {
     constexpr int CHUNKS = TILE_ROWS * TILE_COLS / 4;
-    hipLaunchKernelGGL((helix_tail_reduce_kernel<OutT, TILE_ROWS, TILE_COLS, GROUP>), dim3((CHUNKS + 255) / 256, p.tiles),
+    hipLaunchKernelGGL((helix_tail_reduce_kernel<TILE_ROWS, TILE_COLS, GROUP>), dim3((CHUNKS + 255) / 256, p.tiles),
                        dim3(256), 0, s, ws, C, M, N, ldc, tiles_m, tiles_n, tiles_m * tiles_n - p.tiles, p.splits);
     return (int)hipGetLastError();
 }
