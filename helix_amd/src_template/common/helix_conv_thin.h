@@ -1,5 +1,5 @@
 // FP16 convolution of thin inputs: one to four channels, the first layers of CNNs (3 -> 64, 7x7 stride 2) and of
-// speech models (1 -> 32, 5x20 stride 2).  Used by the FP16 tile libraries' helix_conv2d for such layers whatever
+// speech models (1 -> 32, 5x20 stride 2).  Used by the FP16 tile libraries' helix_conv2d for such layers, whatever
 // their tile parameters are.
 //
 // What bounds such a layer is its output (batch 32, 224 x 224 x 3 -> 64, 7x7 stride 2: 51 MB written, 9.6 MB read, 7.6
@@ -20,9 +20,9 @@
 // A pair that hangs over the end of a filter row takes its second pixel as zero, and chunks beyond the filter read a
 // zeroed slot: exactly the filter's taps contribute, whatever the neighbouring pixels hold.
 //
-// Measured, us per launch, the general path against this one: batch 32, 224 x 224 x 3 -> 64: 7x7 stride 2 62 / 22, 3x3
-// 91 / 36 (5.9 TB/s), 11x11 stride 4 -> 96 54 / 28; batch 20, 180 x 180 x 3, 5x5 53 / 20; batch 1,
-// 7x7 10.5 / 6.7, 3x3 10.0 / 6.3; 4 x 161 x 700 x 1 -> 32, 5x20 stride 2 33 / 14.  What is left of the 7x7 layer: 2.5 us of
+// Measured, us per launch (helix_bench_conv), the general path's fastest configuration against this one: batch 32, 224 x 224
+// x 3 -> 64: 7x7 stride 2 58 / 22, 3x3 88 / 36 (5.9 TB/s), 11x11 stride 4 -> 96 49 / 28; batch 20, 180 x 180 x 3, 5x5 51 / 21;
+// batch 1, 7x7 10.2 / 6.9, 3x3 10.4 / 6.5; 4 x 161 x 700 x 1 -> 32, 5x20 stride 2 33 / 14.  What is left of the 7x7 layer: 2.5 us of
 // launch, about 6 us until weights and patch are in place (all workgroups start together, so nothing overlaps it), then the
 // output at 5.7 TB/s.
 #pragma once
@@ -68,6 +68,18 @@ struct Params {
     FastDiv by_cols, by_row_blocks, by_col_blocks, by_pairs, by_units;   // by_units: units that cover one staged row
 };
 
+// Where the 24 bytes of four three-channel pixels at byte `at` of x (the unit) are loaded from: seven whole dwords from byte
+// `from` on, never beyond the last whole dword of x.  Near the end of x these start in front of the unit's first dword and are
+// moved down by `behind` of them; what then lies behind the end belongs to no pixel of the row.  Where the number of halves is
+// odd, the last one lies in no whole dword: it is read by itself, into dword `last_half` of the moved ones (7 and more: not in
+// this unit).  x holds at least 28 bytes.
+struct Window { int from, behind, last_half; };
+__host__ __device__ __forceinline__ Window window_of(int at, int x_bytes) {
+    const int whole = x_bytes & ~3, first = at & ~3, last = whole - 28;
+    const int from = first < last ? first : last;
+    return Window{from, (first - from) >> 2, (x_bytes & 2) ? (whole - first) >> 2 : 7};
+}
+
 // 16 bytes of LDS at an address that is a multiple of 8
 __device__ __forceinline__ uintx4 read16(const unsigned char* p) {
     const uintx2 lo = *(const uintx2*)p, hi = *(const uintx2*)(p + 8);
@@ -102,8 +114,7 @@ __global__ __launch_bounds__(threads_of(KS), resident_of(KS) * threads_of(KS) / 
     auto first_column = [&](int iw) -> int { return p.unit_pixels == 4 ? iw & ~3 : iw; };
     // x as whole dwords (three channels put a pixel at any even byte: the dwords around a unit are shifted into place);
     // an offset beyond the buffer reads zeros
-    const unsigned rx_bytes = (p.x_bytes + 3) & ~3u;
-    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(p.x), 0, (int)rx_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(p.x), 0, (int)p.x_bytes, 0x00020000);
     auto load_unit = [&](const Block& k, int i) -> Unit {
         Unit v{{0, 0, 0, 0}, {0, 0}};
         const int pr = p.by_units.div(i), u = i - pr * units;
@@ -111,15 +122,18 @@ __global__ __launch_bounds__(threads_of(KS), resident_of(KS) * threads_of(KS) / 
         const bool inside = (i < total_units) & ((unsigned)ih < (unsigned)p.H) & ((unsigned)iw < (unsigned)p.W);
         const int at = (((k.image * p.H + ih) * p.W + iw) * p.IC) * 2;
         if (p.unit_pixels == 4) {
-            // 28 bytes from the dword at or below the unit; near the end of x from its last 28 bytes, then moved down (what
-            // lies behind the end belongs to no pixel of the row)
-            const int last = (int)rx_bytes - 28, from = (at & ~3) < last ? (at & ~3) : last;
-            const uintx4 lo = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(rx, inside ? from : OOB, 0, 0));
-            const uintx3 hi = __builtin_bit_cast(uintx3, __builtin_amdgcn_raw_buffer_load_b96(rx, inside ? from + 16 : OOB, 0, 0));
+            const Window n = window_of(inside ? at : 0, (int)p.x_bytes);
+            const uintx4 lo = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(rx, inside ? n.from : OOB, 0, 0));
+            const uintx3 hi = __builtin_bit_cast(uintx3, __builtin_amdgcn_raw_buffer_load_b96(rx, inside ? n.from + 16 : OOB, 0, 0));
             unsigned w[7] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2]};
-            for (int behind = inside ? (at - from) >> 2 : 0; __any(behind > 0); behind--) {
+            for (int behind = n.behind; __any(behind > 0); behind--) {
 #pragma unroll
                 for (int e = 0; e < 6; e++) w[e] = behind > 0 ? w[e + 1] : w[e];
+            }
+            if (__any(inside && n.last_half < 7)) {
+                const unsigned half = __builtin_amdgcn_raw_buffer_load_b16(rx, (int)p.x_bytes - 2, 0, 0);
+#pragma unroll
+                for (int e = 1; e < 7; e++) w[e] = inside && n.last_half == e ? half : w[e];
             }
 #pragma unroll
             for (int e = 0; e < 4; e++) v.a[e] = __builtin_amdgcn_alignbyte(w[e + 1], w[e], at & 2);
