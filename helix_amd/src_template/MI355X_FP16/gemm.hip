@@ -643,11 +643,13 @@ inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W
                   int stride, int pad, void* ws, size_t ws_bytes, hipStream_t s) {
     if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 1)) return HELIX_ERR_INVALID_VALUE;
     if (IC % 8 != 0) {   // a 16-byte chunk of the implicit gather must stay inside one filter tap
-        // up to four channels: the kernel that stages the input once (1.25 - 2.8 times as fast as the copies below on every
-        // first layer of the benchmark lists); longer filters and wider rows than its LDS holds take the copies
+        // up to four channels: the kernel that stages the input once, 1.5 - 2.7 times as fast as the copies below on the first
+        // layers of the benchmark lists; longer filters and wider rows than its LDS holds take the copies
         helix_conv_thin::Plan thin;
         if ((((uintptr_t)y & 15) == 0 || OC % 8 != 0) && helix_conv_thin::make_plan(thin, batch, H, W, IC, OC, kH, kW, stride, pad)) {
+            // (what the copies refuse is refused here too)
             if (!ws || ws_bytes < conv_workspace_bytes(batch, H, W, IC, OC, kH, kW, stride, pad)) return HELIX_ERR_WORKSPACE;
+            if ((uintptr_t)ws & 15) return HELIX_ERR_INVALID_VALUE;
             return helix_conv_thin::launch(thin, x, w, y, s);
         }
         if (helix_im2col::pads_channels(batch, H, W, IC, 8, 2))
