@@ -80,6 +80,36 @@ def gather_channels(input_channel):
     return padded if 3 * padded <= 8 * input_channel else input_channel
 
 
+# What the kernel for thin inputs takes (src_template/common/helix_conv_thin.h, make_plan).
+THIN_MAX_CHANNELS, THIN_MAX_STEPS, THIN_OC_BLOCK, THIN_STEP_BYTES, THIN_LDS_BYTES = 4, 24, 64, 4096, 160 * 1024
+
+
+def runs_thin(batch, IC, H, W, OC, kH, kW, stride, pad):
+    """Whether a layer runs in the kernel for one to four channels, which is the same in every tile library (same rule,
+    same arithmetic as its host side: the layer's index range, its filter, and one output row or
+    a part of one in LDS)."""
+    OH, OW = (H + 2 * pad - kH) // stride + 1, (W + 2 * pad - kW) // stride + 1
+    pairs = (kW + 1) // 2
+    steps = (kH * pairs + 3) // 4
+    oc_blocks = -(-OC // THIN_OC_BLOCK)
+    if IC > THIN_MAX_CHANNELS or batch * H * W * IC * 2 >= 0x7ffffff0 or steps > THIN_MAX_STEPS:
+        return False
+    pixels = batch * OH * OW
+    if pixels > 0x7fffffff or oc_blocks > 65535:
+        return False
+    raw = -(-THIN_OC_BLOCK * kH * kW * IC * 2 // 16) * 16
+    packed = steps * THIN_STEP_BYTES
+    for halve in range(4 if batch * OH * oc_blocks < 512 else 1):
+        cols = OW if halve == 0 else -(-(OW >> halve) // 16) * 16
+        if halve and (cols >= OW or cols < 16):
+            break
+        patch = 16 + kH * (((cols - 1) * stride + 2 * pairs + 1) // 2 * 2) * 8
+        lds = max(patch, raw + packed) if steps <= 7 else -(-max(patch, raw) // 16) * 16 + packed
+        if lds <= THIN_LDS_BYTES and batch * OH * -(-OW // cols) <= 0x7fffffff:
+            return True
+    return False
+
+
 def conv_kernel_scratch(k, IC=None):
     """Scratch bytes per lane (register spills) of the convolution kernel configuration k runs for this channel count,
     as recorded when the library was built; 0 when the build left no record.  The gather keeps per-copy-slot state
@@ -122,9 +152,15 @@ def ranked_configs(prof_dict, M, N, K, IC=None, top=VERIFY_TOP, pointwise=False)
 
 def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP):
     """The fastest of the cost model's first `top` configurations on this layer (utils.helix_runtime.fastest_of:
-    2 + 5 launches each, the leaders timed again)."""
+    2 + 5 launches each, the leaders timed again); for a layer that runs in the kernel for thin inputs the model's first
+    one without K partitions."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     ICg = gather_channels(input_channel)
+    if runs_thin(batch, input_channel, H, W, output_channel, kH, kW, stride, pad):
+        # every library launches the same kernel: nothing to time.  A library without K partitions asks for the least
+        # workspace; the model's choice among them is what a y off 16 bytes, which takes the other path, runs on
+        ranked = ranked_configs(prof_dict, M, output_channel, ICg * kH * kW, ICg, len(prof_dict))
+        return next((k for k in ranked if k[5] == 0), ranked[0])
 
     def time_config(k, warmup, iters):
         return load(library_for_key(k)).bench_conv(batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
