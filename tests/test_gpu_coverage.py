@@ -88,7 +88,8 @@ def _int_conv_cases(rng, dtype, channel_counts):
 def test_every_fp16_library_integer_exact(keys):
     """Per configuration: two ragged GEMMs (a narrow first K tile, a split-K partition with a remainder) and five
     convolutions -- IC = 128 and 64 (a K tile inside one filter tap when IC is a multiple of BLOCK_K), IC = 8
-    (the general gather), IC = 3 (channel-padded copies in the workspace), and a 1 x 1 stride-1 layer."""
+    (the general gather), IC = 3 (the kernel for thin inputs, the same in every library; the copies in the workspace are
+    swept in test_gpu_conv_copies.py), and a 1 x 1 stride-1 layer."""
     rng = np.random.default_rng(100)
     gemms = _int_gemm_cases(rng, np.float16)
     convs = _int_conv_cases(rng, np.float16, (128, 64, 8, 3))
@@ -345,8 +346,9 @@ def test_extreme_list_members_vs_float64(profiles, shape):
 
 
 def test_extreme_conv_one_channel_wide_filter(profiles):
-    """DeepBench speech layer: one input channel, 5 x 20 filter, stride 2 -- 100 taps through the column-buffer
-    path, and the 32-channel 5 x 10 layer behind it (a K tile spanning several taps)."""
+    """DeepBench speech layer: one input channel, 5 x 20 filter, stride 2 -- 100 taps, in FP32 through the column buffer, in
+    FP16 through whichever of that and the kernel for thin inputs its size selects --, and the 32-channel 5 x 10 layer
+    behind it (a K tile spanning several taps)."""
     prof16, _ = profiles
     for (batch, IC, H, W, OC, kH, kW, stride, pad) in [(1, 1, 161, 700, 32, 5, 20, 2, 0), (2, 32, 79, 341, 32, 5, 10, 2, 0)]:
         x, w = seeded_inputs.conv_operands(batch, IC, H, W, OC, kH, kW)

@@ -382,8 +382,9 @@ def run_conv(lib, x, w, stride, pad, dtype):
 CONV_GEOMS = [(2, 14, 14, 16, 24, 3, 3, 1, 1), (2, 15, 13, 8, 8, 3, 3, 2, 1), (3, 8, 8, 32, 16, 1, 1, 2, 0),
               (1, 12, 12, 8, 40, 5, 5, 1, 2), (2, 9, 9, 64, 64, 3, 3, 1, 1), (1, 7, 7, 24, 16, 3, 3, 1, 0),
               (2, 6, 10, 72, 8, 1, 1, 1, 0)]
-# channel counts that are not a multiple of the gather chunk: channel-padded copies in the workspace (IC = 3, 6,
-# 25; 2 in FP32) or explicit im2col + GEMM through the workspace (IC = 1; 2 in FP16)
+# channel counts that are not a multiple of the gather chunk: channel-padded copies in the workspace (IC = 6, 25; 2, 3 in
+# FP32), explicit im2col + GEMM through the workspace (IC = 1 in FP32) or the kernel for thin inputs (IC = 1 ... 3 in FP16,
+# whose copies and column buffer test_gpu_conv_copies.py holds)
 CONV_GEOMS_ODD = [(2, 20, 20, 3, 16, 7, 7, 2, 3), (1, 9, 11, 1, 8, 5, 5, 2, 0), (2, 8, 8, 25, 24, 5, 5, 1, 2),
                   (1, 10, 10, 6, 10, 3, 3, 1, 1), (3, 13, 13, 3, 96, 11, 11, 4, 0), (2, 7, 9, 2, 8, 3, 3, 1, 1)]
 
@@ -419,8 +420,8 @@ def test_conv_f16_golden_and_special_cases():
     wi = rng.integers(-2, 3, (16, 3, 3, 8)).astype(np.float16)
     want = O.conv2d_nhwc(xi.astype(np.float32), wi.astype(np.float32), 2, 1)
     assert np.array_equal(run_conv(lib, xi, wi, 2, 1, torch.float16).astype(np.float32), want)
-    # IC = 3 runs on channel-padded copies, IC = 1 through the column buffer: exact on integers too, also through a
-    # split-K library, and refused without the workspace rather than mis-computed
+    # IC = 3 and 1 run in the kernel for thin inputs: exact on integers too, also through a split-K library, and refused
+    # without the workspace that the other paths need for them
     xi3 = rng.integers(-2, 3, (2, 9, 8, 3)).astype(np.float16)
     wi3 = rng.integers(-2, 3, (16, 3, 3, 3)).astype(np.float16)
     want3 = O.conv2d_nhwc(xi3.astype(np.float32), wi3.astype(np.float32), 2, 1)
@@ -512,9 +513,9 @@ def test_gemm_random_shapes_vs_oracle():
 
 
 def test_conv_random_geometries_vs_oracle():
-    """Seeded random small convolutions, channel counts 1 ... 20 (implicit gather, channel-padded copies and
-    column-buffer paths all occur), strides 1 ... 3, padding up to the filter size, rectangular images and
-    filters: FP16 and FP32 against the oracle."""
+    """Seeded random small convolutions, channel counts 1 ... 20 (implicit gather and channel-padded copies in both
+    precisions, the column buffer in FP32, the kernel for thin inputs in FP16), strides 1 ... 3, padding up to the filter
+    size, rectangular images and filters: FP16 and FP32 against the oracle."""
     rng = np.random.default_rng(33)
     lib16 = [load(b16.kernel_library("gemm", 2, 64, 64, 32, 32, 64)), load(b16.kernel_library("gemm_splitK", 2, 128, 64, 64, 32, 128))]
     lib32 = [load(b32.sgemm_library(64, 64, 16, 32, 32)), load(b32.sgemm_library(32, 64, 64, 32, 32, 4))]
@@ -539,9 +540,9 @@ def test_conv_random_geometries_vs_oracle():
 
 
 def test_conv_first_layers_full_size_sampled():
-    """The three-channel first layers of AlexNet, GoogleNet and a VGG-style stem at batch 32 and 224 x 224 (the
-    channel-padded path at its real size, corners and image borders included): sampled output pixels against
-    float64, FP16 and FP32."""
+    """The three-channel first layers of AlexNet, GoogleNet and a VGG-style stem at batch 32 and 224 x 224 (FP16: the kernel
+    for thin inputs, FP32: the channel-padded copies, at their real size, corners and image borders included): sampled
+    output pixels against float64."""
     rng = np.random.default_rng(12)
     lib16 = load(b16.kernel_library("gemm", 2, 128, 64, 32, 32, 64))
     lib32 = load(b32.sgemm_library(64, 64, 16, 32, 32))
