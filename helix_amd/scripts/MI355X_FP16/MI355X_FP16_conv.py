@@ -86,8 +86,8 @@ THIN_MAX_CHANNELS, THIN_MAX_STEPS, THIN_OC_BLOCK, THIN_STEP_BYTES, THIN_LDS_BYTE
 
 def runs_thin(batch, IC, H, W, OC, kH, kW, stride, pad):
     """Whether a layer runs in the kernel for one to four channels, which is the same in every tile library (same rule,
-    same arithmetic as its host side: the layer's index range, its filter, and one output row or
-    a part of one in LDS)."""
+    same arithmetic as its host side: the layer's index range, its filter, where that kernel is the faster one, and one output
+    row or a part of one in LDS)."""
     OH, OW = (H + 2 * pad - kH) // stride + 1, (W + 2 * pad - kW) // stride + 1
     pairs = (kW + 1) // 2
     steps = (kH * pairs + 3) // 4
@@ -96,6 +96,13 @@ def runs_thin(batch, IC, H, W, OC, kH, kW, stride, pad):
         return False
     pixels = batch * OH * OW
     if pixels > 0x7fffffff or oc_blocks > 65535:
+        return False
+    staged = ((OH - 1) * stride + kH) * ((OW - 1) * stride + kW) / (OH * OW) * oc_blocks
+    if OC > 512 and pixels * OC * 2 > 256 << 20 and not (IC == 3 and steps >= (2 if OC <= 1024 else 4)):
+        return False
+    if IC == 4 and staged > 96.0:
+        return False
+    if IC < 3 and (staged > 48.0 if steps <= 7 else staged > 24.0 or pixels * IC < 16384 or (steps > 17 and OC > 2 * THIN_OC_BLOCK)):
         return False
     raw = -(-THIN_OC_BLOCK * kH * kW * IC * 2 // 16) * 16
     packed = steps * THIN_STEP_BYTES

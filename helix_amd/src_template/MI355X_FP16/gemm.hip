@@ -644,7 +644,8 @@ inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W
     if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 1)) return HELIX_ERR_INVALID_VALUE;
     if (IC % 8 != 0) {   // a 16-byte chunk of the implicit gather must stay inside one filter tap
         // up to four channels: the kernel that stages the input once, 1.5 - 2.7 times as fast as the copies below on the first
-        // layers of the benchmark lists; longer filters and wider rows than its LDS holds take the copies
+        // layers of the benchmark lists; what it is not the faster path for (helix_conv_thin::is_faster), and longer filters and
+        // wider rows than its LDS holds, takes the copies
         helix_conv_thin::Plan thin;
         if ((((uintptr_t)y & 15) == 0 || OC % 8 != 0) && helix_conv_thin::make_plan(thin, batch, H, W, IC, OC, kH, kW, stride, pad)) {
             // (what the copies refuse is refused here too)

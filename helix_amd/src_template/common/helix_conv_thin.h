@@ -1,6 +1,6 @@
 // FP16 convolution of thin inputs: one to four channels, the first layers of CNNs (3 -> 64, 7x7 stride 2) and of
 // speech models (1 -> 32, 5x20 stride 2).  Used by the FP16 tile libraries' helix_conv2d for such layers, whatever
-// their tile parameters are.
+// their tile parameters are, where it is the faster path (is_faster below).
 //
 // What bounds such a layer is its output (batch 32, 224 x 224 x 3 -> 64, 7x7 stride 2: 51 MB written, 9.6 MB read, 7.6
 // Gflop): the general path copied the activations to eight channels and walked K = kH * kW * 8, 2.7 times the products,
@@ -388,8 +388,30 @@ struct Plan {
 
 inline size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }
 
+// Whether this kernel is the faster path for a layer that it can run.  It stages the input again for every 64 output channels:
+// in units of four pixels for three channels, pixel by pixel for the others, which is what those are bound by once each output
+// pixel has `staged` input pixels moved for it over all channel blocks.  us per launch, the fastest of fifteen configurations of
+// the general path / this kernel, 64 images of 112 x 112, stride 4:
+//   3 -> 1024 channels        3x3  43 / 28, 11x11 123 / 104
+//   4 -> 256 | 512 (staged 56 | 112)    1x1  18 / 17 | 24 / 29, 7x7 33 / 29 | 50 / 55
+//   1 -> 128 | 256 (staged 28 - 37 | 56 - 70)   3x3  12 / 10 | 15 / 14, 7x7 16 / 15 | 19 / 23
+//   1 -> 64 | 256, 11x11 (17 steps)   23 / 16 | 29 / 39; 8 images of 224 x 224, stride 2, 13x13 -> 128 | 256  47 / 32 | 54 / 60
+// Filters of more than seven steps have their weights in LDS and a longer way to the first result: of one channel, 64 x 64 at
+// batch 1 | 2 | 4 | 8, 9x9 8.4 / 8.6 | 8.5 / 8.7 | 11 / 10 | 13 / 10, 11x11 8.7 / 10.5 | 9.0 / 10.5 | 11 / 11 | 18 / 12, of two
+// the same at half as many pixels.
+// Results beyond the 256 MB memory-side cache in rows of more than 512 channels: the 128-byte pieces of a pixel that a
+// workgroup writes reach HBM at 3.9 - 5.0 TB/s, the general path's 512-byte ones faster than it loses by its copies where
+// the filter is 1x1 (4 x 256 x 256 x 3 -> 2048 216 / 277, -> 4096 391 / 516), about level for 3x3 ones from 2048 channels on.
+inline bool is_faster(long long pixels, double staged, int IC, int OC, int steps) {
+    if (OC > 512 && pixels * OC * 2 > (256LL << 20) && !(IC == 3 && steps >= (OC <= 1024 ? 2 : 4))) return false;
+    if (IC == 3) return true;
+    if (IC == 4) return staged <= 96.0;
+    if (steps <= 7) return staged <= 48.0;
+    return staged <= 24.0 && pixels * IC >= 16384 && (steps <= 17 || OC <= 2 * OC_BLOCK);
+}
+
 // The split of a layer over workgroups; false where the layer does not fit this kernel (more than four channels, filters or
-// rows beyond what LDS holds).
+// rows beyond what LDS holds) or another path is the faster one.
 inline bool make_plan(Plan& plan, int batch, int H, int W, int IC, int OC, int kH, int kW, int stride, int pad) {
     if (IC > 4 || (long long)batch * H * W * IC * 2 >= 0x7ffffff0LL) return false;
     const int OH = (H + 2 * pad - kH) / stride + 1, OW = (W + 2 * pad - kW) / stride + 1;
@@ -399,6 +421,9 @@ inline bool make_plan(Plan& plan, int batch, int H, int W, int IC, int OC, int k
     const size_t raw = align16((size_t)OC_BLOCK * kH * kW * IC * 2), packed = (size_t)steps * STEP_BYTES;
     const int oc_blocks = (OC + OC_BLOCK - 1) / OC_BLOCK;
     if (oc_blocks > 65535) return false;
+    // input pixels under the output, borders included, per output pixel and channel block
+    const double staged = ((double)(OH - 1) * stride + kH) * ((double)(OW - 1) * stride + kW) / ((double)OH * OW) * oc_blocks;
+    if (!is_faster((long long)batch * OH * OW, staged, IC, OC, (int)steps)) return false;
     double best = 0.0;
     Params& p = plan.p;
     // candidates: this runs on every call, so a few of them (a search over all rows took longer than the small layers).

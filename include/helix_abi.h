@@ -104,8 +104,8 @@ HELIX_API size_t helix_conv_workspace_bytes(int batch, int H, int W, int IC, int
 
 /* One NHWC convolution on `stream`: implicit GEMM (no column buffer) when IC is a multiple of the gather
  * chunk; FP16 layers of up to four channels run in one kernel that pads the channels on the way into LDS
- * (src_template/common/helix_conv_thin.h; the workspace is asked for all the same, longer filters need it); else the
- * implicit GEMM on copies with the channels zero-padded to the chunk, or (IC = 1; 2 in FP16) im2col
+ * (src_template/common/helix_conv_thin.h; the workspace is asked for all the same, layers that kernel is slower for or a y
+ * off 16 bytes need it); else the implicit GEMM on copies with the channels zero-padded to the chunk, or (IC = 1; 2 in FP16) im2col
  * into the workspace followed by the GEMM, as the reference does for every layer.
  * Replaces: `im2col batch IC H W OC kH kW stride pad` followed by the GEMM executable
  * (scripts/Ampere_FP16/Ampere_FP16_conv.py:431-446, src_template/Ampere_FP16/im2col.cu:38-97). */

@@ -77,6 +77,21 @@ def test_every_library_copies(keys):
             assert np.array_equal(got.astype(np.float32), want), (key, layer)
 
 
+# pairs of layers on either side of each line of the rule (helix_conv_thin::is_faster)
+@pytest.mark.parametrize("layer,thin", [((4, 1, 64, 64, 32, 9, 9, 1, 4), True), ((4, 1, 64, 63, 32, 9, 9, 1, 4), False),
+                                        ((2, 2, 64, 64, 72, 11, 11, 1, 5), True), ((2, 2, 64, 63, 72, 11, 11, 1, 5), False),
+                                        ((4, 1, 64, 64, 128, 13, 13, 1, 6), True), ((4, 1, 64, 64, 136, 13, 13, 1, 6), False),
+                                        ((1, 1, 33, 33, 192, 3, 3, 4, 1), True), ((1, 1, 33, 33, 200, 3, 3, 4, 1), False),
+                                        ((1, 4, 33, 33, 448, 1, 1, 4, 0), True), ((1, 4, 33, 33, 456, 1, 1, 4, 0), False),
+                                        ((1, 3, 33, 33, 1024, 7, 7, 4, 3), True)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_both_sides_of_the_rule(layer, thin):
+    assert c16.runs_thin(*layer) == thin
+    x, w, want = integers(layer)
+    got = run_conv(load(b16.kernel_library(*LIBS[0])), x, w, layer[7], layer[8], torch.float16)
+    assert np.array_equal(got.astype(np.float32), want)
+
+
 @pytest.mark.parametrize("IC", [1, 3, 6])
 def test_workspace_off_16_bytes_is_refused(IC):
     """Whichever path the layer runs on."""

@@ -22,7 +22,7 @@ LAYERS = [(1, 3, 1, 8, 1, 1, 1, 1, 0),            # one row, one output channel
           (2, 3, 40, 44, 64, 7, 7, 2, 3),         # 7 steps
           (1, 3, 30, 170, 24, 7, 7, 1, 3),        # ... with rows cut into column blocks
           (130, 3, 30, 29, 96, 11, 11, 4, 0),     # weights in LDS, several blocks per workgroup
-          (1, 1, 40, 300, 32, 5, 20, 2, 0),       # one channel
+          (1, 1, 40, 300, 32, 5, 20, 2, 0),       # one channel, a long filter: too few pixels, takes the column buffer
           (2, 2, 9, 11, 12, 7, 6, 1, 5),          # two channels, even filter width, padding wider than the image's edge
           (1, 4, 30, 31, 70, 3, 3, 1, 1),
           (600, 3, 20, 20, 8, 3, 3, 1, 1)]        # more blocks than the chip holds at once
