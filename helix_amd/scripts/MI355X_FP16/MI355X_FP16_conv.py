@@ -89,6 +89,8 @@ def runs_thin(batch, IC, H, W, OC, kH, kW, stride, pad):
     same arithmetic as its host side: the layer's index range, its filter, where that kernel is the faster one, and one output
     row or a part of one in LDS)."""
     OH, OW = (H + 2 * pad - kH) // stride + 1, (W + 2 * pad - kW) // stride + 1
+    if OH < 1 or OW < 1:       # a filter beyond the padded image: refused by the library
+        return False
     pairs = (kW + 1) // 2
     steps = (kH * pairs + 3) // 4
     oc_blocks = -(-OC // THIN_OC_BLOCK)

@@ -6,6 +6,7 @@ import subprocess
 import pytest
 
 from utils.helix_runtime import SRC_ROOT, _find_include_dir
+from utils.hip_ctypes import HELIX_ERR_INVALID_VALUE, HelixError
 from MI355X_FP16 import MI355X_FP16_conv as c16
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -47,6 +48,17 @@ def test_host_knows_which_layers_the_thin_kernel_takes(check):
     taken = [line == "1" for line in run.stdout.split()]
     assert len(taken) == len(cases) and 500 < sum(taken) < 2900
     assert [c16.runs_thin(*l) for l in cases] == taken
+
+
+@pytest.mark.parametrize("layer", [(1, 3, 5, 5, 8, 7, 7, 3, 0), (1, 3, 9, 5, 8, 7, 7, 2, 0), (1, 1, 3, 30, 8, 5, 5, 1, 0)])
+def test_filter_beyond_the_image_is_still_refused_by_the_selection(layer, monkeypatch):
+    class Library:
+        def bench_conv(self, *a, **kw):
+            raise HelixError("helix_bench_conv", HELIX_ERR_INVALID_VALUE)
+    assert not c16.runs_thin(*layer)
+    monkeypatch.setattr(c16, "load", lambda path: Library())
+    with pytest.raises(RuntimeError, match="none of"):
+        c16.verified_config({(2, 64, 64, 32, 32, 0, 64): 1e-5}, *layer)
 
 
 def test_selection_of_a_thin_layer_times_nothing(monkeypatch):
