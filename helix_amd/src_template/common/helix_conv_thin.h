@@ -70,14 +70,14 @@ struct Params {
 
 // Where the 24 bytes of four three-channel pixels at byte `at` of x (the unit) are loaded from: seven whole dwords from byte
 // `from` on, never beyond the last whole dword of x.  Near the end of x these start in front of the unit's first dword and are
-// moved down by `behind` of them; what then lies behind the end belongs to no pixel of the row.  Where the number of halves is
-// odd, the last one lies in no whole dword: it is read by itself, into dword `last_half` of the moved ones (7 and more: not in
-// this unit).  x holds at least 28 bytes.
-struct Window { int from, behind, last_half; };
+// moved down by `behind` of them; what then lies behind the end belongs to no pixel of the row.  An odd number of halves leaves
+// the last one in no whole dword: it is read by itself and moved in behind the last of them (a unit that holds it is always
+// moved, by one dword or more).  x holds at least 28 bytes.
+struct Window { int from, behind; };
 __host__ __device__ __forceinline__ Window window_of(int at, int x_bytes) {
     const int whole = x_bytes & ~3, first = at & ~3, last = whole - 28;
     const int from = first < last ? first : last;
-    return Window{from, (first - from) >> 2, (x_bytes & 2) ? (whole - first) >> 2 : 7};
+    return Window{from, (first - from) >> 2};
 }
 
 // 16 bytes of LDS at an address that is a multiple of 8
@@ -122,18 +122,15 @@ __global__ __launch_bounds__(threads_of(KS), resident_of(KS) * threads_of(KS) / 
         const bool inside = (i < total_units) & ((unsigned)ih < (unsigned)p.H) & ((unsigned)iw < (unsigned)p.W);
         const int at = (((k.image * p.H + ih) * p.W + iw) * p.IC) * 2;
         if (p.unit_pixels == 4) {
-            const Window n = window_of(inside ? at : 0, (int)p.x_bytes);
+            const Window n = window_of(at, (int)p.x_bytes);
             const uintx4 lo = __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(rx, inside ? n.from : OOB, 0, 0));
             const uintx3 hi = __builtin_bit_cast(uintx3, __builtin_amdgcn_raw_buffer_load_b96(rx, inside ? n.from + 16 : OOB, 0, 0));
             unsigned w[7] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2]};
-            for (int behind = n.behind; __any(behind > 0); behind--) {
+            for (int behind = inside ? n.behind : 0; __any(behind > 0); behind--) {
 #pragma unroll
                 for (int e = 0; e < 6; e++) w[e] = behind > 0 ? w[e + 1] : w[e];
-            }
-            if (__any(inside && n.last_half < 7)) {
                 const unsigned half = __builtin_amdgcn_raw_buffer_load_b16(rx, (int)p.x_bytes - 2, 0, 0);
-#pragma unroll
-                for (int e = 1; e < 7; e++) w[e] = inside && n.last_half == e ? half : w[e];
+                w[6] = behind > 0 ? half : w[6];
             }
 #pragma unroll
             for (int e = 0; e < 4; e++) v.a[e] = __builtin_amdgcn_alignbyte(w[e + 1], w[e], at & 2);

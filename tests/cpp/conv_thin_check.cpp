@@ -16,15 +16,16 @@ static int windows() {
         for (int pixel = 0; pixel < pixels; pixel++) {
             const int at = pixel * 6;
             const helix_conv_thin::Window n = helix_conv_thin::window_of(at, bytes);
-            if (n.from < 0 || n.from % 4 || n.from + 28 > bytes || n.behind < 0 || n.behind > 6 || n.last_half < 1) {
+            if (n.from < 0 || n.from % 4 || n.from + 28 > bytes || n.behind < 0 || n.behind > 6) {
                 bad++;
                 continue;
             }
             unsigned w[7];
             memcpy(w, x + n.from, 28);
-            for (int b = 0; b < n.behind; b++)
+            for (int b = 0; b < n.behind; b++) {
                 for (int e = 0; e < 6; e++) w[e] = w[e + 1];
-            if (n.last_half < 7) w[n.last_half] = (unsigned)x[bytes - 2] | (unsigned)x[bytes - 1] << 8;
+                w[6] = (unsigned)x[bytes - 2] | (unsigned)x[bytes - 1] << 8;
+            }
             const int held = bytes - at < 24 ? bytes - at : 24;      // what of the unit lies in x
             bad += memcmp((unsigned char*)w + (at & 2), x + at, held) != 0;
         }

@@ -54,3 +54,19 @@ def test_thin_convolution_reads_only_the_filter_window(kW):
     want[max(0, 6 - h):6 + h + 1, max(0, 8 - h):8 + h + 1] = True
     assert np.array_equal(np.isinf(got[0]), np.repeat(want[:, :, None], 8, axis=2))
     assert np.array_equal(got[0][~want], np.zeros_like(got[0][~want]))
+
+
+@pytest.mark.parametrize("layer", [(1, 3, 9, 171, 24, 7, 7, 1, 3), (5, 3, 7, 7, 8, 3, 3, 1, 1), (1, 3, 31, 31, 64, 11, 11, 4, 2),
+                                   (301, 3, 5, 9, 16, 5, 5, 1, 2), (1, 3, 3, 5, 8, 2, 2, 1, 1)], ids=lambda l: "x".join(map(str, l)))
+def test_last_half_of_an_odd_input(layer):
+    """An odd number of halves: the last one lies in no whole dword and is read by itself, in every block whose patch holds
+    its pixel (several rows of blocks, column blocks, weights in registers and in LDS)."""
+    batch, IC, H, W, OC, kH, kW, stride, pad = layer
+    assert batch * IC * H * W % 2 == 1
+    x = np.zeros((batch, H, W, IC), np.float16)
+    x[-1, -1, -1, :] = 1, 2, 4
+    w = np.random.default_rng(7).integers(1, 4, (OC, kH, kW, IC)).astype(np.float16)
+    want = O.conv2d_nhwc(x.astype(np.float32), w.astype(np.float32), stride, pad)
+    assert want.max() > 0
+    got = run_conv(load(b16.kernel_library("gemm", 2, 64, 64, 32, 32, 64)), x, w, stride, pad, torch.float16)
+    assert np.array_equal(got.astype(np.float32), want)
