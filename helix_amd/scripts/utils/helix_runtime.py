@@ -362,14 +362,15 @@ def fastest_of(keys, time_config, what):
     return min(finalists, key=lambda k: best[k])
 
 
-def tuned_config(backend, problem, prof_dict, model_pick, verify):
-    """The configuration a runner launches for `problem`: the recorded winner if the profile still holds it, else
+def tuned_config(backend, problem, prof_dict, model_pick, verify, unprofiled=()):
+    """The configuration a runner launches for `problem`: the recorded winner if the profile still holds it (or `unprofiled`,
+    the keys of configurations that are ranked without a profile), else
     `verify()` (the fastest of the cost model's first candidates, timed now) which is then recorded; with
     HELIX_SELECTION=model always `model_pick()`."""
     if selection_mode() == "model":
         return model_pick()
     key = read_winners(backend, prof_dict).get(tuple(problem))
-    if key is not None and key in prof_dict:
+    if key is not None and (key in prof_dict or key in unprofiled):
         return key
     key = verify()
     store_winner(backend, problem, key, prof_dict)

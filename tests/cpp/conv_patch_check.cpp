@@ -1,0 +1,46 @@
+// Host side of conv_patch.hip, one configuration of it: per layer read (batch IC H W OC kH kW stride pad) one line with the
+// LDS bytes, the staged bytes and the workgroups of its plan, or "none"; exits with 1 when a block of output pixels would
+// write or read beyond what the plan reserves.
+#include "conv_patch.hip"
+
+static int staged_row(const Params& p, int m) {
+    const int t = m / p.by_OW.d, image = t / p.OH;
+    return image * p.image_rows + (t - image * p.OH) * p.stride;
+}
+
+int main() {
+    int l[9];
+    while (scanf("%d %d %d %d %d %d %d %d %d", l, l + 1, l + 2, l + 3, l + 4, l + 5, l + 6, l + 7, l + 8) == 9) {
+        const int kH = l[5], kW = l[6];
+        Params p{};
+        int lds = 0;
+        if (l[2] + 2 * l[8] < kH || l[3] + 2 * l[8] < kW || !tpl::make_plan(p, &lds, l[0], l[2], l[3], l[1], l[4], kH, kW, l[7], l[8])) {
+            printf("none\n");
+            continue;
+        }
+        int most = 0;
+        const bool spare = p.chunks % KT_CHUNKS != 0;
+        for (int m0 = 0; m0 < p.M; m0 += BLOCK_ROWS) {
+            const int last = (m0 + BLOCK_ROWS < p.M ? m0 + BLOCK_ROWS : p.M) - 1, row0 = staged_row(p, m0);
+            const int rows = staged_row(p, last) + kH - row0;
+            if (rows > most) most = rows;
+            // the last staged chunk, and the chunk behind it where there is one
+            const long long wrote = (long long)(rows - 1) * p.row_bytes + (long long)(p.row_pixels - 1) * p.pixel_bytes + (p.group + spare) * 16;
+            long long read = 0;
+            for (int m = m0; m <= last; m++) {      // the last chunk of the last tap
+                const long long at = (long long)(staged_row(p, m) - row0 + kH - 1) * p.row_bytes +
+                                     ((long long)(m % p.by_OW.d) * p.stride + kW - 1) * p.pixel_bytes + (p.group + spare) * 16;
+                if (at > read) read = at;
+            }
+            if (p.patch_offset + wrote > lds || p.patch_offset + read > lds || p.real_pixels > p.W ||
+                p.pad + p.real_pixels > p.row_pixels || (p.real_pixels + p.pad < p.row_pixels && p.real_pixels < p.W)) {
+                printf("out of bounds\n");
+                return 1;
+            }
+        }
+        const long long rows = tpl::staged_rows(p.OH, p.by_OW.d, kH, p.stride, BLOCK_ROWS < p.M ? BLOCK_ROWS : p.M);
+        if (most > rows) return 1;
+        printf("%d %lld %d\n", lds, rows * p.row_bytes, p.blocks);
+    }
+    return 0;
+}
