@@ -13,8 +13,8 @@ import math
 import os
 
 from utils.helix_runtime import load, kernel_resources, tuned_config, fastest_of
-from utils.roofline import NUM_CU
-from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, is_dtl_key, patch_keys, PATCH_BLOCK_K
+from utils.conv_patch import PatchFamily, PATCH_TOP
+from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, is_dtl_key, patch_key, patch_keys, PATCH_POINTS
 from MI355X_FP16.MI355X_FP16_gemm import short_value, config_cost, VERIFY_TOP
 
 root_path = os.getcwd()
@@ -120,82 +120,14 @@ def runs_thin(batch, IC, H, W, OC, kH, kW, stride, pad):
     return False
 
 
-# ---- the family whose input stays in LDS (src_template/MI355X_FP16/conv_patch.hip) ----------------------------------------
-# Clocks at 2.4 GHz, fitted to 318 measured (layer, configuration) pairs, 8 % rms; what decides is the order: the fastest of
-# the first four by this model is 0.24 % behind the fastest of all 22 in the geometric mean over 29 layers, 3.8 % at worst
-# (the first one alone 4.6 and 38 %).
-PATCH_FIXED_CLOCKS = 10300             # launch, first loads, last stores
-PATCH_STAGE_BYTES_PER_CLOCK = 20       # input into LDS, per compute unit
-PATCH_MFMA_CLOCKS = 16 * 1.63          # of one 16 x 16 x 32 product in the loop
-PATCH_LDS_BYTES_PER_CLOCK = 105
-PATCH_WEIGHT_BYTES_PER_CLOCK = 69
-PATCH_TILE_CLOCKS = 117                # of a K tile at least, whatever is in it
-PATCH_SUM_CLOCKS = 34                  # adding one part of K of one 16 x 16 tile; about the same to store a tile
-PATCH_TOP = 4
-PATCH_WAVES = 8            # waves a compute unit holds of a configuration that takes up to 256 registers
-
-
-def patch_layout(key, batch, IC, H, W, OC, kH, kW, stride, pad):
-    """(bytes of LDS, of which staged input, workgroups) of a configuration of the family, None where it cannot run the layer
-    (same arithmetic as make_plan of conv_patch.hip)."""
-    _, rows, cols, wave_rows, wave_cols, groups, _, _ = key
-    OH, OW = (H + 2 * pad - kH) // stride + 1, (W + 2 * pad - kW) // stride + 1
-    K, M = kH * kW * IC, batch * OH * OW
-    if OH < 1 or OW < 1 or IC % 8 or K * 2 > 0x1000000 or batch * H * W * IC * 2 >= 0x40000000 or OC * K * 2 >= 0x40000000:
-        return None
-    image_rows, row_pixels = (OH - 1) * stride + kH, (OW - 1) * stride + kW
-    blocks = -(-M // rows) * -(-OC // cols)
-    if (M > 0x7fffff or W * IC * 2 > 0x7fffff or batch * H > 0x7fffff or batch * image_rows > 0x7fffff or blocks > 0x3fffffff
-            or row_pixels - pad < 1):
-        return None
-    pixels = min(rows, M)
-    if pixels % OW == 0:
-        n = pixels // OW
-        crossings = n // OH - 1 if n % OH == 0 else 0 if OH % n == 0 else (n - 2) // OH + 1
-    else:
-        n = (pixels - 2) // OW + 2
-        crossings = (n - 2) // OH + 1
-    staged_rows = (n - 1) * stride + kH + crossings * max(kH - stride, 0)
-    tiles = -(-(K // 8) // 8)
-    used = IC // 8 + (1 if (K // 8) % 8 else 0)
-    pixel_bytes = 16 * (used + (6 - used % 4) % 4 if stride % 2 else used | 1)
-    waves = rows // wave_rows * (cols // wave_cols) * groups
-    patch = staged_rows * row_pixels * pixel_bytes
-    offset = waves * wave_cols * PATCH_BLOCK_K * 2 + 8 * (tiles + 1) * 4
-    sums = waves * wave_rows * wave_cols * 4 if groups > 1 else 0
-    lds = max(offset + patch, sums)
-    return (lds, patch, blocks) if lds <= LDS_BYTES_PER_CU else None
-
-
-def patch_config_cost(key, batch, IC, H, W, OC, kH, kW, stride, pad):
-    """Predicted seconds of a layer on a configuration of the family; inf where it cannot run it."""
-    layout = patch_layout(key, batch, IC, H, W, OC, kH, kW, stride, pad)
-    if layout is None:
-        return float("inf")
-    lds, patch, blocks = layout
-    _, rows, cols, wave_rows, wave_cols, groups, block_k, _ = key
-    waves = rows // wave_rows * (cols // wave_cols) * groups
-    tm, tn = wave_rows // 16, wave_cols // 16
-    resident = max(1, min(LDS_BYTES_PER_CU // lds, (2 if tm * tn <= 8 else 1) * PATCH_WAVES // waves))
-    tiles = -(-(kH * kW * IC) // block_k)
-    part = -(-tiles // groups)
-
-    def round_clocks(share):                 # workgroups of one round on a compute unit
-        multiply = part * 2 * tm * tn * PATCH_MFMA_CLOCKS * max(1.0, waves * share / 4)
-        read = share * waves * part * (2 * tm + 4 * tn) * 1024 / PATCH_LDS_BYTES_PER_CLOCK
-        weights = share * waves * part * tn * 2048 / PATCH_WEIGHT_BYTES_PER_CLOCK
-        return (patch * share / PATCH_STAGE_BYTES_PER_CLOCK + max(multiply, read, weights, part * PATCH_TILE_CLOCKS)
-                + (PATCH_SUM_CLOCKS * groups * tm * tn if groups > 1 else 0) + PATCH_SUM_CLOCKS * share * tm * tn * waves / groups)
-
-    rounds = -(-blocks // (NUM_CU * resident))
-    last = blocks - (rounds - 1) * NUM_CU * resident
-    return (PATCH_FIXED_CLOCKS + (rounds - 1) * round_clocks(resident) + round_clocks(min(resident, -(-last // NUM_CU)))) / 2.4e9
+# The family whose input stays in LDS (utils/conv_patch.py)
+PATCH = PatchFamily(element_bytes=2, whole_chunks=True, points=PATCH_POINTS, fixed=10300, stage_rate=20, multiply=2 * 16 * 1.63,
+                    lds_rate=105, weight_rate=69, tile=117, add=34)
 
 
 def patch_ranked(layer, top=PATCH_TOP):
-    """The `top` configurations of the family with the lowest predicted time that can run the layer, best first."""
-    costs = sorted((patch_config_cost(k, *layer), k) for k in patch_keys())
-    return [k for cost, k in costs[:top] if cost < float("inf")]
+    """The keys of that family's first `top` configurations for a layer."""
+    return [patch_key(point) for point in PATCH.ranked(layer, top)]
 
 
 def conv_kernel_scratch(k, IC=None):
@@ -239,8 +171,8 @@ def ranked_configs(prof_dict, M, N, K, IC=None, top=VERIFY_TOP, pointwise=False)
 
 
 def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP):
-    """The fastest of the cost model's first `top` configurations on this layer (utils.helix_runtime.fastest_of:
-    2 + 5 launches each, the leaders timed again); for a layer that runs in the kernel for thin inputs the model's first
+    """The fastest of the cost model's first `top` configurations on this layer and the first few of the family whose input
+    stays in LDS (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again); for a layer that runs in the kernel for thin inputs the model's first
     one without K partitions."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     ICg = gather_channels(input_channel)
@@ -313,7 +245,7 @@ def get_MI355X_FP16_conv_Oracle_result(prof_dict, batch, input_channel, H, W, ou
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     flops = 2.0 * M * output_channel * input_channel * kH * kW
     min_cost, best = float("inf"), None
-    for k in list(prof_dict.keys()) + patch_keys():
+    for k in list(prof_dict.keys()) + list(patch_keys()):
         if k[0] == 0 or is_dtl_key(k):
             continue
         try:

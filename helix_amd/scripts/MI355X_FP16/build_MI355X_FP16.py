@@ -199,7 +199,7 @@ def iter_dtl_configs():
                         yield (K_STAGES, BLOCK_ROWS, BLOCK_COLS, WAVE_ROWS, WAVE_COLS, BLOCK_K)
 
 
-# Convolutions whose input stays in LDS (src_template/MI355X_FP16/conv_patch.hip): (BLOCK_ROWS, BLOCK_COLS, WAVE_ROWS,
+# Convolutions whose input stays in LDS (src_template/common/helix_conv_patch.h): (BLOCK_ROWS, BLOCK_COLS, WAVE_ROWS,
 # WAVE_COLS, K_GROUPS) points, of four or eight waves.  All 400 shapes with wave tiles of 16 .. 128 x 16 | 32 | 64 were timed on
 # 50 convolution layers; picked greedily, these are within 0.2 % (geometric mean) of the fastest of all of them over the
 # layers on which the family is no more than 12 % behind the implicit GEMM.
@@ -208,12 +208,18 @@ PATCH_POINTS = [(16, 16, 16, 16, 4), (16, 16, 16, 16, 8), (32, 16, 32, 16, 4), (
                 (64, 32, 64, 32, 4), (96, 32, 96, 16, 4), (32, 128, 32, 32, 2), (64, 128, 64, 32, 1), (80, 128, 80, 32, 1),
                 (160, 32, 80, 32, 2), (112, 64, 112, 32, 2), (112, 64, 112, 32, 4), (112, 128, 112, 32, 1),
                 (112, 128, 112, 32, 2), (224, 64, 112, 32, 1), (224, 128, 112, 32, 1)]
-PATCH_BLOCK_K = 64
+
+
+def patch_key(point):
+    """Key of a point of that family, convolutions only: (2, BLOCK_ROWS, BLOCK_COLS, WAVE_ROWS, WAVE_COLS, K_GROUPS, 64, 2)."""
+    return (2,) + tuple(point) + (64, 2)
+
+
+PATCH_KEYS = tuple(patch_key(point) for point in PATCH_POINTS)
 
 
 def patch_keys():
-    """Keys of that family, convolutions only: (2, BLOCK_ROWS, BLOCK_COLS, WAVE_ROWS, WAVE_COLS, K_GROUPS, 64, 2)."""
-    return [(2,) + point + (PATCH_BLOCK_K, 2) for point in PATCH_POINTS]
+    return PATCH_KEYS
 
 
 def is_patch_key(key):

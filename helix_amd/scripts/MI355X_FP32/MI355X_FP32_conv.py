@@ -6,7 +6,8 @@ import math
 import os
 
 from utils.helix_runtime import load, tuned_config, fastest_of
-from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library
+from utils.conv_patch import PatchFamily, PATCH_TOP
+from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, patch_key, patch_keys, PATCH_POINTS
 from MI355X_FP32.MI355X_FP32_gemm import config_cost, extra_points, VERIFY_TOP
 
 root_path = os.getcwd()
@@ -51,17 +52,28 @@ def ranked_configs(prof_dict, M, N, K, top=VERIFY_TOP):
     return [k for _, k in cand[:top]]
 
 
+# The family whose input stays in LDS (utils/conv_patch.py)
+PATCH = PatchFamily(element_bytes=4, whole_chunks=False, points=PATCH_POINTS, fixed=8460, stage_rate=10, multiply=2 * 4 * 32 * 1.18,
+                    lds_rate=105, weight_rate=69, tile=406, add=92)
+
+
+def patch_ranked(layer, top=PATCH_TOP):
+    """The keys of that family's first `top` configurations for a layer."""
+    return [patch_key(point) for point in PATCH.ranked(layer, top)]
+
+
 def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP):
-    """The fastest of the cost model's first `top` configurations on this layer (utils.helix_runtime.fastest_of:
-    2 + 5 launches each, the leaders timed again)."""
+    """The fastest of the cost model's first `top` configurations on this layer and the first few of the family whose input
+    stays in LDS (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again)."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
 
     def time_config(k, warmup, iters):
         return load(library_for_key(k)).bench_conv(batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
                                                    warmup=warmup, iters=iters)[1]
 
-    return fastest_of(ranked_configs(prof_dict, M, output_channel, gather_channels(input_channel) * kH * kW, top),
-                      time_config, "this layer")
+    layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
+    return fastest_of(ranked_configs(prof_dict, M, output_channel, gather_channels(input_channel) * kH * kW, top)
+                      + patch_ranked(layer, min(top, PATCH_TOP)), time_config, "this layer")
 
 
 def get_MI355X_FP32_conv_Verified_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
@@ -89,7 +101,7 @@ def select_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW,
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return tuned_config("MI355X_FP32", ("conv",) + layer, prof_dict,
                         lambda: layer_cost_model(prof_dict, *layer),
-                        lambda: verified_config(prof_dict, *layer))
+                        lambda: verified_config(prof_dict, *layer), patch_keys())
 
 
 def get_MI355X_FP32_conv_Helix_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,

@@ -80,6 +80,34 @@ def iter_kgroup_configs():
                 yield (BM, BN, BK, WAVE_M, WAVE_N, KG)
 
 
+# Convolutions whose input stays in LDS (src_template/common/helix_conv_patch.h): (BLOCK_ROWS, BLOCK_COLS, WAVE_ROWS, WAVE_COLS,
+# K_GROUPS) points.  200 shapes with wave tiles of 16 .. 128 x 16 | 32 | 64 were timed on 54 convolution layers; picked greedily,
+# these are within 0.3 % (geometric mean) of the fastest of all of them over the 34 layers on which the family is no more than
+# 10 % behind the implicit GEMM.
+PATCH_POINTS = [(16, 16, 16, 16, 4), (16, 16, 16, 16, 8), (16, 32, 16, 16, 4), (32, 32, 16, 16, 1), (64, 16, 16, 16, 1),
+                (32, 32, 32, 16, 4), (64, 64, 32, 16, 1), (128, 32, 32, 16, 1), (48, 16, 48, 16, 8), (48, 32, 48, 16, 2),
+                (96, 64, 48, 16, 1), (192, 16, 48, 16, 1), (256, 32, 64, 16, 1), (80, 32, 80, 16, 4), (160, 16, 80, 16, 4),
+                (160, 32, 80, 16, 1), (160, 64, 80, 16, 1), (160, 32, 80, 32, 2), (112, 64, 112, 16, 1), (112, 128, 112, 32, 1),
+                (224, 64, 112, 32, 1), (512, 16, 128, 16, 2)]
+
+
+def patch_key(point):
+    """Key of a point of that family, convolutions only: (BLOCK_ROWS, BLOCK_COLS, 32, WAVE_ROWS, WAVE_COLS, 0, K_GROUPS, 4);
+    the field of the LDS stages is 0."""
+    return (point[0], point[1], 32, point[2], point[3], 0, point[4], 4)
+
+
+PATCH_KEYS = tuple(patch_key(point) for point in PATCH_POINTS)
+
+
+def patch_keys():
+    return PATCH_KEYS
+
+
+def is_patch_key(key):
+    return key[2] != 0 and key[5] == 0
+
+
 def sgemm_library(BM, BN, BK, WAVE_M, WAVE_N, KG=1):
     suffix = "" if KG == 1 else f"_kg{KG}"
     return f"{bin_dir('fp32')}/libsgemm_{BM}_{BN}_{BK}_{WAVE_M}_{WAVE_N}{suffix}.so"
@@ -100,6 +128,8 @@ def library_for_key(key):
     the GEMV rows, whose first two fields are the activation-row tile and 128 weight rows."""
     if key[2] == 0:
         return kernel_library("gemv_fp32" if key[5] == 0 else "gemv_fp32_splitK")
+    if is_patch_key(key):
+        return kernel_library("conv_patch_" + "_".join(str(key[i]) for i in (0, 1, 3, 4, 6)))
     return sgemm_library(key[0], key[1], key[2], key[3], key[4], key[6])
 
 
@@ -123,9 +153,15 @@ def compile_kernel(kernel_name):
     return (f"{SRC_ROOT}/MI355X_FP32/{src_name}.hip", kernel_library(kernel_name), defines)
 
 
+def patch_job(key):
+    names = ("BLOCK_ROWS", "BLOCK_COLS", "WAVE_ROWS", "WAVE_COLS", "K_GROUPS")
+    return (f"{SRC_ROOT}/MI355X_FP32/conv_patch.hip", library_for_key(key), dict(zip(names, (key[i] for i in (0, 1, 3, 4, 6)))))
+
+
 def build_jobs():
     jobs = [compile_sgemm(*cfg) for cfg in iter_configs()]
     jobs += [compile_sgemm(*cfg) for cfg in iter_kgroup_configs()]
+    jobs += [patch_job(key) for key in patch_keys()]
     jobs.append(compile_kernel("gemv_fp32"))
     jobs.append(compile_kernel("gemv_fp32_splitK"))
     jobs.append(rocblas_job())

@@ -19,17 +19,16 @@ int main() {
             continue;
         }
         int most = 0;
-        const bool spare = p.chunks % KT_CHUNKS != 0;
         for (int m0 = 0; m0 < p.M; m0 += BLOCK_ROWS) {
             const int last = (m0 + BLOCK_ROWS < p.M ? m0 + BLOCK_ROWS : p.M) - 1, row0 = staged_row(p, m0);
             const int rows = staged_row(p, last) + kH - row0;
             if (rows > most) most = rows;
-            // the last staged chunk, and the chunk behind it where there is one
-            const long long wrote = (long long)(rows - 1) * p.row_bytes + (long long)(p.row_pixels - 1) * p.pixel_bytes + (p.group + spare) * 16;
+            // the last staged chunk
+            const long long wrote = (long long)(rows - 1) * p.row_bytes + (long long)(p.row_pixels - 1) * p.pixel_bytes + p.group * 16;
             long long read = 0;
             for (int m = m0; m <= last; m++) {      // the last chunk of the last tap
                 const long long at = (long long)(staged_row(p, m) - row0 + kH - 1) * p.row_bytes +
-                                     ((long long)(m % p.by_OW.d) * p.stride + kW - 1) * p.pixel_bytes + (p.group + spare) * 16;
+                                     ((long long)(m % p.by_OW.d) * p.stride + kW - 1) * p.pixel_bytes + p.group * 16;
                 if (at > read) read = at;
             }
             if (p.patch_offset + wrote > lds || p.patch_offset + read > lds || p.real_pixels > p.W ||

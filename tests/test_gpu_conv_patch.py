@@ -1,5 +1,5 @@
-"""FP16 convolutions whose input stays in LDS (MI355X_FP16/conv_patch.hip): every configuration on layers at the edges of its
-blocks, through the C ABI."""
+"""Convolutions whose input stays in LDS (common/helix_conv_patch.h), FP16 and FP32: every configuration on layers at the edges
+of its blocks, through the C ABI."""
 import numpy as np
 import pytest
 import torch
@@ -8,6 +8,8 @@ from utils.helix_runtime import load
 from utils.hip_ctypes import HELIX_ERR_INVALID_VALUE, HELIX_ERR_UNSUPPORTED
 from MI355X_FP16 import build_MI355X_FP16 as b16
 from MI355X_FP16 import MI355X_FP16_conv as c16
+from MI355X_FP32 import build_MI355X_FP32 as b32
+from MI355X_FP32 import MI355X_FP32_conv as c32
 from oracle import oracle as O
 from gpu_helpers import conv_out_hw, dev, run_conv
 
@@ -25,37 +27,62 @@ LAYERS = [(1, 8, 1, 1, 1, 1, 1, 1, 0),            # one pixel, one channel, K of
           (1, 8, 60, 120, 8, 7, 3, 4, 3)]         # more staged pixels than a thread's batch of loads
 
 
-@pytest.mark.parametrize("layer", LAYERS, ids=lambda l: "x".join(map(str, l)))
-def test_every_configuration_integer_exact(layer):
+# channel counts off the chunk: FP32 only
+LAYERS32 = LAYERS + [(2, 3, 21, 23, 40, 7, 7, 2, 3),     # one chunk per pixel, three floats of it
+                     (1, 1, 9, 17, 5, 3, 3, 1, 1),
+                     (3, 25, 10, 9, 17, 3, 3, 1, 1),     # a last chunk of one float; channels off the store's width
+                     (2, 6, 8, 8, 36, 1, 3, 1, 0),
+                     (1, 7, 1, 3, 16, 1, 1, 1, 0)]
+CASES = [(np.float16, b16, c16, l) for l in LAYERS] + [(np.float32, b32, c32, l) for l in LAYERS32]
+
+
+@pytest.mark.parametrize("dtype,build,conv,layer", CASES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else getattr(v, "__name__", "").split(".")[-1])
+def test_every_configuration_integer_exact(dtype, build, conv, layer):
     """Inputs in {-1, 0, 1}: exact in any order of the sums."""
     batch, IC, H, W, OC, kH, kW, stride, pad = layer
     rng = np.random.default_rng(sum(layer))
-    x = rng.integers(-1, 2, (batch, H, W, IC)).astype(np.float16)
-    w = rng.integers(-1, 2, (OC, kH, kW, IC)).astype(np.float16)
+    x = rng.integers(-1, 2, (batch, H, W, IC)).astype(dtype)
+    w = rng.integers(-1, 2, (OC, kH, kW, IC)).astype(dtype)
     want = O.conv2d_nhwc(x.astype(np.float32), w.astype(np.float32), stride, pad)
     assert np.abs(want).max() < 2048
     ran = 0
-    for key in b16.patch_keys():
-        if c16.patch_layout(key, *layer) is None:
+    for point in build.PATCH_POINTS:
+        if conv.PATCH.layout(point, *layer) is None:
             continue
-        got = run_conv(load(b16.library_for_key(key)), x, w, stride, pad, torch.float16)
-        assert np.array_equal(got.astype(np.float32), want), key
+        got = run_conv(load(build.library_for_key(build.patch_key(point))), x, w, stride, pad, torch.float16 if dtype is np.float16 else torch.float32)
+        assert np.array_equal(got.astype(np.float32), want), point
         ran += 1
     assert ran >= 4
 
 
-@pytest.mark.parametrize("key", b16.patch_keys()[::5], ids=str)
-def test_infinite_pixel_reaches_its_window_only(key):
-    """K has a remainder of five chunks, which multiplies zeros by zeros, whatever lies beside them."""
-    x = np.zeros((2, 12, 16, 8), np.float16)
-    x[1, 6, 8, 3] = np.inf
-    x[1, 11, 15, 7] = np.nan
-    w = np.ones((40, 3, 3, 8), np.float16)
-    got = run_conv(load(b16.library_for_key(key)), x, w, 1, 1, torch.float16)
-    want = np.zeros((2, 12, 16, 1), np.float16)
+@pytest.mark.parametrize("IC", [8, 3])
+@pytest.mark.parametrize("dtype,build", [(np.float16, b16), (np.float32, b32)])
+def test_infinite_pixel_reaches_its_window_only(dtype, build, IC):
+    """K has a remainder, which multiplies zeros by zeros, whatever lies beside them; so have the channels with IC = 3."""
+    if dtype is np.float16 and IC % 8:
+        pytest.skip("whole chunks only")
+    x = np.zeros((2, 12, 16, IC), dtype)
+    x[1, 6, 8, IC - 1] = np.inf
+    x[1, 11, 15, 0] = np.nan
+    w = np.ones((40, 3, 3, IC), dtype)
+    want = np.zeros((2, 12, 16, 1), dtype)
     want[1, 5:8, 7:10] = np.inf
     want[1, 10:, 14:] = np.nan
-    assert np.array_equal(got, np.repeat(want, 40, axis=3), equal_nan=True)
+    for key in build.patch_keys()[::3]:
+        got = run_conv(load(build.library_for_key(key)), x, w, 1, 1, torch.float16 if dtype is np.float16 else torch.float32)
+        assert np.array_equal(got, np.repeat(want, 40, axis=3), equal_nan=True), key
+
+
+def test_infinite_weight_of_the_next_tap():
+    """FP32, three channels: the fourth float of a tap's chunk would be the next tap's first."""
+    x = np.zeros((1, 5, 5, 3), np.float32)
+    x[0, 2, 2] = 1
+    w = np.zeros((16, 3, 3, 3), np.float32)
+    w[:, 1, 1, 0] = np.inf
+    for key in b32.patch_keys()[::3]:
+        got = run_conv(load(b32.library_for_key(key)), x, w, 1, 1, torch.float32)
+        # zero times the infinite weight is NaN at every other pixel; with the zero behind the chunk before it, it is not one here
+        assert np.isposinf(got[0, 2, 2]).all() and np.isnan(got).sum() == 24 * 16, key
 
 
 @pytest.mark.parametrize("offset", [1, 4])
