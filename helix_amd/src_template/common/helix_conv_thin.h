@@ -44,14 +44,14 @@ typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 typedef unsigned uintx3 __attribute__((ext_vector_type(3)));
 typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
 
-constexpr int OC_BLOCK = 64, NT = OC_BLOCK / 16;    // output channels of a workgroup, in 16-wide MFMA tiles
-constexpr int STEP_BYTES = NT * 64 * 16;            // packed weights of one MFMA step
+constexpr int OC_BLOCK = 64;                        // output channels of a workgroup, in 16-wide MFMA tiles (96 for some layers, see make_plan)
+constexpr int step_bytes(int nt) { return nt * 64 * 16; }      // packed weights of one MFMA step
 constexpr int ZERO_BYTES = 16;                      // a zeroed slot in front of the patch
 constexpr int LDS_MAX = 160 * 1024;
 constexpr int MAX_STEPS = 24;
 constexpr int OOB = 0x7fffffff;                     // byte offset beyond any buffer: the load returns zeros
 constexpr int threads_of(int ks) { return ks ? 256 : 512; }    // weights in LDS leave room for one workgroup per CU
-constexpr int resident_of(int ks) { return ks == 7 ? 2 : ks == 4 ? 3 : ks == 0 ? 1 : 4; }   // workgroups per CU the registers allow
+constexpr int resident_of(int ks, int nt) { return (ks == 7 ? 2 : ks == 4 ? 3 : ks == 0 ? 1 : 4) - (nt == 6); }   // workgroups per CU the registers allow
 
 struct Params {
     const _Float16* x;   // NHWC
@@ -90,15 +90,16 @@ __device__ __forceinline__ uintx4 read16(const unsigned char* p) {
 // channels 32 i + 8 q + {0..3} and {4..7} of their pixel.
 __device__ __forceinline__ int channel_of(int j, int r) { return (j >> 1) * 32 + (r >> 2) * 8 + (j & 1) * 4 + (r & 3); }
 
-template <int KS>
-__global__ __launch_bounds__(threads_of(KS), resident_of(KS) * threads_of(KS) / 256) void helix_conv_thin_f16_kernel(const Params p) {
+template <int KS, int NT>
+__global__ __launch_bounds__(threads_of(KS), resident_of(KS, NT) * threads_of(KS) / 256) void helix_conv_thin_f16_kernel(const Params p) {
     constexpr int THREADS = threads_of(KS), WAVES = THREADS / 64;
+    constexpr int STEP_BYTES = step_bytes(NT), CHANNELS = 16 * NT;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, q = lane >> 4;
-    const int oc0 = (int)blockIdx.y * OC_BLOCK;
-    const int ocs = (p.OC - oc0) < OC_BLOCK ? (p.OC - oc0) : OC_BLOCK;
+    const int oc0 = (int)blockIdx.y * CHANNELS;
+    const int ocs = (p.OC - oc0) < CHANNELS ? (p.OC - oc0) : CHANNELS;
 
     // ---- input under a block of output pixels: one unit is unit_pixels pixels of one row, from an input column that is a
     // multiple of unit_pixels --------------------------------------------------------------------------------------------
@@ -164,6 +165,18 @@ __global__ __launch_bounds__(threads_of(KS), resident_of(KS) * threads_of(KS) / 
             put(0, v.a[0], v.a[1]);
         }
     };
+    // ---- weights: as they lie; with more than four steps of them the loads of a thread are all in flight at once (7x7 21.8 ->
+    // 21.1 us, batch 1 6.7 -> 6.4, 11x11 12.7 -> 12.6; of fewer there is one or two, and the plain loop is the shorter one) -----
+    const int taps = p.kH * p.kW, filter = taps * p.IC, halves = ocs * filter;
+    const _Float16* src = p.w + (size_t)oc0 * filter;         // a multiple of 32 filters in: 16-byte aligned
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(src), 0, halves * 2, 0x00020000);
+    constexpr bool AT_ONCE = KS == 0 || KS > 4;
+    constexpr int WF = AT_ONCE ? 6 : 0;
+    uintx4 first[WF + 1];
+    auto load_weights = [&](int i) -> uintx4 {                 // 16 bytes, where all of them are filters of this block
+        return __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(rw, i < halves / 8 ? i * 16 : OOB, 0, 0));
+    };
+
     // the first PF units per thread of a block are requested ahead: the first block's in front of the work on the weights,
     // a later block's in front of the multiplication of the one before it
     constexpr int PF = 4;
@@ -172,38 +185,47 @@ __global__ __launch_bounds__(threads_of(KS), resident_of(KS) * threads_of(KS) / 
 #pragma unroll
     for (int u = 0; u < PF; u++)
         if (u * THREADS < total_units) early[u] = load_unit(block_of(g), tid + u * THREADS);
-
-    // ---- weights: as they lie into LDS, then packed in the order the MFMAs take them -----------------------------
-    const int taps = p.kH * p.kW, filter = taps * p.IC;
-    _Float16* raw = (_Float16*)(smem + p.raw_offset);
-    {
-        const _Float16* src = p.w + (size_t)oc0 * filter;     // a multiple of 64 filters in: 16-byte aligned
-        const int n = ocs * filter;
-        for (int i = tid; i < n / 8; i += THREADS) ((uintx4*)raw)[i] = ((const uintx4*)src)[i];
-        for (int i = (n & ~7) + tid; i < n; i += THREADS) raw[i] = src[i];
+    if constexpr (AT_ONCE) {
+#pragma unroll
+        for (int u = 0; u < WF; u++)
+            if (u * THREADS < halves / 8) first[u] = load_weights(tid + u * THREADS);
     }
+
+    // ---- weights: into LDS, then packed in the order the MFMAs take them --------------------------------------------------
+    _Float16* raw = (_Float16*)(smem + p.raw_offset);
+    if constexpr (AT_ONCE) {
+#pragma unroll
+        for (int u = 0; u < WF; u++)
+            if (tid + u * THREADS < halves / 8) ((uintx4*)raw)[tid + u * THREADS] = first[u];
+    }
+    for (int i = tid + WF * THREADS; i < halves / 8; i += THREADS) ((uintx4*)raw)[i] = ((const uintx4*)src)[i];
+    for (int i = (halves & ~7) + tid; i < halves; i += THREADS) raw[i] = src[i];
     __syncthreads();
     {
-        constexpr int AT_ONCE = WAVES / NT;                    // steps packed at a time: thread = (step, MFMA tile, lane)
-        const int n = channel_of(wave % NT, r);
-        const bool live = n < ocs;
-        const _Float16* of_n = raw + (live ? n : 0) * filter;
-        auto pack = [&](int s) {
+        // one step of one MFMA tile at a time, a lane's pair of pixels in four dwords read around it and shifted into place
+        // (half by half the 7x7 layer spent 2 us here); what lies beyond the pair is read (LDS that the plan reserves) and
+        // masked
+        auto pack = [&](int s, int j) {
             const int chunk = 4 * s + q, kh = p.by_pairs.div(chunk), kw = 2 * (chunk - kh * p.pairs);
-            const bool ok = live && chunk < p.chunks;
-            const _Float16* at = of_n + (ok ? (kh * p.kW + kw) * p.IC : 0);
-            half8 v;
-#pragma unroll
-            for (int e = 0; e < 8; e++) {                      // every read issued (from a valid place), then selected
-                const int c = e & 3, k = e >> 2;
-                const bool has = ok && c < p.IC && kw + k < p.kW;
-                const _Float16 h = at[has ? k * p.IC + c : 0];
-                v[e] = has ? h : (_Float16)0;
-            }
-            *(half8*)(smem + p.packed_offset + s * STEP_BYTES + (tid % (NT * 64)) * 16) = v;
+            const int n = channel_of(j, r);
+            const bool ok = n < ocs && chunk < p.chunks;
+            const int at = ok ? n * filter + (kh * p.kW + kw) * p.IC : 0, odd = (at & 1) * 2;
+            const unsigned* from = (const unsigned*)raw + (at >> 1);
+            const unsigned w0 = from[0], w1 = from[1], w2 = from[2], w3 = from[3];
+            const unsigned h0 = __builtin_amdgcn_alignbyte(w1, w0, odd), h1 = __builtin_amdgcn_alignbyte(w2, w1, odd);
+            const unsigned h2 = __builtin_amdgcn_alignbyte(w3, w2, odd), h3 = w3;      // (four channels: never odd)
+            uintx4 v;
+            if (p.IC == 3) v = uintx4{h0, h1 & 0xffffu, h1 >> 16 | h2 << 16, h2 >> 16};
+            else if (p.IC == 4) v = uintx4{h0, h1, h2, h3};
+            else if (p.IC == 2) v = uintx4{h0, 0, h1, 0};
+            else v = uintx4{h0 & 0xffffu, 0, h0 >> 16, 0};
+            const unsigned one = ok ? 0xffffffffu : 0u, two = ok && kw + 1 < p.kW ? 0xffffffffu : 0u;
+            v[0] &= one, v[1] &= one, v[2] &= two, v[3] &= two;
+            *(uintx4*)(smem + p.packed_offset + s * STEP_BYTES + (j * 64 + lane) * 16) = v;
         };
+        const int items = p.steps * NT;
 #pragma unroll 2
-        for (int s = wave / NT; s < p.steps; s += AT_ONCE) pack(s);
+        for (int i = wave; i < items; i += WAVES) pack(i / NT, i % NT);
     }
     __syncthreads();
     constexpr int KR = KS > 0 ? KS : 1;
@@ -379,8 +401,9 @@ __global__ __launch_bounds__(threads_of(KS), resident_of(KS) * threads_of(KS) / 
 struct Plan {
     Params p;
     int ks;            // kernel variant: 2, 4 or 7 steps of weights in registers, 0: weights in LDS
+    int nt;            // and MFMA tiles of channels per workgroup
     int lds_bytes;
-    int grid;          // workgroups per 64 output channels
+    int grid;          // workgroups per block of output channels
 };
 
 inline size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }
@@ -415,12 +438,18 @@ inline bool make_plan(Plan& plan, int batch, int H, int W, int IC, int OC, int k
     const long long pairs = (kW + 1) / 2, chunks = kH * pairs, steps = (chunks + 3) / 4;
     if (steps > MAX_STEPS || (long long)batch * OH * OW > 0x7fffffffLL) return false;
     const int ks = steps <= 2 ? 2 : steps <= 4 ? 4 : steps <= 7 ? 7 : 0, waves = threads_of(ks) / 64, per_wave = ks ? 1 : 4;
-    const size_t raw = align16((size_t)OC_BLOCK * kH * kW * IC * 2), packed = (size_t)steps * STEP_BYTES;
     const int oc_blocks = (OC + OC_BLOCK - 1) / OC_BLOCK;
     if (oc_blocks > 65535) return false;
     // input pixels under the output, borders included, per output pixel and channel block
     const double staged = ((double)(OH - 1) * stride + kH) * ((double)(OW - 1) * stride + kW) / ((double)OH * OW) * oc_blocks;
     if (!is_faster((long long)batch * OH * OW, staged, IC, OC, (int)steps)) return false;
+    // 96 channels per workgroup where one then holds all of a pixel and there are many: written by two, its 64 and 32 channels
+    // are not whole 128-byte lines, and the input is staged twice.  us per launch at 64 / 96, three channels -> 96: 4 x 224 x 224
+    // 3x3 16.2 / 11.2, 32 x 224 x 224 5x5 stride 2 25.7 / 21.2; 77k pixels 8.4 / 8.3, 900 - 23k pixels 5.0 / 5.8, 5.8 / 6.3; with
+    // seven steps (one workgroup per CU, for the registers) 28.5 / 28.2 at 307k pixels, 9.9 / 10.7 at 30k
+    const int nt = IC == 3 && ks > 0 && ks <= 4 && OC > 64 && OC <= 96 && (long long)batch * OH * OW >= (1 << 17) ? 6 : 4;
+    const int nt_blocks = (OC + 16 * nt - 1) / (16 * nt);
+    const size_t raw = align16((size_t)16 * nt * kH * kW * IC * 2), packed = (size_t)steps * step_bytes(nt);
     double best = 0.0;
     Params& p = plan.p;
     // candidates: this runs on every call, so a few of them (a search over all rows took longer than the small layers).
@@ -442,17 +471,17 @@ inline bool make_plan(Plan& plan, int batch, int H, int W, int IC, int OC, int k
                                      : (long long)align16((size_t)(patch > (long long)raw ? patch : (long long)raw)) + (long long)packed;
             if (lds > LDS_MAX) break;
             int resident = (int)(LDS_MAX / lds);
-            if (resident > resident_of(ks)) resident = resident_of(ks);
+            if (resident > resident_of(ks, nt)) resident = resident_of(ks, nt);
             const long long blocks = (long long)batch * ((OH + rows - 1) / rows) * col_blocks;
             if (blocks > 0x7fffffffLL) continue;
-            const long long slots = 256LL * resident, wgs = blocks * oc_blocks;
+            const long long slots = 256LL * resident, wgs = blocks * nt_blocks;
             const long long rounds = (wgs + slots - 1) / slots, grid = (blocks + rounds - 1) / rounds;
             // cycles: the weights once per workgroup, then per block its patch and its MFMAs, which the workgroups of a
             // compute unit share
-            const long long sharing = (grid * oc_blocks + 255) / 256;
+            const long long sharing = (grid * nt_blocks + 255) / 256;
             const double per_block = (double)patch / 20.0 + 500.0;
             const long long tile_rounds = (((long long)rows * cols + 15) / 16 + waves * per_wave - 1) / (waves * per_wave) * per_wave;
-            const double multiply = (double)tile_rounds * (waves / 4) * (double)steps * NT * 22.0;
+            const double multiply = (double)tile_rounds * (waves / 4) * (double)steps * nt * 22.0;
             const double t = 300.0 * (double)steps + (double)rounds * (per_block + (double)sharing * multiply);
             if (best == 0.0 || t < best) {
                 best = t;
@@ -483,16 +512,17 @@ inline bool make_plan(Plan& plan, int batch, int H, int W, int IC, int OC, int k
     p.by_pairs = helix_fastdiv::make((int)pairs);
     p.by_units = helix_fastdiv::make(units);
     plan.ks = ks;
+    plan.nt = nt;
     return true;
 }
 
-template <int KS>
+template <int KS, int NT>
 inline int launch_steps(const Plan& plan, hipStream_t s) {
-    static int rc = (int)hipFuncSetAttribute((const void*)helix_conv_thin_f16_kernel<KS>,
+    static int rc = (int)hipFuncSetAttribute((const void*)helix_conv_thin_f16_kernel<KS, NT>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     if (rc) return rc;
-    const dim3 grid((unsigned)plan.grid, (unsigned)((plan.p.OC + OC_BLOCK - 1) / OC_BLOCK), 1);
-    hipLaunchKernelGGL(helix_conv_thin_f16_kernel<KS>, grid, dim3(threads_of(KS)), plan.lds_bytes, s, plan.p);
+    const dim3 grid((unsigned)plan.grid, (unsigned)((plan.p.OC + 16 * NT - 1) / (16 * NT)), 1);
+    hipLaunchKernelGGL((helix_conv_thin_f16_kernel<KS, NT>), grid, dim3(threads_of(KS)), plan.lds_bytes, s, plan.p);
     return (int)hipGetLastError();
 }
 
@@ -501,11 +531,13 @@ inline int launch(Plan& plan, const void* x, const void* w, void* y, hipStream_t
     plan.p.x = (const _Float16*)x;
     plan.p.w = (const _Float16*)w;
     plan.p.y = (_Float16*)y;
-    switch (plan.ks) {
-        case 2: return launch_steps<2>(plan, s);
-        case 4: return launch_steps<4>(plan, s);
-        case 7: return launch_steps<7>(plan, s);
-        default: return launch_steps<0>(plan, s);
+    switch (plan.ks * 8 + plan.nt) {
+        case 2 * 8 + 4: return launch_steps<2, 4>(plan, s);
+        case 2 * 8 + 6: return launch_steps<2, 6>(plan, s);
+        case 4 * 8 + 4: return launch_steps<4, 4>(plan, s);
+        case 4 * 8 + 6: return launch_steps<4, 6>(plan, s);
+        case 7 * 8 + 4: return launch_steps<7, 4>(plan, s);
+        default: return launch_steps<0, 4>(plan, s);
     }
 }
 

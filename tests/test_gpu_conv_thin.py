@@ -70,3 +70,10 @@ def test_last_half_of_an_odd_input(layer):
     assert want.max() > 0
     got = run_conv(load(b16.kernel_library("gemm", 2, 64, 64, 32, 32, 64)), x, w, stride, pad, torch.float16)
     assert np.array_equal(got.astype(np.float32), want)
+
+
+@pytest.mark.parametrize("layer", [(3, 3, 210, 211, 72, 3, 3, 1, 1), (2, 3, 257, 257, 96, 5, 5, 1, 2), (9, 3, 242, 243, 65, 4, 4, 2, 2),
+                                   (3, 3, 210, 208, 97, 3, 3, 1, 1)], ids=lambda l: "x".join(map(str, l)))
+def test_many_pixels_of_up_to_96_channels(layer):
+    """96 channels per workgroup from 131072 pixels on (2 and 4 steps), the edges of its channel range and one beyond it."""
+    test_thin_convolution_integer_exact(layer)
