@@ -14,8 +14,8 @@ import os
 
 from utils.helix_runtime import load, kernel_resources, tuned_config, fastest_of
 from utils.conv_patch import PatchFamily, PATCH_TOP
-from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, is_dtl_key, patch_key, patch_keys, PATCH_POINTS
-from MI355X_FP16.MI355X_FP16_gemm import short_value, config_cost, VERIFY_TOP
+from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, is_dtl_key, patch_key, PATCH_KEYS, PATCH_POINTS, RING_KEYS
+from MI355X_FP16.MI355X_FP16_gemm import short_value, config_cost, ring_ranked, VERIFY_TOP
 
 root_path = os.getcwd()
 
@@ -170,10 +170,10 @@ def ranked_configs(prof_dict, M, N, K, IC=None, top=VERIFY_TOP, pointwise=False)
     return [k for _, k in cand[:top]]
 
 
-def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP):
-    """The fastest of the cost model's first `top` configurations on this layer and the first few of the family whose input
-    stays in LDS (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again); for a layer that runs in the kernel for thin inputs the model's first
-    one without K partitions."""
+def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP, families=True):
+    """The fastest of the cost model's first `top` configurations, and with `families` of the unprofiled ones' first, on this layer
+    (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again); for a layer that runs in the kernel for thin
+    inputs the model's first one without K partitions."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     ICg = gather_channels(input_channel)
     if runs_thin(batch, input_channel, H, W, output_channel, kH, kW, stride, pad):
@@ -189,8 +189,17 @@ def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, k
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return fastest_of(ranked_configs(prof_dict, M, output_channel, ICg * kH * kW, ICg, top,
                                      is_pointwise(kH, kW, stride, pad) and input_channel % GATHER_CHUNK == 0)
-                      + patch_ranked(layer, min(top, PATCH_TOP)),
+                      + (unprofiled_ranked(*layer) if families else []),
                       time_config, "this layer")
+
+
+def unprofiled_ranked(batch, input_channel, H, W, output_channel, kH, kW, stride, pad):
+    """The keys of the families without a profile that are timed beside the cost model's candidates: the layers whose input stays
+    in LDS and, for a plain product, the ring tiles."""
+    keys = patch_ranked((batch, input_channel, H, W, output_channel, kH, kW, stride, pad))
+    if is_pointwise(kH, kW, stride, pad) and input_channel % GATHER_CHUNK == 0:
+        keys += ring_ranked(batch * H * W, output_channel, input_channel)
+    return keys
 
 
 def get_MI355X_FP16_conv_Verified_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
@@ -199,7 +208,7 @@ def get_MI355X_FP16_conv_Verified_result(prof_dict, batch, input_channel, H, W, 
     again with the runner's launch counts.  Returns (cost_ms, tflops, key)."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     flops = 2.0 * M * output_channel * input_channel * kH * kW
-    best = verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top)
+    best = verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top, families=False)
     _, cost, _ = load(library_for_key(best)).bench_conv(batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
                                                         warmup=10, iters=10)
     return cost * 1e3, flops / 1e12 / cost, best
@@ -220,7 +229,7 @@ def select_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW,
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return tuned_config("MI355X_FP16", ("conv",) + layer, prof_dict,
                         lambda: layer_cost_model(prof_dict, *layer),
-                        lambda: verified_config(prof_dict, *layer), patch_keys())
+                        lambda: verified_config(prof_dict, *layer), PATCH_KEYS + RING_KEYS)
 
 
 def get_MI355X_FP16_conv_Helix_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
@@ -245,7 +254,7 @@ def get_MI355X_FP16_conv_Oracle_result(prof_dict, batch, input_channel, H, W, ou
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     flops = 2.0 * M * output_channel * input_channel * kH * kW
     min_cost, best = float("inf"), None
-    for k in list(prof_dict.keys()) + list(patch_keys()):
+    for k in list(prof_dict.keys()) + list(PATCH_KEYS + RING_KEYS):
         if k[0] == 0 or is_dtl_key(k):
             continue
         try:

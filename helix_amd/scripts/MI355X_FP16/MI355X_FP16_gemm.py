@@ -9,7 +9,7 @@ import os
 
 from utils.helix_runtime import load, tuned_config, fastest_of
 from utils.roofline import NUM_CU, HBM_BYTES_PER_S, gemm_bytes
-from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, SPLITK_MAX
+from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, SPLITK_MAX, RING_KEYS
 from MI355X_FP16.profile_MI355X_FP16 import PROFILE_K, PROFILE_K_SHORT
 
 root_path = os.getcwd()
@@ -150,6 +150,42 @@ def ranked_configs(prof_dict, M, N, K, top=VERIFY_TOP):
     return [k for k, _ in ranked[:top]]
 
 
+# ---- the family of four-wave tiles over a ring of LDS stages (src_template/MI355X_FP16/gemm_ring.hip) --------------------
+# It has no profile.  Clocks at 2.4 GHz, fitted to 2239 measured (problem, configuration) pairs, 21 % rms; what decides is the
+# order: the fastest of the first four by this model and of the profiled candidates is 0.15 % behind the fastest of all in the
+# geometric mean over 62 problems, 5.6 % at worst.
+RING_TOP = 4
+RING_FIXED_CLOCKS = 3990           # launch, first copies
+RING_STEP_CLOCKS = 32 * 1.84       # the products of a 32 x 32 piece of a workgroup's tile in one K tile of 64
+RING_FEED_BYTES_PER_CLOCK = 31     # L2 into LDS, per compute unit
+RING_STORE_CLOCKS = 476            # the results of a 32 x 32 piece
+RING_BYTES_PER_S = 4.4e12          # operands once and results once
+RING_LDS_BYTES = 160 * 1024
+
+
+def ring_seconds(key, M, N, K):
+    """Predicted seconds of a configuration of that family."""
+    stages, rows, cols = key[:3]
+    tiles = math.ceil(M / rows) * math.ceil(N / cols)
+    pieces, copied = rows * cols // 1024, (rows + cols) * 128
+    by_registers = 4 if pieces <= 8 else 3 if pieces <= 12 else 2 if pieces <= 24 else 1
+    resident = max(1, min(RING_LDS_BYTES // (stages * copied), by_registers))
+
+    def round_clocks(share):       # workgroups of one round on a compute unit
+        step = max(pieces * RING_STEP_CLOCKS, copied / RING_FEED_BYTES_PER_CLOCK)
+        return share * (math.ceil(K / 64) * step + RING_STORE_CLOCKS * pieces)
+
+    rounds = math.ceil(tiles / (NUM_CU * resident))
+    last = tiles - (rounds - 1) * NUM_CU * resident
+    clocks = RING_FIXED_CLOCKS + (rounds - 1) * round_clocks(resident) + round_clocks(min(resident, math.ceil(last / NUM_CU)))
+    return max(clocks / 2.4e9, gemm_bytes(M, N, K, 2) / RING_BYTES_PER_S + 2.5e-6)
+
+
+def ring_ranked(M, N, K, top=RING_TOP):
+    """The `top` configurations of that family with the lowest predicted time, best first."""
+    return sorted(RING_KEYS, key=lambda k: (ring_seconds(k, M, N, K), k))[:top]
+
+
 def padded_k(K):
     """The FP16 kernels load 16-byte chunks along K; a K that is not a multiple of 8 halves is run on
     buffers whose rows are zero-padded to the next multiple (zeros add nothing to the dot products)."""
@@ -185,11 +221,11 @@ def weight_copies(N, K):
     return math.ceil(CACHE_BYTES / weights) if weights >= COLD_WEIGHT_BYTES else 1
 
 
-def verified_config(prof_dict, M, N, K, top=VERIFY_TOP):
-    """The fastest of the cost model's first `top` configurations on this problem (utils.helix_runtime.fastest_of:
-    2 + 5 launches each, the leaders timed again).  Where the copies of the weights do not fit the device beside the
-    problem, one does."""
-    keys = ranked_configs(prof_dict, M, N, K, top)
+def verified_config(prof_dict, M, N, K, top=VERIFY_TOP, families=True):
+    """The fastest of the cost model's first `top` configurations, and with `families` of the ring tiles' first, on this problem
+    (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again).  Where the copies of the weights do not fit
+    the device beside the problem, one does."""
+    keys = ranked_configs(prof_dict, M, N, K, top) + (ring_ranked(M, N, K) if families else [])
 
     def fastest(copies):
         return fastest_of(keys, lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters, copies=copies),
@@ -205,11 +241,11 @@ def verified_config(prof_dict, M, N, K, top=VERIFY_TOP):
 
 
 def select_config(prof_dict, M, N, K):
-    """The configuration the runner launches: the cost model's ranking, settled on the device the first time a
-    problem is met and remembered beside the profile (utils.helix_runtime.tuned_config); the cost model's first
+    """The configuration the runner launches: the cost model's ranking and the ring family's, settled on the device the first time
+    a problem is met and remembered beside the profile (utils.helix_runtime.tuned_config); the cost model's first
     choice alone with HELIX_SELECTION=model."""
     return tuned_config("MI355X_FP16", ("gemm", M, N, K), prof_dict, lambda: cost_model(prof_dict, M, N, K),
-                        lambda: verified_config(prof_dict, M, N, K))
+                        lambda: verified_config(prof_dict, M, N, K), RING_KEYS)
 
 
 def get_MI355X_FP16_gemm_Helix_result(prof_dict, M, N, K, backend="hip"):
@@ -234,7 +270,7 @@ def get_MI355X_FP16_gemm_rocblas_result(M, N, K):
 def get_MI355X_FP16_gemm_Verified_result(prof_dict, M, N, K, top=VERIFY_TOP):
     """The fastest of the cost model's first `top` configurations: each timed briefly, the winner timed again with
     the runner's launch counts.  Returns (cost_ms, tflops, key)."""
-    best = verified_config(prof_dict, M, N, K, top)
+    best = verified_config(prof_dict, M, N, K, top, families=False)
     cost = run_config(best, M, N, K)
     return cost * 1e3, 2 * M * N * K / 1e12 / cost, best
 
@@ -243,7 +279,7 @@ def get_MI355X_FP16_gemm_Oracle_result(prof_dict, M, N, K):
     """Exhaustive per-shape search: run every candidate, keep the fastest
     (benchmark_Ampere_FP16_performance_comparison.py:56-69).  Returns (cost_ms, tflops, key)."""
     min_cost, best = float("inf"), None
-    for k in prof_dict.keys():
+    for k in list(prof_dict.keys()) + list(RING_KEYS):
         if k[0] == 0 and min(M, N) > 16:
             continue   # the weight-streaming kernel re-reads the weights per 16 activation rows
         try:

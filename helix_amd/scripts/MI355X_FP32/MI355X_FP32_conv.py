@@ -7,7 +7,7 @@ import os
 
 from utils.helix_runtime import load, tuned_config, fastest_of
 from utils.conv_patch import PatchFamily, PATCH_TOP
-from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, patch_key, patch_keys, PATCH_POINTS
+from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, patch_key, PATCH_KEYS, PATCH_POINTS
 from MI355X_FP32.MI355X_FP32_gemm import config_cost, extra_points, VERIFY_TOP
 
 root_path = os.getcwd()
@@ -62,9 +62,9 @@ def patch_ranked(layer, top=PATCH_TOP):
     return [patch_key(point) for point in PATCH.ranked(layer, top)]
 
 
-def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP):
-    """The fastest of the cost model's first `top` configurations on this layer and the first few of the family whose input
-    stays in LDS (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again)."""
+def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP, families=True):
+    """The fastest of the cost model's first `top` configurations, and with `families` of the input-in-LDS ones' first, on this layer
+    (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again)."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
 
     def time_config(k, warmup, iters):
@@ -73,7 +73,7 @@ def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, k
 
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return fastest_of(ranked_configs(prof_dict, M, output_channel, gather_channels(input_channel) * kH * kW, top)
-                      + patch_ranked(layer, min(top, PATCH_TOP)), time_config, "this layer")
+                      + (patch_ranked(layer) if families else []), time_config, "this layer")
 
 
 def get_MI355X_FP32_conv_Verified_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
@@ -82,7 +82,7 @@ def get_MI355X_FP32_conv_Verified_result(prof_dict, batch, input_channel, H, W, 
     again with the runner's launch counts.  Returns (cost_ms, tflops, key)."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     flops = 2.0 * M * output_channel * input_channel * kH * kW
-    best = verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top)
+    best = verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top, families=False)
     _, cost, _ = load(library_for_key(best)).bench_conv(batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
                                                         warmup=10, iters=10)
     return cost * 1e3, flops / 1e12 / cost, best
@@ -101,7 +101,7 @@ def select_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW,
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return tuned_config("MI355X_FP32", ("conv",) + layer, prof_dict,
                         lambda: layer_cost_model(prof_dict, *layer),
-                        lambda: verified_config(prof_dict, *layer), patch_keys())
+                        lambda: verified_config(prof_dict, *layer), PATCH_KEYS)
 
 
 def get_MI355X_FP32_conv_Helix_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,

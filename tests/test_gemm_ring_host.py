@@ -1,0 +1,58 @@
+"""Ranking and selection of the four-wave tiles over a ring of LDS stages (MI355X_FP16/gemm_ring.hip), which have no profile."""
+from utils import helix_runtime
+from MI355X_FP16 import build_MI355X_FP16 as b16
+from MI355X_FP16 import profile_MI355X_FP16 as p16
+from MI355X_FP16 import MI355X_FP16_conv as c16
+from MI355X_FP16 import MI355X_FP16_gemm as g16
+
+
+def test_points_fit_the_template():
+    assert len(set(b16.RING_KEYS)) == len(b16.RING_POINTS) == 22 and not set(b16.RING_KEYS) & set(p16.all_keys())
+    for rows, cols, stages in b16.RING_POINTS:
+        assert rows % 32 == cols % 32 == 0 and 32 <= rows <= 256 and 32 <= cols <= 256
+        assert stages * (rows + cols) * 128 <= 160 * 1024 and (stages - 1) * (rows + cols) // 32 <= 63
+        assert 4 * 16 * (cols + 16) <= stages * (rows + cols) * 128            # the strips that the results pass through
+    key = b16.ring_key((224, 160, 3))
+    assert key == (3, 224, 160, 112, 80, 0, 64, 3) and b16.is_ring_key(key) and not b16.is_dtl_key(key) and not b16.is_patch_key(key)
+    assert b16.library_for_key(key).endswith("build/bin_fp16/libgemm_ring_3_224_160.so")
+    assert b16.ring_job(key)[2] == {"K_STAGES": 3, "BLOCK_ROWS": 224, "BLOCK_COLS": 160}
+
+
+def test_ranking_follows_the_rounds():
+    """661 rows in three tiles of 224, and 207 tiles in one round of 256; few rows take small tiles."""
+    assert b16.ring_key((224, 160, 3)) in g16.ring_ranked(661, 11008, 4096, 2)
+    assert all(k[1] <= 64 for k in g16.ring_ranked(19, 1032, 952, 2))
+    assert len(g16.ring_ranked(300, 8192, 4096)) == g16.RING_TOP
+    assert g16.ring_seconds(b16.ring_key((64, 64, 3)), 8192, 8192, 8192) > g16.ring_seconds(b16.ring_key((256, 128, 3)), 8192, 8192, 8192)
+
+
+def test_selection_times_the_family_and_keeps_its_winner(tmp_path, monkeypatch):
+    """For products and for pointwise layers; other layers are not offered to it."""
+    monkeypatch.setattr(helix_runtime, "root_path", str(tmp_path))
+    prof = {(2, 64, 64, 32, 32, 0, 64): 1e-5, (2, 128, 64, 64, 32, 0, 64): 2e-5}
+    timed = []
+
+    def run_config(k, M, N, K, **kw):
+        timed.append(k)
+        return 1e-6 if b16.is_ring_key(k) else 2e-6
+
+    monkeypatch.setattr(g16, "run_config", run_config)
+    key = g16.select_config(prof, 661, 1100, 4096)
+    assert b16.is_ring_key(key) and set(prof) < set(timed) and len(set(timed)) == len(prof) + g16.RING_TOP
+    timed.clear()
+    assert g16.select_config(prof, 661, 1100, 4096) == key and not timed
+    monkeypatch.setenv("HELIX_SELECTION", "model")
+    assert g16.select_config(prof, 661, 1100, 4096) in prof
+    monkeypatch.delenv("HELIX_SELECTION")
+
+    class Library:
+        def __init__(self, path):
+            self.path = path
+
+        def bench_conv(self, *a, **kw):
+            return 0.0, 1e-6 if "gemm_ring" in self.path else 2e-6, 0.0
+
+    monkeypatch.setattr(c16, "load", Library)
+    assert b16.is_ring_key(c16.select_config(prof, 4, 64, 14, 14, 96, 1, 1, 1, 0))
+    assert not b16.is_ring_key(c16.select_config(prof, 4, 64, 14, 14, 96, 3, 3, 1, 1))
+    assert not b16.is_ring_key(c16.select_config(prof, 4, 25, 14, 14, 96, 1, 1, 1, 0))
