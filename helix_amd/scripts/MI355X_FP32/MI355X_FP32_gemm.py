@@ -7,7 +7,7 @@ import os
 from utils.helix_runtime import load, tuned_config, fastest_of
 from utils.hip_ctypes import STATIC_SCRATCH_BYTES
 from utils.roofline import NUM_CU, HBM_BYTES_PER_S, gemm_bytes
-from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library
+from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, RING_KEYS
 from MI355X_FP32.profile_MI355X_FP32 import PROFILE_K, PROFILE_K_SHORT, GEMV_PROFILE_K
 
 root_path = os.getcwd()
@@ -195,6 +195,41 @@ def ranked_configs(prof_dict, M, N, K, top=VERIFY_TOP):
     return [k for k, _ in ranked[:top]]
 
 
+# ---- the family of four-wave tiles over a ring of LDS stages (src_template/MI355X_FP32/gemm_ring.hip) --------------------
+# It has no profile.  Clocks at 2.4 GHz, fitted to 768 measured (problem, configuration) pairs, 13 % rms; what decides is the
+# order: the fastest of the first four by this model and of sgemm.hip's configurations is 0.2 % behind the fastest of all in the
+# geometric mean over 48 problems, 4.3 % at worst.
+RING_TOP = 4
+RING_FIXED_CLOCKS = 5100           # launch, and per round of workgroups: first copies, last stores
+RING_ROUND_CLOCKS = 5000
+RING_STEP_CLOCKS = 128 * 1.127     # the products of a 32 x 32 piece of a workgroup's tile in 16 columns of K
+RING_WAIT_CLOCKS = 76              # what 16 columns take beside them where a compute unit holds one workgroup
+RING_STORE_CLOCKS = 83             # the results of a 32 x 32 piece
+RING_BYTES_PER_S = 3.8e12          # operands once and results once
+RING_LDS_BYTES = 160 * 1024
+
+
+def ring_seconds(key, M, N, K):
+    """Predicted seconds of a configuration of that family."""
+    rows, cols = key[:2]
+    pieces, halves = rows * cols // 1024, math.ceil(K / 16)
+    resident = min(8, RING_LDS_BYTES // ((rows + cols) * 256))
+    per_cu = math.ceil(math.ceil(M / rows) * math.ceil(N / cols) / NUM_CU)
+
+    def round_clocks(share):       # workgroups of one round on a compute unit
+        step = max(share * pieces * RING_STEP_CLOCKS, RING_WAIT_CLOCKS + pieces * RING_STEP_CLOCKS)
+        return halves * step + share * pieces * RING_STORE_CLOCKS + RING_ROUND_CLOCKS
+
+    rounds = (per_cu - 1) // resident
+    clocks = RING_FIXED_CLOCKS + rounds * round_clocks(resident) + round_clocks(per_cu - rounds * resident)
+    return max(clocks / 2.4e9, gemm_bytes(M, N, K, 4) / RING_BYTES_PER_S + 2.5e-6)
+
+
+def ring_ranked(M, N, K, top=RING_TOP):
+    """The `top` configurations of that family with the lowest predicted time, best first."""
+    return sorted(RING_KEYS, key=lambda k: (ring_seconds(k, M, N, K), k))[:top]
+
+
 def run_config(k, M, N, K, warmup=10, iters=10, outer=1):
     """Seconds per launch (mean) on the real M, N, K (edges are predicated in the kernel; the reference
     pads M and N up to the tile instead, Ampere_FP32_gemm.py:103)."""
@@ -207,19 +242,19 @@ def run_config(k, M, N, K, warmup=10, iters=10, outer=1):
     return avg
 
 
-def verified_config(prof_dict, M, N, K, top=VERIFY_TOP):
-    """The fastest of the cost model's first `top` configurations on this problem (utils.helix_runtime.fastest_of:
-    2 + 5 launches each, the leaders timed again)."""
-    return fastest_of(ranked_configs(prof_dict, M, N, K, top),
+def verified_config(prof_dict, M, N, K, top=VERIFY_TOP, families=True):
+    """The fastest of the cost model's first `top` configurations, and with `families` of the ring tiles' first, on this problem
+    (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again)."""
+    return fastest_of(ranked_configs(prof_dict, M, N, K, top) + (ring_ranked(M, N, K) if families else []),
                       lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters), f"{M}x{N}x{K}")
 
 
 def select_config(prof_dict, M, N, K):
-    """The configuration the runner launches: the cost model's ranking, settled on the device the first time a
-    problem is met and remembered beside the profile (utils.helix_runtime.tuned_config); the cost model's first
+    """The configuration the runner launches: the cost model's ranking and the ring family's, settled on the device the first time
+    a problem is met and remembered beside the profile (utils.helix_runtime.tuned_config); the cost model's first
     choice alone with HELIX_SELECTION=model."""
     return tuned_config("MI355X_FP32", ("gemm", M, N, K), prof_dict, lambda: cost_model(prof_dict, M, N, K),
-                        lambda: verified_config(prof_dict, M, N, K))
+                        lambda: verified_config(prof_dict, M, N, K), RING_KEYS)
 
 
 def get_MI355X_FP32_gemm_Helix_result(prof_dict, M, N, K, backend="hip"):
@@ -244,7 +279,7 @@ def get_MI355X_FP32_gemm_rocblas_result(M, N, K):
 def get_MI355X_FP32_gemm_Verified_result(prof_dict, M, N, K, top=VERIFY_TOP):
     """The fastest of the cost model's first `top` configurations: each timed briefly, the winner timed again with
     the runner's launch counts.  Returns (cost_ms, tflops, key)."""
-    best = verified_config(prof_dict, M, N, K, top)
+    best = verified_config(prof_dict, M, N, K, top, families=False)
     cost = run_config(best, M, N, K)
     return cost * 1e3, 2 * M * N * K / 1e12 / cost, best
 
@@ -252,7 +287,7 @@ def get_MI355X_FP32_gemm_Verified_result(prof_dict, M, N, K, top=VERIFY_TOP):
 def get_MI355X_FP32_gemm_Oracle_result(prof_dict, M, N, K):
     """Exhaustive per-shape search.  Returns (cost_ms, tflops, key)."""
     min_cost, best = float("inf"), None
-    for k in prof_dict.keys():
+    for k in list(prof_dict.keys()) + list(RING_KEYS):
         if k[2] == 0 and min(M, N) > 16:
             continue
         try:

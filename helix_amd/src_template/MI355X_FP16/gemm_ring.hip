@@ -31,6 +31,7 @@
 #include <stdio.h>
 
 #include "helix_abi.h"
+#include "helix_ring.h"
 
 #ifndef BLOCK_ROWS
 #define BLOCK_ROWS 224
@@ -44,13 +45,13 @@
 
 namespace {
 
+using namespace helix_ring;
+
 typedef _Float16 half_t;
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef int intx4 __attribute__((ext_vector_type(4)));
 typedef int intx2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) unsigned char* lds_ptr_t;
 
 constexpr int BM = BLOCK_ROWS, BN = BLOCK_COLS, TM = BM / 32, TN = BN / 32, NM = TM * TN, STAGES = K_STAGES, BK = 64;
 constexpr int NTHREADS = 256, ROW_BYTES = BK * 2;
@@ -58,8 +59,6 @@ constexpr int A_BYTES = BM * ROW_BYTES, STAGE_BYTES = (BM + BN) * ROW_BYTES;
 constexpr int COPIES = TM + TN;                     // 1 KiB copies of a wave per K tile
 constexpr int STRIP_LD = 32 * TN + 16, STRIP_BYTES = 16 * STRIP_LD;     // results: 16 rows of a wave's columns, rows padded by 16 bytes
 constexpr int LDS_BYTES = STAGES * STAGE_BYTES;
-constexpr int GROUP_ROWS = 4, NUM_XCD = 8;
-constexpr int OOB_OFFSET = 0x7fffffff;              // byte offset beyond any buffer: zeros
 
 static_assert(BM % 32 == 0 && BN % 32 == 0 && TM >= 1 && TN >= 1 && TM <= 8 && TN <= 8, "wave tiles of 16 x 16 .. 128 x 128");
 static_assert(STAGES >= 2 && (STAGES - 1) * COPIES <= 63, "copies in flight are counted in a 6-bit counter");
@@ -72,28 +71,6 @@ struct Params {
     int M, N, K, lda, ldb, ldc, tiles_m, tiles_n;
 };
 
-// 128-bit buffer descriptor as four dwords: base address (48 bits), stride 0, byte count, raw-buffer flags
-__device__ __forceinline__ intx4 raw_rsrc(const void* base, unsigned bytes) {
-    const unsigned long long a = (unsigned long long)base;
-    return intx4{(int)(unsigned)a, (int)((a >> 32) & 0xffffu), (int)bytes, 0x00020000};
-}
-
-// One 16-byte-per-lane copy into LDS: lane l's data lands at LDS byte lds_addr + 16 l (wave-uniform, through M0), zeros where its
-// offset is beyond the buffer.  From inline assembly, so that the compiler neither orders LDS reads behind it nor counts it in
-// its own waits: completion is waited for by hand, in front of the barrier that publishes it.
-__device__ __forceinline__ void copy16(intx4 rsrc, unsigned lds_addr, int offset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(offset), "s"(rsrc)
-                 : "memory", "m0");
-}
-
-// s_waitcnt vmcnt(COPIES_LEFT), and lgkmcnt(0) where LDS_TOO
-template <int COPIES_LEFT, bool LDS_TOO>
-__device__ __forceinline__ void wait() {
-    __builtin_amdgcn_s_waitcnt((COPIES_LEFT & 15) | (7 << 4) | ((LDS_TOO ? 0 : 15) << 8) | ((COPIES_LEFT >> 4) << 14));
-}
-
 // (the tile parameters are template arguments for the symbol name's sake: a profiler lists configurations separately)
 template <int T_STAGES = STAGES, int T_BM = BM, int T_BN = BN>
 __global__ __launch_bounds__(NTHREADS, 1) void helix_gemm_f16_ring_kernel(const Params p) {
@@ -102,13 +79,9 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_gemm_f16_ring_kernel(const 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_m = wave >> 1, wave_n = wave & 1, r = lane & 15, q = lane >> 4;
 
-    // ids are dealt round-robin to the 8 XCDs: each is given a compact run of tiles, walked in column-major groups of rows
-    const int ntiles = p.tiles_m * p.tiles_n, per_xcd = (ntiles + NUM_XCD - 1) / NUM_XCD;
-    const int slot = (int)(blockIdx.x / NUM_XCD), pid = (int)(blockIdx.x % NUM_XCD) * per_xcd + slot;
-    if (slot >= per_xcd || pid >= ntiles) return;
-    const int group_tiles = GROUP_ROWS * p.tiles_n, first_m = pid / group_tiles * GROUP_ROWS, in_group = pid % group_tiles;
-    const int rows_of_group = (p.tiles_m - first_m) < GROUP_ROWS ? (p.tiles_m - first_m) : GROUP_ROWS;
-    const int m0 = (first_m + in_group % rows_of_group) * BM, n0 = in_group / rows_of_group * BN;
+    int tm, tn;
+    if (!tile_of((int)blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn)) return;
+    const int m0 = tm * BM, n0 = tn * BN;
 
     // ---- copies: piece d of a wave is 8 LDS rows; row r holds its 16-byte chunk c at c ^ (r / 2 mod 8) ------------------
     const int rows_a = (p.M - m0) < BM ? (p.M - m0) : BM, rows_b = (p.N - n0) < BN ? (p.N - n0) : BN;
@@ -185,11 +158,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_gemm_f16_ring_kernel(const 
             __builtin_amdgcn_sched_barrier(0);
         }
         // this wave is done reading tile t, and its copies of tile t + 1 have landed; behind the barrier that holds for all
-        wait<(STAGES - 2) * COPIES, true>();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
+        wait_and_meet<(STAGES - 2) * COPIES>();
 #pragma unroll
         for (int g = 0; g < NM; g++) {
             multiply(g, 1);

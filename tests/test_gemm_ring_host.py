@@ -1,9 +1,13 @@
-"""Ranking and selection of the four-wave tiles over a ring of LDS stages (MI355X_FP16/gemm_ring.hip), which have no profile."""
+"""Ranking and selection of the four-wave tiles over a ring of LDS stages (MI355X_FP16/gemm_ring.hip, MI355X_FP32/gemm_ring.hip),
+which have no profile."""
 from utils import helix_runtime
 from MI355X_FP16 import build_MI355X_FP16 as b16
 from MI355X_FP16 import profile_MI355X_FP16 as p16
 from MI355X_FP16 import MI355X_FP16_conv as c16
 from MI355X_FP16 import MI355X_FP16_gemm as g16
+from MI355X_FP32 import build_MI355X_FP32 as b32
+from MI355X_FP32 import profile_MI355X_FP32 as p32
+from MI355X_FP32 import MI355X_FP32_gemm as g32
 
 
 def test_points_fit_the_template():
@@ -56,3 +60,25 @@ def test_selection_times_the_family_and_keeps_its_winner(tmp_path, monkeypatch):
     assert b16.is_ring_key(c16.select_config(prof, 4, 64, 14, 14, 96, 1, 1, 1, 0))
     assert not b16.is_ring_key(c16.select_config(prof, 4, 64, 14, 14, 96, 3, 3, 1, 1))
     assert not b16.is_ring_key(c16.select_config(prof, 4, 25, 14, 14, 96, 1, 1, 1, 0))
+
+
+def test_fp32_family(tmp_path, monkeypatch):
+    """The same of the FP32 family, which has two stages and takes products only."""
+    assert len(set(b32.RING_KEYS)) == len(b32.RING_POINTS) == 16 and not set(b32.RING_KEYS) & set(p32.all_keys())
+    for rows, cols in b32.RING_POINTS:
+        assert rows % 32 == cols % 32 == 0 and 32 <= rows <= 256 and 32 <= cols <= 256 and (rows + cols) * 256 <= 160 * 1024
+    key = b32.ring_key((96, 160))
+    assert key == (96, 160, 32, 48, 80, 2, 1, 0) and b32.is_ring_key(key) and not b32.is_patch_key(key)
+    assert b32.library_for_key(key).endswith("build/bin_fp32/libgemm_ring_96_160.so")
+    assert b32.ring_job(key)[2] == {"BLOCK_ROWS": 96, "BLOCK_COLS": 160}
+    assert b32.ring_key((64, 64)) in g32.ring_ranked(4000, 2300, 770)
+    assert g32.ring_ranked(196, 512, 256, 1) == [b32.ring_key((32, 32))]
+    monkeypatch.setattr(helix_runtime, "root_path", str(tmp_path))
+    prof = {b32.config_key(64, 64, 16, 32, 32): 1.0, b32.config_key(128, 64, 16, 32, 32): 1.7}
+    timed = []
+    monkeypatch.setattr(g32, "run_config", lambda k, M, N, K, **kw: timed.append(k) or (1e-6 if b32.is_ring_key(k) else 2e-6))
+    key = g32.select_config(prof, 661, 1100, 4096)
+    assert b32.is_ring_key(key) and set(prof) < set(timed) and len(set(timed)) == len(prof) + g32.RING_TOP
+    timed.clear()
+    assert g32.select_config(prof, 661, 1100, 4096) == key and not timed
+    assert g32.verified_config(prof, 661, 1100, 4096, families=False) in prof
