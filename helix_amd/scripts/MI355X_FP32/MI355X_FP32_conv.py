@@ -7,8 +7,8 @@ import os
 
 from utils.helix_runtime import load, tuned_config, fastest_of
 from utils.conv_patch import PatchFamily, PATCH_TOP
-from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, patch_key, PATCH_KEYS, PATCH_POINTS
-from MI355X_FP32.MI355X_FP32_gemm import config_cost, extra_points, VERIFY_TOP
+from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, patch_key, PATCH_KEYS, PATCH_POINTS, RING_KEYS
+from MI355X_FP32.MI355X_FP32_gemm import config_cost, extra_points, ring_first, RING_CONV, RING_CONV_TOP, VERIFY_TOP
 
 root_path = os.getcwd()
 
@@ -62,8 +62,20 @@ def patch_ranked(layer, top=PATCH_TOP):
     return [patch_key(point) for point in PATCH.ranked(layer, top)]
 
 
+RING_MAX_TAPS = 31      # of the ring tiles' convolution (src_template/MI355X_FP32/gemm_ring.hip): a bit of a row's mask each
+
+
+def ring_ranked(layer, top=RING_CONV_TOP):
+    """The keys of the ring tiles' first `top` configurations for a layer, none where they do not take it."""
+    batch, IC, H, W, OC, kH, kW, stride, pad = layer
+    if IC % GATHER_CHUNK or kH * kW > RING_MAX_TAPS:
+        return []
+    M, K = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1), IC * kH * kW
+    return ring_first(M, OC, K, 4 * (batch * IC * H * W + OC * K + M * OC), RING_CONV, top)
+
+
 def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP, families=True):
-    """The fastest of the cost model's first `top` configurations, and with `families` of the input-in-LDS ones' first, on this layer
+    """The fastest of the cost model's first `top` configurations, and with `families` of the unprofiled ones' first, on this layer
     (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again)."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
 
@@ -73,7 +85,7 @@ def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, k
 
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return fastest_of(ranked_configs(prof_dict, M, output_channel, gather_channels(input_channel) * kH * kW, top)
-                      + (patch_ranked(layer) if families else []), time_config, "this layer")
+                      + (patch_ranked(layer) + ring_ranked(layer) if families else []), time_config, "this layer")
 
 
 def get_MI355X_FP32_conv_Verified_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
@@ -101,7 +113,7 @@ def select_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW,
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return tuned_config("MI355X_FP32", ("conv",) + layer, prof_dict,
                         lambda: layer_cost_model(prof_dict, *layer),
-                        lambda: verified_config(prof_dict, *layer), PATCH_KEYS)
+                        lambda: verified_config(prof_dict, *layer), PATCH_KEYS + RING_KEYS)
 
 
 def get_MI355X_FP32_conv_Helix_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,

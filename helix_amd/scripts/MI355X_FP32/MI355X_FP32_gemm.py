@@ -196,38 +196,42 @@ def ranked_configs(prof_dict, M, N, K, top=VERIFY_TOP):
 
 
 # ---- the family of four-wave tiles over a ring of LDS stages (src_template/MI355X_FP32/gemm_ring.hip) --------------------
-# It has no profile.  Clocks at 2.4 GHz, fitted to 768 measured (problem, configuration) pairs, 13 % rms; what decides is the
-# order: the fastest of the first four by this model and of sgemm.hip's configurations is 0.2 % behind the fastest of all in the
-# geometric mean over 48 problems, 4.3 % at worst.
-RING_TOP = 4
-RING_FIXED_CLOCKS = 5100           # launch, and per round of workgroups: first copies, last stores
-RING_ROUND_CLOCKS = 5000
-RING_STEP_CLOCKS = 128 * 1.127     # the products of a 32 x 32 piece of a workgroup's tile in 16 columns of K
-RING_WAIT_CLOCKS = 76              # what 16 columns take beside them where a compute unit holds one workgroup
-RING_STORE_CLOCKS = 83             # the results of a 32 x 32 piece
-RING_BYTES_PER_S = 3.8e12          # operands once and results once
+# It has no profile.  Clocks at 2.4 GHz: launch; per round of workgroups (first copies, last stores); the products of a 32 x 32
+# piece of a workgroup's tile in 16 columns of K, and what they take beside them where a compute unit holds one workgroup; the
+# results of such a piece; operands once and results once, bytes per second.  Fitted to 864 and 792 measured (problem,
+# configuration) pairs, 18 % and 11 % rms; what decides is the order: the fastest of the first five by this model and of the older
+# templates' configurations is 0.2 % behind the fastest of all in the geometric mean over 48 products (5.5 % at worst), that of the
+# first four 0 % over 44 convolutions.
+RING_TOP, RING_CONV_TOP = 5, 4
+RING_GEMM = (4300, 5650, 128 * 1.13, 82, 35, 4.7e12)
+RING_CONV = (9700, 2200, 128 * 1.23, 93, 137, 6.5e12)
 RING_LDS_BYTES = 160 * 1024
 
 
-def ring_seconds(key, M, N, K):
-    """Predicted seconds of a configuration of that family."""
+def ring_seconds(key, M, N, K, moved, constants):
+    """Predicted seconds of a configuration of that family on a problem that moves `moved` bytes."""
+    fixed, per_round, step_clocks, wait_clocks, store_clocks, rate = constants
     rows, cols = key[:2]
-    pieces, halves = rows * cols // 1024, math.ceil(K / 16)
+    pieces, halves = rows * cols / 1024, math.ceil(K / 16)
     resident = min(8, RING_LDS_BYTES // ((rows + cols) * 256))
     per_cu = math.ceil(math.ceil(M / rows) * math.ceil(N / cols) / NUM_CU)
 
     def round_clocks(share):       # workgroups of one round on a compute unit
-        step = max(share * pieces * RING_STEP_CLOCKS, RING_WAIT_CLOCKS + pieces * RING_STEP_CLOCKS)
-        return halves * step + share * pieces * RING_STORE_CLOCKS + RING_ROUND_CLOCKS
+        step = max(share * pieces * step_clocks, wait_clocks + pieces * step_clocks)
+        return halves * step + share * pieces * store_clocks + per_round
 
     rounds = (per_cu - 1) // resident
-    clocks = RING_FIXED_CLOCKS + rounds * round_clocks(resident) + round_clocks(per_cu - rounds * resident)
-    return max(clocks / 2.4e9, gemm_bytes(M, N, K, 4) / RING_BYTES_PER_S + 2.5e-6)
+    clocks = fixed + rounds * round_clocks(resident) + round_clocks(per_cu - rounds * resident)
+    return max(clocks / 2.4e9, moved / rate + 2.5e-6)
+
+
+def ring_first(M, N, K, moved, constants, top):
+    """The `top` configurations of that family with the lowest predicted time, best first."""
+    return sorted(RING_KEYS, key=lambda k: (ring_seconds(k, M, N, K, moved, constants), k))[:top]
 
 
 def ring_ranked(M, N, K, top=RING_TOP):
-    """The `top` configurations of that family with the lowest predicted time, best first."""
-    return sorted(RING_KEYS, key=lambda k: (ring_seconds(k, M, N, K), k))[:top]
+    return ring_first(M, N, K, gemm_bytes(M, N, K, 4), RING_GEMM, top)
 
 
 def run_config(k, M, N, K, warmup=10, iters=10, outer=1):

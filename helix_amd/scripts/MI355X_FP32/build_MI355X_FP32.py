@@ -108,17 +108,18 @@ def is_patch_key(key):
     return key[2] != 0 and key[5] == 0
 
 
-# Four-wave tiles over a ring of direct-to-LDS stages (src_template/MI355X_FP32/gemm_ring.hip): (BLOCK_ROWS, BLOCK_COLS) points.  121
-# of them, with two and three stages, were timed on 48 problems: all of them bring the fastest of both templates to 0.9537 of the
-# fastest sgemm.hip configuration in the geometric mean, these to 0.954 (the first fourteen picked greedily, then the larger
-# squares' favourites); three stages add nothing but where K partitions are faster.
-RING_POINTS = [(32, 32), (32, 64), (64, 32), (32, 96), (96, 32), (32, 128), (128, 32), (32, 160), (160, 32), (224, 32), (64, 64),
-               (128, 64), (64, 256), (96, 160), (160, 96), (128, 128)]
+# Four-wave tiles over a ring of direct-to-LDS stages (src_template/MI355X_FP32/gemm_ring.hip): (BLOCK_ROWS, BLOCK_COLS, WAVES_M)
+# points.  68 of them were timed on 48 products and 44 convolutions; picked greedily, these bring the fastest of all templates to
+# 0.925 of the fastest configuration of the older ones in the geometric mean, where all of them would bring it to 0.924.  Three
+# stages add nothing but where K partitions are faster.
+RING_POINTS = [(16, 64, 1), (32, 32, 2), (32, 64, 2), (32, 96, 2), (32, 128, 1), (64, 16, 4), (64, 48, 4), (64, 64, 2), (64, 80, 4),
+               (64, 96, 2), (64, 112, 4), (64, 128, 4), (64, 256, 1), (96, 32, 2), (96, 64, 2), (96, 160, 2), (128, 64, 4), (160, 32, 2)]
 
 
 def ring_key(point):
     """Key of a point of that family: (BLOCK_ROWS, BLOCK_COLS, 32, WAVE_ROWS, WAVE_COLS, 2, 1, 0); no copy passes a register."""
-    return (point[0], point[1], 32, point[0] // 2, point[1] // 2, 2, 1, 0)
+    rows, cols, waves_m = point
+    return (rows, cols, 32, rows // waves_m, cols * waves_m // 4, 2, 1, 0)
 
 
 RING_KEYS = tuple(ring_key(point) for point in RING_POINTS)
@@ -151,7 +152,7 @@ def library_for_key(key):
     if is_patch_key(key):
         return kernel_library("conv_patch_" + "_".join(str(key[i]) for i in (0, 1, 3, 4, 6)))
     if is_ring_key(key):
-        return kernel_library(f"gemm_ring_{key[0]}_{key[1]}")
+        return kernel_library(f"gemm_ring_{key[0]}_{key[1]}_{key[3]}_{key[4]}")
     return sgemm_library(key[0], key[1], key[2], key[3], key[4], key[6])
 
 
@@ -181,7 +182,8 @@ def patch_job(key):
 
 
 def ring_job(key):
-    return (f"{SRC_ROOT}/MI355X_FP32/gemm_ring.hip", library_for_key(key), {"BLOCK_ROWS": key[0], "BLOCK_COLS": key[1]})
+    return (f"{SRC_ROOT}/MI355X_FP32/gemm_ring.hip", library_for_key(key), 
+            {"BLOCK_ROWS": key[0], "BLOCK_COLS": key[1], "WAVES_M": key[0] // key[3]})
 
 
 def build_jobs():

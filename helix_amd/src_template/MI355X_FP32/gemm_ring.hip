@@ -1,6 +1,7 @@
-// MI355X (gfx950 / CDNA4) FP32 GEMM template: four waves, K tiles copied straight into a ring of LDS stages.
+// MI355X (gfx950 / CDNA4) FP32 GEMM and implicit-GEMM convolution template: four waves, K tiles copied straight into a ring of LDS stages.
 //
 //   C[M x N] = A^T * B with A stored K x M and B stored K x N (row-major FP32): operands and result as in sgemm.hip.
+//   y[B,OH,OW,OC] = conv2d(x[B,H,W,IC], w[OC,kH,kW,IC]), IC a multiple of 4, at most 31 taps.
 //
 // Role in the reference: src_template/Ampere_FP32/sgemm.cu:97-350, whose cp.async stages this is the counterpart of.
 //
@@ -12,18 +13,21 @@
 //     a lane reads four consecutive rows of a k in 16 bytes, one for each of four tiles, and holds four consecutive columns of a result
 //     row in return, which it stores in 16 bytes, a quarter wave 256 bytes together.  The loop for a 96 x 96 wave tile: 288 products,
 //     32 LDS reads, 12 copies, 3 waits, one barrier per 32 columns of K;
-//   * tiles are any multiple of 32 x 32, and the last half K tile is left out where it is empty (K = 770: 784 columns of work).
-// Two stages do (a K tile of the smallest workgroup takes 1000 clocks), which leaves room for up to eight workgroups on a CU: one's
+//   * the four waves lie 2 x 2, or in a row or column, which gives tiles 16 rows or columns apart: 48 and 80 columns for products
+//     and layers of few; and the last half K tile is left out where it is empty (K = 770: 784 columns of work).
+// Two stages do (the products of a K tile take 256 clocks a wave at the least), which leaves room for up to eight workgroups on a CU: one's
 // stores and first copies lie behind another's products.
-// Sums: ascending k, one FMA chain per result, as sgemm.hip's unpartitioned launches; the same bits in every configuration over
-// 300 x 520 x 100, 1000 x 770 x 777 and 513 x 257 x 16.
+// Sums: ascending k, a chain of FMAs per 256 of K, added in order: up to there the bits of an unpartitioned sgemm.hip launch,
+// beyond it less than half of its error (4000 x 2300 x 770, 8134 x 451 x 5225: 5.0e-7 and 13e-7 in the norm there, 3.5e-7 and 9.2e-7 with
+// two K groups); per 128 it is 2.1e-7 and 2.4e-7, and costs 2 - 4 % of the time.
 // Measured, us per launch, the fastest of sgemm.hip's configurations / of these: 4000 x 2300 x 770 120.7 / 107.2 (64 x 64 tiles; 94 are
 // the products at the peak rate), 2048^3 129.9 / 121.4, 4096^3 946 / 925, 661 x 11008 x 1024 128.8 / 116.5, 512 x 3072 x 768 25.7 / 22.6,
-// 8134 x 451 x 5225 326 / 293, 283256 x 72 x 331 196 / 168, 3325 x 1824 x 328 37.5 / 33.1, 196 x 512 x 256 5.4 / 4.6.  Behind where
-// tiles are few and K is long (29 x 1000 x 11976 18.8 / 105): K groups and partitions stay sgemm.hip's, as do convolutions.
+// 8134 x 451 x 5225 326 / 290, 283256 x 72 x 331 196 / 130 (64 x 80 tiles; 168 with the waves 2 x 2), 361104 x 36 x 196 87 / 75 (64 x
+// 48; 92), 3325 x 1824 x 328 37.5 / 33.3, 196 x 512 x 256 5.4 / 4.6; 0.928 in the geometric mean over 48 problems.  Behind where
+// tiles are few and K is long (29 x 1000 x 11976 18.8 / 105): K groups and partitions stay sgemm.hip's.
 //
 // Compile-time parameters (-D, one shared library per combination):
-//   BLOCK_ROWS x BLOCK_COLS   workgroup tile, multiples of 32; a wave's is half of it in both directions
+//   BLOCK_ROWS x BLOCK_COLS   workgroup tile, of WAVES_M x 4 / WAVES_M waves, whole 16 x 16 tiles each
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -31,6 +35,7 @@
 #include <utility>
 
 #include "helix_abi.h"
+#include "helix_fastdiv.h"
 #include "helix_ring.h"
 
 #ifndef BLOCK_ROWS
@@ -38,6 +43,9 @@
 #endif
 #ifndef BLOCK_COLS
 #define BLOCK_COLS 192
+#endif
+#ifndef WAVES_M
+#define WAVES_M 2
 #endif
 
 namespace {
@@ -47,13 +55,25 @@ using namespace helix_ring;
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int BM = BLOCK_ROWS, BN = BLOCK_COLS, TM = BM / 32, TN = BN / 32, NM = TM * TN, STAGES = 2, BK = 32;
+constexpr int BM = BLOCK_ROWS, BN = BLOCK_COLS, WM = WAVES_M, WN = 4 / WM, TM = BM / WM / 16, TN = BN / WN / 16, NM = TM * TN, STAGES = 2, BK = 32;
 constexpr int NTHREADS = 256, STEPS = BK / 8;       // k steps of four in half a K tile
-constexpr int A_BYTES = BM * BK * 4, STAGE_BYTES = (BM + BN) * BK * 4, LDS_BYTES = STAGES * STAGE_BYTES;
-constexpr int COPIES = TM + TN;                     // 1 KiB copies of a wave per K tile
+constexpr int BLOCK_TILES = 8;                      // K tiles whose products are one chain of sums
+constexpr int A_BYTES = BM * BK * 4, STAGE_BYTES = (BM + BN) * BK * 4, RING_BYTES = STAGES * STAGE_BYTES;
+// 1 KiB copies of a K tile, dealt out to the waves, A's from wave 0 on, B's from wave 2 on.  Where a count is no multiple of four
+// the waves it leaves out copy zeros to a place behind the ring: a branch among the products costs more
+constexpr int PIECES_A = BM / 8, PIECES_B = BN / 8, CA = (PIECES_A + 3) / 4, CB = (PIECES_B + 3) / 4, COPIES = CA + CB;
+constexpr bool EVEN = PIECES_A % 4 == 0 && PIECES_B % 4 == 0;
+constexpr int LDS_BYTES = RING_BYTES + (EVEN ? 0 : 1024);
+__device__ __forceinline__ int piece_of(int d, int wave) { return d < CA ? d * 4 + wave : (d - CA) * 4 + (wave ^ 2); }
+__device__ __forceinline__ bool has_piece(int d, int wave) { return EVEN || piece_of(d, wave) < (d < CA ? PIECES_A : PIECES_B); }
+// LDS offset of a wave's piece
+__device__ __forceinline__ int place_of(int d, int wave, int stage) {
+    return has_piece(d, wave) ? stage * STAGE_BYTES + (d < CA ? 0 : A_BYTES) + piece_of(d, wave) * 1024 : RING_BYTES;
+}
 
-static_assert(BM % 32 == 0 && BN % 32 == 0 && TM >= 1 && TN >= 1 && TM <= 8 && TN <= 8, "wave tiles of 16 x 16 .. 128 x 128");
-static_assert((STAGES - 1) * COPIES <= 63, "copies in flight are counted in a 6-bit counter");
+static_assert((WM == 1 || WM == 2 || WM == 4) && BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "whole 16 x 16 tiles in every wave");
+static_assert(TM >= 1 && TN >= 1 && TM <= 8 && TN <= 8, "wave tiles of 16 x 16 .. 128 x 128");
+static_assert(STAGES == 2 && COPIES <= 63, "the wait in a tile's middle is for every copy; a 6-bit counter");
 static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 
 // A wave's T tiles of 16 rows (or columns) lie in groups of 4, 2 and 1: lane r of a group of W holds its W r .. W r + W - 1, in one
@@ -81,6 +101,20 @@ __device__ __forceinline__ void each(F&& f) {
     each<N>(f, std::make_integer_sequence<int, N>{});
 }
 
+__device__ __forceinline__ void clear(floatx4 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+}
+
+__device__ __forceinline__ void add(floatx4 (&sum)[TM][TN], const floatx4 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) sum[i][j] += acc[i][j];
+}
+
 template <int W>
 __device__ __forceinline__ void load(const unsigned char* from, float* to) {
     if (W == 4) {
@@ -100,7 +134,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave_m = wave >> 1, wave_n = wave & 1, r = lane & 15, q = lane >> 4;
+    const int wave_m = wave / WN, wave_n = wave % WN, r = lane & 15, q = lane >> 4;
     int tm, tn;
     if (!tile_of((int)blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn)) return;
     const int m0 = tm * BM, n0 = tn * BN;
@@ -111,9 +145,9 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
     int from[COPIES];
 #pragma unroll
     for (int d = 0; d < COPIES; d++) {
-        const int T = d < TM ? BM : BN, chunk = (d < TM ? wave * TM + d : wave * TN + d - TM) * 64 + lane;
+        const int T = d < CA ? BM : BN, chunk = piece_of(d, wave) * 64 + lane;
         const int row = chunk / (T / 4), col = chunk % (T / 4) * 4;
-        from[d] = (d < TM ? m0 : n0) + col < (d < TM ? p.M : p.N) ? (row * (d < TM ? p.lda : p.ldb) + col) * 4 : OOB_OFFSET;
+        from[d] = has_piece(d, wave) && (d < CA ? m0 : n0) + col < (d < CA ? p.M : p.N) ? (row * (d < CA ? p.lda : p.ldb) + col) * 4 : OOB_OFFSET;
     }
     const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)smem;
     const int ktiles = (p.K + BK - 1) / BK;
@@ -123,8 +157,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
         return raw_rsrc(base + (size_t)k0 * ld + first, t < ktiles ? (unsigned)(((size_t)(p.K - k0) * ld - first) * 4) : 0u);
     };
     auto copy = [&](int d, int stage, const intx4& ra, const intx4& rb) {
-        const int piece = d < TM ? wave * TM + d : wave * TN + d - TM;
-        copy16(d < TM ? ra : rb, lds0 + (unsigned)(stage * STAGE_BYTES + (d < TM ? 0 : A_BYTES) + piece * 1024), from[d]);
+        copy16(d < CA ? ra : rb, lds0 + (unsigned)place_of(d, wave, stage), from[d]);
     };
 #pragma unroll
     for (int u = 0; u < STAGES; u++) {
@@ -139,11 +172,9 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
     for (int g = 0; g < GA; g++) at_a[g] = (q * BM + (wave_m * TM + group_first(TM, g)) * 16 + group_width(TM, g) * r) * 4;
 #pragma unroll
     for (int g = 0; g < GB; g++) at_b[g] = A_BYTES + (q * BN + (wave_n * TN + group_first(TN, g)) * 16 + group_width(TN, g) * r) * 4;
-    floatx4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 acc[TM][TN], sum[TM][TN];                // of this block of K, of the blocks before it
+    clear(acc);
+    clear(sum);
     float fa[2][STEPS][TM], fb[2][STEPS][TN];
     constexpr int READS = STEPS * (GA + GB);
     auto read = [&](int e, int h, int stage) {       // step by step, in the order in which the products take them
@@ -171,35 +202,43 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
     // fragment reads that are out after g products: they end two thirds into a half
     auto due = [](int g, int reads) constexpr -> int { return 3 * g >= 2 * PRODUCTS ? reads : 3 * g * reads / (2 * PRODUCTS); };
 
-    wait<(STAGES - 1) * COPIES, false>();
+    wait<COPIES, false>();                  // the first stage is there
     __syncthreads();
     each<READS>([&](auto e) __attribute__((always_inline)) { read(e, 0, 0); });
     int stage = 0;
     // (whole tiles, and half a one behind the loop where no more is left: a way out in the middle of the loop had the compiler copy
     // every accumulator twice a tile)
     const int halves = (p.K + BK / 2 - 1) / (BK / 2);
-    for (int t = 0; t < halves / 2; t++) {
-        const int next = stage + 1 == STAGES ? 0 : stage + 1;
-        const intx4 ra = rsrc_of(p.A, p.lda, m0, t + STAGES), rb = rsrc_of(p.B, p.ldb, n0, t + STAGES);
-        each<PRODUCTS>([&](auto g) __attribute__((always_inline)) {
-            multiply(g, 0);
+    for (int t = 0, end; t < halves / 2; t = end) {
+        end = t + BLOCK_TILES < halves / 2 ? t + BLOCK_TILES : halves / 2;
+        for (int u = t; u < end; u++) {
+            const int next = stage + 1 == STAGES ? 0 : stage + 1;
+            const intx4 ra = rsrc_of(p.A, p.lda, m0, u + STAGES), rb = rsrc_of(p.B, p.ldb, n0, u + STAGES);
+            each<PRODUCTS>([&](auto g) __attribute__((always_inline)) {
+                multiply(g, 0);
 #pragma unroll
-            for (int e = due(g, READS); e < due(g + 1, READS); e++) read(e, 1, stage);
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        // this wave is done reading tile t, and its copies of tile t + 1 have landed; behind the barrier that holds for all
-        wait_and_meet<(STAGES - 2) * COPIES>();
-        each<PRODUCTS>([&](auto g) __attribute__((always_inline)) {
-            multiply(g, 1);
+                for (int e = due(g, READS); e < due(g + 1, READS); e++) read(e, 1, stage);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            // this wave is done reading tile t, and its copies of tile t + 1 have landed; behind the barrier that holds for all
+            wait_and_meet<0>();
+            each<PRODUCTS>([&](auto g) __attribute__((always_inline)) {
+                multiply(g, 1);
 #pragma unroll
-            for (int e = due(g, READS); e < due(g + 1, READS); e++) read(e, 0, next);   // (past the last tile: zeros, not used)
+                for (int e = due(g, READS); e < due(g + 1, READS); e++) read(e, 0, next);   // (past the last tile: zeros, not used)
 #pragma unroll
-            for (int d = g * COPIES / PRODUCTS; d < (g + 1) * COPIES / PRODUCTS; d++) copy(d, stage, ra, rb);
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        stage = next;
+                for (int d = g * COPIES / PRODUCTS; d < (g + 1) * COPIES / PRODUCTS; d++) copy(d, stage, ra, rb);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            stage = next;
+        }
+        if (end < halves / 2) {
+            add(sum, acc);
+            clear(acc);
+        }
     }
     if (halves & 1) each<PRODUCTS>([&](auto g) __attribute__((always_inline)) { multiply(g, 0); });
+    add(sum, acc);
     wait<0, true>();                                 // no copy is left when the workgroup gives its LDS back
 
     // ---- results: lanes 0 .. 15 of a quarter hold a piece of a row, 256, 128 or 64 bytes long -----------------------------
@@ -218,17 +257,202 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
                 const int col = n0 + (wave_n * TN + j) * 16 + w * r;
                 float* dst = p.C + (size_t)row * p.ldc + col;
                 if (w == 4 && vec == 4 && col + 4 <= p.N) {
-                    __builtin_nontemporal_store(floatx4{acc[i][j][v], acc[i][j + w / 4][v], acc[i][j + w / 2][v], acc[i][j + w - 1][v]},
+                    __builtin_nontemporal_store(floatx4{sum[i][j][v], sum[i][j + w / 4][v], sum[i][j + w / 2][v], sum[i][j + w - 1][v]},
                                                 (floatx4*)dst);
                 } else if (w >= 2 && vec >= 2 && col + w <= p.N) {
 #pragma unroll
                     for (int e = 0; e < w; e += 2)
-                        __builtin_nontemporal_store(floatx2{acc[i][j + e][v], acc[i][j + e + 1][v]}, (floatx2*)(dst + e));
+                        __builtin_nontemporal_store(floatx2{sum[i][j + e][v], sum[i][j + e + 1][v]}, (floatx2*)(dst + e));
                 } else {
 #pragma unroll
                     for (int e = 0; e < w; e++)
-                        if (col + e < p.N) dst[e] = acc[i][j + e][v];
+                        if (col + e < p.N) dst[e] = sum[i][j + e][v];
                 }
+            }
+        }
+    }
+}
+
+// ---- convolutions --------------------------------------------------------------------------------------------------------
+// The implicit GEMM: rows are pixels, columns filters, K the taps' channels, which are contiguous in both operands and stay so in
+// LDS: 32 k of a row in 128 bytes, its 16-byte chunk c at c ^ (row / 2 mod 8), so that a lane reads four k of a row at once, which
+// are the operands of four products.  A copy's lane knows where the first tap of its pixel lies and which taps are inside the
+// image (a bit each); a tile adds the tap's offset, one for all lanes where channels come in 32s, five instructions a copy.
+// Measured, us per launch, the fastest configuration of sgemm.hip and conv_patch.hip / of this (batch x channels x image, filter):
+//   1x1  3 x 256 x 63 x 63 -> 96 12.6 / 9.9    3 x 128 x 49 x 49 -> 192 9.2 / 7.5     2 x 96 x 75 x 75 -> 384 15.5 / 12.6
+//        41 x 128 x 45 x 45 -> 128 32.8 / 28.0  51 x 832 x 15 x 15 -> 160 37.7 / 32.1  45 x 128 x 56 x 56 -> 48 28.8 / 22.3
+//   3x3  11 x 192 x 37 x 37 -> 208 110.6 / 97.8     32 x 256 x 14 x 14 -> 256 83.4 / 72.8    12 x 256 x 27 x 27 -> 160 72.6 / 63.1
+//        7 x 96 x 85 x 85 -> 48 57.3 / 46.3          16 x 128 x 49 x 49 -> 64 57.4 / 51.8
+//   5x5  8 x 16 x 60 x 60 -> 160 44.7 / 39.7        31 x 16 x 109 x 109 -> 48 163 / 126
+// Behind, as in products, where tiles are few and K is long (1 x 256 x 14 x 14 3x3 7.8 / 20.5).  0.922 in the geometric
+// mean over 44 layers.
+
+using helix_fastdiv::FastDiv;
+
+struct ConvParams {
+    const float* x;    // NHWC
+    const float* w;    // [OC][kH][kW][IC]
+    float* y;          // M x N
+    int M, N, K, tiles_m, tiles_n;
+    int H, W, IC, kH, kW, stride, pad;
+    unsigned x_bytes;
+    FastDiv by_OW, by_OH, by_IC, by_kW;
+};
+constexpr int NO_TAP = 31;                          // a bit that no row's mask has
+
+// WHOLE: channels are a multiple of 32, so that a K tile lies in one tap
+template <bool WHOLE, int T_BM = BM, int T_BN = BN>
+__global__ __launch_bounds__(NTHREADS, 1) void helix_conv_f32_ring_kernel(const ConvParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_m = wave / WN, wave_n = wave % WN, r = lane & 15, q = lane >> 4;
+    int tm, tn;
+    if (!tile_of((int)blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn)) return;
+    const int m0 = tm * BM, n0 = tn * BN;
+
+    // ---- copies: piece d of a wave is 8 LDS rows.  Of a pixel: where its first tap lies, and which taps are inside the image ----
+    const int rows_b = (p.N - n0) < BN ? (p.N - n0) : BN;
+    // (a wave's pieces are all even or all odd, so that a lane has one chunk of every row)
+    const int chunk = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
+    int first[CA];
+    unsigned inside[CA];
+#pragma unroll
+    for (int d = 0; d < CA; d++) {
+        const int m = m0 + piece_of(d, wave) * 8 + (lane >> 3);
+        const int t = p.by_OW.div(m), ow = m - t * p.by_OW.d, b = p.by_OH.div(t), oh = t - b * p.by_OH.d;
+        const int ih = oh * p.stride - p.pad, iw = ow * p.stride - p.pad;
+        first[d] = (int)((((unsigned)b * p.H + ih) * p.W + iw) * (unsigned)p.IC * 4u) + (WHOLE ? chunk * 16 : 0);
+        const int left = iw < 0 ? -iw : 0, right = p.W - iw < p.kW ? p.W - iw : p.kW;
+        const unsigned of_row = right > left ? (1u << right) - (1u << left) : 0u;
+        unsigned mask = 0;
+        for (int kh = 0; kh < p.kH; kh++) mask |= (unsigned)(ih + kh) < (unsigned)p.H ? of_row << (kh * p.kW) : 0u;
+        inside[d] = has_piece(d, wave) && m < p.M ? mask : 0u;
+    }
+    int of_b[CB];
+#pragma unroll
+    for (int d = 0; d < CB; d++) {
+        const int row = piece_of(CA + d, wave) * 8 + (lane >> 3);
+        of_b[d] = has_piece(CA + d, wave) && row < rows_b ? row * p.K * 4 + chunk * 16 : OOB_OFFSET;
+    }
+    const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)smem;
+    const int ktiles = (p.K + BK - 1) / BK;
+    const float* base_b = p.w + (size_t)n0 * p.K;
+    const unsigned bytes_b = (unsigned)rows_b * (unsigned)p.K * 4u;
+    const intx4 rx = raw_rsrc(p.x, p.x_bytes);
+    // tap and byte offset behind a row's first tap, of the tile that is copied next: one for all lanes, or by the lane's chunk
+    int tap = 0, offset = 0, kw = 0, c = 0;
+    intx4 rw;
+    auto aim = [&](int t) {
+        rw = raw_rsrc(base_b + (size_t)(t < ktiles ? t : 0) * BK, t < ktiles ? bytes_b - (unsigned)t * (BK * 4u) : 0u);
+        if (WHOLE) return;
+        const int k = t * BK + chunk * 4, at = p.by_IC.div(k), row = p.by_kW.div(at);
+        tap = k < p.K ? at : NO_TAP;
+        offset = ((row * p.W + at - row * p.kW) * p.IC + k - at * p.IC) * 4;
+    };
+    auto step = [&]() {                              // WHOLE: to the next tile
+        c += BK;
+        offset += BK * 4;
+        if (c == p.IC) {
+            c = 0;
+            tap = tap < NO_TAP ? tap + 1 : NO_TAP;
+            if (++kw == p.kW) {
+                kw = 0;
+                offset += (p.W - p.kW) * p.IC * 4;
+            }
+        }
+    };
+    auto copy = [&](int d, int stage) {
+        const unsigned to = lds0 + (unsigned)place_of(d, wave, stage);
+        if (d < CA) copy16(rx, to, (inside[d] >> tap) & 1 ? first[d] + offset : OOB_OFFSET);
+        else copy16(rw, to, !WHOLE && tap == NO_TAP ? OOB_OFFSET : of_b[d - CA]);
+    };
+#pragma unroll
+    for (int u = 0; u < STAGES; u++) {
+        aim(u);
+#pragma unroll
+        for (int d = 0; d < COPIES; d++) copy(d, u);
+        if (WHOLE) step();
+    }
+
+    // ---- fragments: lane (r, q) supplies row r, chunk 4 h + q of half h ------------------------------------------------
+    int at_a[2], at_b[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int chunk = ((h * 4 + q) ^ (r >> 1)) << 4;
+        at_a[h] = (wave_m * TM * 16 + r) * BK * 4 + chunk;
+        at_b[h] = A_BYTES + (wave_n * TN * 16 + r) * BK * 4 + chunk;
+    }
+    floatx4 acc[TM][TN], sum[TM][TN];                // of this block of K, of the blocks before it
+    clear(acc);
+    clear(sum);
+    floatx4 fa[2][TM], fb[2][TN];
+    constexpr int READS = TM + TN, PRODUCTS = 4 * NM;
+    auto read = [&](int e, int h, int stage) {
+        const unsigned char* from = smem + stage * STAGE_BYTES;
+        if (e < TM) fa[h][e] = *(const floatx4*)(from + at_a[h] + e * 16 * BK * 4);
+        else fb[h][e - TM] = *(const floatx4*)(from + at_b[h] + (e - TM) * 16 * BK * 4);
+    };
+    // the filters go first, which leaves a lane with four consecutive columns of one row
+    auto multiply = [&](int g, int h) {
+        const int e = g / NM, i = g % NM % TM, j = g % NM / TM;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[h][j][e], fa[h][i][e], acc[i][j], 0, 0, 0);
+    };
+    auto due = [](int g, int reads) constexpr -> int { return 3 * g >= 2 * PRODUCTS ? reads : 3 * g * reads / (2 * PRODUCTS); };
+
+    wait<COPIES, false>();                  // the first stage is there
+    __syncthreads();
+    each<READS>([&](auto e) __attribute__((always_inline)) { read(e, 0, 0); });
+    int stage = 0;
+    const int halves = (p.K + BK / 2 - 1) / (BK / 2);       // as in the products' loop
+    for (int t = 0, end; t < halves / 2; t = end) {
+        end = t + BLOCK_TILES < halves / 2 ? t + BLOCK_TILES : halves / 2;
+        for (int u = t; u < end; u++) {
+            const int next = stage + 1 == STAGES ? 0 : stage + 1;
+            each<PRODUCTS>([&](auto g) __attribute__((always_inline)) {
+                multiply(g, 0);
+#pragma unroll
+                for (int e = due(g, READS); e < due(g + 1, READS); e++) read(e, 1, stage);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            aim(u + STAGES);
+            wait_and_meet<0>();
+            each<PRODUCTS>([&](auto g) __attribute__((always_inline)) {
+                multiply(g, 1);
+#pragma unroll
+                for (int e = due(g, READS); e < due(g + 1, READS); e++) read(e, 0, next);   // (past the last tile: zeros, not used)
+#pragma unroll
+                for (int d = g * COPIES / PRODUCTS; d < (g + 1) * COPIES / PRODUCTS; d++) copy(d, stage);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if (WHOLE) step();
+            stage = next;
+        }
+        if (end < halves / 2) {
+            add(sum, acc);
+            clear(acc);
+        }
+    }
+    if (halves & 1) each<PRODUCTS>([&](auto g) __attribute__((always_inline)) { multiply(g, 0); });
+    add(sum, acc);
+    wait<0, true>();                                 // no copy is left when the workgroup gives its LDS back
+
+    // ---- results: a quarter's lanes hold 16 bytes of 16 rows ---------------------------------------------------------------
+    const bool wide = (((uintptr_t)p.y >> 2 | (unsigned)p.N) & 3) == 0;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        const int row = m0 + (wave_m * TM + i) * 16 + r;
+        if (row >= p.M) continue;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int col = n0 + (wave_n * TN + j) * 16 + 4 * q;
+            float* dst = p.y + (size_t)row * p.N + col;
+            if (wide && col + 4 <= p.N) {
+                __builtin_nontemporal_store(sum[i][j], (floatx4*)dst);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (col + e < p.N) dst[e] = sum[i][j][e];
             }
         }
     }
@@ -253,8 +477,8 @@ inline const char* info_json() {
                  "\"block_k\": %d, \"k_groups\": 1, \"split_k\": 1, \"direct_to_lds\": 1, \"threads\": %d, \"lds_bytes\": %d, "
                  "\"layout_a\": \"K x M row-major f32\", \"layout_b\": \"K x N row-major f32\", "
                  "\"layout_c\": \"M x N row-major f32\", \"accumulate\": \"f32\", "
-                 "\"k_multiple\": 1, \"ld_multiple\": 4, \"conv\": \"none\"}",
-                 STAGES, BM, BN, BM / 2, BN / 2, BK, NTHREADS, LDS_BYTES);
+                 "\"k_multiple\": 1, \"ld_multiple\": 4, \"conv\": \"NHWC x [OC][kH][kW][IC]; IC a multiple of 4, at most 31 taps\"}",
+                 STAGES, BM, BN, BM / WM, BN / WN, BK, NTHREADS, LDS_BYTES);
         done = true;
     }
     return buf;
@@ -287,8 +511,32 @@ inline int gemm(const void* A, const void* B, void* C, int M, int N, int K, int 
     return (int)hipGetLastError();
 }
 
-inline int conv2d(const void*, const void*, void*, int, int, int, int, int, int, int, int, int, void*, size_t, hipStream_t) {
-    return HELIX_ERR_UNSUPPORTED;
+template <bool WHOLE>
+inline int launch_conv(const ConvParams& p, unsigned grid, hipStream_t s) {
+    static int rc = (int)hipFuncSetAttribute((const void*)helix_conv_f32_ring_kernel<WHOLE>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+    if (rc) return rc;
+    hipLaunchKernelGGL(helix_conv_f32_ring_kernel<WHOLE>, dim3(grid), dim3(NTHREADS), LDS_BYTES, s, p);
+    return (int)hipGetLastError();
+}
+
+inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W, int IC, int OC, int kH, int kW, int stride,
+                  int pad, void*, size_t, hipStream_t s) {
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 3)) return HELIX_ERR_INVALID_VALUE;
+    const int OH = (H + 2 * pad - kH) / stride + 1, OW = (W + 2 * pad - kW) / stride + 1;
+    // a 16-byte chunk lies in one tap, and a row's mask has a bit for each and one to spare
+    if (IC % 4 != 0 || kH > NO_TAP || kW > NO_TAP || kH * kW > NO_TAP) return HELIX_ERR_UNSUPPORTED;
+    const long long M = (long long)batch * OH * OW, K = (long long)kH * kW * IC;
+    const long long xbytes = (long long)batch * H * W * IC * 4;
+    if (M > 0x7fffffffLL - BM || K > 0x7fffffffLL - 4 * BK || xbytes >= 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;
+    if ((long long)BN * K * 4 >= 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;
+    ConvParams p{(const float*)x, (const float*)w, (float*)y, (int)M, OC, (int)K, ((int)M - 1) / BM + 1, (OC - 1) / BN + 1,
+                 H, W, IC, kH, kW, stride, pad, (unsigned)xbytes,
+                 helix_fastdiv::make(OW), helix_fastdiv::make(OH), helix_fastdiv::make(IC), helix_fastdiv::make(kW)};
+    const long long ntiles = (long long)p.tiles_m * p.tiles_n;
+    if (ntiles > 0x3fffffffLL) return HELIX_ERR_INVALID_VALUE;
+    const unsigned grid = (unsigned)((ntiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
+    return IC % BK == 0 ? launch_conv<true>(p, grid, s) : launch_conv<false>(p, grid, s);
 }
 
 }  // namespace tpl

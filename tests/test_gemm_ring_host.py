@@ -7,11 +7,12 @@ from MI355X_FP16 import MI355X_FP16_conv as c16
 from MI355X_FP16 import MI355X_FP16_gemm as g16
 from MI355X_FP32 import build_MI355X_FP32 as b32
 from MI355X_FP32 import profile_MI355X_FP32 as p32
+from MI355X_FP32 import MI355X_FP32_conv as c32
 from MI355X_FP32 import MI355X_FP32_gemm as g32
 
 
 def test_points_fit_the_template():
-    assert len(set(b16.RING_KEYS)) == len(b16.RING_POINTS) == 22 and not set(b16.RING_KEYS) & set(p16.all_keys())
+    assert len(set(b16.RING_KEYS)) == len(b16.RING_POINTS) == 25 and not set(b16.RING_KEYS) & set(p16.all_keys())
     for rows, cols, stages in b16.RING_POINTS:
         assert rows % 32 == cols % 32 == 0 and 32 <= rows <= 256 and 32 <= cols <= 256
         assert stages * (rows + cols) * 128 <= 160 * 1024 and (stages - 1) * (rows + cols) // 32 <= 63
@@ -27,11 +28,12 @@ def test_ranking_follows_the_rounds():
     assert b16.ring_key((224, 160, 3)) in g16.ring_ranked(661, 11008, 4096, 2)
     assert all(k[1] <= 64 for k in g16.ring_ranked(19, 1032, 952, 2))
     assert len(g16.ring_ranked(300, 8192, 4096)) == g16.RING_TOP
-    assert g16.ring_seconds(b16.ring_key((64, 64, 3)), 8192, 8192, 8192) > g16.ring_seconds(b16.ring_key((256, 128, 3)), 8192, 8192, 8192)
+    seconds = lambda point: g16.ring_seconds(b16.ring_key(point), 8192, 8192, 8192, 3 * 8192 ** 2 * 2, g16.RING_GEMM)
+    assert seconds((64, 64, 3)) > seconds((256, 128, 3))
 
 
 def test_selection_times_the_family_and_keeps_its_winner(tmp_path, monkeypatch):
-    """For products and for pointwise layers; other layers are not offered to it."""
+    """For products and for layers of whole chunks of channels; others are not offered to it."""
     monkeypatch.setattr(helix_runtime, "root_path", str(tmp_path))
     prof = {(2, 64, 64, 32, 32, 0, 64): 1e-5, (2, 128, 64, 64, 32, 0, 64): 2e-5}
     timed = []
@@ -58,21 +60,23 @@ def test_selection_times_the_family_and_keeps_its_winner(tmp_path, monkeypatch):
 
     monkeypatch.setattr(c16, "load", Library)
     assert b16.is_ring_key(c16.select_config(prof, 4, 64, 14, 14, 96, 1, 1, 1, 0))
-    assert not b16.is_ring_key(c16.select_config(prof, 4, 64, 14, 14, 96, 3, 3, 1, 1))
+    assert b16.is_ring_key(c16.select_config(prof, 4, 64, 14, 14, 96, 3, 3, 1, 1))
+    assert not b16.is_ring_key(c16.select_config(prof, 4, 64, 14, 14, 96, 4, 8, 1, 1))
     assert not b16.is_ring_key(c16.select_config(prof, 4, 25, 14, 14, 96, 1, 1, 1, 0))
 
 
 def test_fp32_family(tmp_path, monkeypatch):
-    """The same of the FP32 family, which has two stages and takes products only."""
-    assert len(set(b32.RING_KEYS)) == len(b32.RING_POINTS) == 16 and not set(b32.RING_KEYS) & set(p32.all_keys())
-    for rows, cols in b32.RING_POINTS:
-        assert rows % 32 == cols % 32 == 0 and 32 <= rows <= 256 and 32 <= cols <= 256 and (rows + cols) * 256 <= 160 * 1024
-    key = b32.ring_key((96, 160))
-    assert key == (96, 160, 32, 48, 80, 2, 1, 0) and b32.is_ring_key(key) and not b32.is_patch_key(key)
-    assert b32.library_for_key(key).endswith("build/bin_fp32/libgemm_ring_96_160.so")
-    assert b32.ring_job(key)[2] == {"BLOCK_ROWS": 96, "BLOCK_COLS": 160}
-    assert b32.ring_key((64, 64)) in g32.ring_ranked(4000, 2300, 770)
-    assert g32.ring_ranked(196, 512, 256, 1) == [b32.ring_key((32, 32))]
+    """The same of the FP32 family, which has two stages."""
+    assert len(set(b32.RING_KEYS)) == len(b32.RING_POINTS) == 18 and not set(b32.RING_KEYS) & set(p32.all_keys())
+    for rows, cols, waves_m in b32.RING_POINTS:
+        assert waves_m in (1, 2, 4) and rows % (16 * waves_m) == cols % (64 // waves_m) == 0
+        assert rows // waves_m <= 128 and cols * waves_m // 4 <= 128 and (rows + cols) * 256 + 1024 <= 160 * 1024
+    key = b32.ring_key((64, 80, 4))
+    assert key == (64, 80, 32, 16, 80, 2, 1, 0) and b32.is_ring_key(key) and not b32.is_patch_key(key)
+    assert b32.library_for_key(key).endswith("build/bin_fp32/libgemm_ring_64_80_16_80.so")
+    assert b32.ring_job(key)[2] == {"BLOCK_ROWS": 64, "BLOCK_COLS": 80, "WAVES_M": 4}
+    assert b32.ring_key((64, 64, 2)) in g32.ring_ranked(4000, 2300, 770)
+    assert b32.ring_key((64, 80, 4)) in g32.ring_ranked(283256, 72, 331, 1)
     monkeypatch.setattr(helix_runtime, "root_path", str(tmp_path))
     prof = {b32.config_key(64, 64, 16, 32, 32): 1.0, b32.config_key(128, 64, 16, 32, 32): 1.7}
     timed = []
@@ -82,3 +86,15 @@ def test_fp32_family(tmp_path, monkeypatch):
     timed.clear()
     assert g32.select_config(prof, 661, 1100, 4096) == key and not timed
     assert g32.verified_config(prof, 661, 1100, 4096, families=False) in prof
+
+    class Library:
+        def __init__(self, path):
+            self.path = path
+
+        def bench_conv(self, *a, **kw):
+            return 0.0, 1e-6 if "gemm_ring" in self.path else 2e-6, 0.0
+
+    monkeypatch.setattr(c32, "load", Library)
+    assert b32.is_ring_key(c32.select_config(prof, 4, 64, 28, 28, 96, 3, 3, 1, 1))
+    assert not c32.ring_ranked((4, 25, 28, 28, 96, 3, 3, 1, 1)) and not c32.ring_ranked((4, 64, 28, 28, 96, 11, 11, 1, 5))
+    assert len(c32.ring_ranked((4, 4, 28, 28, 96, 5, 6, 1, 0))) == g32.RING_CONV_TOP

@@ -1,4 +1,4 @@
-"""FP32 products on four-wave tiles over a ring of LDS stages (MI355X_FP32/gemm_ring.hip): every configuration at the edges of its
+"""FP32 products and convolutions on four-wave tiles over a ring of LDS stages (MI355X_FP32/gemm_ring.hip): every configuration at the edges of its
 tiles, through the C ABI."""
 import numpy as np
 import pytest
@@ -7,7 +7,8 @@ import torch
 from utils.helix_runtime import load
 from utils.hip_ctypes import HELIX_ERR_INVALID_VALUE, HELIX_ERR_UNSUPPORTED
 from MI355X_FP32 import build_MI355X_FP32 as b32
-from gpu_helpers import dev, run_sgemm_f32
+from oracle import oracle as O
+from gpu_helpers import dev, run_conv, run_sgemm_f32
 
 pytestmark = pytest.mark.gpu
 
@@ -28,13 +29,19 @@ def test_every_configuration_integer_exact(problem):
         assert np.array_equal(got.astype(np.int64), exact), key
 
 
-def test_the_bits_of_sgemm():
-    """Products of a result are added in ascending k, each rounded, as in an unpartitioned launch of sgemm.hip."""
+def test_sums_next_to_sgemm():
+    """Up to 256 of K the products of a result are added in ascending k, each rounded, as in an unpartitioned launch of sgemm.hip;
+    longer chains are cut there, which leaves less error than its two K groups."""
     rng = np.random.default_rng(4)
-    A, B = rng.standard_normal((290, 777)).astype(np.float32), rng.standard_normal((777, 301)).astype(np.float32)
-    want = run_sgemm_f32(load(b32.default_library()), A, B, workspace=False)
+    A, B = rng.standard_normal((290, 2600)).astype(np.float32), rng.standard_normal((2600, 301)).astype(np.float32)
+    short = run_sgemm_f32(load(b32.default_library()), A[:, :255], B[:255], workspace=False)
+    exact = A.astype(np.float64) @ B.astype(np.float64)
+    error = lambda got: np.linalg.norm(got - exact)
+    limit = error(run_sgemm_f32(load(b32.sgemm_library(64, 64, 32, 32, 32, 2)), A, B, workspace=False))
     for key in b32.RING_KEYS:
-        assert np.array_equal(run_sgemm_f32(load(b32.library_for_key(key)), A, B), want), key
+        lib = load(b32.library_for_key(key))
+        assert np.array_equal(run_sgemm_f32(lib, A[:, :255], B[:255]), short), key
+        assert error(run_sgemm_f32(lib, A, B)) <= limit, key
 
 
 def test_many_tiles_integer_exact():
@@ -103,4 +110,40 @@ def test_graph_replays_and_refusals():
         assert np.array_equal(C.cpu().numpy().astype(np.int64), exact)
     assert lib.gemm(*args[:6], 130, *args[7:], check=False) == HELIX_ERR_INVALID_VALUE
     assert lib.gemm(dA.data_ptr() + 4, *args[1:], check=False) == HELIX_ERR_INVALID_VALUE
-    assert lib.conv2d(dA.data_ptr(), dB.data_ptr(), C.data_ptr(), 1, 4, 4, 8, 8, 1, 1, 1, 0, check=False) == HELIX_ERR_UNSUPPORTED
+    conv = (dA.data_ptr(), dB.data_ptr(), C.data_ptr(), 1, 8, 8)
+    assert lib.conv2d(*conv, 6, 8, 1, 1, 1, 0, check=False) == HELIX_ERR_UNSUPPORTED       # chunks across taps
+    assert lib.conv2d(*conv, 4, 8, 4, 8, 1, 0, check=False) == HELIX_ERR_UNSUPPORTED       # 32 taps
+    assert lib.conv2d(dA.data_ptr() + 4, *conv[1:], 8, 8, 1, 1, 1, 0, check=False) == HELIX_ERR_INVALID_VALUE
+
+
+# batch, channels, H, W, filters, kH, kW, stride, pad
+LAYERS = [(1, 4, 1, 1, 1, 1, 1, 1, 0),         # one pixel, one chunk
+          (2, 32, 9, 11, 70, 3, 3, 1, 1),      # a tile is one tap; filters off 4
+          (3, 12, 14, 10, 33, 5, 5, 2, 2),     # a tile over three taps
+          (2, 64, 12, 12, 48, 5, 5, 1, 4),     # rows and columns of taps beyond the image
+          (2, 100, 7, 7, 40, 1, 1, 1, 0),      # half a K tile left over
+          (2, 4, 9, 12, 20, 5, 6, 1, 0),       # 30 taps, eight of them a tile
+          (1, 8, 40, 3, 24, 31, 1, 3, 2),      # 31 taps
+          (2, 96, 20, 23, 260, 3, 2, 3, 1)]    # several tiles both ways, rows off every multiple
+
+
+@pytest.mark.parametrize("layer", LAYERS, ids=lambda l: "x".join(map(str, l)))
+def test_every_configuration_convolves_integer_exact(layer):
+    B, IC, H, W, OC, kH, kW, stride, pad = layer
+    rng = np.random.default_rng(sum(layer))
+    x = rng.integers(-4, 5, (B, H, W, IC)).astype(np.float32)
+    w = rng.integers(-4, 5, (OC, kH, kW, IC)).astype(np.float32)
+    want = O.conv2d_nhwc(x, w, stride, pad)
+    for key in b32.RING_KEYS:
+        assert np.array_equal(run_conv(load(b32.library_for_key(key)), x, w, stride, pad, torch.float32), want), key
+
+
+def test_infinities_in_the_input_reach_their_pixels_only():
+    """Padding, channels beyond the last tile and rows beyond the last pixel are zeros, not what lies beside them."""
+    x = np.zeros((2, 6, 7, 20), np.float32)
+    w = np.ones((35, 3, 3, 20), np.float32)
+    x[0, 5, 6, 19] = np.inf
+    want = np.zeros((2, 6, 7, 35), np.float32)
+    want[0, 4:6, 5:7] = np.inf
+    for key in b32.RING_KEYS:
+        assert np.array_equal(run_conv(load(b32.library_for_key(key)), x, w, 1, 1, torch.float32), want), key
