@@ -9,7 +9,7 @@ import os
 
 from utils.helix_runtime import load, tuned_config, fastest_of
 from utils.roofline import NUM_CU, HBM_BYTES_PER_S, gemm_bytes
-from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, SPLITK_MAX, RING_KEYS
+from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, SPLITK_MAX, RING_KEYS, is_ring_key
 from MI355X_FP16.profile_MI355X_FP16 import PROFILE_K, PROFILE_K_SHORT
 
 root_path = os.getcwd()
@@ -151,39 +151,53 @@ def ranked_configs(prof_dict, M, N, K, top=VERIFY_TOP):
 
 
 # ---- the family of four-wave tiles over a ring of LDS stages (src_template/MI355X_FP16/gemm_ring.hip) --------------------
-# It has no profile.  Clocks at 2.4 GHz, fitted to 2239 measured (problem, configuration) pairs, 21 % rms; what decides is the
-# order: the fastest of the first four by this model and of the profiled candidates is 0.15 % behind the fastest of all in the
-# geometric mean over 62 problems, 5.6 % at worst.
+# It has no profile.  Clocks at 2.4 GHz: launch and first copies; the products of a 32 x 32 piece of a workgroup's tile in one K
+# tile of 64; bytes per clock from L2 into LDS, per compute unit; the results of a piece; operands once and results once, bytes
+# per second; what a K tile takes beside that where a compute unit holds one workgroup.  Fitted to 2239 and 1250 measured (problem,
+# configuration) pairs, 21 % and 18 % rms; what decides is the order: the fastest of the first four by this model and of the
+# older templates' configurations is 0.15 % behind the fastest of all in the geometric mean over 62 products (5.6 % at worst),
+# 0.01 % over 50 convolutions.
 RING_TOP = 4
-RING_FIXED_CLOCKS = 3990           # launch, first copies
-RING_STEP_CLOCKS = 32 * 1.84       # the products of a 32 x 32 piece of a workgroup's tile in one K tile of 64
-RING_FEED_BYTES_PER_CLOCK = 31     # L2 into LDS, per compute unit
-RING_STORE_CLOCKS = 476            # the results of a 32 x 32 piece
-RING_BYTES_PER_S = 4.4e12          # operands once and results once
+RING_GEMM = (3990, 32 * 1.84, 31, 476, 4.4e12, 0)
+RING_CONV = (6700, 53.6, 40, 236, 10e12, 132)
 RING_LDS_BYTES = 160 * 1024
+# The selection repeats a launch on one set of operands, which small ones leave in L2; with three sets in turn these tiles, whose few
+# stages wait for each copy, lose more than the older ones: 127619 x 5 x 458 20.4 / 20.9 us on one set, 26.7 / 24.5 on three; 4096 x
+# 3072 x 768 21.5 / 22.4 and 21.1 / 21.6.  So they have to be ahead by this much.
+RING_HANDICAP = 1.03
 
 
-def ring_seconds(key, M, N, K):
-    """Predicted seconds of a configuration of that family."""
+def ring_seconds(key, M, N, K, moved, constants):
+    """Predicted seconds of a configuration of that family on a problem that moves `moved` bytes."""
+    fixed, step_clocks, feed, store_clocks, rate, wait_clocks = constants
     stages, rows, cols = key[:3]
     tiles = math.ceil(M / rows) * math.ceil(N / cols)
     pieces, copied = rows * cols // 1024, (rows + cols) * 128
     by_registers = 4 if pieces <= 8 else 3 if pieces <= 12 else 2 if pieces <= 24 else 1
     resident = max(1, min(RING_LDS_BYTES // (stages * copied), by_registers))
+    ktiles = math.ceil(K / 64)
 
     def round_clocks(share):       # workgroups of one round on a compute unit
-        step = max(pieces * RING_STEP_CLOCKS, copied / RING_FEED_BYTES_PER_CLOCK)
-        return share * (math.ceil(K / 64) * step + RING_STORE_CLOCKS * pieces)
+        return (share * (ktiles * max(pieces * step_clocks, copied / feed) + store_clocks * pieces) +
+                (ktiles * wait_clocks if share == 1 else 0))
 
     rounds = math.ceil(tiles / (NUM_CU * resident))
     last = tiles - (rounds - 1) * NUM_CU * resident
-    clocks = RING_FIXED_CLOCKS + (rounds - 1) * round_clocks(resident) + round_clocks(min(resident, math.ceil(last / NUM_CU)))
-    return max(clocks / 2.4e9, gemm_bytes(M, N, K, 2) / RING_BYTES_PER_S + 2.5e-6)
+    clocks = fixed + (rounds - 1) * round_clocks(resident) + round_clocks(min(resident, math.ceil(last / NUM_CU)))
+    return max(clocks / 2.4e9, moved / rate + 2.5e-6)
+
+
+def handicap(key):
+    return RING_HANDICAP if is_ring_key(key) else 1.0
+
+
+def ring_first(M, N, K, moved, constants, top):
+    """The `top` configurations of that family with the lowest predicted time, best first."""
+    return sorted(RING_KEYS, key=lambda k: (ring_seconds(k, M, N, K, moved, constants), k))[:top]
 
 
 def ring_ranked(M, N, K, top=RING_TOP):
-    """The `top` configurations of that family with the lowest predicted time, best first."""
-    return sorted(RING_KEYS, key=lambda k: (ring_seconds(k, M, N, K), k))[:top]
+    return ring_first(M, N, K, gemm_bytes(M, N, K, 2), RING_GEMM, top)
 
 
 def padded_k(K):
@@ -228,7 +242,7 @@ def verified_config(prof_dict, M, N, K, top=VERIFY_TOP, families=True):
     keys = ranked_configs(prof_dict, M, N, K, top) + (ring_ranked(M, N, K) if families else [])
 
     def fastest(copies):
-        return fastest_of(keys, lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters, copies=copies),
+        return fastest_of(keys, lambda k, warmup, iters: handicap(k) * run_config(k, M, N, K, warmup=warmup, iters=iters, copies=copies),
                           f"{M}x{N}x{K}")
 
     copies = weight_copies(N, K)

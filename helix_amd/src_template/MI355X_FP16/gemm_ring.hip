@@ -1,7 +1,8 @@
-// MI355X (gfx950 / CDNA4) FP16 GEMM template: four waves, K tiles copied straight into a ring of LDS stages.
+// MI355X (gfx950 / CDNA4) FP16 GEMM and implicit-GEMM convolution template: four waves, K tiles copied straight into a ring of LDS stages.
 //
-//   C[M x N] = A[M x K] * B[N x K]^T, FP16 in, FP32 accumulate (MFMA), FP16 out; operands and result as in gemm.hip.  A 1 x 1
-//   convolution with stride 1 and no padding is this product of the activations as they lie.
+//   C[M x N] = A[M x K] * B[N x K]^T, FP16 in, FP32 accumulate (MFMA), FP16 out; operands and result as in gemm.hip.
+//   y[B,OH,OW,OC] = conv2d(x[B,H,W,IC], w[OC,kH,kW,IC]), IC a multiple of 8, at most 31 taps; a 1 x 1 one with stride 1 and no padding
+//   is the product of the activations as they lie.
 //
 // Role in the reference: src_template/Ampere_FP16/gemm.cu:120-534, whose K_STAGE ring of cp.async stages this is the counterpart
 // of.
@@ -22,6 +23,13 @@
 // two stages).  Level or behind: squares from 4096 on (8192^3
 // 830 / 855; what both wait for there is L2: 48 KiB a K tile come at 27 - 30 bytes per clock and CU, and the larger tiles that would
 // ask for less do not leave room for a third stage), few tiles with long K (split-K libraries).
+// Convolutions: a copy's lane knows where the first tap of its pixel lies and which taps are inside the image (a bit each); a tile
+// adds the tap's offset, one for all lanes where channels come in 64s.  No table and no register on the way from L2 to LDS, where
+// gemm.hip's gather passes staging registers (batch x channels x image, filter; the fastest of gemm.hip and conv_patch.hip / of these):
+//   3x3  21 x 384 x 33 x 33 -> 320 58.3 / 48.2   8 x 256 x 75 x 75 -> 512 103 / 93     22 x 192 x 57 x 57 -> 32 21.9 / 19.3
+//        32 x 64 x 56 x 56 -> 64 14.7 / 13.6     5 x 64 x 26 x 26 -> 128 5.5 / 4.7     49 x 192 x 22 x 22 -> 64 12.3 / 11.3
+// and behind with few tiles and long K, where K is shared out elsewhere (4 x 256 x 14 x 14 7.0 / 9.2); 0.973 in the geometric mean
+// over 50 layers.
 //
 // Compile-time parameters (-D, one shared library per combination):
 //   BLOCK_ROWS x BLOCK_COLS   workgroup tile, multiples of 32; a wave's is half of it in both directions
@@ -31,6 +39,7 @@
 #include <stdio.h>
 
 #include "helix_abi.h"
+#include "helix_fastdiv.h"
 #include "helix_ring.h"
 
 #ifndef BLOCK_ROWS
@@ -71,9 +80,22 @@ struct Params {
     int M, N, K, lda, ldb, ldc, tiles_m, tiles_n;
 };
 
+// A convolution as the implicit GEMM: rows are pixels, columns filters, K the taps' channels
+using helix_fastdiv::FastDiv;
+
+struct ConvParams : Params {
+    int H, W, IC, kH, kW, stride, pad;
+    unsigned x_bytes;
+    FastDiv by_OW, by_OH, by_IC, by_kW;
+};
+constexpr int NO_TAP = 31;                          // a bit that no row's mask has
+
+// What the kernel multiplies: a product, a convolution whose K tiles lie in one tap (channels a multiple of 64), any other
+enum { PRODUCT, WHOLE_TAPS, CHUNKS_OF_TAPS };
+
 // (the tile parameters are template arguments for the symbol name's sake: a profiler lists configurations separately)
-template <int T_STAGES = STAGES, int T_BM = BM, int T_BN = BN>
-__global__ __launch_bounds__(NTHREADS, 1) void helix_gemm_f16_ring_kernel(const Params p) {
+template <int MODE, class P, int T_STAGES = STAGES, int T_BM = BM, int T_BN = BN>
+__global__ __launch_bounds__(NTHREADS, 1) void helix_gemm_f16_ring_kernel(const P p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -83,36 +105,79 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_gemm_f16_ring_kernel(const 
     if (!tile_of((int)blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn)) return;
     const int m0 = tm * BM, n0 = tn * BN;
 
-    // ---- copies: piece d of a wave is 8 LDS rows; row r holds its 16-byte chunk c at c ^ (r / 2 mod 8) ------------------
+    // ---- copies: piece d of a wave is 8 LDS rows; row r holds its 16-byte chunk c at c ^ (r / 2 mod 8).  A wave's pieces are all even
+    // or all odd, so that a lane has one chunk of every row ------------------------------------------------------------------
     const int rows_a = (p.M - m0) < BM ? (p.M - m0) : BM, rows_b = (p.N - n0) < BN ? (p.N - n0) : BN;
-    const half_t* baseA = p.A + (size_t)m0 * p.lda;
+    const half_t* baseA = p.A + (MODE == PRODUCT ? (size_t)m0 * p.lda : 0);
     const half_t* baseB = p.B + (size_t)n0 * p.ldb;
     const unsigned bytesA = (unsigned)(((size_t)(rows_a - 1) * p.lda + p.K) * 2);
     const unsigned bytesB = (unsigned)(((size_t)(rows_b - 1) * p.ldb + p.K) * 2);
-    auto piece_of = [&](int d) -> int { return d < TM ? wave * TM + d : wave * TN + d - TM; };
-    auto chunk_of = [&](int d) -> int { return (lane & 7) ^ ((4 * piece_of(d) + (lane >> 4)) & 7); };
+    auto piece_of = [&](int d) -> int { return (d < TM ? d : d - TM) * 4 + wave; };
+    const int chunk = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
     int from[COPIES];
+    unsigned inside[TM];                             // of a pixel: the taps that are inside the image; `from` is its first tap's place
 #pragma unroll
     for (int d = 0; d < COPIES; d++) {
         const int row = piece_of(d) * 8 + (lane >> 3);
-        from[d] = row < (d < TM ? rows_a : rows_b) ? row * (d < TM ? p.lda : p.ldb) * 2 + chunk_of(d) * 16 : OOB_OFFSET;
+        from[d] = row < (d < TM ? rows_a : rows_b) ? row * (d < TM ? p.lda : p.ldb) * 2 + chunk * 16 : OOB_OFFSET;
+        if constexpr (MODE != PRODUCT) {
+            if (d >= TM) continue;
+            const int m = m0 + row, t = p.by_OW.div(m), ow = m - t * p.by_OW.d, b = p.by_OH.div(t), oh = t - b * p.by_OH.d;
+            const int ih = oh * p.stride - p.pad, iw = ow * p.stride - p.pad;
+            from[d] = (int)((((unsigned)b * p.H + ih) * p.W + iw) * (unsigned)p.IC * 2u) + (MODE == WHOLE_TAPS ? chunk * 16 : 0);
+            const int left = iw < 0 ? -iw : 0, right = p.W - iw < p.kW ? p.W - iw : p.kW;
+            const unsigned of_row = right > left ? (1u << right) - (1u << left) : 0u;
+            unsigned mask = 0;
+            for (int kh = 0; kh < p.kH; kh++) mask |= (unsigned)(ih + kh) < (unsigned)p.H ? of_row << (kh * p.kW) : 0u;
+            inside[d] = m < p.M ? mask : 0u;
+        }
     }
     const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)smem;
-    // where K is not a multiple of 64 the narrow tile comes first, so that only its copies carry a column mask
-    const int ktiles = (p.K + BK - 1) / BK, first_w = p.K % BK ? p.K % BK : BK;
+    // where a product's K is not a multiple of 64 the narrow tile comes first, so that only its copies carry a column mask
+    const int ktiles = (p.K + BK - 1) / BK, first_w = MODE == PRODUCT && p.K % BK ? p.K % BK : BK;
     auto k0_of = [&](int t) -> int { return t == 0 ? 0 : first_w + (t - 1) * BK; };
+    // a convolution's tap and the byte offset behind a row's first tap, of the tile that is copied next: one for all lanes, or by
+    // the lane's chunk
+    int tap = 0, offset = 0, kw = 0, c = 0;
+    intx4 ra, rb;
     // (past the last tile the copies still go out, from empty buffers: the counts stay)
-    auto rsrc_a = [&](int t) -> intx4 { return raw_rsrc(baseA + k0_of(t), t < ktiles ? bytesA - (unsigned)k0_of(t) * 2u : 0u); };
-    auto rsrc_b = [&](int t) -> intx4 { return raw_rsrc(baseB + k0_of(t), t < ktiles ? bytesB - (unsigned)k0_of(t) * 2u : 0u); };
-    auto copy = [&](int d, int stage, const intx4& ra, const intx4& rb, bool narrow) {
-        const int offset = narrow && chunk_of(d) * 8 >= first_w ? OOB_OFFSET : from[d];
-        copy16(d < TM ? ra : rb, lds0 + (unsigned)(stage * STAGE_BYTES + (d < TM ? 0 : A_BYTES) + piece_of(d) * 1024), offset);
+    auto aim = [&](int t) {
+        if constexpr (MODE == PRODUCT) ra = raw_rsrc(baseA + k0_of(t), t < ktiles ? bytesA - (unsigned)k0_of(t) * 2u : 0u);
+        else ra = raw_rsrc(p.A, p.x_bytes);
+        rb = raw_rsrc(baseB + k0_of(t), t < ktiles ? bytesB - (unsigned)k0_of(t) * 2u : 0u);
+        if constexpr (MODE == CHUNKS_OF_TAPS) {
+            const int k = t * BK + chunk * 8, at = p.by_IC.div(k), row = p.by_kW.div(at);
+            tap = k < p.K ? at : NO_TAP;
+            offset = ((row * p.W + at - row * p.kW) * p.IC + k - at * p.IC) * 2;
+        }
+    };
+    auto step = [&]() {                              // to the next tile
+        if constexpr (MODE == WHOLE_TAPS) {
+            c += BK;
+            offset += BK * 2;
+            if (c == p.IC) {
+                c = 0;
+                tap = tap < NO_TAP ? tap + 1 : NO_TAP;
+                if (++kw == p.kW) {
+                    kw = 0;
+                    offset += (p.W - p.kW) * p.IC * 2;
+                }
+            }
+        }
+    };
+    auto copy = [&](int d, int stage, bool narrow) {
+        int at = from[d];
+        if (MODE == PRODUCT) at = narrow && chunk * 8 >= first_w ? OOB_OFFSET : at;
+        else if (d < TM) at = (inside[d] >> tap) & 1 ? at + offset : OOB_OFFSET;
+        else if (MODE == CHUNKS_OF_TAPS) at = tap == NO_TAP ? OOB_OFFSET : at;
+        copy16(d < TM ? ra : rb, lds0 + (unsigned)(stage * STAGE_BYTES + (d < TM ? 0 : A_BYTES) + piece_of(d) * 1024), at);
     };
 #pragma unroll
     for (int u = 0; u < STAGES; u++) {
-        const intx4 ra = rsrc_a(u), rb = rsrc_b(u);
+        aim(u);
 #pragma unroll
-        for (int d = 0; d < COPIES; d++) copy(d, u, ra, rb, u == 0);
+        for (int d = 0; d < COPIES; d++) copy(d, u, u == 0);
+        step();
     }
 
     // ---- fragments: lane (r, q) supplies row r, chunk 4 s + q of step s -----------------------------------------------
@@ -148,7 +213,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_gemm_f16_ring_kernel(const 
     int stage = 0;
     for (int t = 0; t < ktiles; t++) {
         const int next = stage + 1 == STAGES ? 0 : stage + 1;
-        const intx4 ra = rsrc_a(t + STAGES), rb = rsrc_b(t + STAGES);
+        aim(t + STAGES);
 #pragma unroll
         for (int g = 0; g < NM; g++) {
             multiply(g, 0);
@@ -167,9 +232,10 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_gemm_f16_ring_kernel(const 
                 if (e * EARLY / (TM + TN) == g) read(e, 0, next);    // (past the last tile: zeros, not used)
 #pragma unroll
             for (int d = 0; d < COPIES; d++)
-                if (d * NM / COPIES == g) copy(d, stage, ra, rb, false);
+                if (d * NM / COPIES == g) copy(d, stage, false);
             __builtin_amdgcn_sched_barrier(0);
         }
+        step();
         stage = next;
     }
 
@@ -236,7 +302,7 @@ inline const char* info_json() {
                  "\"block_k\": %d, \"split_k\": 1, \"direct_to_lds\": 1, \"threads\": %d, \"lds_bytes\": %d, "
                  "\"layout_a\": \"M x K row-major f16\", \"layout_b\": \"N x K row-major f16\", "
                  "\"layout_c\": \"M x N row-major f16\", \"accumulate\": \"f32\", "
-                 "\"k_multiple\": 8, \"ld_multiple\": 8, \"conv\": \"1 x 1, stride 1, no padding; IC a multiple of 8\"}",
+                 "\"k_multiple\": 8, \"ld_multiple\": 8, \"conv\": \"NHWC x [OC][kH][kW][IC]; IC a multiple of 8, at most 31 taps\"}",
                  STAGES, BM, BN, BM / 2, BN / 2, BK, NTHREADS, LDS_BYTES);
         done = true;
     }
@@ -251,6 +317,15 @@ inline void bench_layout(int M, int N, int K, size_t* ae, size_t* be, size_t* ce
     *lda = K; *ldb = K; *ldc = N;
 }
 
+template <int MODE, class P>
+inline int launch(const P& p, unsigned grid, hipStream_t s) {
+    static int rc = (int)hipFuncSetAttribute((const void*)helix_gemm_f16_ring_kernel<MODE, P>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+    if (rc) return rc;
+    hipLaunchKernelGGL((helix_gemm_f16_ring_kernel<MODE, P>), dim3(grid), dim3(NTHREADS), LDS_BYTES, s, p);
+    return (int)hipGetLastError();
+}
+
 inline int gemm(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, void*, size_t, hipStream_t s) {
     if (K % 8 != 0 || lda % 8 != 0 || ldb % 8 != 0) return HELIX_ERR_INVALID_VALUE;
     if (lda < K || ldb < K || ldc < N) return HELIX_ERR_INVALID_VALUE;
@@ -260,20 +335,30 @@ inline int gemm(const void* A, const void* B, void* C, int M, int N, int K, int 
     Params p{(const half_t*)A, (const half_t*)B, (half_t*)C, M, N, K, lda, ldb, ldc, (M - 1) / BM + 1, (N - 1) / BN + 1};
     const long long ntiles = (long long)p.tiles_m * p.tiles_n;
     if (ntiles > 0x3fffffffLL) return HELIX_ERR_INVALID_VALUE;
-    static int rc = (int)hipFuncSetAttribute((const void*)helix_gemm_f16_ring_kernel<>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-    if (rc) return rc;
-    const unsigned grid = (unsigned)((ntiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
-    hipLaunchKernelGGL(helix_gemm_f16_ring_kernel<>, dim3(grid), dim3(NTHREADS), LDS_BYTES, s, p);
-    return (int)hipGetLastError();
+    return launch<PRODUCT>(p, (unsigned)((ntiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD), s);
 }
 
 inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W, int IC, int OC, int kH, int kW, int stride,
                   int pad, void* ws, size_t ws_bytes, hipStream_t s) {
-    const long long M = (long long)batch * H * W;
-    if (kH != 1 || kW != 1 || stride != 1 || pad != 0 || IC % 8 != 0) return HELIX_ERR_UNSUPPORTED;
-    if (M > 0x7fffffff || M * IC * 2 >= 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;      // as gemm.hip's
-    return gemm(x, w, y, (int)M, OC, IC, IC, IC, OC, ws, ws_bytes, s);
+    const int OH = (H + 2 * pad - kH) / stride + 1, OW = (W + 2 * pad - kW) / stride + 1;
+    const long long M = (long long)batch * OH * OW, K = (long long)kH * kW * IC, xbytes = (long long)batch * H * W * IC * 2;
+    // a 16-byte chunk lies in one tap, and a row's mask has a bit for each and one to spare
+    if (IC % 8 != 0 || kH > NO_TAP || kW > NO_TAP || kH * kW > NO_TAP) return HELIX_ERR_UNSUPPORTED;
+    if (M > 0x7fffffff || xbytes >= 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;      // as gemm.hip's
+    if (kH == 1 && kW == 1 && stride == 1 && pad == 0) return gemm(x, w, y, (int)M, OC, IC, IC, IC, OC, ws, ws_bytes, s);
+    if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 1)) return HELIX_ERR_INVALID_VALUE;
+    if (M > 0x7fffffffLL - BM || K > 0x7fffffffLL - 8 * BK || (long long)BN * K * 2 >= 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;
+    ConvParams p;
+    static_cast<Params&>(p) = Params{(const half_t*)x, (const half_t*)w, (half_t*)y, (int)M, OC, (int)K, 0, (int)K, OC,
+                                     ((int)M - 1) / BM + 1, (OC - 1) / BN + 1};
+    p.H = H; p.W = W; p.IC = IC; p.kH = kH; p.kW = kW; p.stride = stride; p.pad = pad;
+    p.x_bytes = (unsigned)xbytes;
+    p.by_OW = helix_fastdiv::make(OW); p.by_OH = helix_fastdiv::make(OH);
+    p.by_IC = helix_fastdiv::make(IC); p.by_kW = helix_fastdiv::make(kW);
+    const long long ntiles = (long long)p.tiles_m * p.tiles_n;
+    if (ntiles > 0x3fffffffLL) return HELIX_ERR_INVALID_VALUE;
+    const unsigned grid = (unsigned)((ntiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
+    return IC % BK == 0 ? launch<WHOLE_TAPS>(p, grid, s) : launch<CHUNKS_OF_TAPS>(p, grid, s);
 }
 
 }  // namespace tpl

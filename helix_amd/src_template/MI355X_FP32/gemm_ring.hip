@@ -20,10 +20,10 @@
 // Sums: ascending k, a chain of FMAs per 256 of K, added in order: up to there the bits of an unpartitioned sgemm.hip launch,
 // beyond it less than half of its error (4000 x 2300 x 770, 8134 x 451 x 5225: 5.0e-7 and 13e-7 in the norm there, 3.5e-7 and 9.2e-7 with
 // two K groups); per 128 it is 2.1e-7 and 2.4e-7, and costs 2 - 4 % of the time.
-// Measured, us per launch, the fastest of sgemm.hip's configurations / of these: 4000 x 2300 x 770 120.7 / 107.2 (64 x 64 tiles; 94 are
-// the products at the peak rate), 2048^3 129.9 / 121.4, 4096^3 946 / 925, 661 x 11008 x 1024 128.8 / 116.5, 512 x 3072 x 768 25.7 / 22.6,
-// 8134 x 451 x 5225 326 / 290, 283256 x 72 x 331 196 / 130 (64 x 80 tiles; 168 with the waves 2 x 2), 361104 x 36 x 196 87 / 75 (64 x
-// 48; 92), 3325 x 1824 x 328 37.5 / 33.3, 196 x 512 x 256 5.4 / 4.6; 0.928 in the geometric mean over 48 problems.  Behind where
+// Measured, us per launch, the fastest of sgemm.hip's configurations / of these: 4000 x 2300 x 770 120.7 / 111.5 (94 are the products
+// at the peak rate), 2048^3 131.1 / 123.4, 4096^3 944 / 936, 661 x 11008 x 1024 129.0 / 119.4, 512 x 3072 x 768 25.5 / 22.6, 8134 x 451 x
+// 5225 328 / 300, 283256 x 72 x 331 191 / 133 (64 x 80 tiles; 168 with the waves 2 x 2), 361104 x 36 x 196 98 / 78 (64 x 48; 92),
+// 3325 x 1824 x 328 37.6 / 33.9, 196 x 512 x 256 5.4 / 4.6; 0.928 in the geometric mean over 48 problems with one chain of sums.  Behind where
 // tiles are few and K is long (29 x 1000 x 11976 18.8 / 105): K groups and partitions stay sgemm.hip's.
 //
 // Compile-time parameters (-D, one shared library per combination):
@@ -279,11 +279,11 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
 // are the operands of four products.  A copy's lane knows where the first tap of its pixel lies and which taps are inside the
 // image (a bit each); a tile adds the tap's offset, one for all lanes where channels come in 32s, five instructions a copy.
 // Measured, us per launch, the fastest configuration of sgemm.hip and conv_patch.hip / of this (batch x channels x image, filter):
-//   1x1  3 x 256 x 63 x 63 -> 96 12.6 / 9.9    3 x 128 x 49 x 49 -> 192 9.2 / 7.5     2 x 96 x 75 x 75 -> 384 15.5 / 12.6
-//        41 x 128 x 45 x 45 -> 128 32.8 / 28.0  51 x 832 x 15 x 15 -> 160 37.7 / 32.1  45 x 128 x 56 x 56 -> 48 28.8 / 22.3
-//   3x3  11 x 192 x 37 x 37 -> 208 110.6 / 97.8     32 x 256 x 14 x 14 -> 256 83.4 / 72.8    12 x 256 x 27 x 27 -> 160 72.6 / 63.1
-//        7 x 96 x 85 x 85 -> 48 57.3 / 46.3          16 x 128 x 49 x 49 -> 64 57.4 / 51.8
-//   5x5  8 x 16 x 60 x 60 -> 160 44.7 / 39.7        31 x 16 x 109 x 109 -> 48 163 / 126
+//   1x1  3 x 256 x 63 x 63 -> 96 12.9 / 9.8    3 x 128 x 49 x 49 -> 192 9.2 / 7.2     2 x 96 x 75 x 75 -> 384 15.4 / 12.5
+//        41 x 128 x 45 x 45 -> 128 35.1 / 30.2  51 x 832 x 15 x 15 -> 160 39.6 / 33.6  45 x 128 x 56 x 56 -> 48 30.3 / 22.5
+//   3x3  11 x 192 x 37 x 37 -> 208 108.5 / 97.2     32 x 256 x 14 x 14 -> 256 82.7 / 75.1    12 x 256 x 27 x 27 -> 160 70.1 / 63.9
+//        7 x 96 x 85 x 85 -> 48 56.6 / 46.7          16 x 128 x 49 x 49 -> 64 58.3 / 51.5
+//   5x5  8 x 16 x 60 x 60 -> 160 44.0 / 39.1        31 x 16 x 109 x 109 -> 48 164 / 130
 // Behind, as in products, where tiles are few and K is long (1 x 256 x 14 x 14 3x3 7.8 / 20.5).  0.922 in the geometric
 // mean over 44 layers.
 

@@ -1,4 +1,4 @@
-"""FP16 products on four-wave tiles over a ring of LDS stages (MI355X_FP16/gemm_ring.hip): every configuration at the edges of its
+"""FP16 products and convolutions on four-wave tiles over a ring of LDS stages (MI355X_FP16/gemm_ring.hip): every configuration at the edges of its
 tiles, through the C ABI."""
 import numpy as np
 import pytest
@@ -100,9 +100,48 @@ def test_graph_replays_and_refusals():
         assert np.array_equal(C.cpu().numpy().astype(np.int64), exact)
     assert lib.gemm(*args[:5], 199, *args[6:], check=False) == HELIX_ERR_INVALID_VALUE
     assert lib.gemm(dA.data_ptr() + 2, *args[1:], check=False) == HELIX_ERR_INVALID_VALUE
-    assert lib.conv2d(dA.data_ptr(), dB.data_ptr(), C.data_ptr(), 1, 4, 4, 8, 8, 3, 3, 1, 1, check=False) == HELIX_ERR_UNSUPPORTED
+    conv = (dA.data_ptr(), dB.data_ptr(), C.data_ptr(), 1, 8, 8)
+    assert lib.conv2d(*conv, 12, 8, 1, 1, 1, 0, check=False) == HELIX_ERR_UNSUPPORTED      # chunks across taps
+    assert lib.conv2d(*conv, 8, 8, 4, 8, 1, 0, check=False) == HELIX_ERR_UNSUPPORTED       # 32 taps
+    assert lib.conv2d(dA.data_ptr() + 2, *conv[1:], 8, 8, 3, 3, 1, 1, check=False) == HELIX_ERR_INVALID_VALUE
     x = rng.integers(-1, 2, (3, 5, 7, 72)).astype(np.float16)
     w = rng.integers(-1, 2, (40, 1, 1, 72)).astype(np.float16)
     want = O.conv2d_nhwc(x.astype(np.float32), w.astype(np.float32), 1, 0)
     for key in b16.RING_KEYS[::5]:
         assert np.array_equal(run_conv(load(b16.library_for_key(key)), x, w, 1, 0, torch.float16).astype(np.float32), want), key
+
+
+# batch, channels, H, W, filters, kH, kW, stride, pad
+LAYERS = [(1, 8, 3, 3, 1, 3, 3, 1, 0),         # one pixel, nine taps of a chunk in two tiles
+          (2, 64, 9, 11, 70, 3, 3, 1, 1),      # a tile is one tap; filters two at a time
+          (3, 24, 14, 10, 33, 5, 5, 2, 2),     # a tile over three taps
+          (2, 128, 12, 12, 48, 5, 5, 1, 4),    # rows and columns of taps beyond the image
+          (2, 104, 7, 7, 40, 1, 1, 2, 0),      # strided 1 x 1: no plain product
+          (2, 8, 9, 12, 20, 5, 6, 1, 0),       # 30 taps, eight of them a tile
+          (1, 16, 40, 3, 24, 31, 1, 3, 2),     # 31 taps
+          (2, 192, 20, 23, 260, 3, 2, 3, 1)]   # several tiles both ways, rows off every multiple
+
+
+@pytest.mark.parametrize("layer", LAYERS, ids=lambda l: "x".join(map(str, l)))
+def test_every_configuration_convolves_integer_exact(layer):
+    B, IC, H, W, OC, kH, kW, stride, pad = layer
+    rng = np.random.default_rng(sum(layer))
+    x = rng.integers(-1, 2, (B, H, W, IC)).astype(np.float16)
+    w = rng.integers(-1, 2, (OC, kH, kW, IC)).astype(np.float16)
+    want = O.conv2d_nhwc(x.astype(np.float32), w.astype(np.float32), stride, pad)
+    assert np.abs(want).max() < 2048
+    for key in b16.RING_KEYS:
+        got = run_conv(load(b16.library_for_key(key)), x, w, stride, pad, torch.float16)
+        assert np.array_equal(got.astype(np.float32), want), key
+
+
+def test_infinities_in_the_input_reach_their_pixels_only():
+    """Padding, channels beyond the last tile and rows beyond the last pixel are zeros, not what lies beside them."""
+    x = np.zeros((2, 6, 7, 40), np.float16)
+    w = np.ones((35, 3, 3, 40), np.float16)
+    x[0, 5, 6, 39] = np.inf
+    want = np.zeros((2, 6, 7, 35), np.float32)
+    want[0, 4:6, 5:7] = np.inf
+    for key in b16.RING_KEYS:
+        got = run_conv(load(b16.library_for_key(key)), x, w, 1, 1, torch.float16)
+        assert np.array_equal(got.astype(np.float32), want), key
