@@ -260,7 +260,7 @@ def get_MI355X_FP16_conv_Oracle_result(prof_dict, batch, input_channel, H, W, ou
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     flops = 2.0 * M * output_channel * input_channel * kH * kW
     min_cost, best = float("inf"), None
-    for k in list(prof_dict.keys()) + list(PATCH_KEYS + RING_KEYS):
+    for k in prof_dict.keys():
         if k[0] == 0 or is_dtl_key(k):
             continue
         try:

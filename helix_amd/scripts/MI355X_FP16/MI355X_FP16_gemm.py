@@ -293,7 +293,7 @@ def get_MI355X_FP16_gemm_Oracle_result(prof_dict, M, N, K):
     """Exhaustive per-shape search: run every candidate, keep the fastest
     (benchmark_Ampere_FP16_performance_comparison.py:56-69).  Returns (cost_ms, tflops, key)."""
     min_cost, best = float("inf"), None
-    for k in list(prof_dict.keys()) + list(RING_KEYS):
+    for k in prof_dict.keys():
         if k[0] == 0 and min(M, N) > 16:
             continue   # the weight-streaming kernel re-reads the weights per 16 activation rows
         try:

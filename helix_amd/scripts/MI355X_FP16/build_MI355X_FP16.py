@@ -14,7 +14,9 @@ names modulo the backend tag.  Differences that follow from the target:
   * the deeper pipelines of the reference (K_STAGE 3 .. 5 are rings of cp.async stages, gemm.cu:156-198) are the
     direct-to-LDS family, src_template/MI355X_FP16/gemm_dtl.hip: eight-wave tiles whose K tiles go from global
     memory straight into a ring of K_STAGES LDS stages of BLOCK_K columns.  Its prof-dict keys carry a
-    trailing eighth field 1 (DIRECT_TO_LDS); keys of the other families keep seven fields;
+    trailing eighth field 1 (DIRECT_TO_LDS).  Two families without a profile, ranked by models of their own: convolutions whose input
+    stays in LDS (conv_patch.hip, eighth field 2) and four-wave tiles over a ring of LDS stages (gemm_ring.hip, eighth field 3);
+    the other keys keep seven fields;
   * the space is pruned by measurement (keeps_up): points that were never within reach of the fastest configuration
     on a table of 162 problems are not built;
   * compiles run in parallel worker threads instead of one os.system at a time.
