@@ -18,8 +18,8 @@
 // Two stages do (the products of a K tile take 256 clocks a wave at the least), which leaves room for up to eight workgroups on a CU: one's
 // stores and first copies lie behind another's products.
 // Sums: ascending k, a chain of FMAs per 256 of K, added in order: up to there the bits of an unpartitioned sgemm.hip launch,
-// beyond it less than half of its error (4000 x 2300 x 770, 8134 x 451 x 5225: 5.0e-7 and 13e-7 in the norm there, 3.5e-7 and 9.2e-7 with
-// two K groups); per 128 it is 2.1e-7 and 2.4e-7, and costs 2 - 4 % of the time.
+// beyond it 2.8e-7 - 3.0e-7 in the norm from K = 770 to 6160, where one chain leaves 5.0e-7 - 14e-7, sgemm.hip's two K groups 3.5e-7 -
+// 9.9e-7 and its partitions 3.9e-7 - 13e-7 (operands ~ N(0, 1)); per 128 it is 2.1e-7 - 2.4e-7, and costs 2 - 4 % of the time.
 // Measured, us per launch, the fastest of sgemm.hip's configurations / of these: 4000 x 2300 x 770 120.7 / 111.5 (94 are the products
 // at the peak rate), 2048^3 131.1 / 123.4, 4096^3 944 / 936, 661 x 11008 x 1024 129.0 / 119.4, 512 x 3072 x 768 25.5 / 22.6, 8134 x 451 x
 // 5225 328 / 300, 283256 x 72 x 331 191 / 133 (64 x 80 tiles; 168 with the waves 2 x 2), 361104 x 36 x 196 98 / 78 (64 x 48; 92),
