@@ -22,9 +22,10 @@
 //
 // Measured, us per launch (helix_bench_conv), the general path's fastest configuration against this one: batch 32, 224 x 224
 // x 3 -> 64: 7x7 stride 2 58 / 22, 3x3 88 / 36 (5.9 TB/s), 11x11 stride 4 -> 96 49 / 28; batch 20, 180 x 180 x 3, 5x5 51 / 21;
-// batch 1, 7x7 10.2 / 6.9, 3x3 10.4 / 6.5; 4 x 161 x 700 x 1 -> 32, 5x20 stride 2 33 / 14.  What is left of the 7x7 layer: 2.5 us of
-// launch, about 6 us until weights and patch are in place (all workgroups start together, so nothing overlaps it), then the
-// output at 5.7 TB/s.
+// batch 1, 7x7 10.2 / 6.4, 3x3 10.4 / 6.5; 4 x 161 x 700 x 1 -> 32, 5x20 stride 2 33 / 14.  The weights' fragments are packed from
+// four dwords each with all of a thread's loads in flight (half by half out of LDS before: 7x7 at batch 32 21.7 / 21.2 us per call).
+// What is left of the 7x7 layer: 2.5 us of launch, about 5 us until weights and patch are in place (all workgroups start together,
+// so nothing overlaps it), then the output at 5.7 TB/s.
 #pragma once
 
 #include <hip/hip_runtime.h>
