@@ -87,8 +87,8 @@ constexpr int KT_CHUNKS = 8, KT_BYTES = 128;  // K tile: what a wave loads of it
 constexpr int PRODUCTS = F32 ? 4 : 1;         // MFMAs of a step and tile: one 16x16x32, or 16x16x4 ones of one element of each chunk
 constexpr int AHEAD = 2;                      // K tiles of weights in flight in registers
 constexpr int OWN_BYTES = WAVE_COLS * KT_BYTES; // a wave's piece of LDS for its weights
-constexpr int ZERO_BYTES = 16;                // in front of everything in LDS: what K chunks beyond the filter read, at an offset of
-constexpr int BEYOND = -(1 << 24);            // this from any pixel (and of no more than 0 in all)
+constexpr int ZERO_BYTES = 16;                // in front of everything in LDS: what the K chunks of a last tile beyond the filter read,
+constexpr int BEYOND = -(1 << 24);            // at this offset from any pixel (REST, see table_entry and operand_at)
 constexpr int TABLE_OFFSET = ZERO_BYTES + NWAVES * OWN_BYTES;   // LDS offsets of the K chunks from a pixel's corner
 constexpr int SUM_BYTES = K_GROUPS > 1 ? NWAVES * TM * TN * 1024 : 0;
 constexpr int LDS_MAX = 160 * 1024;
@@ -127,7 +127,32 @@ __device__ __forceinline__ uintx4 load16(__amdgpu_buffer_rsrc_t r, int at) {
 
 // n / d: the bits of FastDiv::div through the high word of one 32-bit product, which the staging loop's three divisions a chunk
 // are a third of.
-__device__ __forceinline__ int quotient(const FastDiv& d, int n) { return (int)(__umulhi((unsigned)n << 1, d.mul) >> (d.shift - 31)); }
+__host__ __device__ __forceinline__ int quotient(const FastDiv& d, int n) {
+    return (int)((unsigned)((unsigned long long)((unsigned)n << 1) * d.mul >> 32) >> (d.shift - 31));
+}
+
+// A product of two 24-bit factors
+__host__ __device__ __forceinline__ int times(int a, int b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __mul24(a, b);
+#else
+    return a * b;
+#endif
+}
+
+// LDS offset of K chunk j from a pixel's corner; the table holds those of the K tiles and of one more, which is read ahead (by a wave
+// whose part of K is empty, too) and not multiplied.  Beyond the filter it is the zeros' where a tile has such chunks (REST), else
+// all of them are read ahead only and take the pixel's first chunk, which is a place inside the patch.
+template <bool REST>
+__host__ __device__ __forceinline__ int table_entry(const Params& p, int j) {
+    const int tap = quotient(p.by_group, j), g = j - times(tap, p.group);
+    const int kh = quotient(p.by_kW, tap), kw = tap - times(kh, p.kW);
+    return j < p.chunks ? times(kh, p.row_bytes) + times(kw, p.pixel_bytes) + g * 16 : REST ? BEYOND : 0;
+}
+
+// LDS offset of that chunk of the pixel whose corner is at `at`
+template <bool REST>
+__host__ __device__ __forceinline__ int operand_at(int at, int o) { return !REST || at + o > 0 ? at + o : 0; }
 
 // One chunk of a pixel or of a filter tap.  TAIL (FP32, where an element is a dword): `elements` of it, and not a byte beyond
 // them, which may be the buffer's end.  (No branch on that: one inside the loop over K made every load wait for itself.)
@@ -239,11 +264,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Par
         }
         if (tid == 0) *(uintx4*)smem = uintx4{0, 0, 0, 0};
         // LDS offset of each K chunk from a pixel's corner
-        for (int j = tid; j < KT_CHUNKS * (p.ktiles + 1); j += NTHREADS) {
-            const int tap = quotient(p.by_group, j), g = j - __mul24(tap, p.group);
-            const int kh = quotient(p.by_kW, tap), kw = tap - __mul24(kh, p.kW);
-            ((int*)(smem + TABLE_OFFSET))[j] = j < p.chunks ? __mul24(kh, p.row_bytes) + __mul24(kw, p.pixel_bytes) + g * 16 : BEYOND;
-        }
+        for (int j = tid; j < KT_CHUNKS * (p.ktiles + 1); j += NTHREADS) ((int*)(smem + TABLE_OFFSET))[j] = table_entry<REST>(p, j);
     }
     int at[TM];
 #pragma unroll
@@ -284,7 +305,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Par
     // order); then the loads AHEAD tiles on.  off[s]: LDS offset of the chunks that are read behind step s.
     auto read_operand = [&](int e, int s, int o) {          // weights of the first 16 channels, pixels, other weights
         if (e == 0) b[s][0] = read_b(s, 0);
-        else if (e <= TM) a[s][e - 1] = *(const frag*)(smem + (!REST || at[e - 1] + o > 0 ? at[e - 1] + o : 0));
+        else if (e <= TM) a[s][e - 1] = *(const frag*)(smem + operand_at<REST>(at[e - 1], o));
         else b[s][e - TM] = read_b(s, e - TM);
     };
     constexpr int W = 2 * TN, EARLY = 2 * SLOTS / 3 > 0 ? 2 * SLOTS / 3 : 1;
@@ -491,6 +512,9 @@ inline bool make_plan(Params& p, int* lds_bytes, int batch, int H, int W, int IC
     return true;
 }
 
+// Which variant runs a layer: REST of the kernel
+inline bool has_rest(const Params& p) { return (F32 && p.tail) || p.chunks % KT_CHUNKS; }
+
 template <bool TAIL, bool REST>
 inline int launch(const Params& p, int lds_bytes, hipStream_t s) {
     static int rc = (int)hipFuncSetAttribute((const void*)helix_conv_patch_kernel<TAIL, REST>,
@@ -511,7 +535,7 @@ inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W
     p.wide = OC % STORE == 0 && ((uintptr_t)y & (EB * STORE - 1)) == 0;
     if constexpr (F32)
         if (p.tail) return launch<true, true>(p, lds_bytes, s);
-    if (p.chunks % KT_CHUNKS) return launch<false, true>(p, lds_bytes, s);
+    if (has_rest(p)) return launch<false, true>(p, lds_bytes, s);
     return launch<false, false>(p, lds_bytes, s);
 }
 

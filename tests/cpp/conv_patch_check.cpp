@@ -8,6 +8,18 @@ static int staged_row(const Params& p, int m) {
     return image * p.image_rows + (t - image * p.OH) * p.stride;
 }
 
+// Whether every operand that a lane reads lies inside the plan's LDS: all entries of the table, those of the K tile that is read
+// ahead (and by a wave whose part of K is empty) among them, for pixels whose corners are at `first` .. `last`.
+template <bool REST>
+static bool operands_inside(const Params& p, int first, int last, int lds) {
+    for (int j = 0; j < KT_CHUNKS * (p.ktiles + 1); j++) {
+        const int o = table_entry<REST>(p, j);
+        for (const int at : {operand_at<REST>(first, o), operand_at<REST>(last, o)})
+            if (at < 0 || at + 16 > lds) return false;
+    }
+    return true;
+}
+
 int main() {
     int l[9];
     while (scanf("%d %d %d %d %d %d %d %d %d", l, l + 1, l + 2, l + 3, l + 4, l + 5, l + 6, l + 7, l + 8) == 9) {
@@ -25,13 +37,14 @@ int main() {
             if (rows > most) most = rows;
             // the last staged chunk
             const long long wrote = (long long)(rows - 1) * p.row_bytes + (long long)(p.row_pixels - 1) * p.pixel_bytes + p.group * 16;
-            long long read = 0;
-            for (int m = m0; m <= last; m++) {      // the last chunk of the last tap
-                const long long at = (long long)(staged_row(p, m) - row0 + kH - 1) * p.row_bytes +
-                                     ((long long)(m % p.by_OW.d) * p.stride + kW - 1) * p.pixel_bytes + p.group * 16;
-                if (at > read) read = at;
+            int corner = 0;                         // of the pixel that lies furthest back; the block's first is at 0 or behind
+            for (int m = m0; m <= last; m++) {
+                const int at = (staged_row(p, m) - row0) * p.row_bytes + m % p.by_OW.d * p.stride * p.pixel_bytes;
+                if (at > corner) corner = at;
             }
-            if (p.patch_offset + wrote > lds || p.patch_offset + read > lds || p.real_pixels > p.W ||
+            const bool inside = tpl::has_rest(p) ? operands_inside<true>(p, p.patch_offset, p.patch_offset + corner, lds)
+                                                 : operands_inside<false>(p, p.patch_offset, p.patch_offset + corner, lds);
+            if (p.patch_offset + wrote > lds || !inside || p.real_pixels > p.W ||
                 p.pad + p.real_pixels > p.row_pixels || (p.real_pixels + p.pad < p.row_pixels && p.real_pixels < p.W)) {
                 printf("out of bounds\n");
                 return 1;
