@@ -93,7 +93,7 @@ constexpr int TABLE_OFFSET = ZERO_BYTES + NWAVES * OWN_BYTES;   // LDS offsets o
 constexpr int SUM_BYTES = K_GROUPS > 1 ? NWAVES * TM * TN * 1024 : 0;
 constexpr int LDS_MAX = 160 * 1024;
 constexpr int NUM_XCD = 8;
-constexpr int OOB = 0x40000000;               // byte offset beyond any buffer (they stay below it), twice too: the load returns zeros
+constexpr unsigned OOB = 0x40000000u;         // byte offset beyond any buffer (they stay below it), twice too: the load returns zeros
 
 static_assert(BLOCK_ROWS % WAVE_ROWS == 0 && BLOCK_COLS % WAVE_COLS == 0 && WAVE_ROWS % 16 == 0 && WAVE_COLS % 16 == 0, "tiles");
 static_assert(F32 || TN == 1 || TN % 2 == 0, "a lane's halves are four channels of a single tile or eight of a pair");
@@ -121,8 +121,8 @@ struct Params {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }
-__device__ __forceinline__ uintx4 load16(__amdgpu_buffer_rsrc_t r, int at) {
-    return __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+__device__ __forceinline__ uintx4 load16(__amdgpu_buffer_rsrc_t r, unsigned at) {
+    return __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, 0, 0));
 }
 
 // n / d: the bits of FastDiv::div through the high word of one 32-bit product, which the staging loop's three divisions a chunk
@@ -157,11 +157,11 @@ __host__ __device__ __forceinline__ int operand_at(int at, int o) { return !REST
 // One chunk of a pixel or of a filter tap.  TAIL (FP32, where an element is a dword): `elements` of it, and not a byte beyond
 // them, which may be the buffer's end.  (No branch on that: one inside the loop over K made every load wait for itself.)
 template <bool TAIL>
-__device__ __forceinline__ uintx4 load_chunk(__amdgpu_buffer_rsrc_t r, int at, int elements) {
+__device__ __forceinline__ uintx4 load_chunk(__amdgpu_buffer_rsrc_t r, unsigned at, int elements) {
     if constexpr (!TAIL) return load16(r, at);
     uintx4 v;
 #pragma unroll
-    for (int e = 0; e < 4; e++) v[e] = __builtin_amdgcn_raw_buffer_load_b32(r, e < elements ? at + 4 * e : OOB, 0, 0);
+    for (int e = 0; e < 4; e++) v[e] = __builtin_amdgcn_raw_buffer_load_b32(r, (int)(e < elements ? at + 4 * e : OOB), 0, 0);
     return v;
 }
 
@@ -196,18 +196,18 @@ __global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Par
     const int t_end = t_begin + p.tiles_per_part < p.ktiles ? t_begin + p.tiles_per_part : p.ktiles;
     const int chunk_end = KT_CHUNKS * t_end < p.chunks ? KT_CHUNKS * t_end : p.chunks;
     const __amdgpu_buffer_rsrc_t rw = rsrc(p.w, p.w_bytes);
-    int w_at[2 * TN];                    // 8 rows of a tile at a time: lane l takes chunk l % 8 of row l / 8
+    unsigned w_at[2 * TN];               // 8 rows of a tile at a time: lane l takes chunk l % 8 of row l / 8
 #pragma unroll
     for (int d = 0; d < 2 * TN; d++) {
         const int n = oc0 + channel_of(d >> 1, (d & 1) * 8 + (lane >> 3));
-        w_at[d] = n < p.OC ? n * (p.taps * p.channel_bytes) : OOB;
+        w_at[d] = n < p.OC ? (unsigned)(n * (p.taps * p.channel_bytes)) : OOB;
     }
-    struct At { int offset, elements; };
+    struct At { unsigned offset; int elements; };
     auto tile_at = [&](int t) -> At {
         const int c = KT_CHUNKS * t + (lane & 7);
-        if (!TAIL) return At{c < chunk_end ? c * 16 : OOB, 4};
+        if (!TAIL) return At{c < chunk_end ? (unsigned)c * 16 : OOB, 4};
         const int tap = quotient(p.by_group, c), g = c - __mul24(tap, p.group);
-        return At{c < chunk_end ? __mul24(tap, p.channel_bytes) + g * 16 : OOB, g == p.group - 1 ? p.tail : 4};
+        return At{c < chunk_end ? (unsigned)(__mul24(tap, p.channel_bytes) + g * 16) : OOB, g == p.group - 1 ? p.tail : 4};
     };
     uintx4 st[AHEAD][2 * TN];
 #pragma unroll
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Par
                 const int px = quotient(p.by_group, c), g = c - __mul24(px, p.group);
                 const bool inside = (i < total) & ((unsigned)ih < (unsigned)p.H);
                 const int in_row = TAIL ? __mul24(px, p.channel_bytes) + g * 16 : c * 16;
-                v[u] = load_chunk<TAIL>(rx, inside ? __mul24(__mul24(image, p.H) + ih, image_row_bytes) + in_row : OOB, g == p.group - 1 ? p.tail : 4);
+                v[u] = load_chunk<TAIL>(rx, inside ? (unsigned)(__mul24(__mul24(image, p.H) + ih, image_row_bytes) + in_row) : OOB, g == p.group - 1 ? p.tail : 4);
                 dst[u] = i < total ? __mul24(row, p.row_bytes) + c * 16 + __mul24(px, gap) : -1;
             }
             unsigned char* first = patch + p.pad * p.pixel_bytes;

@@ -3,6 +3,11 @@
 // write or read beyond what the plan reserves.
 #include "conv_patch.hip"
 
+// A weight of a channel that is not there in a K chunk that is not there either: its offset is the sum of two that read zeros, in
+// defined arithmetic (a signed sum would be none, and no constant), and reads zeros itself, up to the last byte of a load.
+constexpr auto TWICE_OUT = OOB + OOB;
+static_assert((unsigned long long)TWICE_OUT >= (unsigned long long)OOB && TWICE_OUT <= 0xffffffffu - 15, "beyond any buffer");
+
 static int staged_row(const Params& p, int m) {
     const int t = m / p.by_OW.d, image = t / p.OH;
     return image * p.image_rows + (t - image * p.OH) * p.stride;
