@@ -91,6 +91,12 @@ struct Params {
     int M, N, K, lda, ldb, ldc, tiles_m, tiles_n;
 };
 
+// Bytes of the rows that a K tile has of an operand, from column `first` on, with `rows` of K left: an operand may have 4 GiB, a tile's
+// buffer stays below the offset that reads zeros
+__host__ __device__ __forceinline__ unsigned tile_bytes(int rows, int ld, int first) {
+    return (unsigned)(((size_t)(rows < BK ? rows : BK) * ld - first) * 4);
+}
+
 // f(0) .. f(N - 1) with constant arguments: the K loop's several hundred steps are more than `#pragma unroll` takes in nested loops
 template <int N, class F, int... I>
 __device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) {
@@ -154,7 +160,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
     // (past the last tile the copies still go out, from empty buffers: the counts stay)
     auto rsrc_of = [&](const float* base, int ld, int first, int t) -> intx4 {
         const int k0 = t < ktiles ? t * BK : 0;
-        return raw_rsrc(base + (size_t)k0 * ld + first, t < ktiles ? (unsigned)(((size_t)(p.K - k0) * ld - first) * 4) : 0u);
+        return raw_rsrc(base + (size_t)k0 * ld + first, t < ktiles ? tile_bytes(p.K - k0, ld, first) : 0u);
     };
     auto copy = [&](int d, int stage, const intx4& ra, const intx4& rb) {
         copy16(d < CA ? ra : rb, lds0 + (unsigned)place_of(d, wave, stage), from[d]);
@@ -493,13 +499,14 @@ inline void bench_layout(int M, int N, int K, size_t* ae, size_t* be, size_t* ce
     *lda = Mp; *ldb = Np; *ldc = Np;
 }
 
+// Rows of `ld` floats as an operand: byte offsets inside one K tile are 31-bit, in all as sgemm.hip takes them
+inline bool operand_fits(int K, int ld) { return (long long)K * ld * 4 < 0xffffffffLL && (long long)BK * ld * 4 < 0x7fffffffLL; }
+
 inline int gemm(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc, void*, size_t, hipStream_t s) {
     if (lda % 4 != 0 || ldb % 4 != 0) return HELIX_ERR_INVALID_VALUE;  // 16-byte copies along M and N
     if (lda < M || ldb < N || ldc < N) return HELIX_ERR_INVALID_VALUE;
     if (((uintptr_t)A & 15) || ((uintptr_t)B & 15) || ((uintptr_t)C & 3)) return HELIX_ERR_INVALID_VALUE;
-    // byte offsets inside one K tile are 32-bit, and a buffer descriptor spans at most 4 GiB
-    if ((long long)K * lda * 4 >= 0xffffffffLL || (long long)K * ldb * 4 >= 0xffffffffLL) return HELIX_ERR_INVALID_VALUE;
-    if ((long long)BK * lda * 4 >= 0x7fffffffLL || (long long)BK * ldb * 4 >= 0x7fffffffLL) return HELIX_ERR_INVALID_VALUE;
+    if (!operand_fits(K, lda) || !operand_fits(K, ldb)) return HELIX_ERR_INVALID_VALUE;
     Params p{(const float*)A, (const float*)B, (float*)C, M, N, K, lda, ldb, ldc, (M - 1) / BM + 1, (N - 1) / BN + 1};
     const long long ntiles = (long long)p.tiles_m * p.tiles_n;
     if (ntiles > 0x3fffffffLL) return HELIX_ERR_INVALID_VALUE;

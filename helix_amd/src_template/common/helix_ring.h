@@ -10,7 +10,7 @@ typedef int intx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) unsigned char* lds_ptr_t;
 
 constexpr int GROUP_ROWS = 4, NUM_XCD = 8;
-constexpr int OOB_OFFSET = 0x7fffffff;              // byte offset beyond any buffer: zeros
+constexpr int OOB_OFFSET = 0x7ffffff0;              // byte offset, of a whole copy, beyond any buffer (less than 2 GiB each): zeros
 
 // 128-bit buffer descriptor as four dwords: base address (48 bits), stride 0, byte count, raw-buffer flags
 __device__ __forceinline__ intx4 raw_rsrc(const void* base, unsigned bytes) {

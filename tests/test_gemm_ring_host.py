@@ -1,5 +1,8 @@
 """Ranking and selection of the four-wave tiles over a ring of LDS stages (MI355X_FP16/gemm_ring.hip, MI355X_FP32/gemm_ring.hip),
-which have no profile."""
+which have no profile, and the limits of their operands."""
+import os
+import subprocess
+
 from utils import helix_runtime
 from MI355X_FP16 import build_MI355X_FP16 as b16
 from MI355X_FP16 import profile_MI355X_FP16 as p16
@@ -98,3 +101,18 @@ def test_fp32_family(tmp_path, monkeypatch):
     assert b32.is_ring_key(c32.select_config(prof, 4, 64, 28, 28, 96, 3, 3, 1, 1))
     assert not c32.ring_ranked((4, 25, 28, 28, 96, 3, 3, 1, 1)) and not c32.ring_ranked((4, 64, 28, 28, 96, 11, 11, 1, 5))
     assert len(c32.ring_ranked((4, 4, 28, 28, 96, 5, 6, 1, 0))) == g32.RING_CONV_TOP
+
+
+def test_zeros_are_read_beyond_every_operand(tmp_path):
+    """The offset of what a copy has not got lies behind a K tile of the largest operand that the FP32 tiles take, 4 GiB, aligned as a
+    copy is."""
+    exe, key = str(tmp_path / "check"), b32.ring_key((32, 64, 2))
+    defines = [f"-D{k}={v}" for k, v in b32.ring_job(key)[2].items()]
+    build = subprocess.run(["hipcc", "-O1", "-w", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                            f"-I{helix_runtime._find_include_dir()}", f"-I{os.path.join(helix_runtime.SRC_ROOT, 'common')}",
+                            f"-I{os.path.join(helix_runtime.SRC_ROOT, 'MI355X_FP32')}", *defines,
+                            os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "gemm_ring_check.cpp"), "-o", exe],
+                           capture_output=True, text=True)
+    assert build.returncode == 0, build.stderr[-2000:]
+    run = subprocess.run([exe], capture_output=True, text=True)
+    assert run.returncode == 0, run.stdout[-200:]

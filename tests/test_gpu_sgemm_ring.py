@@ -56,6 +56,22 @@ def test_many_tiles_integer_exact():
         assert torch.equal(C, want), key
 
 
+def test_operand_beyond_2_gib_integer_exact():
+    """A of 2.4 GB: what a copy has not got (columns beyond M and N, pieces that a wave has not) reads zeros behind a tile's rows, not
+    data of the operand."""
+    M, N, K = 1800003, 20, 331
+    gen = torch.Generator(device="cuda:0").manual_seed(9)
+    dA = torch.randint(-8, 9, (K, M + 1), generator=gen, device="cuda:0", dtype=torch.float32)
+    dB = torch.randint(-8, 9, (K, N), generator=gen, device="cuda:0", dtype=torch.float32)
+    dA[:, M] = float("inf")
+    want = torch.cat([(dA[:, at:min(at + 200000, M)].double().t().contiguous() @ dB.double()).float() for at in range(0, M, 200000)])
+    C = torch.empty((M, N), dtype=torch.float32, device="cuda:0")
+    for key in b32.RING_KEYS[::2]:
+        C.fill_(float("nan"))
+        load(b32.library_for_key(key)).gemm(dA.data_ptr(), dB.data_ptr(), C.data_ptr(), M, N, K, M + 1, N, N)
+        assert torch.equal(C, want), key
+
+
 def test_results_stay_inside_their_rows():
     """lda, ldb and ldc beyond M and N, and a C off the vector alignment; neighbours keep what they held, and what lies in the padding
     of A and B (infinities) reaches no result."""
