@@ -7,6 +7,7 @@ LDS_BYTES = 160 * 1024
 K_TILE_BYTES = 128
 PATCH_TOP = 4
 LARGE_WAVE_TILES = 8       # 16 x 16 tiles of a wave beyond which its registers leave a compute unit 8 waves instead of 16
+LARGEST_WAVE_TILES_F32 = 10    # and in FP32, with two sets of accumulators, 4
 
 
 class PatchFamily:
@@ -69,7 +70,8 @@ class PatchFamily:
         rows, cols, wave_rows, wave_cols, groups = point
         waves = rows // wave_rows * (cols // wave_cols) * groups
         tm, tn = wave_rows // 16, wave_cols // 16
-        resident = max(1, min(LDS_BYTES // lds, (16 if tm * tn <= LARGE_WAVE_TILES else 8) // waves))
+        of_registers = 4 if self.element_bytes == 4 and tm * tn > LARGEST_WAVE_TILES_F32 else 16 if tm * tn <= LARGE_WAVE_TILES else 8
+        resident = max(1, min(LDS_BYTES // lds, of_registers // waves))
         part = -(-self.k_tiles(IC, kH, kW) // groups)
 
         def round_clocks(share):             # workgroups of one round on a compute unit

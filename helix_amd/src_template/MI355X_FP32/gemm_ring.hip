@@ -11,20 +11,21 @@
 //     BLOCK_ROWS and BLOCK_COLS floats as they are in memory, and rows from K on are beyond the buffer, hence zeros;
 //   * v_mfma_f32_16x16x4_f32 takes one float of a row per lane; it does not matter which row of the wave's tile is lane r's, so
 //     a lane reads four consecutive rows of a k in 16 bytes, one for each of four tiles, and holds four consecutive columns of a result
-//     row in return, which it stores in 16 bytes, a quarter wave 256 bytes together.  The loop for a 96 x 96 wave tile: 288 products,
-//     32 LDS reads, 12 copies, 3 waits, one barrier per 32 columns of K;
+//     row in return, which it stores in 16 bytes, a quarter wave 256 bytes together.  The loop for a 64 x 64 wave tile (64 x 256
+//     in all): 128 products, 16 LDS reads, 10 copies, one barrier per 32 columns of K;
 //   * the four waves lie 2 x 2, or in a row or column, which gives tiles 16 rows or columns apart: 48 and 80 columns for products
 //     and layers of few; and the last half K tile is left out where it is empty (K = 770: 784 columns of work).
 // Two stages do (the products of a K tile take 256 clocks a wave at the least), which leaves room for up to eight workgroups on a CU: one's
 // stores and first copies lie behind another's products.
-// Sums: ascending k, a chain of FMAs per 256 of K, added in order: up to there the bits of an unpartitioned sgemm.hip launch,
-// beyond it 2.8e-7 - 3.0e-7 in the norm from K = 770 to 6160, where one chain leaves 5.0e-7 - 14e-7, sgemm.hip's two K groups 3.5e-7 -
-// 9.9e-7 and its partitions 3.9e-7 - 13e-7 (operands ~ N(0, 1)); per 128 it is 2.1e-7 - 2.4e-7, and costs 2 - 4 % of the time.
-// Measured, us per launch, the fastest of sgemm.hip's configurations / of these: 4000 x 2300 x 770 120.7 / 111.5 (94 are the products
-// at the peak rate), 2048^3 131.1 / 123.4, 4096^3 944 / 936, 661 x 11008 x 1024 129.0 / 119.4, 512 x 3072 x 768 25.5 / 22.6, 8134 x 451 x
-// 5225 328 / 300, 283256 x 72 x 331 191 / 133 (64 x 80 tiles; 168 with the waves 2 x 2), 361104 x 36 x 196 98 / 78 (64 x 48; 92),
-// 3325 x 1824 x 328 37.6 / 33.9, 196 x 512 x 256 5.4 / 4.6; 0.928 in the geometric mean over 48 problems with one chain of sums.  Behind where
-// tiles are few and K is long (29 x 1000 x 11976 18.8 / 105): K groups and partitions stay sgemm.hip's.
+// Sums (common/helix_sums.h): ascending k, of many results a chain of FMAs per 256 of K, added in order: up to there the bits of an
+// unpartitioned sgemm.hip launch.  2.9e-7 - 3.0e-7 in the norm from K = 770 to 6160, where one chain leaves 5.0e-7 - 14e-7, sgemm.hip's
+// two K groups 3.5e-7 - 9.9e-7 and its partitions 3.9e-7 - 13e-7 (operands ~ N(0, 1)).  Of few results a chain per 16, as exact as sgemm.hip's
+// four and eight K groups: 1.1e-7 - 1.5e-7 from K = 256 to 776.
+// Measured, us per launch, the fastest of sgemm.hip's configurations / of these: 4000 x 2300 x 770 119.3 / 109.4 (94 are the products
+// at the peak rate), 2048^3 130.0 / 123.5, 4096^3 941 / 940, 661 x 11008 x 1024 127.7 / 117.9, 512 x 3072 x 768 25.1 / 23.0, 8134 x 451 x
+// 5225 326 / 298, 283256 x 72 x 331 197 / 137 (64 x 80 tiles; 168 with the waves 2 x 2), 361104 x 36 x 196 92 / 74 (64 x 48; 92),
+// 3325 x 1824 x 328 37.8 / 35.2, 196 x 512 x 256 5.3 / 4.8, 369 x 320 x 608 8.8 / 8.3.  Behind where tiles are few and K is long (29 x 1000 x
+// 11976 18.8 / 147): K groups and partitions stay sgemm.hip's.
 //
 // Compile-time parameters (-D, one shared library per combination):
 //   BLOCK_ROWS x BLOCK_COLS   workgroup tile, of WAVES_M x 4 / WAVES_M waves, whole 16 x 16 tiles each
@@ -37,12 +38,13 @@
 #include "helix_abi.h"
 #include "helix_fastdiv.h"
 #include "helix_ring.h"
+#include "helix_sums.h"
 
 #ifndef BLOCK_ROWS
-#define BLOCK_ROWS 192
+#define BLOCK_ROWS 64
 #endif
 #ifndef BLOCK_COLS
-#define BLOCK_COLS 192
+#define BLOCK_COLS 64
 #endif
 #ifndef WAVES_M
 #define WAVES_M 2
@@ -51,13 +53,13 @@
 namespace {
 
 using namespace helix_ring;
+using helix_sums::Sums;
 
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int BM = BLOCK_ROWS, BN = BLOCK_COLS, WM = WAVES_M, WN = 4 / WM, TM = BM / WM / 16, TN = BN / WN / 16, NM = TM * TN, STAGES = 2, BK = 32;
 constexpr int NTHREADS = 256, STEPS = BK / 8;       // k steps of four in half a K tile
-constexpr int BLOCK_TILES = 8;                      // K tiles whose products are one chain of sums
 constexpr int A_BYTES = BM * BK * 4, STAGE_BYTES = (BM + BN) * BK * 4, RING_BYTES = STAGES * STAGE_BYTES;
 // 1 KiB copies of a K tile, dealt out to the waves, A's from wave 0 on, B's from wave 2 on.  Where a count is no multiple of four
 // the waves it leaves out copy zeros to a place behind the ring: a branch among the products costs more
@@ -107,20 +109,6 @@ __device__ __forceinline__ void each(F&& f) {
     each<N>(f, std::make_integer_sequence<int, N>{});
 }
 
-__device__ __forceinline__ void clear(floatx4 (&acc)[TM][TN]) {
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-}
-
-__device__ __forceinline__ void add(floatx4 (&sum)[TM][TN], const floatx4 (&acc)[TM][TN]) {
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) sum[i][j] += acc[i][j];
-}
-
 template <int W>
 __device__ __forceinline__ void load(const unsigned char* from, float* to) {
     if (W == 4) {
@@ -135,8 +123,8 @@ __device__ __forceinline__ void load(const unsigned char* from, float* to) {
 }
 
 // (the tile parameters are template arguments for the symbol name's sake: a profiler lists configurations separately)
-template <int T_BM = BM, int T_BN = BN>
-__global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const Params p) {
+template <int SUMS, int T_BM = BM, int T_BN = BN>
+__global__ __launch_bounds__(NTHREADS, SUMS == helix_sums::BLOCKS ? 1 : 2) void helix_sgemm_f32_ring_kernel(const Params p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -178,9 +166,9 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
     for (int g = 0; g < GA; g++) at_a[g] = (q * BM + (wave_m * TM + group_first(TM, g)) * 16 + group_width(TM, g) * r) * 4;
 #pragma unroll
     for (int g = 0; g < GB; g++) at_b[g] = A_BYTES + (q * BN + (wave_n * TN + group_first(TN, g)) * 16 + group_width(TN, g) * r) * 4;
-    floatx4 acc[TM][TN], sum[TM][TN];                // of this block of K, of the blocks before it
-    clear(acc);
-    clear(sum);
+    Sums<TM, TN, SUMS> sums;
+    sums.start();
+    constexpr int BLOCK = sums.BLOCK_TILES;
     float fa[2][STEPS][TM], fb[2][STEPS][TN];
     constexpr int READS = STEPS * (GA + GB);
     auto read = [&](int e, int h, int stage) {       // step by step, in the order in which the products take them
@@ -203,7 +191,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
     constexpr int PRODUCTS = STEPS * NM;
     auto multiply = [&](int g, int h) {
         const int s = g / NM, i = g % NM % TM, j = g % NM / TM;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[h][s][i], fb[h][s][j], acc[i][j], 0, 0, 0);
+        sums.multiply(i, j, h * STEPS + s, fa[h][s][i], fb[h][s][j]);
     };
     // fragment reads that are out after g products: they end two thirds into a half
     auto due = [](int g, int reads) constexpr -> int { return 3 * g >= 2 * PRODUCTS ? reads : 3 * g * reads / (2 * PRODUCTS); };
@@ -216,7 +204,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
     // every accumulator twice a tile)
     const int halves = (p.K + BK / 2 - 1) / (BK / 2);
     for (int t = 0, end; t < halves / 2; t = end) {
-        end = t + BLOCK_TILES < halves / 2 ? t + BLOCK_TILES : halves / 2;
+        end = BLOCK && t + BLOCK < halves / 2 ? t + BLOCK : halves / 2;
         for (int u = t; u < end; u++) {
             const int next = stage + 1 == STAGES ? 0 : stage + 1;
             const intx4 ra = rsrc_of(p.A, p.lda, m0, u + STAGES), rb = rsrc_of(p.B, p.ldb, n0, u + STAGES);
@@ -238,13 +226,11 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
             });
             stage = next;
         }
-        if (end < halves / 2) {
-            add(sum, acc);
-            clear(acc);
-        }
+        if constexpr (BLOCK > 0)
+            if (end < halves / 2 || ((halves & 1) && end - t == BLOCK)) sums.end_block();
     }
     if (halves & 1) each<PRODUCTS>([&](auto g) __attribute__((always_inline)) { multiply(g, 0); });
-    add(sum, acc);
+    sums.finish(halves & 1);
     wait<0, true>();                                 // no copy is left when the workgroup gives its LDS back
 
     // ---- results: lanes 0 .. 15 of a quarter hold a piece of a row, 256, 128 or 64 bytes long -----------------------------
@@ -263,16 +249,16 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
                 const int col = n0 + (wave_n * TN + j) * 16 + w * r;
                 float* dst = p.C + (size_t)row * p.ldc + col;
                 if (w == 4 && vec == 4 && col + 4 <= p.N) {
-                    __builtin_nontemporal_store(floatx4{sum[i][j][v], sum[i][j + w / 4][v], sum[i][j + w / 2][v], sum[i][j + w - 1][v]},
+                    __builtin_nontemporal_store(floatx4{sums.sum[i][j][v], sums.sum[i][j + w / 4][v], sums.sum[i][j + w / 2][v], sums.sum[i][j + w - 1][v]},
                                                 (floatx4*)dst);
                 } else if (w >= 2 && vec >= 2 && col + w <= p.N) {
 #pragma unroll
                     for (int e = 0; e < w; e += 2)
-                        __builtin_nontemporal_store(floatx2{sum[i][j + e][v], sum[i][j + e + 1][v]}, (floatx2*)(dst + e));
+                        __builtin_nontemporal_store(floatx2{sums.sum[i][j + e][v], sums.sum[i][j + e + 1][v]}, (floatx2*)(dst + e));
                 } else {
 #pragma unroll
                     for (int e = 0; e < w; e++)
-                        if (col + e < p.N) dst[e] = sum[i][j + e][v];
+                        if (col + e < p.N) dst[e] = sums.sum[i][j + e][v];
                 }
             }
         }
@@ -285,13 +271,12 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_sgemm_f32_ring_kernel(const
 // are the operands of four products.  A copy's lane knows where the first tap of its pixel lies and which taps are inside the
 // image (a bit each); a tile adds the tap's offset, one for all lanes where channels come in 32s, five instructions a copy.
 // Measured, us per launch, the fastest configuration of sgemm.hip and conv_patch.hip / of this (batch x channels x image, filter):
-//   1x1  3 x 256 x 63 x 63 -> 96 12.9 / 9.8    3 x 128 x 49 x 49 -> 192 9.2 / 7.2     2 x 96 x 75 x 75 -> 384 15.4 / 12.5
-//        41 x 128 x 45 x 45 -> 128 35.1 / 30.2  51 x 832 x 15 x 15 -> 160 39.6 / 33.6  45 x 128 x 56 x 56 -> 48 30.3 / 22.5
-//   3x3  11 x 192 x 37 x 37 -> 208 108.5 / 97.2     32 x 256 x 14 x 14 -> 256 82.7 / 75.1    12 x 256 x 27 x 27 -> 160 70.1 / 63.9
-//        7 x 96 x 85 x 85 -> 48 56.6 / 46.7          16 x 128 x 49 x 49 -> 64 58.3 / 51.5
-//   5x5  8 x 16 x 60 x 60 -> 160 44.0 / 39.1        31 x 16 x 109 x 109 -> 48 164 / 130
-// Behind, as in products, where tiles are few and K is long (1 x 256 x 14 x 14 3x3 7.8 / 20.5).  0.922 in the geometric
-// mean over 44 layers.
+//   1x1  3 x 256 x 63 x 63 -> 96 12.6 / 10.1   3 x 128 x 49 x 49 -> 192 9.2 / 7.3     2 x 96 x 75 x 75 -> 384 15.0 / 12.5
+//        41 x 128 x 45 x 45 -> 128 32.1 / 28.5  51 x 832 x 15 x 15 -> 160 37.6 / 33.8  45 x 128 x 56 x 56 -> 48 30.3 / 22.7
+//   3x3  11 x 192 x 37 x 37 -> 208 107.5 / 96.2     32 x 256 x 14 x 14 -> 256 81.1 / 73.4    12 x 256 x 27 x 27 -> 160 68.6 / 63.1
+//        7 x 96 x 85 x 85 -> 48 55.2 / 46.0          16 x 128 x 49 x 49 -> 64 56.1 / 51.1
+//   5x5  8 x 16 x 60 x 60 -> 160 42.3 / 40.2        31 x 16 x 109 x 109 -> 48 163 / 129
+// Behind, as in products, where tiles are few and K is long (1 x 256 x 14 x 14 3x3 8.0 / 20.9).
 
 using helix_fastdiv::FastDiv;
 
@@ -307,8 +292,8 @@ struct ConvParams {
 constexpr int NO_TAP = 31;                          // a bit that no row's mask has
 
 // WHOLE: channels are a multiple of 32, so that a K tile lies in one tap
-template <bool WHOLE, int T_BM = BM, int T_BN = BN>
-__global__ __launch_bounds__(NTHREADS, 1) void helix_conv_f32_ring_kernel(const ConvParams p) {
+template <bool WHOLE, int SUMS, int T_BM = BM, int T_BN = BN>
+__global__ __launch_bounds__(NTHREADS, SUMS == helix_sums::BLOCKS ? 1 : 2) void helix_conv_f32_ring_kernel(const ConvParams p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -357,14 +342,23 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_conv_f32_ring_kernel(const 
         offset = ((row * p.W + at - row * p.kW) * p.IC + k - at * p.IC) * 4;
     };
     auto step = [&]() {                              // WHOLE: to the next tile
-        c += BK;
-        offset += BK * 4;
-        if (c == p.IC) {
-            c = 0;
-            tap = tap < NO_TAP ? tap + 1 : NO_TAP;
-            if (++kw == p.kW) {
-                kw = 0;
-                offset += (p.W - p.kW) * p.IC * 4;
+        // by selection where around a branch the compiler holds the accumulators twice; elsewhere the branch is the shorter way
+        if constexpr (SUMS == helix_sums::FINE || (SUMS == helix_sums::HALVES && NM > 4)) {
+            const bool next_tap = c + BK == p.IC, next_row = next_tap && kw + 1 == p.kW;
+            c = next_tap ? 0 : c + BK;
+            tap += next_tap && tap < NO_TAP ? 1 : 0;
+            kw = next_row ? 0 : next_tap ? kw + 1 : kw;
+            offset += BK * 4 + (next_row ? (p.W - p.kW) * p.IC * 4 : 0);
+        } else {
+            c += BK;
+            offset += BK * 4;
+            if (c == p.IC) {
+                c = 0;
+                tap = tap < NO_TAP ? tap + 1 : NO_TAP;
+                if (++kw == p.kW) {
+                    kw = 0;
+                    offset += (p.W - p.kW) * p.IC * 4;
+                }
             }
         }
     };
@@ -389,9 +383,9 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_conv_f32_ring_kernel(const 
         at_a[h] = (wave_m * TM * 16 + r) * BK * 4 + chunk;
         at_b[h] = A_BYTES + (wave_n * TN * 16 + r) * BK * 4 + chunk;
     }
-    floatx4 acc[TM][TN], sum[TM][TN];                // of this block of K, of the blocks before it
-    clear(acc);
-    clear(sum);
+    Sums<TM, TN, SUMS> sums;
+    sums.start();
+    constexpr int BLOCK = sums.BLOCK_TILES;
     floatx4 fa[2][TM], fb[2][TN];
     constexpr int READS = TM + TN, PRODUCTS = 4 * NM;
     auto read = [&](int e, int h, int stage) {
@@ -402,7 +396,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_conv_f32_ring_kernel(const 
     // the filters go first, which leaves a lane with four consecutive columns of one row
     auto multiply = [&](int g, int h) {
         const int e = g / NM, i = g % NM % TM, j = g % NM / TM;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[h][j][e], fa[h][i][e], acc[i][j], 0, 0, 0);
+        sums.multiply(i, j, h * 4 + e, fb[h][j][e], fa[h][i][e]);
     };
     auto due = [](int g, int reads) constexpr -> int { return 3 * g >= 2 * PRODUCTS ? reads : 3 * g * reads / (2 * PRODUCTS); };
 
@@ -412,7 +406,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_conv_f32_ring_kernel(const 
     int stage = 0;
     const int halves = (p.K + BK / 2 - 1) / (BK / 2);       // as in the products' loop
     for (int t = 0, end; t < halves / 2; t = end) {
-        end = t + BLOCK_TILES < halves / 2 ? t + BLOCK_TILES : halves / 2;
+        end = BLOCK && t + BLOCK < halves / 2 ? t + BLOCK : halves / 2;
         for (int u = t; u < end; u++) {
             const int next = stage + 1 == STAGES ? 0 : stage + 1;
             each<PRODUCTS>([&](auto g) __attribute__((always_inline)) {
@@ -434,13 +428,11 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_conv_f32_ring_kernel(const 
             if (WHOLE) step();
             stage = next;
         }
-        if (end < halves / 2) {
-            add(sum, acc);
-            clear(acc);
-        }
+        if constexpr (BLOCK > 0)
+            if (end < halves / 2 || ((halves & 1) && end - t == BLOCK)) sums.end_block();
     }
     if (halves & 1) each<PRODUCTS>([&](auto g) __attribute__((always_inline)) { multiply(g, 0); });
-    add(sum, acc);
+    sums.finish(halves & 1);
     wait<0, true>();                                 // no copy is left when the workgroup gives its LDS back
 
     // ---- results: a quarter's lanes hold 16 bytes of 16 rows ---------------------------------------------------------------
@@ -454,11 +446,11 @@ __global__ __launch_bounds__(NTHREADS, 1) void helix_conv_f32_ring_kernel(const 
             const int col = n0 + (wave_n * TN + j) * 16 + 4 * q;
             float* dst = p.y + (size_t)row * p.N + col;
             if (wide && col + 4 <= p.N) {
-                __builtin_nontemporal_store(sum[i][j], (floatx4*)dst);
+                __builtin_nontemporal_store(sums.sum[i][j], (floatx4*)dst);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    if (col + e < p.N) dst[e] = sum[i][j][e];
+                    if (col + e < p.N) dst[e] = sums.sum[i][j][e];
             }
         }
     }
@@ -499,6 +491,15 @@ inline void bench_layout(int M, int N, int K, size_t* ae, size_t* be, size_t* ce
     *lda = Mp; *ldb = Np; *ldc = Np;
 }
 
+template <int SUMS>
+inline int launch_gemm(const Params& p, unsigned grid, hipStream_t s) {
+    static int rc = (int)hipFuncSetAttribute((const void*)helix_sgemm_f32_ring_kernel<SUMS>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+    if (rc) return rc;
+    hipLaunchKernelGGL(helix_sgemm_f32_ring_kernel<SUMS>, dim3(grid), dim3(NTHREADS), LDS_BYTES, s, p);
+    return (int)hipGetLastError();
+}
+
 // Rows of `ld` floats as an operand: byte offsets inside one K tile are 31-bit, in all as sgemm.hip takes them
 inline bool operand_fits(int K, int ld) { return (long long)K * ld * 4 < 0xffffffffLL && (long long)BK * ld * 4 < 0x7fffffffLL; }
 
@@ -510,21 +511,26 @@ inline int gemm(const void* A, const void* B, void* C, int M, int N, int K, int 
     Params p{(const float*)A, (const float*)B, (float*)C, M, N, K, lda, ldb, ldc, (M - 1) / BM + 1, (N - 1) / BN + 1};
     const long long ntiles = (long long)p.tiles_m * p.tiles_n;
     if (ntiles > 0x3fffffffLL) return HELIX_ERR_INVALID_VALUE;
-    static int rc = (int)hipFuncSetAttribute((const void*)helix_sgemm_f32_ring_kernel<>,
+    const unsigned grid = (unsigned)((ntiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
+    switch (helix_sums::mode_of(M, N, K)) {
+        case helix_sums::FINE: return launch_gemm<helix_sums::finest(TM, TN)>(p, grid, s);
+        case helix_sums::HALVES: return launch_gemm<helix_sums::HALVES>(p, grid, s);
+        default: return launch_gemm<helix_sums::BLOCKS>(p, grid, s);
+    }
+}
+
+template <bool WHOLE, int SUMS>
+inline int launch_conv(const ConvParams& p, unsigned grid, hipStream_t s) {
+    static int rc = (int)hipFuncSetAttribute((const void*)helix_conv_f32_ring_kernel<WHOLE, SUMS>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
     if (rc) return rc;
-    const unsigned grid = (unsigned)((ntiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
-    hipLaunchKernelGGL(helix_sgemm_f32_ring_kernel<>, dim3(grid), dim3(NTHREADS), LDS_BYTES, s, p);
+    hipLaunchKernelGGL((helix_conv_f32_ring_kernel<WHOLE, SUMS>), dim3(grid), dim3(NTHREADS), LDS_BYTES, s, p);
     return (int)hipGetLastError();
 }
 
-template <bool WHOLE>
+template <int SUMS>
 inline int launch_conv(const ConvParams& p, unsigned grid, hipStream_t s) {
-    static int rc = (int)hipFuncSetAttribute((const void*)helix_conv_f32_ring_kernel<WHOLE>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-    if (rc) return rc;
-    hipLaunchKernelGGL(helix_conv_f32_ring_kernel<WHOLE>, dim3(grid), dim3(NTHREADS), LDS_BYTES, s, p);
-    return (int)hipGetLastError();
+    return p.IC % BK == 0 ? launch_conv<true, SUMS>(p, grid, s) : launch_conv<false, SUMS>(p, grid, s);
 }
 
 inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W, int IC, int OC, int kH, int kW, int stride,
@@ -543,7 +549,11 @@ inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W
     const long long ntiles = (long long)p.tiles_m * p.tiles_n;
     if (ntiles > 0x3fffffffLL) return HELIX_ERR_INVALID_VALUE;
     const unsigned grid = (unsigned)((ntiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
-    return IC % BK == 0 ? launch_conv<true>(p, grid, s) : launch_conv<false>(p, grid, s);
+    switch (helix_sums::mode_of(M, OC, K)) {
+        case helix_sums::FINE: return launch_conv<helix_sums::finest(TM, TN)>(p, grid, s);
+        case helix_sums::HALVES: return launch_conv<helix_sums::HALVES>(p, grid, s);
+        default: return launch_conv<helix_sums::BLOCKS>(p, grid, s);
+    }
 }
 
 }  // namespace tpl

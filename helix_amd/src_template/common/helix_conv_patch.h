@@ -20,21 +20,23 @@
 //     MFMA's order through a piece of LDS that is its own: no barrier between the first product and the last.  (Loaded in the
 //     MFMA's order, 16 rows x 64 bytes per instruction, they come at a quarter of the rate: 15.7 instead of 53 bytes per clock
 //     and CU, one cache line looked up for each lane.)
-//   * results leave from registers, 16 bytes per lane.
+//   * results leave from registers, 16 bytes per lane;
+//   * FP32 sums are cut as common/helix_sums.h says: few results as exactly as sgemm.hip's K groups (1.1e-7 in the norm at 2 x 128 x 7 x 7
+//     3x3 -> 96, where a chain per part of K left 2.3e-7), many in chains of 256 (2.8e-7 at 32 x 128 x 28 x 28, 6.0e-7 in one).
 //
 // Measured (us per launch, the fastest configuration of the implicit GEMM / of this family; batch x channels x image, filter):
 //   FP16  4 x 256 x 14 x 14 3x3 -> 256 10.1 / 6.6    2 x 512 x 16 x 16 3x3 -> 256 10.1 / 6.5    2 x 112 x 14 x 14 3x3 -> 208 7.4 / 4.7
 //         1 x 256 x 13 x 13 3x3 -> 160 7.7 / 5.0     2 x 96 x 15 x 15 5x5 -> 512 9.4 / 6.6      4 x 192 x 9 x 9 3x3 -> 48 6.7 / 4.6
 //         32 x 64 x 56 x 56 3x3 -> 64 15.1 / 14.5    32 x 256 x 14 x 14 3x3 -> 256 15.2 / 13.5  16 x 48 x 40 x 40 5x5 -> 96 13.0 / 11.3
-//   FP32  32 x 128 x 28 x 28 3x3 -> 128 68.6 / 66.8  4 x 256 x 14 x 14 3x3 -> 256 18.4 / 16.2   5 x 32 x 64 x 64 5x5 -> 64 27.8 / 23.3
-//         1 x 24 x 10 x 10 3x3 -> 256 7.2 / 4.4      2 x 128 x 7 x 7 3x3 -> 96 9.0 / 5.7        2 x 25 x 70 x 70 1x1 -> 16 8.5 / 5.0
-//         22 x 3 x 154 x 154 5x5 stride 4 -> 64 21.1 / 12.8, 2 x 3 x 122 x 122 5x5 stride 2 -> 32 9.0 / 5.8
+//   FP32  32 x 128 x 28 x 28 3x3 -> 128 69.3 / 67.7  4 x 256 x 14 x 14 3x3 -> 256 18.8 / 17.2   5 x 32 x 64 x 64 5x5 -> 64 27.3 / 23.5
+//         1 x 24 x 10 x 10 3x3 -> 256 7.3 / 4.5      2 x 128 x 7 x 7 3x3 -> 96 9.0 / 5.9        2 x 25 x 70 x 70 1x1 -> 16 8.5 / 5.0
+//         22 x 3 x 154 x 154 5x5 stride 4 -> 64 21.1 / 13.4, 2 x 3 x 122 x 122 5x5 stride 2 -> 32 9.1 / 6.0
 // Slower, and left to the implicit GEMM by the selection, which times both: FP16 filters with stride 2 on large images; images or
 // channel counts that leave room for few pixels in LDS (FP16 9 x 96 x 106 x 106 3x3 -> 128 32 / 50).  Strips of columns and passes
 // over the channels, which would fit those, were built in FP16 and measured: never ahead there, half a microsecond slower
 // everywhere else.  What bounds it where it runs: small layers launch, first loads and staging (2.6 + 2 us); large FP16 ones LDS (22
 // KB read and written per 28 products of a 112 x 32 wave tile), with staging and stores in front of and behind the loop over K, not
-// beside it; FP32 ones the matrix pipes, at 0.8 of their rate.
+// beside it; FP32 ones the matrix pipes, at 0.75 of their rate.
 //
 // Compile-time parameters (-D, one shared library per combination):
 //   BLOCK_ROWS x BLOCK_COLS   output pixels x channels of a workgroup
@@ -50,6 +52,7 @@
 
 #include "helix_abi.h"
 #include "helix_fastdiv.h"
+#include "helix_sums.h"
 
 #ifndef BLOCK_ROWS
 #define BLOCK_ROWS 32
@@ -176,8 +179,9 @@ __device__ __forceinline__ int channel_of(int j, int r) {
 __device__ __forceinline__ int pixel_of(int r) { return r < 4 ? r : r < 12 ? r + 4 : r - 8; }
 
 // (REST: K is not whole tiles.  The tile parameters are template arguments for the symbol name's sake: a profiler lists configurations separately)
-template <bool TAIL, bool REST, int T_BM = BLOCK_ROWS, int T_BN = BLOCK_COLS, int T_WM = WAVE_ROWS, int T_WN = WAVE_COLS, int T_KG = K_GROUPS, bool T_F32 = F32>
-__global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Params p) {
+// (wave tiles of more than ten have no room for two sets of FP32 accumulators in 256 registers; one of their workgroups fills a CU)
+template <bool TAIL, bool REST, int SUMS, int T_BM = BLOCK_ROWS, int T_BN = BLOCK_COLS, int T_WM = WAVE_ROWS, int T_WN = WAVE_COLS, int T_KG = K_GROUPS, bool T_F32 = F32>
+__global__ __launch_bounds__(NTHREADS, F32 && TM * TN > 10 ? 1 : 2) void helix_conv_patch_kernel(const Params p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int block = (int)(blockIdx.x % NUM_XCD) * p.blocks_per_xcd + (int)(blockIdx.x / NUM_XCD);
     if (block >= p.blocks) return;
@@ -277,11 +281,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Par
     __syncthreads();
 
     // ---- products ----------------------------------------------------------------------------------------------------
-    floatx4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    helix_sums::Sums<TM, TN, SUMS> sums;
+    sums.start();
     const int* table = (const int*)(smem + TABLE_OFFSET) + q;
     typedef std::conditional<F32, floatx4, half8>::type frag;
     // rows of 128 bytes, 16-byte chunk c of row r at c ^ (r / 2 mod 8): reads and writes free of bank conflicts
@@ -295,8 +296,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Par
     constexpr int SLOTS = TM * TN * PRODUCTS;
     auto multiply = [&](int g, int s) {
         const int i = g % TM, j = g / TM % TN, e = g / (TM * TN);
-        if constexpr (F32) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[s][j][e], a[s][i][e], acc[i][j], 0, 0, 0);
-        else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[s][j], a[s][i], acc[i][j], 0, 0, 0);
+        if constexpr (F32) sums.multiply(i, j, s * PRODUCTS + e, b[s][j][e], a[s][i][e]);
+        else sums.sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[s][j], a[s][i], sums.sum[i][j], 0, 0, 0);
     };
     // One K tile, st holding the weights of the next one.  Behind each MFMA its share of the other instructions, in the order in
     // which the products take them and in the first two thirds of the step, so that the last ones have arrived when the next
@@ -357,14 +358,33 @@ __global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Par
     const bool half = REST && chunk_end > KT_CHUNKS * t_begin && (chunk_end - 1) % KT_CHUNKS < 4;
     const int t_whole = t_end - half;
     int t = t_begin;
-    for (; t + AHEAD <= t_whole; t += AHEAD) {
-        tile(t, st[1]);
-        tile(t + 1, st[0]);
+    if constexpr (sums.BLOCK_TILES == 0) {
+        for (; t + AHEAD <= t_whole; t += AHEAD) {
+            tile(t, st[1]);
+            tile(t + 1, st[0]);
+        }
+    } else {
+        constexpr int BLOCK_TILES = sums.BLOCK_TILES;
+        static_assert(BLOCK_TILES == 1 || BLOCK_TILES % AHEAD == 0, "blocks of sums end between tiles");
+        for (int end; t + AHEAD <= t_whole; ) {
+            end = BLOCK_TILES == 1 || BLOCK_TILES > t_whole - t ? t + (t_whole - t) / AHEAD * AHEAD : t + BLOCK_TILES;
+            for (; t < end; t += AHEAD) {
+                tile(t, st[1]);
+                if constexpr (BLOCK_TILES == 1) sums.end_block();
+                tile(t + 1, st[0]);
+                if constexpr (BLOCK_TILES == 1) sums.end_block();
+            }
+            if (BLOCK_TILES > 1 && (t < t_whole || half)) sums.end_block();
+        }
     }
-    if (t < t_whole) tile(t, st[1]);
+    if (t < t_whole) {
+        tile(t, st[1]);
+        if constexpr (sums.BLOCK_TILES == 1) sums.end_block();
+    }
     if (half)
 #pragma unroll
         for (int g = 0; g < SLOTS; g++) multiply(g, 0);
+    sums.finish(half);
 
     // ---- results -----------------------------------------------------------------------------------------------------
     constexpr int PAIR = F32 || TN % 2 ? 1 : 2, UNITS = TM * (TN / PAIR);
@@ -392,26 +412,26 @@ __global__ __launch_bounds__(NTHREADS, 2) void helix_conv_patch_kernel(const Par
             for (int jj = 0; jj < TN / PAIR; jj++) {
                 floatx4 v[PAIR];
 #pragma unroll
-                for (int e = 0; e < PAIR; e++) v[e] = acc[i][jj * PAIR + e];
+                for (int e = 0; e < PAIR; e++) v[e] = sums.sum[i][jj * PAIR + e];
                 store(i, jj, v);
             }
     } else {
         // parts of K: added through LDS in their order, the units of a wave's tile shared out over its parts
         __syncthreads();
-        floatx4* sums = (floatx4*)smem + (size_t)(wave_m * WAVES_N + wave_n) * K_GROUPS * (TM * TN * 64);
+        floatx4* parts = (floatx4*)smem + (size_t)(wave_m * WAVES_N + wave_n) * K_GROUPS * (TM * TN * 64);
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) sums[(part * (TM * TN) + i * TN + j) * 64 + lane] = acc[i][j];
+            for (int j = 0; j < TN; j++) parts[(part * (TM * TN) + i * TN + j) * 64 + lane] = sums.sum[i][j];
         __syncthreads();
         for (int u = part; u < UNITS; u += K_GROUPS) {
             const int i = u / (TN / PAIR), jj = u % (TN / PAIR);
             floatx4 v[PAIR];
 #pragma unroll
-            for (int e = 0; e < PAIR; e++) v[e] = sums[(i * TN + jj * PAIR + e) * 64 + lane];
+            for (int e = 0; e < PAIR; e++) v[e] = parts[(i * TN + jj * PAIR + e) * 64 + lane];
             for (int k = 1; k < K_GROUPS; k++)
 #pragma unroll
-                for (int e = 0; e < PAIR; e++) v[e] += sums[(k * (TM * TN) + i * TN + jj * PAIR + e) * 64 + lane];
+                for (int e = 0; e < PAIR; e++) v[e] += parts[(k * (TM * TN) + i * TN + jj * PAIR + e) * 64 + lane];
             store(i, jj, v);
         }
     }
@@ -515,13 +535,21 @@ inline bool make_plan(Params& p, int* lds_bytes, int batch, int H, int W, int IC
 // Which variant runs a layer: REST of the kernel
 inline bool has_rest(const Params& p) { return (F32 && p.tail) || p.chunks % KT_CHUNKS; }
 
-template <bool TAIL, bool REST>
+template <bool TAIL, bool REST, int SUMS>
 inline int launch(const Params& p, int lds_bytes, hipStream_t s) {
-    static int rc = (int)hipFuncSetAttribute((const void*)helix_conv_patch_kernel<TAIL, REST>,
+    static int rc = (int)hipFuncSetAttribute((const void*)helix_conv_patch_kernel<TAIL, REST, SUMS>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     if (rc) return rc;
-    hipLaunchKernelGGL((helix_conv_patch_kernel<TAIL, REST>), dim3((unsigned)(NUM_XCD * p.blocks_per_xcd)), dim3(NTHREADS), lds_bytes, s, p);
+    hipLaunchKernelGGL((helix_conv_patch_kernel<TAIL, REST, SUMS>), dim3((unsigned)(NUM_XCD * p.blocks_per_xcd)), dim3(NTHREADS), lds_bytes, s, p);
     return (int)hipGetLastError();
+}
+
+template <int SUMS>
+inline int launch_variant(const Params& p, int lds_bytes, hipStream_t s) {
+    // (with a tail the compiler holds the accumulators of HALVES twice)
+    if constexpr (F32)
+        if (p.tail) return launch<true, true, SUMS == helix_sums::HALVES && TM * TN >= 8 ? helix_sums::TILES : SUMS>(p, lds_bytes, s);
+    return has_rest(p) ? launch<false, true, SUMS>(p, lds_bytes, s) : launch<false, false, SUMS>(p, lds_bytes, s);
 }
 
 inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W, int IC, int OC, int kH, int kW, int stride,
@@ -533,10 +561,15 @@ inline int conv2d(const void* x, const void* w, void* y, int batch, int H, int W
     p.x = (const elem*)x; p.w = (const elem*)w; p.y = (elem*)y;
     constexpr int STORE = F32 || TN == 1 ? 4 : 8;      // channels of a lane's store
     p.wide = OC % STORE == 0 && ((uintptr_t)y & (EB * STORE - 1)) == 0;
-    if constexpr (F32)
-        if (p.tail) return launch<true, true>(p, lds_bytes, s);
-    if (has_rest(p)) return launch<false, true>(p, lds_bytes, s);
-    return launch<false, false>(p, lds_bytes, s);
+    if constexpr (F32) {
+        switch (helix_sums::mode_of(p.M, OC, (long long)p.taps * IC, K_GROUPS)) {
+            case helix_sums::FINE: return launch_variant<helix_sums::finest(TM, TN)>(p, lds_bytes, s);
+            case helix_sums::HALVES: return launch_variant<helix_sums::HALVES>(p, lds_bytes, s);
+            default: return launch_variant<helix_sums::BLOCKS>(p, lds_bytes, s);
+        }
+    } else {
+        return launch_variant<helix_sums::CHAIN>(p, lds_bytes, s);
+    }
 }
 
 }  // namespace tpl

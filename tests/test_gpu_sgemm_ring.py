@@ -7,8 +7,9 @@ import torch
 from utils.helix_runtime import load
 from utils.hip_ctypes import HELIX_ERR_INVALID_VALUE, HELIX_ERR_UNSUPPORTED
 from MI355X_FP32 import build_MI355X_FP32 as b32
+from MI355X_FP32 import MI355X_FP32_conv as c32
 from oracle import oracle as O
-from gpu_helpers import dev, run_conv, run_sgemm_f32
+from gpu_helpers import conv_out_hw, dev, run_conv, run_gemv_f32, run_sgemm_f32
 
 pytestmark = pytest.mark.gpu
 
@@ -30,18 +31,59 @@ def test_every_configuration_integer_exact(problem):
 
 
 def test_sums_next_to_sgemm():
-    """Up to 256 of K the products of a result are added in ascending k, each rounded, as in an unpartitioned launch of sgemm.hip;
-    longer chains are cut there, which leaves less error than its two K groups."""
+    """Results beyond 5 x 2^20: up to 256 of K their products are added in ascending k, each rounded, as in an unpartitioned launch of
+    sgemm.hip; longer chains are cut there, half a K tile behind them included (the error of one product behind 256 is that of 257).  That leaves
+    less error than its two K groups."""
     rng = np.random.default_rng(4)
+    A, B = rng.standard_normal((2600, 272)).astype(np.float32), rng.standard_normal((272, 2500)).astype(np.float32)
+    for K in (255, 256, 257, 272):
+        plain = run_sgemm_f32(load(b32.default_library()), A[:, :K], B[:K], workspace=False)
+        exact = A[:, :K].astype(np.float64) @ B[:K].astype(np.float64)
+        for key in b32.RING_KEYS:
+            got = run_sgemm_f32(load(b32.library_for_key(key)), A[:, :K], B[:K])
+            assert np.array_equal(got, plain) if K <= 256 else error(got, exact) <= 1.01 * error(plain, exact), (key, K)
     A, B = rng.standard_normal((290, 2600)).astype(np.float32), rng.standard_normal((2600, 301)).astype(np.float32)
-    short = run_sgemm_f32(load(b32.default_library()), A[:, :255], B[:255], workspace=False)
     exact = A.astype(np.float64) @ B.astype(np.float64)
-    error = lambda got: np.linalg.norm(got - exact)
-    limit = error(run_sgemm_f32(load(b32.sgemm_library(64, 64, 32, 32, 32, 2)), A, B, workspace=False))
+    limit = error(run_sgemm_f32(load(b32.sgemm_library(64, 64, 32, 32, 32, 2)), A, B, workspace=False), exact)
     for key in b32.RING_KEYS:
-        lib = load(b32.library_for_key(key))
-        assert np.array_equal(run_sgemm_f32(lib, A[:, :255], B[:255]), short), key
-        assert error(run_sgemm_f32(lib, A, B)) <= limit, key
+        assert error(run_sgemm_f32(load(b32.library_for_key(key)), A, B), exact) <= limit, key
+
+
+def error(got, exact):
+    return np.linalg.norm(got - exact) / np.linalg.norm(exact)
+
+
+# The norm of n results' errors scatters by sqrt(1 / 2 n) of itself between two ways of summing that are equally exact: four times that
+def scatter(n):
+    return 1 + 4 * (0.5 / n) ** 0.5
+
+
+def wave_tiles(key):
+    """16 x 16 tiles of a wave."""
+    return (key[3] // 16) * (key[4] // 16)
+
+
+@pytest.mark.parametrize("K", [200, 256, 257, 272, 480, 800])
+def test_few_results_are_as_exact_as_k_groups(K):
+    """Where sgemm.hip's fastest configurations have four or eight K groups; K = 257 and 272 end half a K tile behind a whole one."""
+    rng = np.random.default_rng(K)
+    A, B = rng.standard_normal((290, K)).astype(np.float32), rng.standard_normal((K, 301)).astype(np.float32)
+    exact = A.astype(np.float64) @ B.astype(np.float64)
+    limit = min(error(run_sgemm_f32(load(b32.sgemm_library(*c)), A, B, workspace=False), exact)
+                for c in b32.iter_kgroup_configs() if c[5] in (4, 8))
+    for key in b32.RING_KEYS:
+        assert error(run_sgemm_f32(load(b32.library_for_key(key)), A, B), exact) <= limit * scatter(290 * 301), key
+
+
+@pytest.mark.parametrize("K", [260, 500, 1400])
+def test_few_columns_are_as_exact_as_the_gemv(K):
+    rng = np.random.default_rng(K)
+    A, B = rng.standard_normal((3000, K)).astype(np.float32), rng.standard_normal((K, 7)).astype(np.float32)
+    exact = A.astype(np.float64) @ B.astype(np.float64)
+    limit = error(run_gemv_f32(load(b32.kernel_library("gemv_fp32")), B.T, A.T).T, exact)
+    for key in b32.RING_KEYS:
+        if wave_tiles(key) <= 4:                         # what such problems are run on
+            assert error(run_sgemm_f32(load(b32.library_for_key(key)), A, B), exact) <= limit * scatter(3000 * 7), key
 
 
 def test_many_tiles_integer_exact():
@@ -163,3 +205,37 @@ def test_infinities_in_the_input_reach_their_pixels_only():
     want[0, 4:6, 5:7] = np.inf
     for key in b32.RING_KEYS:
         assert np.array_equal(run_conv(load(b32.library_for_key(key)), x, w, 1, 1, torch.float32), want), key
+
+
+# batch, channels, H, W, filters, kH, kW, stride, pad: K = 75, 300, 800, 1200
+EXACT_LAYERS = [(3, 3, 40, 40, 33, 5, 5, 2, 2), (2, 12, 20, 20, 33, 5, 5, 1, 2), (1, 32, 24, 24, 64, 5, 5, 1, 2), (1, 48, 20, 20, 96, 5, 5, 1, 2)]
+
+
+@pytest.mark.parametrize("layer", EXACT_LAYERS, ids=lambda l: "x".join(map(str, l)))
+def test_convolutions_are_as_exact_as_k_groups(layer):
+    """The ring tiles and the family whose input stays in LDS, next to sgemm.hip's four and eight K groups."""
+    B, IC, H, W, OC, kH, kW, stride, pad = layer
+    rng = np.random.default_rng(sum(layer))
+    x, w = rng.standard_normal((B, H, W, IC)).astype(np.float32), rng.standard_normal((OC, kH, kW, IC)).astype(np.float32)
+    exact = np.zeros((B, *conv_out_hw(H, W, kH, kW, stride, pad), OC))
+    xp = np.pad(x.astype(np.float64), ((0, 0), (pad, pad), (pad, pad), (0, 0)))
+    for i in range(kH):
+        for j in range(kW):
+            exact += xp[:, i:, j:][:, :(exact.shape[1] - 1) * stride + 1:stride, :(exact.shape[2] - 1) * stride + 1:stride] @ w[:, i, j].T.astype(np.float64)
+    keys = [k for k in b32.patch_keys() if c32.PATCH.layout((k[0], k[1], k[3], k[4], k[6]), *layer)] + (list(b32.RING_KEYS) if IC % 4 == 0 else [])
+
+    def result(lib):
+        dx, dw, dy = dev(x), dev(w), torch.empty(exact.shape, dtype=torch.float32, device="cuda:0")
+        # without a workspace K is not partitioned beside; a channel count off 4 needs it for its copies
+        wsb = lib.conv_workspace_bytes(B, H, W, IC, OC, kH, kW, stride, pad) if IC % 4 else 0
+        ws = torch.empty(max(wsb, 16), dtype=torch.uint8, device="cuda:0")
+        lib.conv2d(dx.data_ptr(), dw.data_ptr(), dy.data_ptr(), B, H, W, IC, OC, kH, kW, stride, pad, ws.data_ptr() if wsb else 0, wsb)
+        return dy.cpu().numpy()
+
+    errors = {}
+    for c in b32.iter_kgroup_configs():
+        errors[c[5]] = min(errors.get(c[5], 1.0), error(result(load(b32.sgemm_library(*c))), exact))
+    for key in keys:
+        # wave tiles of eight and more add a chain per K tile where channels are off 4, and are held to two groups there
+        limit = errors[2] if IC % 4 and wave_tiles(key) >= 8 else min(errors[4], errors[8])
+        assert error(result(load(b32.library_for_key(key))), exact) <= limit * scatter(exact.size), key
