@@ -12,10 +12,10 @@ repack + GEMM), all on one stream and timed as one.
 import math
 import os
 
-from utils.helix_runtime import load, kernel_resources, tuned_config, fastest_of
+from utils.helix_runtime import load, kernel_resources, tuned_config, fastest_of, operand_sets
 from utils.conv_patch import PatchFamily, PATCH_TOP
 from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, is_dtl_key, patch_key, PATCH_KEYS, PATCH_POINTS, RING_KEYS
-from MI355X_FP16.MI355X_FP16_gemm import short_value, config_cost, handicap, ring_first, ring_ranked, RING_CONV, RING_TOP, VERIFY_TOP
+from MI355X_FP16.MI355X_FP16_gemm import short_value, config_cost, ring_first, ring_ranked, RING_CONV, RING_TOP, VERIFY_TOP
 
 root_path = os.getcwd()
 
@@ -183,14 +183,19 @@ def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, k
         return next((k for k in ranked if k[5] == 0), ranked[0])
 
     def time_config(k, warmup, iters):
-        return handicap(k) * load(library_for_key(k)).bench_conv(batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
-                                                                 warmup=warmup, iters=iters)[1]
+        return load(library_for_key(k)).bench_conv(*layer, warmup=warmup, iters=iters, sets=operand_sets(layer_bytes(*layer)))[1]
 
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return fastest_of(ranked_configs(prof_dict, M, output_channel, ICg * kH * kW, ICg, top,
                                      is_pointwise(kH, kW, stride, pad) and input_channel % GATHER_CHUNK == 0)
                       + (unprofiled_ranked(*layer) if families else []),
                       time_config, "this layer")
+
+
+def layer_bytes(batch, input_channel, H, W, output_channel, kH, kW, stride, pad):
+    """Input, weights and results of a layer."""
+    M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
+    return 2 * (batch * input_channel * H * W + output_channel * input_channel * kH * kW + M * output_channel)
 
 
 RING_MAX_TAPS = 31      # of the ring tiles' convolution (src_template/MI355X_FP16/gemm_ring.hip): a bit of a row's mask each
@@ -202,7 +207,7 @@ def unprofiled_ranked(batch, input_channel, H, W, output_channel, kH, kW, stride
     keys = patch_ranked((batch, input_channel, H, W, output_channel, kH, kW, stride, pad))
     if input_channel % GATHER_CHUNK == 0 and kH * kW <= RING_MAX_TAPS:
         M, K = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1), input_channel * kH * kW
-        moved = 2 * (batch * input_channel * H * W + output_channel * K + M * output_channel)
+        moved = layer_bytes(batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
         keys += (ring_ranked(M, output_channel, K) if is_pointwise(kH, kW, stride, pad) else
                  ring_first(M, output_channel, K, moved, RING_CONV, RING_TOP))
     return keys

@@ -7,9 +7,9 @@ has no counterpart: the only backend value is "hip".
 import math
 import os
 
-from utils.helix_runtime import load, tuned_config, fastest_of
+from utils.helix_runtime import load, tuned_config, fastest_of, operand_sets, CACHE_BYTES
 from utils.roofline import NUM_CU, HBM_BYTES_PER_S, gemm_bytes
-from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, SPLITK_MAX, RING_KEYS, is_ring_key
+from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, SPLITK_MAX, RING_KEYS
 from MI355X_FP16.profile_MI355X_FP16 import PROFILE_K, PROFILE_K_SHORT
 
 root_path = os.getcwd()
@@ -161,11 +161,6 @@ RING_TOP = 4
 RING_GEMM = (3990, 32 * 1.84, 31, 476, 4.4e12, 0)
 RING_CONV = (6700, 53.6, 40, 236, 10e12, 132)
 RING_LDS_BYTES = 160 * 1024
-# The selection repeats a launch on one set of operands, which small ones leave in L2; with three sets in turn these tiles, whose few
-# stages wait for each copy, lose more than the older ones: 127619 x 5 x 458 20.4 / 20.9 us on one set, 26.7 / 24.5 on three; 4096 x
-# 3072 x 768 21.5 / 22.4 and 21.1 / 21.6.  So they have to be ahead by this much.
-RING_HANDICAP = 1.03
-
 
 def ring_seconds(key, M, N, K, moved, constants):
     """Predicted seconds of a configuration of that family on a problem that moves `moved` bytes."""
@@ -187,10 +182,6 @@ def ring_seconds(key, M, N, K, moved, constants):
     return max(clocks / 2.4e9, moved / rate + 2.5e-6)
 
 
-def handicap(key):
-    return RING_HANDICAP if is_ring_key(key) else 1.0
-
-
 def ring_first(M, N, K, moved, constants, top):
     """The `top` configurations of that family with the lowest predicted time, best first."""
     return sorted(RING_KEYS, key=lambda k: (ring_seconds(k, M, N, K, moved, constants), k))[:top]
@@ -206,16 +197,17 @@ def padded_k(K):
     return math.ceil(K / 8) * 8
 
 
-def run_config(k, M, N, K, warmup=10, iters=10, outer=1, copies=1):
+def run_config(k, M, N, K, warmup=10, iters=10, outer=1, copies=0):
     """Seconds per launch (mean) of configuration k on the real, unpadded M and N.  The reference pads
     M and N up to the tile (Ampere_FP16_gemm.py:438) because its kernel has no bounds checks; the
-    MI355X kernels predicate their edges instead.  `copies`: copies of the second operand that the launches
-    take in turn."""
+    MI355X kernels predicate their edges instead.  `copies`: of the second operand that the launches take in turn; one: sets
+    of all operands in turn, as many as operand_sets says; none: one launch after the other on the same operands."""
     lib = load(library_for_key(k))
     if k[0] == 0 and M > N:
         M, N = N, M   # the GEMV kernel streams its second operand; gemv.cu:384-386 swaps the same way
     rotate = copies * N * padded_k(K) * 2 if copies > 1 else 0
-    _, avg, _ = lib.bench(M, N, padded_k(K), warmup=warmup, iters=iters, outer=outer, rotate_bytes=rotate)
+    sets = operand_sets(gemm_bytes(M, N, padded_k(K), 2)) if copies == 1 else 1
+    _, avg, _ = lib.bench(M, N, padded_k(K), warmup=warmup, iters=iters, outer=outer, rotate_bytes=rotate, sets=sets)
     return avg
 
 
@@ -224,9 +216,9 @@ def run_config(k, M, N, K, warmup=10, iters=10, outer=1, copies=1):
 # on as many copies of the weights as fill the cache (none beyond it: weights of its size are out of cache by themselves).
 # What the pick loses against the best of its twelve candidates, out of cache when timed in cache / in cache when timed out
 # of it, mean and worst: weights of 75 - 142 MB (16 problems, 8 - 8192 rows) 6.1 and 35 % (400 x 6144 x 6144) / 1.8 and
-# 6.6 % (661 x 8192 x 8192); 34 - 52 MB (7 problems) 2.7 and 7 % / 2.0 and 4 %, about even, hence the line.  FP32 problems
-# of 67 - 180 MB, bound by the matrix pipes, 2.8 and 6 % / 2.6 and 12 %: they stay timed in cache.
-COLD_WEIGHT_BYTES, CACHE_BYTES = 64 << 20, 256 << 20
+# 6.6 % (661 x 8192 x 8192); 34 - 52 MB (7 problems) 2.7 and 7 % / 2.0 and 4 %, about even, hence the line.  Below it, and in FP32
+# (67 - 180 MB, bound by the matrix pipes: 2.8 and 6 % / 2.6 and 12 %), sets of all operands in turn (helix_runtime.operand_sets).
+COLD_WEIGHT_BYTES = 64 << 20
 
 
 def weight_copies(N, K):
@@ -242,7 +234,7 @@ def verified_config(prof_dict, M, N, K, top=VERIFY_TOP, families=True):
     keys = ranked_configs(prof_dict, M, N, K, top) + (ring_ranked(M, N, K) if families else [])
 
     def fastest(copies):
-        return fastest_of(keys, lambda k, warmup, iters: handicap(k) * run_config(k, M, N, K, warmup=warmup, iters=iters, copies=copies),
+        return fastest_of(keys, lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters, copies=copies),
                           f"{M}x{N}x{K}")
 
     copies = weight_copies(N, K)

@@ -5,7 +5,7 @@ point pads the channels to a multiple of 4 in its workspace first (IC = 1: FP32 
 import math
 import os
 
-from utils.helix_runtime import load, tuned_config, fastest_of
+from utils.helix_runtime import load, tuned_config, fastest_of, operand_sets
 from utils.conv_patch import PatchFamily, PATCH_TOP
 from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, patch_key, PATCH_KEYS, PATCH_POINTS, RING_KEYS
 from MI355X_FP32.MI355X_FP32_gemm import config_cost, extra_points, ring_first, RING_CONV, RING_CONV_TOP, VERIFY_TOP
@@ -62,6 +62,12 @@ def patch_ranked(layer, top=PATCH_TOP):
     return [patch_key(point) for point in PATCH.ranked(layer, top)]
 
 
+def layer_bytes(batch, input_channel, H, W, output_channel, kH, kW, stride, pad):
+    """Input, weights and results of a layer."""
+    M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
+    return 4 * (batch * input_channel * H * W + output_channel * input_channel * kH * kW + M * output_channel)
+
+
 RING_MAX_TAPS = 31      # of the ring tiles' convolution (src_template/MI355X_FP32/gemm_ring.hip): a bit of a row's mask each
 
 
@@ -71,7 +77,7 @@ def ring_ranked(layer, top=RING_CONV_TOP):
     if IC % GATHER_CHUNK or kH * kW > RING_MAX_TAPS:
         return []
     M, K = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1), IC * kH * kW
-    return ring_first(M, OC, K, 4 * (batch * IC * H * W + OC * K + M * OC), RING_CONV, top)
+    return ring_first(M, OC, K, layer_bytes(*layer), RING_CONV, top)
 
 
 def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad, top=VERIFY_TOP, families=True):
@@ -80,8 +86,7 @@ def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, k
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
 
     def time_config(k, warmup, iters):
-        return load(library_for_key(k)).bench_conv(batch, input_channel, H, W, output_channel, kH, kW, stride, pad,
-                                                   warmup=warmup, iters=iters)[1]
+        return load(library_for_key(k)).bench_conv(*layer, warmup=warmup, iters=iters, sets=operand_sets(layer_bytes(*layer)))[1]
 
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
     return fastest_of(ranked_configs(prof_dict, M, output_channel, gather_channels(input_channel) * kH * kW, top)

@@ -4,7 +4,7 @@ the TVM alternative backend (:16-86, :108-136) has no counterpart."""
 import math
 import os
 
-from utils.helix_runtime import load, tuned_config, fastest_of
+from utils.helix_runtime import load, tuned_config, fastest_of, operand_sets
 from utils.hip_ctypes import STATIC_SCRATCH_BYTES
 from utils.roofline import NUM_CU, HBM_BYTES_PER_S, gemm_bytes
 from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, RING_KEYS
@@ -234,23 +234,24 @@ def ring_ranked(M, N, K, top=RING_TOP):
     return ring_first(M, N, K, gemm_bytes(M, N, K, 4), RING_GEMM, top)
 
 
-def run_config(k, M, N, K, warmup=10, iters=10, outer=1):
+def run_config(k, M, N, K, warmup=10, iters=10, outer=1, sets=1):
     """Seconds per launch (mean) on the real M, N, K (edges are predicated in the kernel; the reference
-    pads M and N up to the tile instead, Ampere_FP32_gemm.py:103)."""
+    pads M and N up to the tile instead, Ampere_FP32_gemm.py:103).  `sets`: of operands and results that the launches take in turn."""
     lib = load(library_for_key(k))
     if k[2] == 0:
         if M > N:
             M, N = N, M
         K = math.ceil(K / 4) * 4
-    _, avg, _ = lib.bench(M, N, K, warmup=warmup, iters=iters, outer=outer, rotate_bytes=0)
+    _, avg, _ = lib.bench(M, N, K, warmup=warmup, iters=iters, outer=outer, sets=sets)
     return avg
 
 
 def verified_config(prof_dict, M, N, K, top=VERIFY_TOP, families=True):
     """The fastest of the cost model's first `top` configurations, and with `families` of the ring tiles' first, on this problem
     (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again)."""
+    sets = operand_sets(gemm_bytes(M, N, K, 4))
     return fastest_of(ranked_configs(prof_dict, M, N, K, top) + (ring_ranked(M, N, K) if families else []),
-                      lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters), f"{M}x{N}x{K}")
+                      lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters, sets=sets), f"{M}x{N}x{K}")
 
 
 def select_config(prof_dict, M, N, K):

@@ -333,6 +333,17 @@ def forget_winners(backend):
         os.remove(winners_path(backend))
 
 
+# A selection times on several sets of operands in turn, as a program's calls come with others' between them: one set that is launched
+# on again lies in L2, which flatters kernels that wait for their loads.  Sets that fill the memory-side cache push each other
+# out by themselves.
+CACHE_BYTES, OPERAND_SETS = 256 << 20, 3
+
+
+def operand_sets(set_bytes):
+    """Sets of operands and results that a selection's launches take in turn."""
+    return OPERAND_SETS if set_bytes < CACHE_BYTES else 1
+
+
 SETTLE_FINALISTS = 4        # candidates timed a second time ...
 SETTLE_WITHIN = 1.10        # ... those within this factor of the fastest of the first pass
 

@@ -26,6 +26,8 @@ ABI_SYMBOLS = (
     "helix_conv2d_timed",
     "helix_bench",
     "helix_bench_conv",
+    "helix_bench_sets",
+    "helix_bench_conv_sets",
 )
 
 _vp = ctypes.c_void_p
@@ -67,6 +69,10 @@ class HelixLib:
         L.helix_bench.restype = _i
         L.helix_bench_conv.argtypes = [_i] * 12 + [_dp, _dp, _dp]
         L.helix_bench_conv.restype = _i
+        L.helix_bench_sets.argtypes = [_i] * 6 + [_dp]
+        L.helix_bench_sets.restype = _i
+        L.helix_bench_conv_sets.argtypes = [_i] * 12 + [_dp]
+        L.helix_bench_conv_sets.restype = _i
         self._lib = L
         self._info = None
 
@@ -124,19 +130,28 @@ class HelixLib:
             raise HelixError("helix_conv2d_timed", rc)
         return avg.value
 
-    # -- self-contained measurements: (min_s, avg_s, max_s) per launch -------------------------------
-    def bench(self, M, N, K, warmup=10, iters=10, outer=1, rotate_bytes=0):
+    # -- self-contained measurements: (min_s, avg_s, max_s) per launch; on several sets of operands in turn, each
+    #    of them once at least before the launches that count, the mean alone -----------------------------------------------
+    def bench(self, M, N, K, warmup=10, iters=10, outer=1, rotate_bytes=0, sets=1):
         mn, av, mx = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()
-        rc = self._lib.helix_bench(M, N, K, warmup, iters, outer, rotate_bytes, ctypes.byref(mn), ctypes.byref(av),
-                                   ctypes.byref(mx))
+        if sets > 1:
+            rc = self._lib.helix_bench_sets(M, N, K, max(warmup, sets), iters, sets, ctypes.byref(av))
+            mn = mx = av
+        else:
+            rc = self._lib.helix_bench(M, N, K, warmup, iters, outer, rotate_bytes, ctypes.byref(mn), ctypes.byref(av),
+                                       ctypes.byref(mx))
         if rc != 0:
             raise HelixError("helix_bench", rc)
         return mn.value, av.value, mx.value
 
-    def bench_conv(self, batch, IC, H, W, OC, kH, kW, stride, pad, warmup=10, iters=10, outer=1):
+    def bench_conv(self, batch, IC, H, W, OC, kH, kW, stride, pad, warmup=10, iters=10, outer=1, sets=1):
         mn, av, mx = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()
-        rc = self._lib.helix_bench_conv(batch, IC, H, W, OC, kH, kW, stride, pad, warmup, iters, outer,
-                                        ctypes.byref(mn), ctypes.byref(av), ctypes.byref(mx))
+        layer = (batch, IC, H, W, OC, kH, kW, stride, pad)
+        if sets > 1:
+            rc = self._lib.helix_bench_conv_sets(*layer, max(warmup, sets), iters, sets, ctypes.byref(av))
+            mn = mx = av
+        else:
+            rc = self._lib.helix_bench_conv(*layer, warmup, iters, outer, ctypes.byref(mn), ctypes.byref(av), ctypes.byref(mx))
         if rc != 0:
             raise HelixError("helix_bench_conv", rc)
         return mn.value, av.value, mx.value

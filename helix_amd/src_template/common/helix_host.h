@@ -74,13 +74,32 @@ inline int fill(void* p, size_t n_elems, int elem_bytes, float scale, uint32_t s
 
 struct DeviceBuffers {
     std::vector<void*> ptrs;
+    unsigned char* next = nullptr;    // of one allocation for many buffers, and what is left of it
+    size_t left = 0;
     ~DeviceBuffers() {
         for (void* p : ptrs)
             if (p) (void)hipFree(p);
     }
+    static size_t place(size_t bytes) { return (bytes + 0xffff) & ~(size_t)0xffff; }
+    // The buffers that follow, of `bytes` in all in place()s, come out of one allocation
+    int reserve(size_t bytes) {
+        void* p;
+        const int rc = alloc(&p, bytes);
+        if (rc == 0) {
+            next = (unsigned char*)p;
+            left = bytes;
+        }
+        return rc;
+    }
     int alloc(void** out, size_t bytes) {
         *out = nullptr;
         if (bytes == 0) bytes = 256;
+        if (place(bytes) <= left) {
+            *out = next;
+            next += place(bytes);
+            left -= place(bytes);
+            return 0;
+        }
         hipError_t e = hipMalloc(out, bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();   // reported here: not by the next launch as well
@@ -242,42 +261,20 @@ int helix_conv2d_timed(const void* x, const void* w, void* y, int batch, int H, 
     return helix_host::time_launches(launch, s, warmup, iters, avg_s);
 }
 
-int helix_bench(int M, int N, int K, int warmup, int iters, int outer, size_t rotate_bytes, double* min_s,
-                double* avg_s, double* max_s) {
-    if (M <= 0 || N <= 0 || K <= 0 || iters <= 0 || outer <= 0 || warmup < 0) return HELIX_ERR_INVALID_VALUE;
-    size_t ae, be, ce;
-    int lda, ldb, ldc;
-    tpl::bench_layout(M, N, K, &ae, &be, &ce, &lda, &ldb, &ldc);
-    const int eb = tpl::kElemBytes;
-    size_t nrot = 1;
-    if (rotate_bytes > 0 && be * eb > 0) {
-        nrot = (rotate_bytes + be * eb - 1) / (be * eb);
-        if (nrot < 1) nrot = 1;
-        if (nrot > 64) nrot = 64;
-    }
-    helix_host::DeviceBuffers bufs;
-    void *A, *C, *ws;
-    std::vector<void*> Bs(nrot);
-    int rc;
-    if ((rc = bufs.alloc(&A, ae * eb))) return rc;
-    for (size_t r = 0; r < nrot; r++)
-        if ((rc = bufs.alloc(&Bs[r], be * eb))) return rc;
-    if ((rc = bufs.alloc(&C, ce * eb))) return rc;
-    size_t wsb = tpl::workspace_bytes(M, N, K);
-    if ((rc = bufs.alloc(&ws, wsb))) return rc;
-    if ((rc = helix_host::fill(A, ae, eb, 0.5f, 1u, nullptr))) return rc;
-    for (size_t r = 0; r < nrot; r++)
-        if ((rc = helix_host::fill(Bs[r], be, eb, 0.5f, 2u + (uint32_t)r, nullptr))) return rc;
-    if ((rc = helix_host::fill(C, ce, eb, 0.0f, 3u, nullptr))) return rc;
-    HELIX_HIP_TRY(hipDeviceSynchronize());
+}  // extern "C"
 
-    auto launch = [&](int i) {
-        return tpl::gemm(A, Bs[(size_t)i % nrot], C, M, N, K, lda, ldb, ldc, ws, wsb, nullptr);
-    };
+namespace helix_host {
+namespace {
+
+constexpr int kMaxSets = 64;    // of operands that launches take in turn
+
+// Mean seconds of `outer` groups of launches: least, mean and largest
+template <typename Launch>
+int time_groups(Launch&& launch, int warmup, int iters, int outer, double* min_s, double* avg_s, double* max_s) {
     double mn = DBL_MAX, mx = 0.0, tot = 0.0;
     for (int o = 0; o < outer; o++) {
         double t;
-        rc = helix_host::time_launches(launch, nullptr, o == 0 ? warmup : 0, iters, &t);
+        const int rc = time_launches(launch, nullptr, o == 0 ? warmup : 0, iters, &t);
         if (rc) return rc;
         mn = t < mn ? t : mn;
         mx = t > mx ? t : mx;
@@ -289,8 +286,49 @@ int helix_bench(int M, int N, int K, int warmup, int iters, int outer, size_t ro
     return 0;
 }
 
-int helix_bench_conv(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup,
-                     int iters, int outer, double* min_s, double* avg_s, double* max_s) {
+// Allocates and fills one operand `sets` times
+inline int alloc_sets(DeviceBuffers& bufs, void* (&out)[kMaxSets], int sets, size_t n_elems, int eb, float scale, uint32_t seed) {
+    int rc;
+    for (int i = 0; i < sets; i++) {
+        if ((rc = bufs.alloc(&out[i], n_elems * eb))) return rc;
+        if ((rc = fill(out[i], n_elems, eb, scale, seed + (uint32_t)i, nullptr))) return rc;
+    }
+    return 0;
+}
+
+// `sets` sets of operands and results in turn, of the second operand as many as make `rotate_bytes`
+inline int bench_gemm(int M, int N, int K, int warmup, int iters, int outer, int sets, size_t rotate_bytes, double* min_s, double* avg_s,
+                      double* max_s) {
+    size_t ae, be, ce;
+    int lda, ldb, ldc;
+    tpl::bench_layout(M, N, K, &ae, &be, &ce, &lda, &ldb, &ldc);
+    const int eb = tpl::kElemBytes;
+    size_t nrot = (size_t)sets;
+    if (rotate_bytes > 0 && be * eb > 0) {
+        nrot = (rotate_bytes + be * eb - 1) / (be * eb);
+        if (nrot < 1) nrot = 1;
+        if (nrot > (size_t)kMaxSets) nrot = kMaxSets;
+    }
+    DeviceBuffers bufs;
+    void *As[kMaxSets], *Bs[kMaxSets], *Cs[kMaxSets], *ws;
+    const size_t wsb = tpl::workspace_bytes(M, N, K);
+    int rc;
+    // (a selection meets its candidates with new buffers each: one allocation instead of ten halves its time)
+    if (sets > 1 && (rc = bufs.reserve(sets * (bufs.place(ae * eb) + bufs.place(be * eb) + bufs.place(ce * eb)) + bufs.place(wsb)))) return rc;
+    if ((rc = alloc_sets(bufs, As, sets, ae, eb, 0.5f, 1u))) return rc;
+    if ((rc = alloc_sets(bufs, Bs, (int)nrot, be, eb, 0.5f, 2u))) return rc;
+    if ((rc = alloc_sets(bufs, Cs, sets, ce, eb, 0.0f, 3u))) return rc;
+    if ((rc = bufs.alloc(&ws, wsb))) return rc;
+    HELIX_HIP_TRY(hipDeviceSynchronize());
+
+    auto launch = [&](int i) {
+        return tpl::gemm(As[(size_t)(i % sets)], Bs[(size_t)i % nrot], Cs[(size_t)(i % sets)], M, N, K, lda, ldb, ldc, ws, wsb, nullptr);
+    };
+    return time_groups(launch, warmup, iters, outer, min_s, avg_s, max_s);
+}
+
+inline int bench_conv(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup, int iters, int outer,
+                      int sets, double* min_s, double* avg_s, double* max_s) {
     if (batch <= 0 || IC <= 0 || H <= 0 || W <= 0 || OC <= 0 || kH <= 0 || kW <= 0 || stride <= 0 || pad < 0 ||
         iters <= 0 || outer <= 0 || warmup < 0)
         return HELIX_ERR_INVALID_VALUE;
@@ -298,32 +336,48 @@ int helix_bench_conv(int batch, int IC, int H, int W, int OC, int kH, int kW, in
     int OH = (H + 2 * pad - kH) / stride + 1, OW = (W + 2 * pad - kW) / stride + 1;
     size_t xe = (size_t)batch * H * W * IC, we = (size_t)OC * kH * kW * IC, ye = (size_t)batch * OH * OW * OC;
     const int eb = tpl::kElemBytes;
-    helix_host::DeviceBuffers bufs;
-    void *x, *w, *y, *ws;
+    DeviceBuffers bufs;
+    void *xs[kMaxSets], *ws[kMaxSets], *ys[kMaxSets], *scratch;
+    const size_t scratch_bytes = tpl::conv_workspace_bytes(batch, H, W, IC, OC, kH, kW, stride, pad);
     int rc;
-    if ((rc = bufs.alloc(&x, xe * eb))) return rc;
-    if ((rc = bufs.alloc(&w, we * eb))) return rc;
-    if ((rc = bufs.alloc(&y, ye * eb))) return rc;
-    size_t wsb = tpl::conv_workspace_bytes(batch, H, W, IC, OC, kH, kW, stride, pad);
-    if ((rc = bufs.alloc(&ws, wsb))) return rc;
-    if ((rc = helix_host::fill(x, xe, eb, 0.5f, 1u, nullptr))) return rc;
-    if ((rc = helix_host::fill(w, we, eb, 0.5f, 2u, nullptr))) return rc;
-    if ((rc = helix_host::fill(y, ye, eb, 0.0f, 3u, nullptr))) return rc;
+    if (sets > 1 && (rc = bufs.reserve(sets * (bufs.place(xe * eb) + bufs.place(we * eb) + bufs.place(ye * eb)) + bufs.place(scratch_bytes)))) return rc;
+    if ((rc = alloc_sets(bufs, xs, sets, xe, eb, 0.5f, 1u))) return rc;
+    if ((rc = alloc_sets(bufs, ws, sets, we, eb, 0.5f, 2u))) return rc;
+    if ((rc = alloc_sets(bufs, ys, sets, ye, eb, 0.0f, 3u))) return rc;
+    if ((rc = bufs.alloc(&scratch, scratch_bytes))) return rc;
     HELIX_HIP_TRY(hipDeviceSynchronize());
-    auto launch = [&](int) { return tpl::conv2d(x, w, y, batch, H, W, IC, OC, kH, kW, stride, pad, ws, wsb, nullptr); };
-    double mn = DBL_MAX, mx = 0.0, tot = 0.0;
-    for (int o = 0; o < outer; o++) {
-        double t;
-        rc = helix_host::time_launches(launch, nullptr, o == 0 ? warmup : 0, iters, &t);
-        if (rc) return rc;
-        mn = t < mn ? t : mn;
-        mx = t > mx ? t : mx;
-        tot += t;
-    }
-    if (min_s) *min_s = mn;
-    if (avg_s) *avg_s = tot / outer;
-    if (max_s) *max_s = mx;
-    return 0;
+    auto launch = [&](int i) {
+        return tpl::conv2d(xs[(size_t)(i % sets)], ws[(size_t)(i % sets)], ys[(size_t)(i % sets)], batch, H, W, IC, OC, kH, kW, stride, pad,
+                           scratch, scratch_bytes, nullptr);
+    };
+    return time_groups(launch, warmup, iters, outer, min_s, avg_s, max_s);
+}
+
+}  // namespace
+}  // namespace helix_host
+
+extern "C" {
+
+int helix_bench(int M, int N, int K, int warmup, int iters, int outer, size_t rotate_bytes, double* min_s,
+                double* avg_s, double* max_s) {
+    if (M <= 0 || N <= 0 || K <= 0 || iters <= 0 || outer <= 0 || warmup < 0) return HELIX_ERR_INVALID_VALUE;
+    return helix_host::bench_gemm(M, N, K, warmup, iters, outer, 1, rotate_bytes, min_s, avg_s, max_s);
+}
+
+int helix_bench_sets(int M, int N, int K, int warmup, int iters, int sets, double* avg_s) {
+    if (M <= 0 || N <= 0 || K <= 0 || iters <= 0 || warmup < 0 || sets <= 0 || sets > helix_host::kMaxSets) return HELIX_ERR_INVALID_VALUE;
+    return helix_host::bench_gemm(M, N, K, warmup, iters, 1, sets, 0, nullptr, avg_s, nullptr);
+}
+
+int helix_bench_conv(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup,
+                     int iters, int outer, double* min_s, double* avg_s, double* max_s) {
+    return helix_host::bench_conv(batch, IC, H, W, OC, kH, kW, stride, pad, warmup, iters, outer, 1, min_s, avg_s, max_s);
+}
+
+int helix_bench_conv_sets(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup, int iters, int sets,
+                          double* avg_s) {
+    if (sets <= 0 || sets > helix_host::kMaxSets) return HELIX_ERR_INVALID_VALUE;
+    return helix_host::bench_conv(batch, IC, H, W, OC, kH, kW, stride, pad, warmup, iters, 1, sets, nullptr, avg_s, nullptr);
 }
 
 }  // extern "C"

@@ -1,0 +1,67 @@
+"""The sets of operands that a selection's launches take in turn (utils.helix_runtime.operand_sets)."""
+import pytest
+
+from utils import helix_runtime
+from MI355X_FP16 import build_MI355X_FP16 as b16
+from MI355X_FP16 import MI355X_FP16_conv as c16
+from MI355X_FP16 import MI355X_FP16_gemm as g16
+from MI355X_FP32 import build_MI355X_FP32 as b32
+from MI355X_FP32 import MI355X_FP32_conv as c32
+from MI355X_FP32 import MI355X_FP32_gemm as g32
+
+PROF16 = {(2, 64, 64, 32, 32, 0, 64): 1e-5, (2, 128, 64, 64, 32, 0, 64): 2e-5}
+PROF32 = {b32.config_key(64, 64, 16, 32, 32): 1.0, b32.config_key(128, 64, 16, 32, 32): 1.7}
+# m, n, k: sets in turn; the memory-side cache is full of one; FP16 weights that are copied instead
+PRODUCTS = [((269, 2376, 1376), 3, 3), ((127619, 5, 458), 3, 3), ((8192, 8192, 8192), 1, 1), ((661, 11008, 4096), 1, 3)]
+LAYERS = [((32, 64, 56, 56, 64, 3, 3, 1, 1), 3), ((64, 64, 150, 150, 64, 1, 1, 1, 0), 1)]
+
+
+def libraries(monkeypatch, modules, ring_seconds):
+    """Libraries whose ring tiles take `ring_seconds` and all others 1 s; what they are asked to time."""
+    asked = []
+
+    class Library:
+        def __init__(self, path):
+            self.seconds = ring_seconds if "gemm_ring" in path else 1.0
+
+        def bench(self, M, N, K, warmup, iters, outer=1, rotate_bytes=0, sets=1):
+            asked.append((sets, rotate_bytes))
+            return self.seconds, self.seconds, self.seconds
+
+        def bench_conv(self, *layer, warmup, iters, sets=1):
+            asked.append((sets, 0))
+            return self.seconds, self.seconds, self.seconds
+
+    for module in modules:
+        monkeypatch.setattr(module, "load", Library)
+    return asked
+
+
+@pytest.mark.parametrize("problem,sets16,sets32", PRODUCTS)
+def test_products_are_timed_on_sets_in_turn(problem, sets16, sets32, monkeypatch):
+    asked = libraries(monkeypatch, (g16, g32), 0.99)
+    assert b16.is_ring_key(g16.verified_config(PROF16, *problem))         # a hundredth ahead is ahead
+    copies = g16.weight_copies(*problem[1:])
+    assert {s for s, _ in asked} == {sets16} and {bool(r) for _, r in asked} == {copies > 1}
+    asked.clear()
+    assert b32.is_ring_key(g32.verified_config(PROF32, *problem))
+    assert set(asked) == {(sets32, 0)}
+
+
+@pytest.mark.parametrize("layer,sets", LAYERS)
+def test_layers_are_timed_on_sets_in_turn(layer, sets, monkeypatch):
+    asked = libraries(monkeypatch, (c16, c32), 0.99)
+    assert b16.is_ring_key(c16.verified_config(PROF16, *layer)) and b32.is_ring_key(c32.verified_config(PROF32, *layer))
+    assert set(asked) == {(sets, 0)}
+
+
+def test_rows_of_the_reports_are_timed_on_one_set(monkeypatch):
+    asked = libraries(monkeypatch, (g16, g32), 0.99)
+    g16.run_config((2, 64, 64, 32, 32, 0, 64), 269, 2376, 1376)
+    g32.run_config(b32.config_key(64, 64, 16, 32, 32), 269, 2376, 1376)
+    assert asked == [(1, 0), (1, 0)]
+
+
+def test_sets_end_where_they_fill_the_cache():
+    assert helix_runtime.operand_sets(1) == helix_runtime.OPERAND_SETS == 3
+    assert helix_runtime.operand_sets(helix_runtime.CACHE_BYTES - 1) == 3 and helix_runtime.operand_sets(helix_runtime.CACHE_BYTES) == 1
