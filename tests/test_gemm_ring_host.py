@@ -103,6 +103,17 @@ def test_fp32_family(tmp_path, monkeypatch):
     assert len(c32.ring_ranked((4, 4, 28, 28, 96, 5, 6, 1, 0))) == g32.RING_CONV_TOP
 
 
+def test_few_rows_of_long_k_are_left_to_the_others(monkeypatch):
+    """Decode products: a selection neither ranks nor times the ring tiles, which are never ahead there."""
+    for g, build, prof, problem in ((g16, b16, {(2, 64, 64, 32, 32, 0, 64): 1e-5}, (16, 28672, 8192)),
+                                    (g32, b32, {b32.config_key(64, 64, 16, 32, 32): 1.0}, (4, 11008, 4096))):
+        timed = []
+        monkeypatch.setattr(g, "run_config", lambda k, *a, **kw: timed.append(k) or 1e-6)
+        assert g.verified_config(prof, *problem) in prof
+        assert set(timed) == set(prof) and not any(build.is_ring_key(k) for k in timed)
+        assert len(g.ring_ranked(17, 4096, 4096)) == len(g.ring_ranked(16, 4096, 1016)) == len(g.ring_ranked(30000, 16, 2000)) == g.RING_TOP
+
+
 def test_zeros_are_read_beyond_every_operand(tmp_path):
     """The offset of what a copy has not got lies behind a K tile of the largest operand that the FP32 tiles take, 4 GiB, aligned as a
     copy is."""
