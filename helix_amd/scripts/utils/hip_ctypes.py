@@ -5,6 +5,8 @@ counterpart of one executable of the reference (`os.popen(f"{exe} {M} {N} {K}")`
 scripts/Ampere_FP16/profile_Ampere_FP16.py:36-38).  Loading a library that does not exist raises
 FileNotFoundError: there is no CPU fallback.
 """
+import contextlib
+import contextvars
 import ctypes
 import json
 import os
@@ -28,6 +30,7 @@ ABI_SYMBOLS = (
     "helix_bench_conv",
     "helix_bench_sets",
     "helix_bench_conv_sets",
+    "helix_bench_release",
 )
 
 _vp = ctypes.c_void_p
@@ -40,6 +43,30 @@ class HelixError(RuntimeError):
     def __init__(self, fn, code):
         super().__init__(f"{fn} failed with code {code}")
         self.code = code
+
+
+class _Buffers(ctypes.Structure):
+    """helix_bench_buffers of include/helix_abi.h."""
+    COUNT = 200
+    _fields_ = [("device", _vp * COUNT), ("bytes", _sz * COUNT)]
+    library = None      # one that has used them
+
+
+_buffers = contextvars.ContextVar("helix_bench_buffers", default=None)
+
+
+@contextlib.contextmanager
+def shared_buffers():
+    """Within it (this thread's calls) every measurement of HelixLib.bench and bench_conv uses the same buffers, whatever the library,
+    which are given back at its end: what differs between two of them is the kernel, not where its operands lie."""
+    buffers = _Buffers()
+    token = _buffers.set(buffers)
+    try:
+        yield
+    finally:
+        _buffers.reset(token)
+        if buffers.library:
+            buffers.library.helix_bench_release(ctypes.byref(buffers))
 
 
 class HelixLib:
@@ -69,10 +96,12 @@ class HelixLib:
         L.helix_bench.restype = _i
         L.helix_bench_conv.argtypes = [_i] * 12 + [_dp, _dp, _dp]
         L.helix_bench_conv.restype = _i
-        L.helix_bench_sets.argtypes = [_i] * 6 + [_dp]
+        L.helix_bench_sets.argtypes = [_i] * 6 + [_sz, ctypes.POINTER(_Buffers), _dp]
         L.helix_bench_sets.restype = _i
-        L.helix_bench_conv_sets.argtypes = [_i] * 12 + [_dp]
+        L.helix_bench_conv_sets.argtypes = [_i] * 12 + [ctypes.POINTER(_Buffers), _dp]
         L.helix_bench_conv_sets.restype = _i
+        L.helix_bench_release.argtypes = [ctypes.POINTER(_Buffers)]
+        L.helix_bench_release.restype = _i
         self._lib = L
         self._info = None
 
@@ -130,12 +159,20 @@ class HelixLib:
             raise HelixError("helix_conv2d_timed", rc)
         return avg.value
 
-    # -- self-contained measurements: (min_s, avg_s, max_s) per launch; on several sets of operands in turn, each
-    #    of them once at least before the launches that count, the mean alone -----------------------------------------------
+    # -- self-contained measurements: (min_s, avg_s, max_s) per launch; on several sets of operands in turn (each of them once at
+    #    least before the launches that count) or in shared_buffers the mean alone, of one group --------------------------------
+    def _shared_buffers(self):
+        buffers = _buffers.get()
+        if buffers is None:
+            return None
+        buffers.library = self._lib
+        return ctypes.pointer(buffers)
+
     def bench(self, M, N, K, warmup=10, iters=10, outer=1, rotate_bytes=0, sets=1):
         mn, av, mx = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()
-        if sets > 1:
-            rc = self._lib.helix_bench_sets(M, N, K, max(warmup, sets), iters, sets, ctypes.byref(av))
+        buffers = self._shared_buffers()
+        if sets > 1 or buffers:
+            rc = self._lib.helix_bench_sets(M, N, K, max(warmup, sets), iters, sets, rotate_bytes, buffers, ctypes.byref(av))
             mn = mx = av
         else:
             rc = self._lib.helix_bench(M, N, K, warmup, iters, outer, rotate_bytes, ctypes.byref(mn), ctypes.byref(av),
@@ -147,8 +184,9 @@ class HelixLib:
     def bench_conv(self, batch, IC, H, W, OC, kH, kW, stride, pad, warmup=10, iters=10, outer=1, sets=1):
         mn, av, mx = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()
         layer = (batch, IC, H, W, OC, kH, kW, stride, pad)
-        if sets > 1:
-            rc = self._lib.helix_bench_conv_sets(*layer, max(warmup, sets), iters, sets, ctypes.byref(av))
+        buffers = self._shared_buffers()
+        if sets > 1 or buffers:
+            rc = self._lib.helix_bench_conv_sets(*layer, max(warmup, sets), iters, sets, buffers, ctypes.byref(av))
             mn = mx = av
         else:
             rc = self._lib.helix_bench_conv(*layer, warmup, iters, outer, ctypes.byref(mn), ctypes.byref(av), ctypes.byref(mx))

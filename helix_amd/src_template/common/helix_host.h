@@ -72,40 +72,46 @@ inline int fill(void* p, size_t n_elems, int elem_bytes, float scale, uint32_t s
     return (int)hipGetLastError();
 }
 
+constexpr size_t kLentUnit = (size_t)2 << 20;    // of lent buffers' sizes, so that the paddings of one problem's layouts fit the same ones
+
 struct DeviceBuffers {
     std::vector<void*> ptrs;
-    unsigned char* next = nullptr;    // of one allocation for many buffers, and what is left of it
-    size_t left = 0;
+    helix_bench_buffers* lent = nullptr;    // the caller's, taken in order instead of new ones
+    int taken = 0;
     ~DeviceBuffers() {
         for (void* p : ptrs)
             if (p) (void)hipFree(p);
     }
-    static size_t place(size_t bytes) { return (bytes + 0xffff) & ~(size_t)0xffff; }
-    // The buffers that follow, of `bytes` in all in place()s, come out of one allocation
-    int reserve(size_t bytes) {
-        void* p;
-        const int rc = alloc(&p, bytes);
-        if (rc == 0) {
-            next = (unsigned char*)p;
-            left = bytes;
-        }
-        return rc;
-    }
     int alloc(void** out, size_t bytes) {
         *out = nullptr;
         if (bytes == 0) bytes = 256;
-        if (place(bytes) <= left) {
-            *out = next;
-            next += place(bytes);
-            left -= place(bytes);
-            return 0;
-        }
+        if (lent) return take(out, (bytes + kLentUnit - 1) / kLentUnit * kLentUnit);
         hipError_t e = hipMalloc(out, bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();   // reported here: not by the next launch as well
             return (int)e;
         }
         ptrs.push_back(*out);
+        return 0;
+    }
+    // The next of the caller's buffers, replaced by a larger one where it is too small
+    int take(void** out, size_t bytes) {
+        if (taken >= HELIX_BENCH_BUFFERS) return HELIX_ERR_INVALID_VALUE;
+        void*& p = lent->device[taken];
+        size_t& size = lent->bytes[taken];
+        if (size < bytes) {
+            if (p) (void)hipFree(p);
+            size = 0;
+            const hipError_t e = hipMalloc(&p, bytes);
+            if (e != hipSuccess) {
+                (void)hipGetLastError();
+                p = nullptr;
+                return (int)e;
+            }
+            size = bytes;
+        }
+        taken++;
+        *out = p;
         return 0;
     }
 };
@@ -267,6 +273,7 @@ namespace helix_host {
 namespace {
 
 constexpr int kMaxSets = 64;    // of operands that launches take in turn
+static_assert(HELIX_BENCH_BUFFERS >= 3 * kMaxSets + 1, "operands, results and a workspace");
 
 // Mean seconds of `outer` groups of launches: least, mean and largest
 template <typename Launch>
@@ -297,8 +304,8 @@ inline int alloc_sets(DeviceBuffers& bufs, void* (&out)[kMaxSets], int sets, siz
 }
 
 // `sets` sets of operands and results in turn, of the second operand as many as make `rotate_bytes`
-inline int bench_gemm(int M, int N, int K, int warmup, int iters, int outer, int sets, size_t rotate_bytes, double* min_s, double* avg_s,
-                      double* max_s) {
+inline int bench_gemm(int M, int N, int K, int warmup, int iters, int outer, int sets, size_t rotate_bytes, helix_bench_buffers* buffers,
+                      double* min_s, double* avg_s, double* max_s) {
     size_t ae, be, ce;
     int lda, ldb, ldc;
     tpl::bench_layout(M, N, K, &ae, &be, &ce, &lda, &ldb, &ldc);
@@ -313,8 +320,7 @@ inline int bench_gemm(int M, int N, int K, int warmup, int iters, int outer, int
     void *As[kMaxSets], *Bs[kMaxSets], *Cs[kMaxSets], *ws;
     const size_t wsb = tpl::workspace_bytes(M, N, K);
     int rc;
-    // (a selection meets its candidates with new buffers each: one allocation instead of ten halves its time)
-    if (sets > 1 && (rc = bufs.reserve(sets * (bufs.place(ae * eb) + bufs.place(be * eb) + bufs.place(ce * eb)) + bufs.place(wsb)))) return rc;
+    bufs.lent = buffers;
     if ((rc = alloc_sets(bufs, As, sets, ae, eb, 0.5f, 1u))) return rc;
     if ((rc = alloc_sets(bufs, Bs, (int)nrot, be, eb, 0.5f, 2u))) return rc;
     if ((rc = alloc_sets(bufs, Cs, sets, ce, eb, 0.0f, 3u))) return rc;
@@ -328,7 +334,7 @@ inline int bench_gemm(int M, int N, int K, int warmup, int iters, int outer, int
 }
 
 inline int bench_conv(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup, int iters, int outer,
-                      int sets, double* min_s, double* avg_s, double* max_s) {
+                      int sets, helix_bench_buffers* buffers, double* min_s, double* avg_s, double* max_s) {
     if (batch <= 0 || IC <= 0 || H <= 0 || W <= 0 || OC <= 0 || kH <= 0 || kW <= 0 || stride <= 0 || pad < 0 ||
         iters <= 0 || outer <= 0 || warmup < 0)
         return HELIX_ERR_INVALID_VALUE;
@@ -340,7 +346,7 @@ inline int bench_conv(int batch, int IC, int H, int W, int OC, int kH, int kW, i
     void *xs[kMaxSets], *ws[kMaxSets], *ys[kMaxSets], *scratch;
     const size_t scratch_bytes = tpl::conv_workspace_bytes(batch, H, W, IC, OC, kH, kW, stride, pad);
     int rc;
-    if (sets > 1 && (rc = bufs.reserve(sets * (bufs.place(xe * eb) + bufs.place(we * eb) + bufs.place(ye * eb)) + bufs.place(scratch_bytes)))) return rc;
+    bufs.lent = buffers;
     if ((rc = alloc_sets(bufs, xs, sets, xe, eb, 0.5f, 1u))) return rc;
     if ((rc = alloc_sets(bufs, ws, sets, we, eb, 0.5f, 2u))) return rc;
     if ((rc = alloc_sets(bufs, ys, sets, ye, eb, 0.0f, 3u))) return rc;
@@ -361,23 +367,34 @@ extern "C" {
 int helix_bench(int M, int N, int K, int warmup, int iters, int outer, size_t rotate_bytes, double* min_s,
                 double* avg_s, double* max_s) {
     if (M <= 0 || N <= 0 || K <= 0 || iters <= 0 || outer <= 0 || warmup < 0) return HELIX_ERR_INVALID_VALUE;
-    return helix_host::bench_gemm(M, N, K, warmup, iters, outer, 1, rotate_bytes, min_s, avg_s, max_s);
+    return helix_host::bench_gemm(M, N, K, warmup, iters, outer, 1, rotate_bytes, nullptr, min_s, avg_s, max_s);
 }
 
-int helix_bench_sets(int M, int N, int K, int warmup, int iters, int sets, double* avg_s) {
+int helix_bench_sets(int M, int N, int K, int warmup, int iters, int sets, size_t rotate_bytes, helix_bench_buffers* buffers, double* avg_s) {
     if (M <= 0 || N <= 0 || K <= 0 || iters <= 0 || warmup < 0 || sets <= 0 || sets > helix_host::kMaxSets) return HELIX_ERR_INVALID_VALUE;
-    return helix_host::bench_gemm(M, N, K, warmup, iters, 1, sets, 0, nullptr, avg_s, nullptr);
+    return helix_host::bench_gemm(M, N, K, warmup, iters, 1, sets, rotate_bytes, buffers, nullptr, avg_s, nullptr);
 }
 
 int helix_bench_conv(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup,
                      int iters, int outer, double* min_s, double* avg_s, double* max_s) {
-    return helix_host::bench_conv(batch, IC, H, W, OC, kH, kW, stride, pad, warmup, iters, outer, 1, min_s, avg_s, max_s);
+    return helix_host::bench_conv(batch, IC, H, W, OC, kH, kW, stride, pad, warmup, iters, outer, 1, nullptr, min_s, avg_s, max_s);
 }
 
 int helix_bench_conv_sets(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup, int iters, int sets,
-                          double* avg_s) {
+                          helix_bench_buffers* buffers, double* avg_s) {
     if (sets <= 0 || sets > helix_host::kMaxSets) return HELIX_ERR_INVALID_VALUE;
-    return helix_host::bench_conv(batch, IC, H, W, OC, kH, kW, stride, pad, warmup, iters, 1, sets, nullptr, avg_s, nullptr);
+    return helix_host::bench_conv(batch, IC, H, W, OC, kH, kW, stride, pad, warmup, iters, 1, sets, buffers, nullptr, avg_s, nullptr);
+}
+
+int helix_bench_release(helix_bench_buffers* buffers) {
+    int rc = 0;
+    for (int i = 0; buffers && i < HELIX_BENCH_BUFFERS; i++) {
+        const hipError_t e = buffers->device[i] ? hipFree(buffers->device[i]) : hipSuccess;
+        if (e != hipSuccess && rc == 0) rc = (int)e;
+        buffers->device[i] = nullptr;
+        buffers->bytes[i] = 0;
+    }
+    return rc;
 }
 
 }  // extern "C"

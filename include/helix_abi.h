@@ -141,12 +141,22 @@ HELIX_API int helix_bench(int M, int N, int K, int warmup, int iters, int outer,
 HELIX_API int helix_bench_conv(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup,
                      int iters, int outer, double* min_s, double* avg_s, double* max_s);
 
-/* The same for `sets` (1 .. 64) sets of operands and results that the launches take in turn, as a program's calls come with others' between
- * them: what the launch before left in the caches is another set's.  The mean of one group of launches.
+/* The same for comparing libraries: `sets` (1 .. 64) sets of operands and results that the launches take in turn, as a program's calls
+ * come with others' between them (what the launch before left in the caches is another set's), and all of it in buffers that the
+ * next library's call uses again (where they lie moves a kernel's time by several per cent).  The caller's `buffers`, all zero at first,
+ * are allocated and enlarged as needed, and given back with helix_bench_release of any library; null: the call's own.  The mean of
+ * one group of launches.
  * No counterpart in the reference, which times one set (src_template/Ampere_FP16/gemm.cu:636-652). */
-HELIX_API int helix_bench_sets(int M, int N, int K, int warmup, int iters, int sets, double* avg_s);
+#define HELIX_BENCH_BUFFERS 200
+typedef struct {
+    void* device[HELIX_BENCH_BUFFERS];
+    size_t bytes[HELIX_BENCH_BUFFERS];
+} helix_bench_buffers;
+HELIX_API int helix_bench_sets(int M, int N, int K, int warmup, int iters, int sets, size_t rotate_bytes, helix_bench_buffers* buffers,
+                               double* avg_s);
 HELIX_API int helix_bench_conv_sets(int batch, int IC, int H, int W, int OC, int kH, int kW, int stride, int pad, int warmup, int iters,
-                                    int sets, double* avg_s);
+                                    int sets, helix_bench_buffers* buffers, double* avg_s);
+HELIX_API int helix_bench_release(helix_bench_buffers* buffers);
 
 #ifdef __cplusplus
 }

@@ -1,7 +1,7 @@
 """The sets of operands that a selection's launches take in turn (utils.helix_runtime.operand_sets)."""
 import pytest
 
-from utils import helix_runtime
+from utils import helix_runtime, hip_ctypes
 from MI355X_FP16 import build_MI355X_FP16 as b16
 from MI355X_FP16 import MI355X_FP16_conv as c16
 from MI355X_FP16 import MI355X_FP16_gemm as g16
@@ -60,6 +60,23 @@ def test_rows_of_the_reports_are_timed_on_one_set(monkeypatch):
     g16.run_config((2, 64, 64, 32, 32, 0, 64), 269, 2376, 1376)
     g32.run_config(b32.config_key(64, 64, 16, 32, 32), 269, 2376, 1376)
     assert asked == [(1, 0), (1, 0)]
+
+
+def test_candidates_of_a_selection_share_their_buffers():
+    """All passes of one selection, and nothing outside it; the next selection has buffers of its own, also after an error."""
+    seen = []
+
+    def time_config(k, warmup, iters):
+        seen.append(hip_ctypes._buffers.get())
+        if k == "c":
+            raise RuntimeError("cannot run")
+        return {"a": 1.0, "b": 1.01}[k]
+
+    assert helix_runtime.fastest_of(["a", "b", "c"], time_config, "p") == "a" and hip_ctypes._buffers.get() is None
+    assert len(seen) == 7 and seen[0] is not None and len({id(s) for s in seen}) == 1
+    with pytest.raises(RuntimeError):
+        helix_runtime.fastest_of(["c"], time_config, "p")
+    assert hip_ctypes._buffers.get() is None and seen[-1] is not seen[0] and seen[-1] is not None
 
 
 def test_sets_end_where_they_fill_the_cache():
