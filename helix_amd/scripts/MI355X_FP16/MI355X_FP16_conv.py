@@ -12,7 +12,7 @@ repack + GEMM), all on one stream and timed as one.
 import math
 import os
 
-from utils.helix_runtime import load, kernel_resources, tuned_config, fastest_of, operand_sets
+from utils.helix_runtime import load, kernel_resources, tuned_config, fastest_in_turn
 from utils.conv_patch import PatchFamily, PATCH_TOP
 from MI355X_FP16.build_MI355X_FP16 import library_for_key, kernel_library, is_dtl_key, patch_key, PATCH_KEYS, PATCH_POINTS, RING_KEYS
 from MI355X_FP16.MI355X_FP16_gemm import short_value, config_cost, ring_first, ring_ranked, RING_CONV, RING_TOP, VERIFY_TOP
@@ -182,14 +182,14 @@ def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, k
         ranked = ranked_configs(prof_dict, M, output_channel, ICg * kH * kW, ICg, len(prof_dict))
         return next((k for k in ranked if k[5] == 0), ranked[0])
 
-    def time_config(k, warmup, iters):
-        return load(library_for_key(k)).bench_conv(*layer, warmup=warmup, iters=iters, sets=operand_sets(layer_bytes(*layer)))[1]
+    def time_config(k, warmup, iters, sets):
+        return load(library_for_key(k)).bench_conv(*layer, warmup=warmup, iters=iters, sets=sets)[1]
 
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
-    return fastest_of(ranked_configs(prof_dict, M, output_channel, ICg * kH * kW, ICg, top,
-                                     is_pointwise(kH, kW, stride, pad) and input_channel % GATHER_CHUNK == 0)
-                      + (unprofiled_ranked(*layer) if families else []),
-                      time_config, "this layer")
+    keys = (ranked_configs(prof_dict, M, output_channel, ICg * kH * kW, ICg, top,
+                           is_pointwise(kH, kW, stride, pad) and input_channel % GATHER_CHUNK == 0)
+            + (unprofiled_ranked(*layer) if families else []))
+    return fastest_in_turn(layer_bytes(*layer), keys, time_config, "this layer")
 
 
 def layer_bytes(batch, input_channel, H, W, output_channel, kH, kW, stride, pad):

@@ -237,21 +237,20 @@ def weight_copies(N, K):
 
 def verified_config(prof_dict, M, N, K, top=VERIFY_TOP, families=True):
     """The fastest of the cost model's first `top` configurations, and with `families` of the ring tiles' first, on this problem
-    (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again).  Where the copies of the weights do not fit
-    the device beside the problem, one does."""
+    (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again).  Where the copies of the weights, or the
+    sets of operands, do not fit the device beside the problem, one does."""
     keys = ranked_configs(prof_dict, M, N, K, top) + (ring_ranked(M, N, K) if families else [])
 
     def fastest(copies):
         return fastest_of(keys, lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters, copies=copies),
                           f"{M}x{N}x{K}")
 
-    copies = weight_copies(N, K)
-    if copies > 1:
+    for copies in (weight_copies(N, K), 1):
         try:
             return fastest(copies)
         except RuntimeError:
             pass
-    return fastest(1)
+    return fastest(0)
 
 
 def select_config(prof_dict, M, N, K):

@@ -5,7 +5,7 @@ point pads the channels to a multiple of 4 in its workspace first (IC = 1: FP32 
 import math
 import os
 
-from utils.helix_runtime import load, tuned_config, fastest_of, operand_sets
+from utils.helix_runtime import load, tuned_config, fastest_in_turn
 from utils.conv_patch import PatchFamily, PATCH_TOP
 from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, patch_key, PATCH_KEYS, PATCH_POINTS, RING_KEYS
 from MI355X_FP32.MI355X_FP32_gemm import config_cost, extra_points, ring_first, RING_CONV, RING_CONV_TOP, VERIFY_TOP
@@ -85,12 +85,13 @@ def verified_config(prof_dict, batch, input_channel, H, W, output_channel, kH, k
     (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again)."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
 
-    def time_config(k, warmup, iters):
-        return load(library_for_key(k)).bench_conv(*layer, warmup=warmup, iters=iters, sets=operand_sets(layer_bytes(*layer)))[1]
+    def time_config(k, warmup, iters, sets):
+        return load(library_for_key(k)).bench_conv(*layer, warmup=warmup, iters=iters, sets=sets)[1]
 
     layer = (batch, input_channel, H, W, output_channel, kH, kW, stride, pad)
-    return fastest_of(ranked_configs(prof_dict, M, output_channel, gather_channels(input_channel) * kH * kW, top)
-                      + (patch_ranked(layer) + ring_ranked(layer) if families else []), time_config, "this layer")
+    keys = (ranked_configs(prof_dict, M, output_channel, gather_channels(input_channel) * kH * kW, top)
+            + (patch_ranked(layer) + ring_ranked(layer) if families else []))
+    return fastest_in_turn(layer_bytes(*layer), keys, time_config, "this layer")
 
 
 def get_MI355X_FP32_conv_Verified_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad,

@@ -4,7 +4,7 @@ the TVM alternative backend (:16-86, :108-136) has no counterpart."""
 import math
 import os
 
-from utils.helix_runtime import load, tuned_config, fastest_of, operand_sets
+from utils.helix_runtime import load, tuned_config, fastest_in_turn
 from utils.hip_ctypes import STATIC_SCRATCH_BYTES
 from utils.roofline import NUM_CU, HBM_BYTES_PER_S, gemm_bytes
 from MI355X_FP32.build_MI355X_FP32 import library_for_key, kernel_library, RING_KEYS
@@ -257,9 +257,8 @@ def run_config(k, M, N, K, warmup=10, iters=10, outer=1, sets=1):
 def verified_config(prof_dict, M, N, K, top=VERIFY_TOP, families=True):
     """The fastest of the cost model's first `top` configurations, and with `families` of the ring tiles' first, on this problem
     (utils.helix_runtime.fastest_of: 2 + 5 launches each, the leaders timed again)."""
-    sets = operand_sets(gemm_bytes(M, N, K, 4))
-    return fastest_of(ranked_configs(prof_dict, M, N, K, top) + (ring_ranked(M, N, K) if families else []),
-                      lambda k, warmup, iters: run_config(k, M, N, K, warmup=warmup, iters=iters, sets=sets), f"{M}x{N}x{K}")
+    return fastest_in_turn(gemm_bytes(M, N, K, 4), ranked_configs(prof_dict, M, N, K, top) + (ring_ranked(M, N, K) if families else []),
+                           lambda k, warmup, iters, sets: run_config(k, M, N, K, warmup=warmup, iters=iters, sets=sets), f"{M}x{N}x{K}")
 
 
 def select_config(prof_dict, M, N, K):

@@ -335,7 +335,7 @@ def forget_winners(backend):
 
 # A selection times on several sets of operands in turn, as a program's calls come with others' between them: one set that is launched
 # on again lies in L2, which flatters kernels that wait for their loads.  Sets that fill the memory-side cache push each other
-# out by themselves.
+# out by themselves.  Where the sets do not fit the device beside what a program holds there, one does (fastest_in_turn).
 CACHE_BYTES, OPERAND_SETS = 256 << 20, 3
 
 
@@ -357,6 +357,18 @@ def fastest_of(keys, time_config, what):
     same library moves by up to 15 % with where its operands lie (16 x 28672 x 8192 78, 84 and 90 us in three allocations)."""
     with shared_buffers():
         return _fastest_of(keys, time_config, what)
+
+
+def fastest_in_turn(set_bytes, keys, time_config, what):
+    """fastest_of on operand_sets(set_bytes) sets of operands, which time_config takes as its last argument; on one where none of `keys`
+    can run on them."""
+    sets = operand_sets(set_bytes)
+    if sets > 1:
+        try:
+            return fastest_of(keys, lambda k, warmup, iters: time_config(k, warmup, iters, sets), what)
+        except RuntimeError:
+            pass
+    return fastest_of(keys, lambda k, warmup, iters: time_config(k, warmup, iters, 1), what)
 
 
 def _fastest_of(keys, time_config, what):

@@ -16,21 +16,26 @@ PRODUCTS = [((269, 2376, 1376), 3, 3), ((127619, 5, 458), 3, 3), ((8192, 8192, 8
 LAYERS = [((32, 64, 56, 56, 64, 3, 3, 1, 1), 3), ((64, 64, 150, 150, 64, 1, 1, 1, 0), 1)]
 
 
-def libraries(monkeypatch, modules, ring_seconds):
-    """Libraries whose ring tiles take `ring_seconds` and all others 1 s; what they are asked to time."""
+def libraries(monkeypatch, modules, ring_seconds, room=True):
+    """Libraries whose ring tiles take `ring_seconds` and all others 1 s; what they are asked to time.  Without `room` the device holds
+    one set of operands and no more."""
     asked = []
+
+    def answer(sets, rotate_bytes, seconds):
+        asked.append((sets, rotate_bytes))
+        if not room and (sets > 1 or rotate_bytes):
+            raise hip_ctypes.HelixError("helix_bench_sets", 2)          # out of memory
+        return seconds, seconds, seconds
 
     class Library:
         def __init__(self, path):
             self.seconds = ring_seconds if "gemm_ring" in path else 1.0
 
         def bench(self, M, N, K, warmup, iters, outer=1, rotate_bytes=0, sets=1):
-            asked.append((sets, rotate_bytes))
-            return self.seconds, self.seconds, self.seconds
+            return answer(sets, rotate_bytes, self.seconds)
 
         def bench_conv(self, *layer, warmup, iters, sets=1):
-            asked.append((sets, 0))
-            return self.seconds, self.seconds, self.seconds
+            return answer(sets, 0, self.seconds)
 
     for module in modules:
         monkeypatch.setattr(module, "load", Library)
@@ -53,6 +58,20 @@ def test_layers_are_timed_on_sets_in_turn(layer, sets, monkeypatch):
     asked = libraries(monkeypatch, (c16, c32), 0.99)
     assert b16.is_ring_key(c16.verified_config(PROF16, *layer)) and b32.is_ring_key(c32.verified_config(PROF32, *layer))
     assert set(asked) == {(sets, 0)}
+
+
+@pytest.mark.parametrize("problem", [p[0] for p in PRODUCTS])
+def test_products_whose_sets_do_not_fit_are_timed_on_one(problem, monkeypatch):
+    asked = libraries(monkeypatch, (g16, g32), 0.99, room=False)
+    for verified_config, prof, is_ring in ((g16.verified_config, PROF16, b16.is_ring_key), (g32.verified_config, PROF32, b32.is_ring_key)):
+        assert is_ring(verified_config(prof, *problem)) and asked[-1] == (1, 0)
+
+
+@pytest.mark.parametrize("layer", [l[0] for l in LAYERS])
+def test_layers_whose_sets_do_not_fit_are_timed_on_one(layer, monkeypatch):
+    asked = libraries(monkeypatch, (c16, c32), 0.99, room=False)
+    assert b16.is_ring_key(c16.verified_config(PROF16, *layer)) and b32.is_ring_key(c32.verified_config(PROF32, *layer))
+    assert asked[-1] == (1, 0)
 
 
 def test_rows_of_the_reports_are_timed_on_one_set(monkeypatch):
