@@ -5,7 +5,7 @@
 // Error x 1e7 of the fastest configuration of those / one chain / these:
 //   BLOCKS  a chain per 256 of K, in order                     4000 x 2300 x 770 4.8 / 5.0 / 2.9; 422 x 4016 x 4456 8.5 / 12 / 3.0
 //   HALVES  a chain per 16                                     196 x 512 x 256 1.5 / 2.9 / 1.1; 314 x 360 x 776 1.6 / 5.0 / 1.5
-//   FINE    chains of 8, added over 32, those by Kahan's summation    40000 x 7 x 500 0.85 / 4.0 / 0.75
+//   FINE    chains of 8, added over 32, those with what each addition loses added up beside    40000 x 7 x 500 0.85 / 4.0 / 0.75
 //   TILES   a chain per 32, where there are no registers for HALVES
 // HALVES takes 2 - 4 % of the time of a launch that BLOCKS would do (196 x 512 x 256 4.7 / 4.8 us, 369 x 320 x 608 7.8 / 8.1; wave tiles of
 // six and more 5 %), FINE 5 % on the tall products that it is for (14.2 / 15.0).
@@ -97,16 +97,18 @@ struct HalfSums {
 template <int TM, int TN>
 struct FineSums {
     static constexpr int BLOCK_TILES = 0;             // no blocks
-    Tiles<TM, TN> acc, tile, sum, low;               // of a chain that is not a tile's first, of a tile, of the tiles before it; what sum lacks
+    Tiles<TM, TN> acc, tile, sum, low;               // of a chain that is not a tile's first, of a tile, of the tiles before it; what sum lost
     __device__ __forceinline__ void start() {
         clear<TM, TN>(acc);
         clear<TM, TN>(tile);
         clear<TM, TN>(sum);
         clear<TM, TN>(low);
     }
-    __device__ __forceinline__ void add_tile(int i, int j) {     // Kahan's summation
-        const floatx4 y = tile[i][j] - low[i][j], t = sum[i][j] + y;
-        low[i][j] = (t - sum[i][j]) - y;
+    // What an addition loses is added up beside the sum, the Kahan-Babuska way, and not taken off the next tile as Kahan does: there an infinite
+    // sum would be NaN behind the next one (inf - inf), and asking for that each time costs 1 - 8 %
+    __device__ __forceinline__ void add_tile(int i, int j) {
+        const floatx4 t = sum[i][j] + tile[i][j];
+        low[i][j] += tile[i][j] - (t - sum[i][j]);
         sum[i][j] = t;
     }
     // a chain is added when the next one begins, a round of products later
@@ -124,7 +126,12 @@ struct FineSums {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) add_tile(i, j);
+            for (int j = 0; j < TN; j++) {
+                add_tile(i, j);
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (__builtin_fabsf(sum[i][j][e]) < __builtin_inff()) sum[i][j][e] += low[i][j][e];
+            }
     }
 };
 

@@ -86,6 +86,47 @@ def test_few_columns_are_as_exact_as_the_gemv(K):
             assert error(run_sgemm_f32(load(b32.library_for_key(key)), A, B), exact) <= limit * scatter(3000 * 7), key
 
 
+def infinite_sums(A, B):
+    """Products of positive operands whose rows 5, 9, 11 and 13 of the first end in inf, -inf, NaN and beyond the largest float."""
+    K = A.shape[1]
+    for k in (3, K // 2, K - 1):            # first, a middle and the last K tile, chains of different places in it
+        A[5, k], A[9, k] = np.inf, -np.inf
+    A[11, 20], A[11, 40] = np.inf, -np.inf
+    A[13, 8:200:16] = 3e38
+    with np.errstate(all="ignore"):
+        want = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
+    assert np.isinf(want).sum() == 3 * B.shape[1] and np.isnan(want).sum() == B.shape[1]
+    return want
+
+
+@pytest.mark.parametrize("K", [256, 500, 1400])
+@pytest.mark.parametrize("few_rows", [False, True])
+def test_infinite_sums_of_few_rows_or_columns(few_rows, K):
+    """What a compensated sum lacks has no value once the sum is infinite: it stays so, and is NaN only where products of both signs are."""
+    rng = np.random.default_rng(K)
+    A, B = rng.integers(1, 9, (300, K)).astype(np.float32), rng.integers(1, 9, (K, 7)).astype(np.float32)
+    want = infinite_sums(A, B)
+    for key in b32.RING_KEYS:
+        lib = load(b32.library_for_key(key))
+        got = run_sgemm_f32(lib, B.T, A.T).T if few_rows else run_sgemm_f32(lib, A, B)
+        assert np.array_equal(got, want, equal_nan=True), key
+
+
+@pytest.mark.parametrize("IC", [32, 36, 29])
+def test_infinite_sums_of_few_channels(IC):
+    """The same in convolutions, the ring tiles' (IC a multiple of 4) and those whose input stays in LDS; the finite results are exact."""
+    rng = np.random.default_rng(IC)
+    x, w = rng.integers(0, 3, (2, 10, 11, IC)).astype(np.float32), rng.integers(1, 4, (13, 3, 3, IC)).astype(np.float32)
+    want = O.conv2d_nhwc(x, w, 1, 1)
+    x[0, 3, 4, IC - 1], want[0, 2:5, 3:6] = np.inf, np.inf
+    x[1, 9, 10, 0], want[1, 8:, 9:] = -np.inf, -np.inf
+    x[1, 0, 0, 7], want[1, :2, :2] = np.nan, np.nan
+    for key in (b32.RING_KEYS if IC % 4 == 0 else ()) + b32.patch_keys():
+        if b32.is_patch_key(key) and c32.PATCH.layout((key[0], key[1], key[3], key[4], key[6]), 2, IC, 10, 11, 13, 3, 3, 1, 1) is None:
+            continue
+        assert np.array_equal(run_conv(load(b32.library_for_key(key)), x, w, 1, 1, torch.float32), want, equal_nan=True), key
+
+
 def test_many_tiles_integer_exact():
     """More workgroups than the chip holds at once, many K tiles; the whole result against the product in 64 bits on the device."""
     M, N, K = 3000, 3080, 500
