@@ -334,14 +334,17 @@ def forget_winners(backend):
 
 
 # A selection times on several sets of operands in turn, as a program's calls come with others' between them: one set that is launched
-# on again lies in L2, which flatters kernels that wait for their loads.  Sets that fill the memory-side cache push each other
-# out by themselves.  Where the sets do not fit the device beside what a program holds there, one does (fastest_in_turn).
-CACHE_BYTES, OPERAND_SETS = 256 << 20, 3
+# on again lies in L2, which flatters kernels that wait for their loads.  Sets beyond the memory-side cache push each other out by
+# themselves, but where one lies moves the time of some kernels and not of others (16 x 28672 x 8192, operands in five places: the GEMV
+# that partitions K 79 and 90 us, the one that does not 79 - 81): on one set the first was picked in 8 of 24 selections, on three in 1 of 32.
+# Beyond LARGE_SET_BYTES, where launches are long and walk many places, one set does, as where three do not fit the device
+# beside what a program holds there (fastest_in_turn).
+CACHE_BYTES, LARGE_SET_BYTES, OPERAND_SETS = 256 << 20, 1 << 30, 3
 
 
 def operand_sets(set_bytes):
     """Sets of operands and results that a selection's launches take in turn."""
-    return OPERAND_SETS if set_bytes < CACHE_BYTES else 1
+    return OPERAND_SETS if set_bytes < LARGE_SET_BYTES else 1
 
 
 SETTLE_FINALISTS = 4        # candidates timed a second time ...

@@ -11,9 +11,10 @@ from MI355X_FP32 import MI355X_FP32_gemm as g32
 
 PROF16 = {(2, 64, 64, 32, 32, 0, 64): 1e-5, (2, 128, 64, 64, 32, 0, 64): 2e-5}
 PROF32 = {b32.config_key(64, 64, 16, 32, 32): 1.0, b32.config_key(128, 64, 16, 32, 32): 1.7}
-# m, n, k: sets in turn; the memory-side cache is full of one; FP16 weights that are copied instead
-PRODUCTS = [((269, 2376, 1376), 3, 3), ((127619, 5, 458), 3, 3), ((8192, 8192, 8192), 1, 1), ((661, 11008, 4096), 1, 3)]
-LAYERS = [((32, 64, 56, 56, 64, 3, 3, 1, 1), 3), ((64, 64, 150, 150, 64, 1, 1, 1, 0), 1)]
+# m, n, k: sets in turn, also where the memory-side cache is full of one; beyond a GiB; FP16 weights that are copied instead
+PRODUCTS = [((269, 2376, 1376), 3, 3), ((127619, 5, 458), 3, 3), ((8192, 8192, 8192), 1, 3), ((40, 28672, 8192), 3, 3),
+            ((32768, 32768, 8192), 1, 1), ((661, 11008, 4096), 1, 3)]
+LAYERS = [((32, 64, 56, 56, 64, 3, 3, 1, 1), 3), ((64, 64, 150, 150, 64, 1, 1, 1, 0), 3), ((256, 64, 150, 150, 64, 1, 1, 1, 0), 1)]
 
 
 def libraries(monkeypatch, modules, ring_seconds, room=True):
@@ -98,6 +99,6 @@ def test_candidates_of_a_selection_share_their_buffers():
     assert hip_ctypes._buffers.get() is None and seen[-1] is not seen[0] and seen[-1] is not None
 
 
-def test_sets_end_where_they_fill_the_cache():
+def test_sets_end_at_a_gib():
     assert helix_runtime.operand_sets(1) == helix_runtime.OPERAND_SETS == 3
-    assert helix_runtime.operand_sets(helix_runtime.CACHE_BYTES - 1) == 3 and helix_runtime.operand_sets(helix_runtime.CACHE_BYTES) == 1
+    assert helix_runtime.operand_sets((1 << 30) - 1) == 3 and helix_runtime.operand_sets(1 << 30) == 1
