@@ -99,6 +99,18 @@ def test_candidates_of_a_selection_share_their_buffers():
     assert hip_ctypes._buffers.get() is None and seen[-1] is not seen[0] and seen[-1] is not None
 
 
+def test_leaders_are_timed_until_the_device_has_come_to_rest():
+    """Two rounds, and more while the fastest of a round is ahead of all before it; six at most."""
+    def picks(times):
+        left = {k: list(t) for k, t in times.items()}
+        pick = helix_runtime.fastest_of(list(times), lambda k, warmup, iters: 1.0 if iters == 5 else left[k].pop(0), "p")
+        return pick, {len(times[k]) - len(left[k]) for k in times}
+
+    assert picks({"a": [1.2, 1.1, 1.0, 1.0, 0.1], "b": [1.3, 1.12, 0.97, 0.965, 2.0]}) == ("b", {4})
+    assert picks({"a": [1.0, 0.995, 0.1], "b": [1.01, 1.0, 0.1]}) == ("a", {2})
+    assert picks({"a": [2.0 ** -i for i in range(9)], "b": [1.1 * 2.0 ** -i for i in range(9)]}) == ("a", {6})
+
+
 def test_sets_end_at_a_gib():
     assert helix_runtime.operand_sets(1) == helix_runtime.OPERAND_SETS == 3
     assert helix_runtime.operand_sets((1 << 30) - 1) == 3 and helix_runtime.operand_sets(1 << 30) == 1
