@@ -260,7 +260,7 @@ def get_MI355X_FP16_conv_Helix_result(prof_dict, batch, input_channel, H, W, out
 
 
 def get_MI355X_FP16_conv_Oracle_result(prof_dict, batch, input_channel, H, W, output_channel, kH, kW, stride, pad):
-    """Exhaustive per-layer search: run every configuration that has a conv entry, keep the fastest (the conv
+    """Exhaustive per-layer search: run every profiled configuration that has a conv entry, keep the fastest (the conv
     counterpart of benchmark_Ampere_FP16_performance_comparison.py:56-69).  Returns (cost_ms, tflops, key)."""
     M = batch * ((H + 2 * pad - kH) // stride + 1) * ((W + 2 * pad - kW) // stride + 1)
     flops = 2.0 * M * output_channel * input_channel * kH * kW

@@ -289,7 +289,7 @@ def get_MI355X_FP16_gemm_Verified_result(prof_dict, M, N, K, top=VERIFY_TOP):
 
 
 def get_MI355X_FP16_gemm_Oracle_result(prof_dict, M, N, K):
-    """Exhaustive per-shape search: run every candidate, keep the fastest
+    """Exhaustive per-shape search: run every profiled configuration, keep the fastest
     (benchmark_Ampere_FP16_performance_comparison.py:56-69).  Returns (cost_ms, tflops, key)."""
     min_cost, best = float("inf"), None
     for k in prof_dict.keys():

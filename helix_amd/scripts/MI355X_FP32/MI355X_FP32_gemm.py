@@ -297,7 +297,7 @@ def get_MI355X_FP32_gemm_Verified_result(prof_dict, M, N, K, top=VERIFY_TOP):
 
 
 def get_MI355X_FP32_gemm_Oracle_result(prof_dict, M, N, K):
-    """Exhaustive per-shape search.  Returns (cost_ms, tflops, key)."""
+    """Exhaustive per-shape search over the profiled configurations.  Returns (cost_ms, tflops, key)."""
     min_cost, best = float("inf"), None
     for k in prof_dict.keys():
         if k[2] == 0 and min(M, N) > 16:

@@ -23,9 +23,11 @@
 // Measured, us per launch (helix_bench_conv), the general path's fastest configuration against this one: batch 32, 224 x 224
 // x 3 -> 64: 7x7 stride 2 58 / 22, 3x3 88 / 36 (5.9 TB/s), 11x11 stride 4 -> 96 49 / 28; batch 20, 180 x 180 x 3, 5x5 51 / 21;
 // batch 1, 7x7 10.2 / 6.4, 3x3 10.4 / 6.5; 4 x 161 x 700 x 1 -> 32, 5x20 stride 2 33 / 14.  The weights' fragments are packed from
-// four dwords each with all of a thread's loads in flight (half by half out of LDS before: 7x7 at batch 32 21.7 / 21.2 us per call).
-// What is left of the 7x7 layer: 2.5 us of launch, about 5 us until weights and patch are in place (all workgroups start together,
-// so nothing overlaps it), then the output at 5.7 TB/s.
+// four dwords each with all of a thread's loads in flight; half by half out of LDS before, on the same memory in turn, one set of
+// operands and three: 7x7 at batch 32 21.2 / 21.0 and 21.2 / 20.8 (single rounds 20.4 - 23), at batch 1 6.7 / 6.45, 11x11 31.5 / 30.8 and
+// 32.5 / 31.6, at batch 1 11.0 / 10.0; 3x3 36.1 / 36.1 and 46.2 / 46.7.  Two cards put the 7x7 layer at 19.7 and 21.5.
+// What is left of it: 2.5 us of launch, about 5 us until weights and patch are in place (all workgroups start together, so nothing
+// overlaps it), then 51 MB of results at some 3.7 TB/s, where 5.7 would take 9 us; what holds these up has not been found.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -166,8 +168,8 @@ __global__ __launch_bounds__(threads_of(KS), resident_of(KS, NT) * threads_of(KS
             put(0, v.a[0], v.a[1]);
         }
     };
-    // ---- weights: as they lie; with more than four steps of them the loads of a thread are all in flight at once (7x7 21.8 ->
-    // 21.1 us, batch 1 6.7 -> 6.4, 11x11 12.7 -> 12.6; of fewer there is one or two, and the plain loop is the shorter one) -----
+    // ---- weights: as they lie; with more than four steps of them the loads of a thread are all in flight at once (7x7 at
+    // batch 32 21.3 -> 20.8 us, at 1 6.66 -> 6.47, 11x11 level; of fewer there is one or two, and the plain loop is the shorter one) -----
     const int taps = p.kH * p.kW, filter = taps * p.IC, halves = ocs * filter;
     const _Float16* src = p.w + (size_t)oc0 * filter;         // a multiple of 32 filters in: 16-byte aligned
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(src), 0, halves * 2, 0x00020000);
@@ -447,7 +449,8 @@ inline bool make_plan(Plan& plan, int batch, int H, int W, int IC, int OC, int k
     // 96 channels per workgroup where one then holds all of a pixel and there are many: written by two, its 64 and 32 channels
     // are not whole 128-byte lines, and the input is staged twice.  us per launch at 64 / 96, three channels -> 96: 4 x 224 x 224
     // 3x3 16.2 / 11.2, 32 x 224 x 224 5x5 stride 2 25.7 / 21.2; 77k pixels 8.4 / 8.3, 900 - 23k pixels 5.0 / 5.8, 5.8 / 6.3; with
-    // seven steps (one workgroup per CU, for the registers) 28.5 / 28.2 at 307k pixels, 9.9 / 10.7 at 30k
+    // seven steps (one workgroup per CU, for the registers) 28.5 / 28.2 at 307k pixels, 9.9 / 10.7 at 30k.  One, two and four channels
+    // have not been measured at 96 and stay at 64
     const int nt = IC == 3 && ks > 0 && ks <= 4 && OC > 64 && OC <= 96 && (long long)batch * OH * OW >= (1 << 17) ? 6 : 4;
     const int nt_blocks = (OC + 16 * nt - 1) / (16 * nt);
     const size_t raw = align16((size_t)16 * nt * kH * kW * IC * 2), packed = (size_t)steps * step_bytes(nt);

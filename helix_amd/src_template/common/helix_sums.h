@@ -1,11 +1,12 @@
 // The FP32 sums of one wave's tiles of v_mfma_f32_16x16x4_f32 products (MI355X_FP32/gemm_ring.hip, common/helix_conv_patch.h).
 //
 // A sum of K products leaves an error that grows with the root of the products in a chain and of the partial sums that are added in
-// turn: about 0.18e-7 x sqrt(chain + partial sums) in the norm, against 64 bits, operands ~ N(0, 1).  The K groups and K partitions of sgemm.hip and the lanes of the GEMV keep both short on small problems; what takes their place has to, too.
+// turn: about 0.18e-7 x sqrt(chain + partial sums) in the norm, against 64 bits, operands ~ N(0, 1).  The K groups and K partitions of
+// sgemm.hip and the lanes of the GEMV keep both short on small problems; what takes their place has to, too.
 // Error x 1e7 of the fastest configuration of those / one chain / these:
 //   BLOCKS  a chain per 256 of K, in order                     4000 x 2300 x 770 4.8 / 5.0 / 2.9; 422 x 4016 x 4456 8.5 / 12 / 3.0
 //   HALVES  a chain per 16                                     196 x 512 x 256 1.5 / 2.9 / 1.1; 314 x 360 x 776 1.6 / 5.0 / 1.5
-//   FINE    chains of 8, added over 32, those with what each addition loses added up beside    40000 x 7 x 500 0.85 / 4.0 / 0.75
+//   FINE    chains of 8, added over 32, those with what each addition loses added up beside    40000 x 7 x 500 0.85 / 4.0 / 0.73
 //   TILES   a chain per 32, where there are no registers for HALVES
 // HALVES takes 2 - 4 % of the time of a launch that BLOCKS would do (196 x 512 x 256 4.7 / 4.8 us, 369 x 320 x 608 7.8 / 8.1; wave tiles of
 // six and more 5 %), FINE 5 % on the tall products that it is for (14.2 / 15.0).
